@@ -32,7 +32,7 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0
 
 
 TRAFFIC_PROFILE = os.path.join('profiles', 'bench_cfg2_hbm_traffic_pmc.txt')
-KERNEL_SOURCES = ('kernels_mfma.hip', 'tk_mfma.h', 'tk_common.h')     # what the expand kernel is compiled from
+KERNEL_SOURCES = ('kernels_mfma.hip', 'lora_kernels.h', 'tk_mfma.h', 'tk_common.h')     # what the expand kernel is compiled from
 
 
 def kernel_source_digest():

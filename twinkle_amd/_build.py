@@ -3,6 +3,8 @@ from __future__ import annotations
 
 import os
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'csrc')
 INCLUDE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), 'include')
@@ -11,20 +13,30 @@ SOURCES = ['api.hip', 'kernels_segments.hip', 'kernels_generic.hip', 'kernels_mf
 
 # -packed-fp32-ops is switched off on purpose: the compiler must not form packed fp32 VALU ops.
 HIPCC_FLAGS = [
-    '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared', '-Xclang', '-target-feature', '-Xclang',
+    '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-Xclang', '-target-feature', '-Xclang',
     '-packed-fp32-ops', '-Wno-unused-command-line-argument',
 ]
 
 
 def build_library(verbose: bool = False) -> str:
-    """Compile every HIP source into ``csrc/libtwinkle_amd.so`` and return its path."""
+    """Compile every HIP source (side by side) and link ``csrc/libtwinkle_amd.so``; returns its path."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
-    cmd = [hipcc, *HIPCC_FLAGS, '-I', INCLUDE, '-I', CSRC, *[os.path.join(CSRC, s) for s in SOURCES], '-o', LIB_PATH]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError('hipcc failed:\n' + ' '.join(cmd) + '\n' + proc.stdout + proc.stderr)
+
+    def run(cmd) -> str:
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError('hipcc failed:\n' + ' '.join(cmd) + '\n' + proc.stdout + proc.stderr)
+        return proc.stderr
+
+    with tempfile.TemporaryDirectory() as tmp:
+        objects = [os.path.join(tmp, s.replace('.hip', '.o')) for s in SOURCES]
+        compiles = [[hipcc, *HIPCC_FLAGS, '-I', INCLUDE, '-I', CSRC, '-c', os.path.join(CSRC, s), '-o', o]
+                    for s, o in zip(SOURCES, objects)]
+        with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+            notes = list(pool.map(run, compiles))
+        notes.append(run([hipcc, '--offload-arch=gfx950', '-shared', *objects, '-o', LIB_PATH]))
     if verbose:
-        print(proc.stderr)
+        print('\n'.join(n for n in notes if n))
     return LIB_PATH
 
 
