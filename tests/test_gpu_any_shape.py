@@ -1,0 +1,84 @@
+"""The kernels for fp32 and for odd shapes (kernels_generic.hip) at the edges of their tiles, against the CPU oracle.
+
+Bars as in test_gpu_lora.py: fp32 1e-5, bf16 2e-2 of the largest value.  fp32: products are exact and sums of at most
+1100 terms carry at most 1100 * 2^-24 = 7e-5 of the sum of magnitudes in the worst case, about sqrt(1100) * 2^-24 = 2e-6
+in the usual one.
+"""
+import pytest
+import torch
+
+import oracle
+from conftest import max_rel_err
+from twinkle_amd import AdapterGroups, build_segments, lora_bwd_, lora_fwd_
+from test_gpu_lora import TOL, _problem
+
+pytestmark = pytest.mark.gpu
+
+
+def _strided(t, dtype, dev, pad):
+    """`t` as a view one element into rows that are `pad` elements longer: rows start at any element address."""
+    wide = torch.zeros(t.shape[0], t.shape[1] + pad, dtype=dtype, device=dev)
+    view = wide[:, 1:1 + t.shape[1]] if pad else wide
+    view.copy_(t.to(dtype))
+    return view
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('t,k,m,ranks,pad', [
+    (5, 1, 1, [1, 1], 0),                            # a width inside one piece
+    (64, 31, 33, [3, 5, 1], 0),                      # one element short of a step, one past it
+    (130, 63, 127, [16, 7], 3),                      # the largest cut piece; rows at odd addresses
+    (200, 65, 129, [17, 32], 2),
+    (300, 257, 255, [33, 64, 2], 5),                 # four waves of steps and one element
+    (300, 512, 256, [40, 64], 1),                    # whole widths at odd row starts
+    (450, 513, 640, [128, 65, 100], 3),              # several slices of the source, the largest rank
+    (1100, 1100, 72, [20, 128, 1, 0, 64], 0),        # ranks of every class in one call, one adapter not live
+    (4700, 72, 1031, [24, 8], 0),                    # groups of several chunks
+])
+def test_edges(dev, dtype, t, k, m, ranks, pad):
+    max_r = max(ranks)
+    x, base, dy, a, b, ids, _, scales = _problem(t, k, m, len(ranks), max_r, ranks, seed=t + k)
+    ids[ids == 1] = 0 if t < 100 else 1              # the smallest ones leave an adapter without rows
+    xd, dyd = _strided(x, dtype, dev, pad), _strided(dy, dtype, dev, pad)
+    yd, dxd = _strided(base, dtype, dev, pad), _strided(torch.zeros(t, k), dtype, dev, pad)
+    ad, bd = [w.to(dtype).to(dev) for w in a], [w.to(dtype).to(dev) for w in b]
+    seg = build_segments(ids.to(torch.int32).to(dev), len(ranks), check=True)
+    groups = AdapterGroups(ad, bd, ranks, scales)
+    h = lora_fwd_(xd, yd, seg, groups)
+    ga, gb = [torch.zeros_like(w) for w in ad], [torch.zeros_like(w) for w in bd]
+    pa, pb = (torch.tensor([w.data_ptr() for w in g], dtype=torch.int64, device=dev) for g in (ga, gb))
+    lora_bwd_(dyd, xd, h, dxd, pa, pb, seg, groups)
+    f64 = lambda v: v.to(dtype).double()  # noqa: E731
+    yo, dxo, dao, dbo = oracle.multi_lora_linear_grads(f64(x), f64(base), ids, [f64(w) for w in a], [f64(w) for w in b],
+                                                        ranks, scales, f64(dy))
+    tol = TOL[dtype]
+    assert max_rel_err(yd, yo) < tol and max_rel_err(dxd, dxo) < tol
+    for g, r in enumerate(ranks):
+        if r:
+            assert max_rel_err(ga[g], dao[g]) < tol, f'dA[{g}]'
+            assert max_rel_err(gb[g], dbo[g]) < tol, f'dB[{g}]'
+    for view in (yd, dxd):                            # what lies around the rows is untouched
+        if pad:
+            wide = view._base
+            assert torch.count_nonzero(wide[:, 0]) == 0 and torch.count_nonzero(wide[:, 1 + view.shape[1]:]) == 0
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_an_infinite_row_stays_with_its_adapter(dev, dtype):
+    """Row 0 is what the kernels read in place of a padding slot: an infinity in it reaches its own adapter only."""
+    x, base, dy, a, b, _, ranks, scales = _problem(100, 40, 24, 3, 8, [8, 3, 5], seed=3)
+    ids = torch.arange(100) % 3
+    x[0, 5] = float('inf')
+    dy[0, 7] = float('inf')
+    ad, bd = [w.to(dtype).to(dev) for w in a], [w.to(dtype).to(dev) for w in b]
+    seg = build_segments(ids.to(torch.int32).to(dev), 3)
+    groups = AdapterGroups(ad, bd, ranks, scales)
+    xd, yd, dyd = (v.to(dtype).to(dev) for v in (x, base, dy))
+    dxd = torch.zeros_like(xd)
+    h = lora_fwd_(xd, yd, seg, groups)
+    ga, gb = [torch.zeros_like(w) for w in ad], [torch.zeros_like(w) for w in bd]
+    pa, pb = (torch.tensor([w.data_ptr() for w in g], dtype=torch.int64, device=dev) for g in (ga, gb))
+    lora_bwd_(dyd, xd, h, dxd, pa, pb, seg, groups)
+    assert torch.isfinite(yd[1:]).all() and torch.isfinite(dxd[1:]).all()
+    for g in (1, 2):
+        assert torch.isfinite(ga[g]).all() and torch.isfinite(gb[g]).all()

@@ -1,121 +1,333 @@
-// Shape-agnostic kernels for the segmented LoRA pass: fp32 or bf16 storage,
-// fp32 accumulation on the vector ALUs, any width / stride / rank <= 128.
-// They carry the fp32 configuration and every shape the MFMA kernels do not
-// take (odd widths, unaligned strides), and share all buffers and tables with
-// them, so the two families are interchangeable per launch.
+// Kernels of the segmented LoRA pass for fp32 and for every shape the kernels of lora_kernels.h do not take (odd
+// widths, strides that are no multiple of 16 bytes): any width / stride / rank <= 128, on the matrix cores, fp32
+// accumulation.  They share all buffers and tables with those kernels, so the two families are interchangeable per
+// launch.
+//
+// One body serves both types because it counts in pieces of 16 bytes, E = 8 bf16 or 4 fp32 elements.  A piece per lane
+// is one operand of v_mfma_f32_16x16x32_bf16, or of four v_mfma_f32_16x16x4_f32 (exact fp32 products and sums, the
+// operand components taken one after the other); either way 16 lanes are 16 rows or columns and the four lane groups
+// kb = lane / 16 are consecutive pieces of the contraction index, 4 E in all.  Pieces are loaded from any element
+// address (global loads need no 16-byte alignment on this part); where the width ends inside a piece its elements are
+// loaded one by one, so nothing past a row's end is touched.
 #include <algorithm>
+#include <type_traits>
 
-#include "tk_device.h"
+#include "tk_mfma.h"
 
 namespace tk {
 
 namespace {
 
-constexpr int kKC = 64;   // source columns staged per step in the shrink kernel
-
-// hT[n][slot] = scale_g * sum_k src[row(slot)][k] * W_g[n][k]   for the 32 slots of one tile
 template <typename T>
-__global__ __launch_bounds__(256) void k_shrink_generic(PassArgs a, const int32_t* __restrict__ tile_group,
-                                                        const int32_t* __restrict__ slot_rows) {
-  extern __shared__ float lds_f[];
-  const int tile_id = blockIdx.x;
-  const int g = checked_group(tile_group[tile_id], a.tb);
-  if (g < 0) return;
-  const int r = class_rank(a.rank[g], a.rank_lo, a.rpad);
-  if (a.class_mode && r <= 0) return;  // a group of another rank class: its tiles belong to another launch
-  const int rpad = a.rpad;
-  float* xs = lds_f;                          // [32][kKC + 1]
-  float* ws = lds_f + kTileRows * (kKC + 1);  // [rpad][kKC + 1]
-  __shared__ int rows_s[kTileRows];
-  const int tid = threadIdx.x;
-  const int slot0 = tile_id * kTileRows;
-  if (tid < kTileRows) rows_s[tid] = checked_row(slot_rows[slot0 + tid], a.tb);
-  __syncthreads();
-  const T* src = (const T*)a.src;
-  const T* W = group_weight<T>(a.w_shrink, a.w_shrink_base, a.shrink_group_stride, g);
-  const int row = tid & 31;   // tile row this thread accumulates
-  const int ng = tid >> 5;    // rank indices ng, ng + 8, ...
-  float acc[TK_MAX_RANK / 8];
+struct Piece {
+  static constexpr int E = 16 / (int)sizeof(T);  // elements of a piece
+};
+
+// E consecutive elements from an address that is a multiple of the element size only
+typedef u32x4_t u32x4_any __attribute__((aligned(2)));
+template <typename T>
+__device__ inline uint4 ld_piece(const T* p) {
+  // (weights are reached through pointers read from memory: said to be global, or the loads would be flat)
+  const u32x4_t v = *(const __attribute__((address_space(1))) u32x4_any*)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+// the same for data that is touched once per pass (see ld16_nt)
+template <typename T>
+__device__ inline uint4 ld_piece_nt(const T* p) {
+  const u32x4_t v = __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x4_any*)p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <typename T>
+__device__ inline void st_piece_nt(T* p, uint4 v) {
+  const u32x4_t w = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(w, (__attribute__((address_space(1))) u32x4_any*)p);
+}
+// the first `keep` of them (zeros behind); nothing past them is read
+template <typename T>
+__device__ inline uint4 ld_piece(const T* p, int keep) {
+  constexpr int E = Piece<T>::E;
+  if (keep >= E) return ld_piece(p);
+  uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int j = 0; j < TK_MAX_RANK / 8; ++j) acc[j] = 0.f;
-  const int nacc = (rpad + 7) / 8;
-  for (int k0 = 0; k0 < a.width_src; k0 += kKC) {
-    for (int i = tid; i < kTileRows * kKC; i += 256) {
-      const int rr = i / kKC, kk = i % kKC;
-      const int k = k0 + kk;
-      xs[rr * (kKC + 1) + kk] =
-          (k < a.width_src && rows_s[rr] >= 0) ? to_f32(src[(int64_t)rows_s[rr] * a.ld_src + k]) : 0.f;
+  for (int i = 0; i < E; ++i)
+    if (i < keep) {
+      if constexpr (sizeof(T) == 4) w[i] = __builtin_bit_cast(uint32_t, p[i]);
+      else w[i >> 1] |= (uint32_t)p[i] << (16 * (i & 1));
     }
-    for (int i = tid; i < rpad * kKC; i += 256) {
-      const int n = i / kKC, kk = i % kKC;
-      const int k = k0 + kk;
-      ws[n * (kKC + 1) + kk] = (n < r && k < a.width_src) ? to_f32(W[(int64_t)n * a.ld_shrink + k]) : 0.f;
-    }
-    __syncthreads();
-    for (int kk = 0; kk < kKC; ++kk) {
-      const float xv = xs[row * (kKC + 1) + kk];
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ inline float part_f32(const uint4& v, int i) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  return __uint_as_float(w[i]);
+}
+
+// acc += A B over the 4 E contraction indices of one piece per lane
+template <typename T>
+__device__ inline f32x4 mma_piece(const uint4& a, const uint4& b, f32x4 acc) {
+  if constexpr (sizeof(T) == 4) {
 #pragma unroll
-      for (int j = 0; j < TK_MAX_RANK / 8; ++j)
-        if (j < nacc) acc[j] += xv * ws[(ng + 8 * j) * (kKC + 1) + kk];
-    }
-    __syncthreads();
+    for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(part_f32(a, i), part_f32(b, i), acc, 0, 0, 0);
+    return acc;
+  } else {
+    return mfma16(a, b, acc);
   }
-  const float sc = r > 0 ? a.scale[g] : 0.f;
+}
+
+// h of one tile from its sums (element (row, n) from `sum`): slot-major and rank-major copies; exact zeros in padding
+// slots and at rank indices past the group's rank, so that the row contractions and the expand need no masks there
+template <typename T, typename Sum>
+__device__ inline void write_h(const PassArgs& a, int slot0, int cnt, int r, float sc, int n0, int nn, const Sum& sum) {
   T* hT = (T*)a.hT;
-  T* hrow = hT + (int64_t)rpad * a.ldh;
-  // padding slots hold exact zeros so that the row-contraction kernels need no masks
+  T* hrow = hT + (int64_t)a.rpad * a.ldh;
+  for (int idx = threadIdx.x; idx < kTileRows * nn; idx += 256) {
+    const int row = idx / nn, n = idx % nn;
+    T v;
+    from_f32(row < cnt && n0 + n < r ? sum(row, n) * sc : 0.f, &v);
+    hrow[(int64_t)(slot0 + row) * a.rpad + n0 + n] = v;
+  }
+  for (int idx = threadIdx.x; idx < kTileRows * nn; idx += 256) {
+    const int row = idx & 31, n = idx >> 5;
+    T v;
+    from_f32(row < cnt && n0 + n < r ? sum(row, n) * sc : 0.f, &v);
+    hT[(int64_t)(n0 + n) * a.ldh + slot0 + row] = v;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Shrink: h[slot][n] = scale_g * sum_k src[row(slot)][k] * W_g[n][k].  A block of four waves owns (tile of 32 slots,
+// slice of the source columns); its waves take steps of 8 E columns (128 bytes of every row) in turn, so a slice is a
+// few memory latencies long, and their sums meet in LDS.  (The form on the vector ALUs before it walked all columns in
+// one block, 64 at a time behind two barriers each: 4096 rows x 4096 columns of fp32 at rank 16 took 1010 us against
+// 20 + 4 for the slice sums, 3.4 TB/s; 3001 x 1000 bf16 at rank 24 390 against 13.)  With several slices (the plan of the split shrink, whose
+// buffer lies behind h) the block leaves its sums for k_shrink_any_finish.
+// ---------------------------------------------------------------------------
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_shrink_any(PassArgs a, int slice_cols, const int32_t* __restrict__ tile_group,
+                                                    const int32_t* __restrict__ slot_rows) {
+  constexpr int E = Piece<T>::E, RP = 16 * NB;
+  constexpr int NBS = NB < 4 ? NB : 4;  // rank blocks that leave through LDS together
+  constexpr int PF = NB == 1 ? 4 : (NB == 2 ? 2 : 1);
+  __shared__ float part[4][kTileRows][16 * NBS + 1];
+  const int nth = blockIdx.x / a.kslices, ks = blockIdx.x - nth * a.kslices;
+  const int tile_id = checked_tile(work_item(a.wl_tiles, nth), a.tb);
+  if (tile_id < 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
+  const int slot0 = tile_id * kTileRows;
+  const int g = checked_group(tile_group[tile_id], a.tb);
+  int ra = checked_row(slot_rows[slot0 + li], a.tb), rb = checked_row(slot_rows[slot0 + 16 + li], a.tb);
+  if (g < 0) return;
+  const int r = class_rank(a.rank[g], a.rank_lo, RP);
+  if (r <= 0) return;  // (uniform over the block, like the returns above)
+  const int cnt = __popcll(__ballot(ra >= 0) & 0xffffull) + __popcll(__ballot(rb >= 0) & 0xffffull);
+  const T* src = (const T*)a.src;
+  const T* xr[2] = {src + (int64_t)max(ra, 0) * a.ld_src, src + (int64_t)max(rb, 0) * a.ld_src};
+  const T* W = group_weight<T>(a.w_shrink, a.w_shrink_base, a.shrink_group_stride, g);
+  const T* wr[NB];
 #pragma unroll
-  for (int j = 0; j < TK_MAX_RANK / 8; ++j) {
-    const int n = ng + 8 * j;
-    if (n < rpad) {
-      T hv;
-      from_f32((n < r && rows_s[row] >= 0) ? acc[j] * sc : 0.f, &hv);
-      hT[(int64_t)n * a.ldh + slot0 + row] = hv;
-      hrow[(int64_t)(slot0 + row) * rpad + n] = hv;
+  for (int nb = 0; nb < NB; ++nb) wr[nb] = W + (int64_t)min(16 * nb + li, r - 1) * a.ld_shrink;  // (masked below)
+  f32x4 acc[2][NB];
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int k0 = ks * slice_cols, k1 = min(a.width_src, k0 + slice_cols);
+  constexpr int STEP = 8 * E;
+  int c = k0 + wave * STEP;
+  // whole steps: loads of PF steps side by side, no guards
+  for (; c + (PF - 1) * 4 * STEP + STEP <= k1; c += PF * 4 * STEP) {
+    uint4 x[PF][2][2], w[PF][NB][2];
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      const int cc = c + 4 * j * STEP + 2 * E * kb;
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) x[j][tt][p] = ld_piece(xr[tt] + cc + p * E);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) w[j][nb][p] = ld_piece(wr[nb] + cc + p * E);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (left alone the compiler pairs each load with its use, one latency each)
+#pragma unroll
+    for (int j = 0; j < PF; ++j)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) acc[tt][nb] = mma_piece<T>(x[j][tt][p], w[j][nb][p], acc[tt][nb]);
+  }
+  for (; c < k1; c += 4 * STEP) {  // the steps left, the last of them perhaps cut by the width
+    const int cc = c + 2 * E * kb;
+    uint4 x[2][2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) x[tt][p] = ld_piece(xr[tt] + cc + p * E, k1 - cc - p * E);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const uint4 w = ld_piece(wr[nb] + cc + p * E, k1 - cc - p * E);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mma_piece<T>(x[tt][p], w, acc[tt][nb]);
+      }
+  }
+  const float sc = a.scale[g];
+#pragma unroll
+  for (int b = 0; b < NB; b += NBS) {
+    if (b) __syncthreads();
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int nb = 0; nb < NBS; ++nb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[wave][16 * tt + 4 * kb + v][16 * nb + li] = acc[tt][b + nb][v];
+    __syncthreads();
+    auto sum = [&](int row, int n) { return ((part[0][row][n] + part[1][row][n]) + part[2][row][n]) + part[3][row][n]; };
+    if (a.kslices > 1) {
+      float* mine = a.hpart + ((int64_t)tile_id * a.kslices + ks) * (kTileRows * RP) + 16 * b;
+      for (int idx = tid; idx < kTileRows * 16 * NBS; idx += 256) {
+        const int row = idx / (16 * NBS), n = idx % (16 * NBS);
+        mine[row * RP + n] = sum(row, n);
+      }
+    } else {
+      write_h<T>(a, slot0, cnt, r, sc, 16 * b, 16 * NBS, sum);
     }
   }
 }
 
-// dst[row(slot)][c] += sum_n hT[n][slot] * W_g[c][n]   for the 32 slots of one tile
+// Adds the slices in slice order and writes h: a block per (tile, 16 rank indices).
 template <typename T>
-__global__ __launch_bounds__(256) void k_expand_generic(PassArgs a, const int32_t* __restrict__ tile_group,
-                                                        const int32_t* __restrict__ slot_rows) {
-  extern __shared__ float lds_f[];  // hs[rpad][32]
-  const int tile_id = blockIdx.x;
+__global__ __launch_bounds__(256) void k_shrink_any_finish(PassArgs a, const int32_t* __restrict__ tile_group,
+                                                           const int32_t* __restrict__ slot_rows) {
+  __shared__ float part[kTileRows][17];
+  const int tile_id = checked_tile(work_item(a.wl_tiles, blockIdx.x), a.tb);
+  if (tile_id < 0) return;
+  const int tid = threadIdx.x, slot0 = tile_id * kTileRows, n0 = 16 * blockIdx.y;
   const int g = checked_group(tile_group[tile_id], a.tb);
+  const int my_row = checked_row(slot_rows[slot0 + (tid & 31)], a.tb);
   if (g < 0) return;
   const int r = class_rank(a.rank[g], a.rank_lo, a.rpad);
   if (r <= 0) return;
-  __shared__ int rows_s[kTileRows];
-  const int tid = threadIdx.x;
-  const int slot0 = tile_id * kTileRows;
-  if (tid < kTileRows) rows_s[tid] = checked_row(slot_rows[slot0 + tid], a.tb);
-  const T* hT = (const T*)a.hT;
-  for (int i = tid; i < r * kTileRows; i += 256) {
-    const int n = i / kTileRows, rr = i % kTileRows;
-    lds_f[i] = to_f32(hT[(int64_t)n * a.ldh + slot0 + rr]);
+  const int cnt = __popcll(__ballot(my_row >= 0) & 0xffffffffull);  // padding is at the end of a tile
+  const int64_t slice = (int64_t)kTileRows * a.rpad;
+  const float* p = a.hpart + (int64_t)tile_id * a.kslices * slice + n0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int idx = tid + 256 * i, row = idx >> 4, n = idx & 15;
+    const float* q = p + row * a.rpad + n;
+    float s = 0.f;
+    for (int k0 = 0; k0 < a.kslices; k0 += 8) {  // eight slices are requested together and added in slice order
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = k0 + k < a.kslices ? q[(k0 + k) * slice] : 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+    part[row][n] = s;
   }
   __syncthreads();
+  write_h<T>(a, slot0, cnt, r, a.scale[g], n0, 16, [&](int row, int n) { return part[row][n]; });
+}
+
+// ---------------------------------------------------------------------------
+// Expand: dst[row(slot)][c] += sum_n h[slot][n] * W_g[c][n].  A wave owns (tile, 16 E columns): column c0 + E li + q is
+// output column li of the q-th product, so a lane updates E consecutive columns of eight rows, 16 bytes each, and a
+// wave-wide access covers four rows of 256 bytes.  The rows are requested before the contraction starts; its operands
+// (h of the tile, 16 E rows of W) come from L2.  4096 x 4096 fp32 at rank 16: 245 -> 29 us (4.6 TB/s of y).
+// ---------------------------------------------------------------------------
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* __restrict__ tile_group,
+                                                    const int32_t* __restrict__ slot_rows,
+                                                    const int32_t* __restrict__ tile_walk, int num_items) {
+  constexpr int E = Piece<T>::E, RP = 16 * NB;
+  constexpr int NKS = (RP + 4 * E - 1) / (4 * E);  // contraction steps
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kb = lane >> 4;
+  const int ngroups = (a.width_dst + 16 * E - 1) / (16 * E);
+  const int item = blockIdx.x * 4 + wave;
+  if (item >= num_items) return;
+  const int nth = item / ngroups;
+  const int tile_id = checked_tile(a.wl_tiles.ids ? work_item(a.wl_tiles, nth) : (tile_walk ? tile_walk[nth] : nth), a.tb);
+  if (tile_id < 0) return;
+  const int slot0 = tile_id * kTileRows;
+  const int g = checked_group(tile_group[tile_id], a.tb);
+  const int4 r0 = *reinterpret_cast<const int4*>(slot_rows + slot0 + 4 * kb);
+  const int4 r1 = *reinterpret_cast<const int4*>(slot_rows + slot0 + 16 + 4 * kb);
+  if (g < 0) return;
+  const int r = class_rank(a.rank[g], a.rank_lo, RP);
+  if (r <= 0) return;
+  const int rows[2][4] = {{r0.x, r0.y, r0.z, r0.w}, {r1.x, r1.y, r1.z, r1.w}};
+  const int c = (item - nth * ngroups) * (16 * E) + E * li;  // this lane's columns
+  const int keep = min(E, a.width_dst - c);                  // <= 0: none
+  T* dst = (T*)a.dst + c;
   const T* W = group_weight<T>(a.w_expand, a.w_expand_base, a.expand_group_stride, g);
-  T* dst = (T*)a.dst;
-  for (int c = tid; c < a.width_dst; c += 256) {
-    float acc[kTileRows];
+  const T* h = (const T*)a.hT + (int64_t)a.rpad * a.ldh + (int64_t)slot0 * RP;
+  uint4 y[2][4];
+  f32x4 d[2][E];
 #pragma unroll
-    for (int rr = 0; rr < kTileRows; ++rr) acc[rr] = 0.f;
-    const T* wrow = W + (int64_t)c * a.ld_expand;
-    for (int n = 0; n < r; ++n) {
-      const float b = to_f32(wrow[n]);
+  for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int rr = 0; rr < kTileRows; ++rr) acc[rr] += lds_f[n * kTileRows + rr] * b;
-    }
+    for (int q = 0; q < E; ++q) d[tt][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // whole: every lane has its E columns and the rank is whole pieces, so that nothing is guarded (rows of padding
+  // slots read row 0, rank indices past the rank read index 0 and are zeroed)
+  auto body = [&](auto whole) {
 #pragma unroll
-    for (int rr = 0; rr < kTileRows; ++rr) {
-      if (rows_s[rr] >= 0) {
-        T* o = dst + (int64_t)rows_s[rr] * a.ld_dst + c;
-        from_f32(to_f32(*o) + acc[rr], o);
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const T* row = dst + (int64_t)max(checked_row(rows[tt][v], a.tb), 0) * a.ld_dst;
+        y[tt][v] = whole ? ld_piece_nt(row) : ld_piece(row, keep);
+      }
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int n0 = 4 * E * ks + E * kb;
+      if (ks && 4 * E * ks >= r) break;  // (uniform over the block)
+      uint4 hop[2], w[E];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) hop[tt] = n0 < RP ? ld_piece(h + (16 * tt + li) * RP + n0) : zero4();
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        if constexpr (whole) {
+          w[q] = ld_piece(W + (int64_t)(c + q) * a.ld_expand + (n0 < r ? n0 : 0));
+        } else {
+          w[q] = q < keep ? ld_piece(W + (int64_t)(c + q) * a.ld_expand + n0, r - n0) : zero4();
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        if (whole && n0 >= r) w[q] = zero4();
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) d[tt][q] = mma_piece<T>(hop[tt], w[q], d[tt][q]);
       }
     }
-  }
+  };
+  if ((c - E * li) + 16 * E <= a.width_dst && r % E == 0) body(std::true_type{});
+  else body(std::false_type{});
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = checked_row(rows[tt][v], a.tb);
+      if (row < 0 || keep <= 0) continue;
+      T* o = dst + (int64_t)row * a.ld_dst;
+      T e[E];
+      __builtin_memcpy(e, &y[tt][v], 16);
+#pragma unroll
+      for (int q = 0; q < E; ++q) from_f32(to_f32(e[q]) + d[tt][q][v], &e[q]);
+      if (keep == E) {
+        uint4 out;
+        __builtin_memcpy(&out, e, 16);
+        st_piece_nt(o, out);
+      } else {
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+          if (q < keep) o[q] = e[q];
+      }
+    }
 }
 
 template <typename T>
@@ -130,57 +342,141 @@ __device__ inline void store_grad(const WgradArgs& a, int g, int n, int c, float
   from_f32(v, o);
 }
 
-// One chunk of one group, 256 columns per block, walked in passes of 512 slots:
-// out[n][c] = sum_{slot in chunk} hT[n][slot] * src[row(slot)][c], slots ascending.
-template <typename T>
-__global__ __launch_bounds__(256) void k_wgrad_generic(WgradArgs a, const ChunkInfo* __restrict__ chunks,
-                                                       const int32_t* __restrict__ slot_rows) {
-  constexpr int kPass = kChunkTilesMin * kTileRows;
-  __shared__ float hs[16][kPass];
-  __shared__ int rows_s[kPass];
-  const ChunkInfo ci = checked_chunk(chunks[blockIdx.x], a.tb);
+// ---------------------------------------------------------------------------
+// Row contraction: out[n][c] = sum over the slots of a chunk of hT[n][slot] * src[row(slot)][c].  A wave owns (chunk,
+// 16 E columns, 16 NB rank indices) and walks the chunk's tiles, the next tile's rows in flight while one is consumed.
+// A lane loads a piece (E columns) of eight rows 8 kb .. 8 kb + 7; column c0 + E li + q is row li of the q-th product.
+// In fp32 component q of the eight pieces is that product's operand as it stands (row 8 kb + i in step i); in bf16 the
+// 8 x 8 block is transposed inside the lane first.  The sums leave through LDS as whole rows (16-byte
+// stores of 64 separate rows instead: 36 against 25 us).  4096 x 4096 fp32 at rank 16: 81 -> 25 us.
+// ---------------------------------------------------------------------------
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_wgrad_any(WgradArgs a, const ChunkInfo* __restrict__ chunks,
+                                                   const int32_t* __restrict__ slot_rows) {
+  constexpr int E = Piece<T>::E, HP = 8 / E;  // pieces of a lane's eight slots of hT
+  constexpr int CW = 16 * E, SS = CW + 4;  // columns of a wave, row stride of its staged sums
+  __shared__ __attribute__((aligned(16))) float stage[4][16 * SS];
+  extern __shared__ __attribute__((aligned(16))) int32_t rows_s[];  // the chunk's row indices
+  // column blocks of one chunk are neighbours (they read neighbouring pieces of the same rows and the same h), the
+  // blocks of one column range and other rank indices too (they read the same pieces)
+  const int nz = a.rpad / (16 * NB), ncb = (a.width + 4 * CW - 1) / (4 * CW);
+  const int z = blockIdx.x % nz, cb = (blockIdx.x / nz) % ncb;
+  const int cidx = work_item(a.wl_chunks, blockIdx.x / (nz * ncb));
+  if (cidx < 0) return;
+  const ChunkInfo ci = checked_chunk(chunks[cidx], a.tb);
   const int g = ci.group;
   if (g < 0) return;
   const int r = class_rank(a.rank[g], a.rank_lo, a.rpad);
-  if (r <= 0) return;
-  const int tid = threadIdx.x;
-  const int c = blockIdx.y * 256 + tid;
-  const int total = ci.ntiles * kTileRows;
-  const T* src = (const T*)a.src;
-  const T* hT = (const T*)a.hT;
-  for (int n0 = 0; n0 < r; n0 += 16) {
-    float acc[16];
+  const int nb0 = 16 * NB * z;  // first rank index of this block
+  if (r <= nb0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
+  const int nt = ci.ntiles;
+  for (int i = tid; i < nt * kTileRows; i += 256) rows_s[i] = checked_row(slot_rows[ci.tile0 * kTileRows + i], a.tb);
+  __syncthreads();
+  const int c0 = (cb * 4 + wave) * CW;
+  if (c0 >= a.width) return;  // (no barrier follows)
+  const int c = c0 + E * li;
+  const int keep = min(E, a.width - c);  // <= 0: none
+  const T* src = (const T*)a.src + c;
+  const T* hT = (const T*)a.hT + (int64_t)(nb0 + li) * a.ldh + (int64_t)ci.tile0 * kTileRows + 8 * kb;
+  const bool full = c0 + CW <= a.width;  // every lane has its E columns (uniform over the wave)
+  struct Tile {
+    uint4 x[8], h[NB][HP];
+    uint32_t live;  // bit i: row i of this lane is a real row
+  };
+  auto issue = [&](int t, Tile& t_) {
+    const int4 ra = *reinterpret_cast<const int4*>(rows_s + t * kTileRows + 8 * kb);
+    const int4 rb = *reinterpret_cast<const int4*>(rows_s + t * kTileRows + 8 * kb + 4);
+    const int rows[8] = {ra.x, ra.y, ra.z, ra.w, rb.x, rb.y, rb.z, rb.w};
+    t_.live = 0;
+    if (full) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0.f;
-    for (int p0 = 0; p0 < total; p0 += kPass) {
-      const int slot0 = ci.tile0 * kTileRows + p0;
-      const int len = min(kPass, total - p0);
-      __syncthreads();
-      for (int i = tid; i < len; i += 256) rows_s[i] = checked_row(slot_rows[slot0 + i], a.tb);
-      for (int i = tid; i < 16 * len; i += 256) {
-        const int j = i / len, pp = i % len;
-        hs[j][pp] = (n0 + j) < r ? to_f32(hT[(int64_t)(n0 + j) * a.ldh + slot0 + pp]) : 0.f;
-      }
-      __syncthreads();
-      if (c < a.width) {
-        for (int pp = 0; pp < len; ++pp) {
-          if (rows_s[pp] < 0) continue;
-          const float xv = to_f32(src[(int64_t)rows_s[pp] * a.ld_src + c]);
+      for (int i = 0; i < 8; ++i) t_.x[i] = ld_piece(src + (int64_t)max(rows[i], 0) * a.ld_src);
+    } else {
 #pragma unroll
-          for (int j = 0; j < 16; ++j) acc[j] += hs[j][pp] * xv;
+      for (int i = 0; i < 8; ++i) t_.x[i] = ld_piece(src + (int64_t)max(rows[i], 0) * a.ld_src, keep);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t_.live |= rows[i] >= 0 ? (1u << i) : 0u;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int p = 0; p < HP; ++p) t_.h[nb][p] = ld_piece(hT + (int64_t)(16 * nb) * a.ldh + t * kTileRows + E * p);
+  };
+  f32x4 acc[E][NB];
+#pragma unroll
+  for (int q = 0; q < E; ++q)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[q][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto consume = [&](Tile& t_) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!((t_.live >> i) & 1u)) t_.x[i] = zero4();
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            acc[q][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(part_f32(t_.x[i], q), part_f32(t_.h[nb][i >> 2], i & 3),
+                                                             acc[q][nb], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const uint32_t sel = (q & 1) ? 0x07060302u : 0x05040100u;
+        uint32_t e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t w[4] = {t_.x[i].x, t_.x[i].y, t_.x[i].z, t_.x[i].w};
+          e[i] = w[q >> 1];
         }
+        const uint4 tr = make_uint4(__builtin_amdgcn_perm(e[1], e[0], sel), __builtin_amdgcn_perm(e[3], e[2], sel),
+                                    __builtin_amdgcn_perm(e[5], e[4], sel), __builtin_amdgcn_perm(e[7], e[6], sel));
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[q][nb] = mfma16(tr, t_.h[nb][0], acc[q][nb]);
       }
     }
-    if (c < a.width) {
+  };
+  Tile A, B;
+  if (nt > 0) issue(0, A);
+  for (int t = 0; t < nt; t += 2) {
+    if (t + 1 < nt) issue(t + 1, B);
+    consume(A);
+    if (t + 1 >= nt) break;
+    if (t + 2 < nt) issue(t + 2, A);
+    consume(B);
+  }
+  // 16 rank indices at a time through the wave's stage, [n][column], so that whole rows leave
+  float* st = stage[wave];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int n = n0 + j;
-        if (n < r) {
-          if (ci.partial >= 0)
-            a.partial[partial_index(ci.partial, n, c, a.rpad, a.width)] = acc[j];
-          else
-            store_grad<T>(a, g, n, c, acc[j]);
-        }
+  for (int nb = 0; nb < NB; ++nb) {
+    const int n_first = nb0 + 16 * nb;
+    if (n_first >= r) break;
+    if (nb) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int q = 0; q < E; q += 4)
+        *reinterpret_cast<float4*>(st + li * SS + E * (4 * kb + v) + q) =
+            make_float4(acc[q][nb][v], acc[q + 1][nb][v], acc[q + 2][nb][v], acc[q + 3][nb][v]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    if (ci.partial >= 0) {  // (columns past the width lie inside the buffer's blocks of 128)
+      float* p = a.partial + partial_index(ci.partial, n_first, c0, a.rpad, a.width);
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const int idx = lane + 64 * i, n = idx / (CW / 4), cc = 4 * (idx % (CW / 4));
+        if (n_first + n < r) *reinterpret_cast<float4*>(p + n * 128 + cc) = *reinterpret_cast<const float4*>(st + n * SS + cc);
+      }
+    } else if (a.transposed) {
+      for (int idx = lane; idx < 16 * CW; idx += 64) {
+        const int cc = idx >> 4, n = idx & 15;
+        if (n_first + n < r && c0 + cc < a.width) store_grad<T>(a, g, n_first + n, c0 + cc, st[n * SS + cc]);
+      }
+    } else {
+      for (int idx = lane; idx < 16 * CW; idx += 64) {
+        const int n = idx / CW, cc = idx % CW;
+        if (n_first + n < r && c0 + cc < a.width) store_grad<T>(a, g, n_first + n, c0 + cc, st[n * SS + cc]);
       }
     }
   }
@@ -355,30 +651,45 @@ __global__ __launch_bounds__(256) void k_wgrad_reduce_multi(WgradReduceJobs jobs
   else wgrad_reduce_body<T, false>(a, n0, chunk_first, partial_first);
 }
 
-// bT_g[n][m] = B_g[m][n], aT_g[k][n] = A_g[n][k]; zero for n >= rank[g].
+// bT_g[n][m] = B_g[m][n], aT_g[k][n] = A_g[n][k]; zero for n >= rank[g].  A block turns 64 features x rpad rank indices
+// over in LDS: both the reads and the writes run along the contiguous index of their matrix (element by element along
+// one of them: 71 against 31 us for four adapters of rank 128, 4096 x 4096).
 // (TS: the adapters' element type, T: that of the copies; they differ for fp32 adapters under bf16 activations)
 template <typename TS, typename T>
 __global__ __launch_bounds__(256) void k_transpose_weights(tk_lora_desc d, int rpad, int rank_lo, T* __restrict__ bT,
                                                            T* __restrict__ aT) {
+  extern __shared__ float turn_s[];  // [64][rpad + 1]
   const int g = blockIdx.y;
   const int r = class_rank(d.rank[g], rank_lo, rpad);
   if (rank_lo > 0 && r <= 0) return;  // a group of a lower rank class: no launch of this class reads its copies
-  const TS* A = (const TS*)d.lora_A[g];
-  const TS* B = (const TS*)d.lora_B[g];
-  const int64_t nb = (int64_t)rpad * d.out_features, na = (int64_t)rpad * d.in_features;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nb + na; i += (int64_t)gridDim.x * 256) {
-    if (i < nb) {
-      const int n = (int)(i / d.out_features), m = (int)(i % d.out_features);
-      T v = (T)0;
-      if (n < r) from_f32(to_f32(B[(int64_t)m * d.ldb + n]), &v);
-      bT[(int64_t)g * nb + i] = v;
-    } else {
-      const int64_t q = i - nb;
-      const int k = (int)(q / rpad), n = (int)(q % rpad);
-      T v = (T)0;
-      if (n < r) from_f32(to_f32(A[(int64_t)n * d.lda + k]), &v);
-      aT[(int64_t)g * na + q] = v;
+  const int blocks_b = (d.out_features + 63) >> 6;
+  const bool is_b = (int)blockIdx.x < blocks_b;
+  const int width = is_b ? d.out_features : d.in_features;
+  const int f0 = ((int)blockIdx.x - (is_b ? 0 : blocks_b)) << 6, nf = min(64, width - f0);
+  const int total = 64 * rpad, shift = __ffs(rpad) - 1, ls = rpad + 1;  // rpad is a power of two
+  if (is_b) {
+    const TS* B = (const TS*)d.lora_B[g] + (int64_t)f0 * d.ldb;
+    for (int i = threadIdx.x; i < total; i += 256) {
+      const int f = i >> shift, n = i & (rpad - 1);
+      turn_s[f * ls + n] = f < nf && n < r ? to_f32(B[(int64_t)f * d.ldb + n]) : 0.f;
     }
+  } else {
+    const TS* A = (const TS*)d.lora_A[g] + f0;
+    for (int i = threadIdx.x; i < total; i += 256) {
+      const int n = i >> 6, f = i & 63;
+      turn_s[f * ls + n] = f < nf && n < r ? to_f32(A[(int64_t)n * d.lda + f]) : 0.f;
+    }
+  }
+  __syncthreads();
+  if (is_b) {
+    T* o = bT + (int64_t)g * rpad * width + f0;
+    for (int i = threadIdx.x; i < total; i += 256) {
+      const int n = i >> 6, f = i & 63;
+      if (f < nf) from_f32(turn_s[f * ls + n], &o[(int64_t)n * width + f]);
+    }
+  } else {
+    T* o = aT + ((int64_t)g * width + f0) * rpad;
+    for (int i = threadIdx.x; i < nf * rpad; i += 256) from_f32(turn_s[(i >> shift) * ls + (i & (rpad - 1))], &o[i]);
   }
 }
 
@@ -484,34 +795,60 @@ int launch_convert_weights(const tk_lora_desc& d, void* stage, bool want_a, bool
   return launch_convert_weights_multi(&dp, &stage, 1, want_a, want_b, s);
 }
 
+namespace {
+
+template <typename T, int NB>
+void launch_pass_any(const PassArgs& a, const SegView& seg, const SegLayout& L, int phases, hipStream_t s) {
+  constexpr int E = Piece<T>::E;
+  const int32_t* rows = seg.slot_table(a.map_rows);
+  if (phases & 1) {
+    // the slices of the split shrink's plan (its buffer holds kslices slices of every tile)
+    const int slice_cols = (int)round_up(ceil_div(a.width_src, a.kslices), 8 * E);
+    hipLaunchKernelGGL((k_shrink_any<T, NB>), dim3((unsigned)(L.max_tiles * a.kslices)), dim3(256), 0, s, a, slice_cols,
+                       seg.tile_group, rows);
+    if (a.kslices > 1)
+      hipLaunchKernelGGL(k_shrink_any_finish<T>, dim3((unsigned)L.max_tiles, NB), dim3(256), 0, s, a, seg.tile_group,
+                         rows);
+  }
+  if (a.dst && (phases & 2)) {
+    const int64_t items = L.max_tiles * ceil_div(a.width_dst, 16 * E);
+    hipLaunchKernelGGL((k_expand_any<T, NB>), dim3((unsigned)ceil_div(items, 4)), dim3(256), 0, s, a, seg.tile_group,
+                       rows, seg.tile_walk(a.map_rows), (int)items);
+  }
+}
+
+template <typename T>
+void launch_pass_any(const PassArgs& a, const SegView& seg, const SegLayout& L, int phases, hipStream_t s) {
+  if (a.rpad <= 16) launch_pass_any<T, 1>(a, seg, L, phases, s);
+  else if (a.rpad <= 32) launch_pass_any<T, 2>(a, seg, L, phases, s);
+  else if (a.rpad <= 64) launch_pass_any<T, 4>(a, seg, L, phases, s);
+  else launch_pass_any<T, 8>(a, seg, L, phases, s);
+}
+
+template <typename T>
+void launch_wgrad_any(const WgradArgs& a, const SegView& seg, const SegLayout& L, hipStream_t s) {
+  const size_t dyn = (size_t)L.chunk_tiles * kTileRows * sizeof(int32_t);
+  // at most 32 rank indices per block: with 64 the accumulators leave one wave per SIMD (bf16: and spill)
+  const int nb = a.rpad <= 16 ? 1 : 2;
+  const dim3 grid((unsigned)(a.rpad / (16 * nb) * ceil_div(a.width, 64 * Piece<T>::E) * L.max_chunks));
+  const auto kernel = nb == 1 ? k_wgrad_any<T, 1> : k_wgrad_any<T, 2>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), dyn, s, a, seg.chunks, seg.slot_table(a.map_rows));
+}
+
+}  // namespace
+
 int launch_pass_generic(const PassArgs& a, const SegView& seg, const SegLayout& L, int dtype, int phases,
                         hipStream_t s) {
   if (L.rows == 0) return TK_OK;
-  const unsigned grid = (unsigned)L.max_tiles;
-  const int32_t* rows = seg.slot_table(a.map_rows);
-  const size_t lds_shrink = sizeof(float) * (size_t)(kTileRows + a.rpad) * (kKC + 1);
-  const size_t lds_expand = sizeof(float) * (size_t)a.rpad * kTileRows;
-  if (dtype == TK_DTYPE_F32) {
-    if (phases & 1)
-      hipLaunchKernelGGL(k_shrink_generic<float>, dim3(grid), dim3(256), lds_shrink, s, a, seg.tile_group, rows);
-    if (a.dst && (phases & 2))
-      hipLaunchKernelGGL(k_expand_generic<float>, dim3(grid), dim3(256), lds_expand, s, a, seg.tile_group, rows);
-  } else {
-    if (phases & 1)
-      hipLaunchKernelGGL(k_shrink_generic<bf16_t>, dim3(grid), dim3(256), lds_shrink, s, a, seg.tile_group, rows);
-    if (a.dst && (phases & 2))
-      hipLaunchKernelGGL(k_expand_generic<bf16_t>, dim3(grid), dim3(256), lds_expand, s, a, seg.tile_group, rows);
-  }
+  if (dtype == TK_DTYPE_F32) launch_pass_any<float>(a, seg, L, phases, s);
+  else launch_pass_any<bf16_t>(a, seg, L, phases, s);
   return check_launch();
 }
 
 int launch_wgrad_generic(const WgradArgs& a, const SegView& seg, const SegLayout& L, int dtype, hipStream_t s) {
   if (L.rows == 0) return TK_OK;
-  const dim3 grid((unsigned)L.max_chunks, (unsigned)ceil_div(a.width, 256));
-  if (dtype == TK_DTYPE_F32)
-    hipLaunchKernelGGL(k_wgrad_generic<float>, grid, dim3(256), 0, s, a, seg.chunks, seg.slot_table(a.map_rows));
-  else
-    hipLaunchKernelGGL(k_wgrad_generic<bf16_t>, grid, dim3(256), 0, s, a, seg.chunks, seg.slot_table(a.map_rows));
+  if (dtype == TK_DTYPE_F32) launch_wgrad_any<float>(a, seg, L, s);
+  else launch_wgrad_any<bf16_t>(a, seg, L, s);
   return check_launch();
 }
 
@@ -555,16 +892,16 @@ int launch_wgrad_reduce_multi(const WgradArgs* sets, int n, const SegView& seg, 
 int launch_transpose_weights(const tk_lora_desc& d, int rank_lo, void* bT, void* aT, hipStream_t s) {
   if (d.num_groups == 0) return TK_OK;
   const int rpad = rank_pad(d.max_rank);
-  const int64_t per_group = (int64_t)rpad * (d.out_features + d.in_features);
-  const dim3 grid((unsigned)std::min<int64_t>(ceil_div(per_group, 256), 64), (unsigned)d.num_groups);
+  const dim3 grid((unsigned)(ceil_div(d.out_features, 64) + ceil_div(d.in_features, 64)), (unsigned)d.num_groups);
+  const size_t lds = sizeof(float) * 64 * (size_t)(rpad + 1);
   if (d.dtype == TK_DTYPE_F32)
-    hipLaunchKernelGGL((k_transpose_weights<float, float>), grid, dim3(256), 0, s, d, rpad, rank_lo, (float*)bT,
+    hipLaunchKernelGGL((k_transpose_weights<float, float>), grid, dim3(256), lds, s, d, rpad, rank_lo, (float*)bT,
                        (float*)aT);
   else if (mixed_weights(d))
-    hipLaunchKernelGGL((k_transpose_weights<float, bf16_t>), grid, dim3(256), 0, s, d, rpad, rank_lo,
+    hipLaunchKernelGGL((k_transpose_weights<float, bf16_t>), grid, dim3(256), lds, s, d, rpad, rank_lo,
                        (bf16_t*)bT, (bf16_t*)aT);
   else
-    hipLaunchKernelGGL((k_transpose_weights<bf16_t, bf16_t>), grid, dim3(256), 0, s, d, rpad, rank_lo, (bf16_t*)bT,
+    hipLaunchKernelGGL((k_transpose_weights<bf16_t, bf16_t>), grid, dim3(256), lds, s, d, rpad, rank_lo, (bf16_t*)bT,
                        (bf16_t*)aT);
   return check_launch();
 }

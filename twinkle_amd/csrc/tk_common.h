@@ -517,7 +517,7 @@ int launch_unpermute_wgrad(const void* dout, int64_t ld_dout, const void* rows_,
                            const void* ws, int64_t rows, int64_t tokens, int32_t width, int32_t groups, int dtype,
                            hipStream_t s);
 
-// kernels_generic.hip : any shape / stride, fp32 and bf16, VALU
+// kernels_generic.hip : any shape / stride, fp32 and bf16
 int launch_pass_generic(const PassArgs& a, const SegView& seg, const SegLayout& L, int dtype, int phases,
                         hipStream_t s);
 int launch_wgrad_generic(const WgradArgs& a, const SegView& seg, const SegLayout& L, int dtype, hipStream_t s);
