@@ -222,6 +222,12 @@ int tk_lora_bwd(const tk_lora_desc* desc, const void* dy_device, int64_t lddy, c
                 const void* h_device, void* dx_device, int64_t lddx, void* const* grad_A, void* const* grad_B,
                 int32_t accumulate, void* workspace_device, int64_t workspace_bytes, tk_stream_t stream);
 
+/* tk_lora_bwd with dx written instead of added onto: dx[row] = scale_g * (dy[row] B_g) A_g, zeros in the rows of no
+ * live group, for a dx that holds nothing yet (saves its zero fill and a read of it). */
+int tk_lora_bwd_store(const tk_lora_desc* desc, const void* dy_device, int64_t lddy, const void* x_device, int64_t ldx,
+                      const void* h_device, void* dx_device, int64_t lddx, void* const* grad_A, void* const* grad_B,
+                      int32_t accumulate, void* workspace_device, int64_t workspace_bytes, tk_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Multi-tenant optimizer step over adapter tensors (one launch set for all tenants).
  *

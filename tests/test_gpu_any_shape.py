@@ -82,3 +82,30 @@ def test_an_infinite_row_stays_with_its_adapter(dev, dtype):
     assert torch.isfinite(yd[1:]).all() and torch.isfinite(dxd[1:]).all()
     for g in (1, 2):
         assert torch.isfinite(ga[g]).all() and torch.isfinite(gb[g]).all()
+
+
+@pytest.mark.parametrize('dtype,t,k,m,ranks', [
+    (torch.bfloat16, 900, 256, 1024, [16, 3, 0, 9]),        # one pass over dy, flat expand
+    (torch.bfloat16, 1500, 384, 640, [64, 20, 0, 33]),      # the expand above rank 16
+    (torch.bfloat16, 1500, 384, 640, [64, 8, 0, 20]),       # three rank classes
+    (torch.bfloat16, 333, 41, 24, [8, 0, 5, 3]),            # odd shapes
+    (torch.float32, 333, 40, 24, [8, 0, 5, 3]),
+    (torch.float32, 200, 40, 24, [0, 0, 0, 0]),             # no live adapter at all
+])
+def test_a_dx_that_is_written_equals_one_that_starts_at_zero(dev, dtype, t, k, m, ranks):
+    """tk_lora_bwd_store into a buffer of NaN and tk_lora_bwd onto zeros: the same bits, zeros in the rows of dead
+    adapters and of no adapter."""
+    from twinkle_amd.ops import _lora_bwd
+    x, base, dy, a, b, ids, _, scales = _problem(t, k, m, len(ranks), max(max(ranks), 1), ranks, seed=t)
+    ids[::7] = -1
+    ids[:70] = len(ranks)
+    xd, yd, dyd = (v.to(dtype).to(dev) for v in (x, base, dy))
+    seg = build_segments(ids.to(torch.int32).to(dev), len(ranks))
+    groups = AdapterGroups([w.to(dtype).to(dev) for w in a], [w.to(dtype).to(dev) for w in b], ranks, scales)
+    h = lora_fwd_(xd, yd, seg, groups)
+    added, written = torch.zeros_like(xd), torch.full_like(xd, float('nan'))
+    _lora_bwd('tk_lora_bwd', dyd, xd, h, added, None, None, seg, groups)
+    _lora_bwd('tk_lora_bwd_store', dyd, xd, h, written, None, None, seg, groups)
+    assert torch.equal(added, written)
+    dead = (ids < 0) | (ids >= len(ranks)) | (torch.tensor(ranks + [0])[ids.clamp(0, len(ranks))] == 0)
+    assert torch.count_nonzero(written[dead.to(dev)]) == 0

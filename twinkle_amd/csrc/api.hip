@@ -614,7 +614,7 @@ int tk_lora_expand(const tk_lora_desc* d, const void* h, void* y, int64_t ldy, t
 // The backward of the groups of one rank class (d: the class's descriptor; every group when there is one class).
 static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, const void* dy, int64_t lddy,
                           const void* x, int64_t ldx, const void* h, void* dx, int64_t lddx, void* const* grad_A,
-                          void* const* grad_B, int32_t accumulate, void* ws, hipStream_t s, bool may_fork) {
+                          void* const* grad_B, int32_t accumulate, bool store_dx, void* ws, hipStream_t s, bool may_fork) {
   const int rank_lo = P.rc[c].lo, class_mode = P.n > 1;
   BwdLayout B(*d);
   SegLayout L(d->rows, d->num_groups);
@@ -623,6 +623,7 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   const bool need_wT = dx || grad_A;
   BwdPlan plan = bwd_plan(d, B, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate, ws, rank_lo, class_mode);
   use_lists(P, c, L, &plan.a, &plan.ga, &plan.gb);
+  plan.a.dst_store = store_dx ? 1 : 0;
   WgradArgs &ga = plan.ga, &gb = plan.gb;
   PassArgs& a = plan.a;
   const TransposeJob& tr = plan.tr;
@@ -698,11 +699,17 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   return rc;
 }
 
-int tk_lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
-                void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, void* ws,
-                int64_t ws_bytes, tk_stream_t stream) {
+static int lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
+                    void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, bool store_dx,
+                    void* ws, int64_t ws_bytes, tk_stream_t stream) {
   if (!desc_ok(d)) return TK_ERR_INVALID;
-  if (d->rows == 0 || d->max_rank == 0) return TK_OK;
+  if (d->rows == 0 || (d->max_rank == 0 && !(store_dx && dx))) return TK_OK;
+  if (d->max_rank == 0) {  // every row is written: zeros
+    if (lddx < d->in_features) return TK_ERR_INVALID;
+    SegLayout L(d->rows, d->num_groups);
+    return launch_zero_rows(dx, lddx, d->in_features, d->dtype, d->rank, 0, d->map_rows, SegView(d->seg_ws, L), L,
+                            (hipStream_t)stream);
+  }
   if (!dy || lddy < d->out_features || !ws) return TK_ERR_INVALID;
   if (dx && lddx < d->in_features) return TK_ERR_INVALID;
   if (grad_A && (!x || ldx < d->in_features)) return TK_ERR_INVALID;
@@ -712,7 +719,10 @@ int tk_lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void*
   {
     SegLayout L(d->rows, d->num_groups);
     SegView V(d->seg_ws, L);
-    const int rc = build_lists(P, d, (char*)ws + P.ws_core_total, V, L, (hipStream_t)stream);
+    int rc = build_lists(P, d, (char*)ws + P.ws_core_total, V, L, (hipStream_t)stream);
+    if (rc == TK_OK && store_dx && dx)
+      rc = launch_zero_rows(dx, lddx, d->in_features, d->dtype, d->rank, d->max_rank, d->map_rows, V, L,
+                            (hipStream_t)stream);
     if (rc != TK_OK) return rc;
   }
   // Every rank class reads and writes the rows and the gradients of its own groups only, in its own region of the
@@ -720,8 +730,20 @@ int tk_lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void*
   // whose row stride does not depend on the padded rank, up to its own padded rank.
   return for_each_class(P.n, (hipStream_t)stream, [&](int c, hipStream_t cs, bool forked) {
     return lora_bwd_class(&P.d[c], P, c, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate,
-                          (char*)ws + P.ws_off[c], cs, !forked);
+                          store_dx, (char*)ws + P.ws_off[c], cs, !forked);
   });
+}
+
+int tk_lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
+                void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, void* ws,
+                int64_t ws_bytes, tk_stream_t stream) {
+  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate, false, ws, ws_bytes, stream);
+}
+
+int tk_lora_bwd_store(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
+                      void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, void* ws,
+                      int64_t ws_bytes, tk_stream_t stream) {
+  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate, true, ws, ws_bytes, stream);
 }
 
 // ---- packed experts: grouped base GEMM (+ LoRA term) ---------------------------------------------------------------

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const T* row = dst + (int64_t)max(checked_row(rows[tt][v], a.tb), 0) * a.ld_dst;
-        y[tt][v] = whole ? ld_piece_nt(row) : ld_piece(row, keep);
+        y[tt][v] = a.dst_store ? zero4() : (whole ? ld_piece_nt(row) : ld_piece(row, keep));
       }
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -328,6 +328,20 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
           if (q < keep) o[q] = e[q];
       }
     }
+}
+
+// Zeros in the rows whose group is not live, next to an expand that writes the others instead of adding onto them.
+template <typename T>
+__global__ __launch_bounds__(256) void k_zero_rows(T* dst, int64_t ld, int width, const int32_t* __restrict__ rank,
+                                                   int max_rank, TableBounds tb, const int32_t* __restrict__ tile_group,
+                                                   const int32_t* __restrict__ slot_rows) {
+  const int g = checked_group(tile_group[blockIdx.x], tb);
+  if (g >= 0 && class_rank(rank[g], 0, max_rank) > 0) return;
+  for (int i = 0; i < kTileRows; ++i) {
+    const int row = checked_row(slot_rows[blockIdx.x * kTileRows + i], tb);
+    if (row < 0) continue;
+    for (int c = threadIdx.x; c < width; c += 256) dst[(int64_t)row * ld + c] = (T)0;
+  }
 }
 
 template <typename T>
@@ -842,6 +856,20 @@ int launch_pass_generic(const PassArgs& a, const SegView& seg, const SegLayout& 
   if (L.rows == 0) return TK_OK;
   if (dtype == TK_DTYPE_F32) launch_pass_any<float>(a, seg, L, phases, s);
   else launch_pass_any<bf16_t>(a, seg, L, phases, s);
+  return check_launch();
+}
+
+int launch_zero_rows(void* dst, int64_t ld, int width, int dtype, const int32_t* rank, int max_rank, int map_rows,
+                     const SegView& seg, const SegLayout& L, hipStream_t s) {
+  if (L.rows == 0) return TK_OK;
+  const dim3 grid((unsigned)L.max_tiles);
+  const int32_t* rows = seg.slot_table(map_rows);
+  if (dtype == TK_DTYPE_F32)
+    hipLaunchKernelGGL(k_zero_rows<float>, grid, dim3(256), 0, s, (float*)dst, ld, width, rank, max_rank,
+                       table_bounds(L), seg.tile_group, rows);
+  else
+    hipLaunchKernelGGL(k_zero_rows<bf16_t>, grid, dim3(256), 0, s, (bf16_t*)dst, ld, width, rank, max_rank,
+                       table_bounds(L), seg.tile_group, rows);
   return check_launch();
 }
 

@@ -326,7 +326,8 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
   if constexpr (NB > 1) {
     constexpr int TPI = 4;
     const int64_t blocks = ceil_div(L.max_tiles, TPI) * ceil_div(ngroups, 4);
-    const auto kernel = a.wl_sets.ids ? k_expand_multi<NB, TPI, true> : k_expand_multi<NB, TPI, false>;
+    const auto kernel = a.dst_store ? (a.wl_sets.ids ? k_expand_multi<NB, TPI, true, true> : k_expand_multi<NB, TPI, false, true>)
+                                    : (a.wl_sets.ids ? k_expand_multi<NB, TPI, true, false> : k_expand_multi<NB, TPI, false, false>);
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, hrow, seg.tile_group, rows,
                        seg.set_walk(a.map_rows), seg.header, seg.round_moved,
                        (int)std::min<int64_t>(L.sort_blocks, 64), (int)L.max_tiles);

@@ -513,7 +513,7 @@ __device__ __forceinline__ void expand_flat_body(const PassArgs& a, const bf16_t
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) y[tt][v] = rok[tt][v] ? ld16_nt(yp[tt][v]) : zero4();
+    for (int v = 0; v < 4; ++v) y[tt][v] = rok[tt][v] && !a.dst_store ? ld16_nt(yp[tt][v]) : zero4();
 #pragma unroll
   for (int q = 0; q < 8; ++q)
 #pragma unroll
@@ -565,7 +565,8 @@ __global__ __launch_bounds__(256) void k_expand_mfma(PassArgs a, const bf16_t* _
 // CLS: the launch serves one of several rank classes (work list of sets, ranks outside the class skipped).  A
 // compile-time switch because this kernel's schedule is touchy: with the two forms in one body the single-class
 // launch measured 10 % slower (config 5's q projection: 116 against 106 us).
-template <int NB, int TPI, bool CLS>
+// STORE: dst_store, for the same reason.
+template <int NB, int TPI, bool CLS, bool STORE>
 __global__ __launch_bounds__(256) void k_expand_multi(PassArgs a, const bf16_t* __restrict__ hrow,
                                                       const int32_t* __restrict__ tile_group,
                                                       const int32_t* __restrict__ slot_rows,
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(256) void k_expand_multi(PassArgs a, const bf16_t* 
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         T.rows[tt][v] = (unsigned)rr[tt][v] < row_limit ? rr[tt][v] : -1;
-        T.y[tt][v] = T.rows[tt][v] >= 0 ? ld16_nt(dst + (int64_t)T.rows[tt][v] * a.ld_dst) : zero4();
+        T.y[tt][v] = T.rows[tt][v] >= 0 && !STORE ? ld16_nt(dst + (int64_t)T.rows[tt][v] * a.ld_dst) : zero4();
       }
     }
   };

@@ -375,6 +375,8 @@ struct PassArgs {
   // groups whose rank is not in (rank_lo, rpad] are skipped (see class_rank); class_mode != 0 says that such groups
   // may exist, and kernels then look at the rank before they request a tile's rows
   int32_t rank_lo, class_mode;
+  // 1: rows are written (dst = h W2^T) instead of added onto; the rows of no live group are left to launch_zero_rows
+  int32_t dst_store;
   WorkList wl_tiles, wl_pairs, wl_octs, wl_sets;  // class_mode: the items of this class (see WorkList)
   TableBounds tb;
 };
@@ -520,6 +522,9 @@ int launch_unpermute_wgrad(const void* dout, int64_t ld_dout, const void* rows_,
 // kernels_generic.hip : any shape / stride, fp32 and bf16
 int launch_pass_generic(const PassArgs& a, const SegView& seg, const SegLayout& L, int dtype, int phases,
                         hipStream_t s);
+// zeros in the rows of `dst` whose group is not live (no group, rank 0, rank above max_rank)
+int launch_zero_rows(void* dst, int64_t ld, int width, int dtype, const int32_t* rank, int max_rank, int map_rows,
+                     const SegView& seg, const SegLayout& L, hipStream_t s);
 int launch_wgrad_generic(const WgradArgs& a, const SegView& seg, const SegLayout& L, int dtype, hipStream_t s);
 // sums the chunk partials of up to two contractions (dA, dB; either may be null) in one launch
 int launch_wgrad_reduce(const WgradArgs* a0, const WgradArgs* a1, const SegView& seg, const SegLayout& L, int dtype,

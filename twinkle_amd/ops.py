@@ -306,6 +306,12 @@ def lora_bwd_(dy: torch.Tensor, x: Optional[torch.Tensor], h: Optional[torch.Ten
               groups: AdapterGroups, map_rows: bool = True, accumulate: bool = False,
               workspace: Optional[torch.Tensor] = None) -> None:
     """``dx += ...`` in place, weight gradients through the pointer arrays (see ``tk_lora_bwd``)."""
+    _lora_bwd('tk_lora_bwd', dy, x, h, dx, grad_a_ptrs, grad_b_ptrs, seg, groups, map_rows, accumulate, workspace)
+
+
+def _lora_bwd(entry: str, dy, x, h, dx, grad_a_ptrs, grad_b_ptrs, seg, groups, map_rows=True, accumulate=False,
+              workspace=None) -> None:
+    """``entry``: ``tk_lora_bwd``, or ``tk_lora_bwd_store`` for a ``dx`` that holds nothing yet."""
     _check_rows(dy, 'dy', seg.rows, groups.out_features, groups.dtype)
     if x is not None:
         _check_rows(x, 'x', seg.rows, groups.in_features, groups.dtype)
@@ -315,13 +321,13 @@ def lora_bwd_(dy: torch.Tensor, x: Optional[torch.Tensor], h: Optional[torch.Ten
     lib = _lib.load()
     if workspace is None:
         workspace = torch.empty(lora_bwd_workspace_bytes(seg, groups), dtype=torch.uint8, device=dy.device)
-    code = lib.tk_lora_bwd(ctypes.byref(d), dy.data_ptr(), dy.stride(0), x.data_ptr() if x is not None else None,
-                           x.stride(0) if x is not None else 0, h.data_ptr() if h is not None else None,
-                           dx.data_ptr() if dx is not None else None, dx.stride(0) if dx is not None else 0,
-                           grad_a_ptrs.data_ptr() if grad_a_ptrs is not None else None,
-                           grad_b_ptrs.data_ptr() if grad_b_ptrs is not None else None, 1 if accumulate else 0,
-                           workspace.data_ptr(), workspace.numel(), _lib.stream_ptr())
-    _lib.check(code, 'tk_lora_bwd')
+    code = getattr(lib, entry)(ctypes.byref(d), dy.data_ptr(), dy.stride(0), x.data_ptr() if x is not None else None,
+                               x.stride(0) if x is not None else 0, h.data_ptr() if h is not None else None,
+                               dx.data_ptr() if dx is not None else None, dx.stride(0) if dx is not None else 0,
+                               grad_a_ptrs.data_ptr() if grad_a_ptrs is not None else None,
+                               grad_b_ptrs.data_ptr() if grad_b_ptrs is not None else None, 1 if accumulate else 0,
+                               workspace.data_ptr(), workspace.numel(), _lib.stream_ptr())
+    _lib.check(code, entry)
 
 
 def grouped_linear_(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTable, groups_per_expert: int = 1,
@@ -406,9 +412,9 @@ class _LoraDelta(torch.autograd.Function):
         na, nb = len(groups.a_tensors), len(groups.b_tensors)
         needs_a = any(ctx.needs_input_grad[5:5 + na])
         needs_b = any(ctx.needs_input_grad[5 + na:5 + na + nb])
-        dx = torch.zeros_like(x) if ctx.needs_input_grad[0] else None
+        dx = torch.empty_like(x) if ctx.needs_input_grad[0] else None
         arena_a, arena_b, pa, pb = _weight_grads(groups, needs_a, needs_b, dy.device)
-        lora_bwd_(dy, x, h, dx, pa, pb, seg, groups, ctx.map_rows, accumulate=False)
+        _lora_bwd('tk_lora_bwd_store', dy, x, h, dx, pa, pb, seg, groups, ctx.map_rows)
         ga = groups.grad_views(arena_a, 'a') if needs_a else [None] * na
         gb = groups.grad_views(arena_b, 'b') if needs_b else [None] * nb
         return (dx, dy, None, None, None, *ga, *gb)
