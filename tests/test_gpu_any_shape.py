@@ -109,3 +109,28 @@ def test_a_dx_that_is_written_equals_one_that_starts_at_zero(dev, dtype, t, k, m
     assert torch.equal(added, written)
     dead = (ids < 0) | (ids >= len(ranks)) | (torch.tensor(ranks + [0])[ids.clamp(0, len(ranks))] == 0)
     assert torch.count_nonzero(written[dead.to(dev)]) == 0
+
+
+@pytest.mark.parametrize('max_r,ranks', [(8, [8, 8, 8]), (8, [8, 4, 8]), (8, [8, 0, 8]), (24, [24, 24, 24])])
+def test_gradients_of_adapters_without_rows_are_zero(dev, max_r, ranks):
+    """The gradient arena starts uninitialised where every live block is written: also the block of an adapter that no
+    row of the batch uses, and never one past a smaller rank.  The freed block before it holds NaN."""
+    from twinkle_amd import multi_lora_delta
+    x, base, dy, a, b, _, _, scales = _problem(300, 128, 256, 3, max_r, ranks, seed=8)
+    ids = torch.zeros(300, dtype=torch.int32)               # adapter 2 is live and has no row
+    ad, bd = ([w.bfloat16().to(dev).requires_grad_(True) for w in ws] for ws in (a, b))
+    groups = AdapterGroups(ad, bd, ranks, scales)
+    xd, yd = x.bfloat16().to(dev).requires_grad_(True), base.bfloat16().to(dev)
+    y = multi_lora_delta(xd, yd, build_segments(ids.to(dev), 3), groups)
+    stale = [torch.full((n,), float('nan'), dtype=torch.bfloat16, device=dev)
+             for n in (groups.a_arena_elems, groups.b_arena_elems, groups.a_arena_elems + groups.b_arena_elems) * 2]
+    del stale
+    y.backward(dy.bfloat16().to(dev))
+    for g in range(3):
+        for w in (ad[g], bd[g]):
+            if ranks[g] == 0:
+                assert w.grad is None
+            else:
+                assert torch.isfinite(w.grad).all()
+                if g == 2:
+                    assert torch.count_nonzero(w.grad) == 0

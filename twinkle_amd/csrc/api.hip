@@ -77,6 +77,9 @@ struct SideStream {
   std::mutex use;  // held while a call enqueues its fork .. join sequence: the events are shared per device
 };
 
+// x and dy together below this: the backward stays on the caller's stream (see lora_bwd_class)
+constexpr int64_t kSideStreamBytes = 192ll << 20;
+
 SideStream* side_stream() {
   static const bool enabled = [] {
     const char* e = getenv("TK_BWD_STREAMS");
@@ -649,7 +652,11 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   // Separate kernels.  Two chains that meet only at the end: dB (reads dy and h) runs on a side stream,
   // the dy shrink -> dX on the caller's; dA follows the shrink on the side stream, next to the expand.
   // Without a side stream everything runs in the same order on the caller's stream.
-  SideStream* side = (grad_B && need_wT && may_fork) ? side_stream() : nullptr;
+  // Small problems stay on one stream: the fork and the join are six calls of the runtime (30 us of host time) and a wait
+  // on each side, more than two kernels of a few microseconds gain from running side by side.
+  const int64_t bytes = d->rows * ((int64_t)d->in_features + d->out_features) * elt_bytes(d->dtype);
+  const bool large = bytes >= kSideStreamBytes;
+  SideStream* side = (grad_B && need_wT && may_fork && large) ? side_stream() : nullptr;
   hipStream_t s2 = side ? side->stream : s;
   // two host threads must not interleave their records and waits on the device's one set of events
   std::unique_lock<std::mutex> side_guard;
