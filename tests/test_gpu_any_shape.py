@@ -134,3 +134,14 @@ def test_gradients_of_adapters_without_rows_are_zero(dev, max_r, ranks):
                 assert torch.isfinite(w.grad).all()
                 if g == 2:
                     assert torch.count_nonzero(w.grad) == 0
+
+
+@pytest.mark.parametrize('t,k,m,ranks', [
+    (2304, 2048, 1024, [128, 65]),                  # long groups: weights shared in LDS, chunks in pairs
+    (2304, 1024, 512, [100, 128]),                  # the narrowest source of that kernel
+    (700, 256, 384, [128, 70, 128]),                # short groups: tile by tile
+    (2600, 2048, 256, [128, 16, 40, 0]),            # rank classes next to rank 128
+])
+def test_rank_128(dev, t, k, m, ranks):
+    from test_gpu_lora import _run
+    _run(dev, torch.bfloat16, *_problem(t, k, m, len(ranks), 128, ranks, seed=t + m))

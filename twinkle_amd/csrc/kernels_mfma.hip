@@ -514,7 +514,6 @@ int launch_wgrad_coop_multi(const SharedWgradArgs& a0, const SegView& seg, const
 }
 
 bool pass_mfma_supported(const PassArgs& a) {
-  if (a.rpad > 64) return false;
   if (a.width_src % 64 != 0 || a.ld_src % 8 != 0 || !aligned16(a.src)) return false;
   if (a.dst && (a.width_dst % 128 != 0 || a.ld_dst % 8 != 0 || !aligned16(a.dst))) return false;
   if (a.ld_shrink % 8 != 0 || a.ld_expand % 8 != 0 || a.ldh % 8 != 0) return false;
@@ -527,12 +526,12 @@ int launch_pass_mfma(const PassArgs& a, const SegView& seg, const SegLayout& L, 
   if (L.rows == 0) return TK_OK;
   if (a.rpad <= 16) launch_pass<1>(a, seg, L, phases, s);
   else if (a.rpad <= 32) launch_pass<2>(a, seg, L, phases, s);
-  else launch_pass<4>(a, seg, L, phases, s);
+  else if (a.rpad <= 64) launch_pass<4>(a, seg, L, phases, s);
+  else return launch_pass_rank128(a, seg, L, phases, s);
   return check_launch();
 }
 
 bool wgrad_mfma_supported(const WgradArgs& a) {
-  if (a.rpad > 64) return false;
   if (a.width % 128 != 0 || a.ld_src % 8 != 0 || a.ldh % 8 != 0 || !aligned16(a.src) || !aligned16(a.hT)) return false;
   return true;
 }
@@ -541,7 +540,8 @@ int launch_wgrad_mfma(const WgradArgs& a, const SegView& seg, const SegLayout& L
   if (L.rows == 0) return TK_OK;
   if (a.rpad <= 16) launch_wgrad_pipe<1, TK_WGRAD_STAGES>(a, seg, L, s);
   else if (a.rpad <= 32) launch_wgrad_coop<2>(a, seg, L, s);
-  else launch_wgrad_coop<4>(a, seg, L, s);
+  else if (a.rpad <= 64) launch_wgrad_coop<4>(a, seg, L, s);
+  else return launch_wgrad_rank128(a, seg, L, s);
   return check_launch();
 }
 

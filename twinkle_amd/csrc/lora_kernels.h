@@ -258,7 +258,10 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
   constexpr int RP = 16 * NB;
   constexpr int WS = 72;                    // row stride of a staged weight block in bf16 (144 B: conflict-free)
   constexpr int NLD = (RP * 8 + 255) / 256;  // 16-byte pieces of a weight block per thread
-  constexpr int S = NB == 4 ? 2 : 3;  // steps of activations in registers (rank 64: the accumulators take the room)
+  constexpr int S = NB >= 4 ? 2 : 3;  // steps of activations in registers (from rank 64 on the accumulators take the room)
+  // steps the weights are requested ahead: at rank 128 one block of four waves has a CU to itself, and nothing else
+  // covers the latency of its 16 KB of weights per step
+  constexpr int WD = NB == 8 ? 2 : 1;
   __shared__ __attribute__((aligned(16))) bf16_t wbuf[2][RP * WS];
   __shared__ int32_t gts[8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
@@ -332,10 +335,11 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[u][tt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    uint4 wr[NLD];
-    auto step = [&](int s, const Step& X, Step& Xnext) {
+    uint4 wr[WD][NLD];
+    // (w_cur: the weights of step s + 1, w_next: where those of step s + WD go; one and the same for WD = 1)
+    auto step = [&](int s, const Step& X, Step& Xnext, const uint4 (&w_cur)[NLD], uint4 (&w_next)[NLD]) {
       lds_barrier();  // block s is complete; the other buffer has been read by everyone
-      stage_load(s + 1, wr);
+      stage_load(s + WD, w_next);
       if (active) issue(s + S - 1, Xnext);
       if (active) {
         const bf16_t* wb = wbuf[s & 1] + li * WS + 16 * kb;
@@ -351,23 +355,25 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
             }
         }
       }
-      stage_store((s + 1) & 1, wr);  // block s + 1 (zeros past the slice), visible behind the next barrier
+      stage_store((s + 1) & 1, w_cur);  // block s + 1 (zeros past the slice), visible behind the next barrier
     };
     Step T[S];
-    stage_load(0, wr);
+    static_assert(S % WD == 0, "the loop's unrolling names the weight registers");
+    stage_load(0, wr[0]);
+    if constexpr (WD > 1) stage_load(1, wr[1]);
     if (active) {
 #pragma unroll
       for (int i = 0; i < S - 1; ++i) issue(i, T[i]);
     }
-    stage_store(0, wr);
+    stage_store(0, wr[0]);
     int s = 0;
     for (; s + S <= ns; s += S) {
 #pragma unroll
-      for (int i = 0; i < S; ++i) step(s + i, T[i], T[(i + S - 1) % S]);
+      for (int i = 0; i < S; ++i) step(s + i, T[i], T[(i + S - 1) % S], wr[(i + 1) % WD], wr[i % WD]);
     }
 #pragma unroll
     for (int i = 0; i < S - 1; ++i)
-      if (s + i < ns) step(s + i, T[i], T[(i + S - 1) % S]);  // block-uniform
+      if (s + i < ns) step(s + i, T[i], T[(i + S - 1) % S], wr[(i + 1) % WD], wr[i % WD]);  // block-uniform
     lds_barrier();  // the next run's first block goes into buffer 0
     if (!active) continue;
 #pragma unroll
@@ -385,7 +391,8 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
 }
 
 template <int NB>
-__global__ __launch_bounds__(256, 2) void k_shrink_quad(PassArgs a, const int32_t* __restrict__ tile_group,
+// (NB = 8: one block per CU, or the accumulators spill)
+__global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void k_shrink_quad(PassArgs a, const int32_t* __restrict__ tile_group,
                                                      const int32_t* __restrict__ slot_rows, int max_tiles) {
   shrink_quad_body<NB>(a, tile_group, slot_rows, max_tiles, blockIdx.x);
 }
@@ -983,18 +990,22 @@ __global__ __launch_bounds__(64) void k_wgrad_pipe(WgradArgs a, const ChunkInfo*
 // PAIRS: pairs of waves per block (1 or 2).  Two pairs take neighbouring column blocks of the same chunk: they load
 // the same h operands at about the same time, so the second pair's come from the CU's cache instead of from L2
 // (every 128-column block of a chunk re-reads the chunk's h: a third of this kernel's L2 reads at rank 64).
+// NB = 8 (rank 128): four waves share a tile, each with a quarter of the rank indices and of the tile's rows, so that the
+// accumulators stay at 64 registers per wave; the result is staged 16 rank indices at a time.
 template <int NB, int S, int PAIRS = 1>
 __device__ __forceinline__ void wgrad_coop_body(const WgradArgs& a, const ChunkInfo* __restrict__ chunks,
                                                 const int32_t* __restrict__ slot_rows, int bx, int by, int nx) {
-  constexpr int RS = 2, NBW = NB / 2;
+  constexpr int RS = NB == 8 ? 4 : 2, NBW = NB / RS, PR = 8 / RS;  // waves per tile, rank blocks and rows of each
+  constexpr int NBS = NB == 8 ? 1 : NBW;  // rank blocks a wave stages together
   constexpr int OS = kWgradStageStride;
   constexpr int XS = 136;  // row stride of a staged tile in bf16 (272 B)
   // the tile buffers are dead when the result is staged: one array serves both
-  constexpr int kLdsFloats = 16 * NB * OS > kTileRows * XS ? 16 * NB * OS : kTileRows * XS;  // >= two staged bf16 tiles
+  constexpr int kLdsFloats = 16 * RS * NBS * OS > kTileRows * XS ? 16 * RS * NBS * OS : kTileRows * XS;  // >= two staged bf16 tiles
   __shared__ __attribute__((aligned(16))) float lds_all[PAIRS * kLdsFloats];
   float* const lds = lds_all + (PAIRS > 1 ? (threadIdx.x >> 7) * kLdsFloats : 0);
   extern __shared__ __attribute__((aligned(16))) int32_t rows_s[];  // the chunk's row indices (same for both pairs)
-  const int tid = threadIdx.x & 127, lane = tid & 63, li = lane & 15, kb = lane >> 4, rs = tid >> 6;
+  static_assert(PAIRS == 1 || RS == 2, "");
+  const int tid = threadIdx.x & (64 * RS - 1), lane = tid & 63, li = lane & 15, kb = lane >> 4, rs = tid >> 6;
   if (by < a.tr.y_blocks) {  // side job: the first rows of the grid transpose the adapter weights
     transpose_weights_job(a.tr, a.rank, a.rpad, ((int64_t)by * nx + bx) * (RS * 64) + tid,
                           (int64_t)a.tr.y_blocks * nx * (RS * 64));
@@ -1031,17 +1042,17 @@ __device__ __forceinline__ void wgrad_coop_body(const WgradArgs& a, const ChunkI
     for (int nb = 0; nb < NBW; ++nb) acc[q][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   struct Piece {
-    uint4 x[4];      // rows 8 kb + 4 rs + i of the tile, columns 8 li .. 8 li + 7
+    uint4 x[PR];     // rows 8 kb + PR rs + i of the tile, columns 8 li .. 8 li + 7
     uint4 h[NBW];
     uint32_t live;
   };
   auto issue = [&](int t, Piece& P) {
     const int tc = min(t, nt - 1);
-    const int4 rr = *reinterpret_cast<const int4*>(rows_s + tc * kTileRows + 8 * kb + 4 * rs);
-    const int rows[4] = {rr.x, rr.y, rr.z, rr.w};
+    int rows[PR];
+    __builtin_memcpy(rows, __builtin_assume_aligned(rows_s + tc * kTileRows + 8 * kb + PR * rs, 4 * PR), 4 * PR);
     P.live = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < PR; ++i) {
       const int row = checked_row(rows[i], a.tb);
       P.x[i] = ld16(src + (int64_t)max(row, 0) * a.ld_src);
       P.live |= row >= 0 ? (1u << i) : 0u;
@@ -1052,8 +1063,8 @@ __device__ __forceinline__ void wgrad_coop_body(const WgradArgs& a, const ChunkI
   auto consume = [&](int t, const Piece& P) {
     bf16_t* buf = tiles + (t & 1) * (kTileRows * XS);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      st16(buf + (8 * kb + 4 * rs + i) * XS + 8 * li, (P.live >> i) & 1u ? P.x[i] : zero4());
+    for (int i = 0; i < PR; ++i)
+      st16(buf + (8 * kb + PR * rs + i) * XS + 8 * li, (P.live >> i) & 1u ? P.x[i] : zero4());
     lds_barrier();
     if (!mine) return;
     uint4 x[8];
@@ -1095,11 +1106,22 @@ __device__ __forceinline__ void wgrad_coop_body(const WgradArgs& a, const ChunkI
   for (int i = 0; i < S - 1; ++i)
     if (t + i < nt) consume(t + i, T[i]);
   __syncthreads();  // the last tile has been read everywhere: its buffer becomes the staging area
-  if (mine) wgrad_store<NBW>(acc, lds + n_base * OS, a, ci, g, r, c0, lane, n_base);
+  if constexpr (NBS == NBW) {
+    if (mine) wgrad_store<NBW>(acc, lds + n_base * OS, a, ci, g, r, c0, lane, n_base);
+  } else {
+#pragma unroll
+    for (int nb = 0; nb < NBW; ++nb) {
+      if (r <= n_base + 16 * nb) break;
+      f32x4 one[8][1];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) one[q][0] = acc[q][nb];
+      wgrad_store<1>(one, lds + rs * 16 * OS, a, ci, g, r, c0, lane, n_base + 16 * nb);
+    }
+  }
 }
 
 template <int NB, int S, int PAIRS>
-__global__ __launch_bounds__(128 * PAIRS) void k_wgrad_coop(WgradArgs a, const ChunkInfo* __restrict__ chunks,
+__global__ __launch_bounds__((NB == 8 ? 256 : 128) * PAIRS) void k_wgrad_coop(WgradArgs a, const ChunkInfo* __restrict__ chunks,
                                                               const int32_t* __restrict__ slot_rows) {
   wgrad_coop_body<NB, S, PAIRS>(a, chunks, slot_rows, blockIdx.x * PAIRS + (PAIRS > 1 ? threadIdx.x >> 7 : 0), blockIdx.y,
                                 gridDim.x * PAIRS);

@@ -538,6 +538,10 @@ int launch_opt_adamw(const tk_opt_tensor* tensors, int n_tensors, const tk_opt_t
                      int dtype, const float* clip, int flags, hipStream_t s);
 int64_t opt_partial_floats(int n_tensors, int64_t max_numel);
 
+// kernels_rank128.hip : the same at padded rank 128
+int launch_pass_rank128(const PassArgs& a, const SegView& seg, const SegLayout& L, int phases, hipStream_t s);
+int launch_wgrad_rank128(const WgradArgs& a, const SegView& seg, const SegLayout& L, hipStream_t s);
+
 // kernels_mfma.hip : bf16, aligned shapes, MFMA
 bool pass_mfma_supported(const PassArgs& a);
 // `phases` (bit mask): 1 = shrink, 2 = expand (h already written), 4 = only the last step of a split shrink
