@@ -145,3 +145,16 @@ def test_gradients_of_adapters_without_rows_are_zero(dev, max_r, ranks):
 def test_rank_128(dev, t, k, m, ranks):
     from test_gpu_lora import _run
     _run(dev, torch.bfloat16, *_problem(t, k, m, len(ranks), 128, ranks, seed=t + m))
+
+
+@pytest.mark.parametrize('t,k,m,ranks', [
+    (1, 1024, 128, [16]),                           # one row, two slices
+    (33, 1088, 256, [16, 5, 0]),                    # a last slice of one step, a dead adapter
+    (300, 4096, 1024, [16, 8, 1]),                  # eight slices; dy in two
+    (2500, 2048, 1152, [16, 16]),                   # few blocks for the shrink, too many readings for the expand
+    (2304, 2112, 384, [64, 40]),                    # rank 64, eight waves: slices that end in half a step
+    (2400, 1024, 512, [32, 20, 32]),                # ... and rank 32, runs of several groups in eight tiles
+])
+def test_few_tiles_and_slices(dev, t, k, m, ranks):
+    from test_gpu_lora import _run
+    _run(dev, torch.bfloat16, *_problem(t, k, m, len(ranks), max(ranks), ranks, seed=t + m))

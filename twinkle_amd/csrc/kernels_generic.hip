@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void k_shrink_any(PassArgs a, int slice_cols, 
                                                     const int32_t* __restrict__ slot_rows) {
   constexpr int E = Piece<T>::E, RP = 16 * NB;
   constexpr int NBS = NB < 4 ? NB : 4;  // rank blocks that leave through LDS together
-  constexpr int PF = NB == 1 ? 4 : (NB == 2 ? 2 : 1);
+  constexpr int PF = NB == 1 && sizeof(T) == 4 ? 4 : (NB <= 2 ? 2 : 1);  // a slice of 512 columns in one go
   __shared__ float part[4][kTileRows][16 * NBS + 1];
   const int nth = blockIdx.x / a.kslices, ks = blockIdx.x - nth * a.kslices;
   const int tile_id = checked_tile(work_item(a.wl_tiles, nth), a.tb);

@@ -37,13 +37,13 @@ __global__ __launch_bounds__(NW * 64) void k_shrink_pair_multi(PassJobs jobs, in
 
 // The same for up to kMaxShared projections that read the same source (see shared_source_item).
 template <int NB>
-__global__ __launch_bounds__(256, 2) void k_shrink_quad_multi(PassJobs jobs, int nproj, int items,
+__global__ __launch_bounds__(512) void k_shrink_oct_multi(PassJobs jobs, int nproj, int items,
                                                            const int32_t* __restrict__ tile_group,
                                                            const int32_t* __restrict__ slot_rows, int max_tiles) {
   int p, item;
   shared_source_item(blockIdx.x, nproj, p, item);
   if (item >= items) return;
-  shrink_quad_body<NB>(jobs.p[p], tile_group, slot_rows, max_tiles, item);
+  shrink_oct_body<NB>(jobs.p[p], tile_group, slot_rows, max_tiles, item);
 }
 
 // The same for up to kMaxShared projections of padded rank 16 in one launch: blockIdx.y selects the projection.
@@ -305,20 +305,34 @@ __global__ __launch_bounds__(256) void k_dy_fused_multi(DyFusedJobs jobs, const 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Few tiles at padded rank 16.  k_shrink_few: up to nine waves per CU (16 adapters of rank 16, 4096 columns, with the
+// sum of the slices, few against pair: 32 rows 7.0 / 9.1 us, 1024 8.7 / 10.1, 4096 14.4 / 15.7, 8192 21.0 / 20.2; 14336
+// columns: 1024 rows 16.9 / 18.0, 2048 21.5 / 21.5, 4096 33.1 / 30.6).
+constexpr int64_t kFewShrinkBlocks = 9 * 256;  // (tile, slice) pairs
+// The expand adds the slices itself up to 8192 readings of a tile's slice (2 KB each, from L2): a launch less, which is
+// what a small eager call is bound by (a decode step of 32 rows: 33 -> 30 us a pass).  On the GPU alone it is 0.5 us
+// faster at 32 rows x 4096 and slower from 256 rows on (by 0.5 us; 1.3 us at 1024).
+constexpr int64_t kFewFinishReads = 8192;
+
 template <int NB>
 void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int phases, hipStream_t s) {
   bf16_t* hrow = (bf16_t*)a.hT + (int64_t)a.rpad * a.ldh;  // second half of the h buffer
   const int32_t* rows = seg.slot_table(a.map_rows);
   constexpr int NW = NB == 1 ? 1 : (NB == 2 ? 2 : 4);  // shrink_waves(16 * NB)
   if (phases & 1) {
-    if (NB > 1 && a.quad_steps > 0)  // see shrink_plan
-      hipLaunchKernelGGL((k_shrink_quad<NB>), dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(256), 0, s,
+    if (NB > 1 && a.oct_steps > 0)  // see shrink_plan
+      hipLaunchKernelGGL((k_shrink_oct<NB == 1 ? 2 : NB>), dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(512), 0, s,
                          a, seg.tile_group, rows, (int)L.max_tiles);
+    else if (NB == 1 && L.max_tiles * a.kslices <= kFewShrinkBlocks)
+      hipLaunchKernelGGL(k_shrink_few, dim3((unsigned)(L.max_tiles * a.kslices)), dim3(64), 0, s, a, hrow, seg.tile_group,
+                         rows);
     else
       hipLaunchKernelGGL((k_shrink_pair<NB, NW>), dim3((unsigned)(ceil_div(L.max_tiles, 2) * a.kslices)),
                          dim3(NW * 64), 0, s, a, hrow, seg.tile_group, rows, (int)L.max_tiles);
   }
-  if ((phases & 5) && a.kslices > 1)
+  const bool fin = NB == 1 && (phases & 5) && (phases & 2) && a.dst && a.kslices > 1 && !a.class_mode &&
+                   L.max_tiles * (a.width_dst >> 7) * a.kslices <= kFewFinishReads;
+  if ((phases & 5) && a.kslices > 1 && !fin)
     hipLaunchKernelGGL((k_shrink_finish<NB>), dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group,
                        rows);
   if (!a.dst || !(phases & 2)) return;
@@ -333,8 +347,9 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
                        (int)std::min<int64_t>(L.sort_blocks, 64), (int)L.max_tiles);
   } else {
     const int64_t items = L.max_tiles * ngroups;
-    hipLaunchKernelGGL((k_expand_mfma<NB>), dim3((unsigned)ceil_div(items, 4)), dim3(256), 0, s, a, hrow,
-                       seg.tile_group, rows, seg.tile_walk(a.map_rows), (int)items);
+    const auto kernel = fin ? k_expand_mfma<NB, true> : k_expand_mfma<NB, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(items, 4)), dim3(256), 0, s, a, hrow, seg.tile_group, rows,
+                       seg.tile_walk(a.map_rows), (int)items);
   }
 }
 
@@ -463,15 +478,15 @@ int launch_shrink_multi(const PassArgs* a, int n, const SegView& seg, const SegL
   PassJobs J{};
   for (int p = 0; p < n; ++p) J.p[p] = a[p];
   const int32_t* rows = seg.slot_table(a[0].map_rows);
-  const bool quad = a[0].quad_steps > 0;
+  const bool quad = a[0].oct_steps > 0;
   const int items = (int)(ceil_div(L.max_tiles, quad ? 8 : 2) * a[0].kslices);
   const dim3 grid((unsigned)(ceil_div(items, 8) * 8 * n));
   if (quad) {  // the single-projection launch makes the same choice: same sums, same bits
     if (a[0].rpad <= 32)
-      hipLaunchKernelGGL((k_shrink_quad_multi<2>), grid, dim3(256), 0, s, J, n, items, seg.tile_group, rows,
+      hipLaunchKernelGGL((k_shrink_oct_multi<2>), grid, dim3(512), 0, s, J, n, items, seg.tile_group, rows,
                          (int)L.max_tiles);
     else
-      hipLaunchKernelGGL((k_shrink_quad_multi<4>), grid, dim3(256), 0, s, J, n, items, seg.tile_group, rows,
+      hipLaunchKernelGGL((k_shrink_oct_multi<4>), grid, dim3(512), 0, s, J, n, items, seg.tile_group, rows,
                          (int)L.max_tiles);
   } else if (a[0].rpad <= 32) {
     hipLaunchKernelGGL((k_shrink_pair_multi<2, 2>), grid, dim3(128), 0, s, J, n, items, seg.tile_group, rows,

@@ -7,7 +7,7 @@
 // wave-wide load covers whole 128-byte lines and every activation byte crosses
 // HBM once per pass.
 //
-//   k_shrink_pair / k_shrink_quad / k_shrink_finish   h = scale * x A^T (split over column slices when x is wide)
+//   k_shrink_pair / k_shrink_oct / k_shrink_finish    h = scale * x A^T (split over column slices when x is wide)
 //   k_expand_mfma / k_expand_multi                     y += h B^T in place (rank <= 16 / above)
 //   k_wgrad_pipe / k_wgrad_coop                        dA, dB: contraction over the rows of a chunk (rank <= 16 / above)
 //   transpose_weights_job                              B^T, A^T copies for the backward shrink / expand
@@ -103,11 +103,11 @@ __device__ inline void shrink_epilogue(const float* part, int planes, const Pass
 // twice: slot-major (hrow, the expand kernel's A operand) and rank-major (hT, read by the
 // weight-gradient kernels); padding slots get exact zeros.
 // ---------------------------------------------------------------------------
-template <int NB, int NW, int TT>
+// PF: steps whose loads are issued together
+template <int NB, int NW, int TT, int PF = 2>
 __device__ inline void shrink_tiles(const PassArgs& a, bf16_t* __restrict__ hrow, const int32_t* __restrict__ slot_rows,
                                     const int (&tiles)[TT], int g, int ks, float (*part)[kTileRows][16 * NB + 1]) {
   constexpr int RP = 16 * NB;
-  constexpr int PF = 2;  // steps whose loads are issued together
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
   const bf16_t* src = (const bf16_t*)a.src;
   const bf16_t *xa[TT], *xb[TT];
@@ -164,6 +164,7 @@ __device__ inline void shrink_tiles(const PassArgs& a, bf16_t* __restrict__ hrow
         w1[j][nb] = (wv[nb] && ok) ? ld16(wp[nb] + c + 8) : zero4();
       }
     }
+    if constexpr (PF == kShrinkSteps) __builtin_amdgcn_sched_barrier(0);  // (or the loads are spread over the products)
 #pragma unroll
     for (int j = 0; j < PF; ++j)
 #pragma unroll
@@ -238,30 +239,46 @@ __global__ __launch_bounds__(NW * 64) void k_shrink_pair(PassArgs a, bf16_t* __r
   shrink_pair_body<NB, NW>(a, hrow, tile_group, slot_rows, max_tiles, blockIdx.x);
 }
 
+// The shrink of few tiles at padded rank 16: one wave per (tile, slice) requests its whole slice, eight steps, at once.
+// There are too few blocks to cover latencies with each other, so the launch takes as long as one block, and that as
+// many memory latencies as it has batches (five with k_shrink_pair's).  Same products in the same order: same bits.
+__global__ __launch_bounds__(64) void k_shrink_few(PassArgs a, bf16_t* __restrict__ hrow,
+                                                   const int32_t* __restrict__ tile_group,
+                                                   const int32_t* __restrict__ slot_rows) {
+  __shared__ float part[1][kTileRows][17];
+  const int nth = blockIdx.x / a.kslices, ks = blockIdx.x - nth * a.kslices;
+  const int tile = checked_tile(work_item(a.wl_tiles, nth), a.tb);
+  if (tile < 0) return;
+  const int g = checked_group(tile_group[tile], a.tb);
+  if (g < 0) return;
+  const int tiles[1] = {tile};
+  shrink_tiles<1, 1, 1, kShrinkSteps>(a, hrow, slot_rows, tiles, g, ks, part);
+}
+
 // ---------------------------------------------------------------------------
 // Shrink with the weights shared through LDS, for groups of many tiles.  In k_shrink_pair every wave fetches the
 // weight columns of its own steps, 16 * NB rank indices for 64 rows: at rank 64 as many bytes of weights (from L2)
 // as of activations (from memory), and the two share the path between L2 and the CUs, which is what sets the pace
-// (measured at rank 64: 536 MB of L2 reads for 268 MB of activations, 7.6 TB/s together).  Here a block of four
-// waves owns (eight consecutive tiles, slice of 64 * STEPS columns): wave w takes tiles 2 w and 2 w + 1 of the
-// eight through all steps, and the weight block of a step (16 * NB x 64) is fetched once per block, 16 B per
-// thread, into a double-buffered LDS tile from which every wave reads its MFMA operands: a quarter of the weight
-// traffic.  One LDS-only barrier per step: a buffer is overwritten one step after the barrier behind its last
-// reader.  The eight tiles are taken in runs of equal group (almost always one run); waves whose tiles lie
-// outside the run still help to stage the weights.  The slice length (a.quad_steps) is chosen per launch.  Activations: three steps in registers per wave, loads two
-// steps ahead.  Every block leaves its sums as one slice of the split-shrink buffer (k_shrink_finish follows);
-// each entry is the sum of one wave's MFMA chain, so results do not depend on timing.
+// (measured at rank 64: 536 MB of L2 reads for 268 MB of activations, 7.6 TB/s together).  Here a block of eight
+// waves owns (eight consecutive tiles, slice of columns): wave w takes tile w through all steps of 128 columns, and
+// the weight block of a step (16 * NB x 128) is fetched once per block, 16 B per thread and piece, into a
+// double-buffered LDS tile from which every wave reads its MFMA operands.  One LDS-only barrier per step: a buffer is
+// overwritten one step after the barrier behind its last reader.  The eight tiles are taken in runs of equal group
+// (almost always one run); waves whose tile lies outside the run still help to stage the weights.  What bounds it is
+// memory latency: a wave keeps S - 1 steps (8 KB each: 256 contiguous bytes of 32 rows) in flight and the weights are
+// requested two steps ahead.  (Four waves of two tiles and 64 columns a step before, 128 bytes of a row at a time:
+// 6000 x 4096 at rank 64 28 against 20 us, 32768 x 4096 about 80 both, 3.5 TB/s of source.)  Every block leaves its sums as one slice of the split-shrink buffer (k_shrink_finish
+// follows); each entry is the sum of one wave's MFMA chain, so results do not depend on timing.
 // ---------------------------------------------------------------------------
 template <int NB>
-__device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_t* __restrict__ tile_group,
-                                                 const int32_t* __restrict__ slot_rows, int max_tiles, int item) {
+__device__ __forceinline__ void shrink_oct_body(const PassArgs& a, const int32_t* __restrict__ tile_group,
+                                                const int32_t* __restrict__ slot_rows, int max_tiles, int item) {
   constexpr int RP = 16 * NB;
-  constexpr int WS = 72;                    // row stride of a staged weight block in bf16 (144 B: conflict-free)
-  constexpr int NLD = (RP * 8 + 255) / 256;  // 16-byte pieces of a weight block per thread
-  constexpr int S = NB >= 4 ? 2 : 3;  // steps of activations in registers (from rank 64 on the accumulators take the room)
-  // steps the weights are requested ahead: at rank 128 one block of four waves has a CU to itself, and nothing else
-  // covers the latency of its 16 KB of weights per step
-  constexpr int WD = NB == 8 ? 2 : 1;
+  constexpr int WS = 136;             // row stride of a staged weight block in bf16 (272 B: conflict-free)
+  constexpr int NLD = RP * 16 / 512;  // 16-byte pieces of a weight block per thread
+  constexpr int S = NB == 8 ? 2 : (NB == 4 ? 3 : 4);  // steps of activations in registers (above, the accumulators take the room)
+  constexpr int WD = S == 3 ? 3 : 2;  // steps the weights are requested ahead
+  static_assert(NB >= 2 && S % WD == 0, "the loop's unrolling names the weight registers");
   __shared__ __attribute__((aligned(16))) bf16_t wbuf[2][RP * WS];
   __shared__ int32_t gts[8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
@@ -270,20 +287,18 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
   if (set < 0) return;  // past the end of this rank class's list (uniform over the block)
   const int t_first = set * 8;
   if (tid < 8) gts[tid] = t_first + tid < max_tiles ? checked_group(tile_group[t_first + tid], a.tb) : -1;
-  const int nsteps = a.width_src >> 6;
-  const int s0 = ks * a.quad_steps;
-  const int ns = min(a.quad_steps, nsteps - s0);  // >= 1 for every slice
-  // this wave's two tiles
-  const bf16_t* src = (const bf16_t*)a.src;
-  const bf16_t *xa[2], *xb[2];
+  const int s0 = ks * a.oct_steps;                                 // in 64-column steps
+  const int n64 = min(a.oct_steps, (a.width_src >> 6) - s0);       // >= 1 for every slice
+  const int ns = (n64 + 1) >> 1;                                   // steps of 128 columns, the last perhaps half
+  // this wave's tile
+  const bf16_t* x_row[2];
+  {
+    const int t = min(t_first + wave, max_tiles - 1);
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int t = min(t_first + 2 * wave + u, max_tiles - 1);
-    int ra = slot_rows[t * kTileRows + li], rb = slot_rows[t * kTileRows + 16 + li];
-    ra = min(max(ra, 0), a.src_rows - 1);
-    rb = min(max(rb, 0), a.src_rows - 1);
-    xa[u] = src + (int64_t)ra * a.ld_src + 16 * kb + (int64_t)s0 * 64;
-    xb[u] = src + (int64_t)rb * a.ld_src + 16 * kb + (int64_t)s0 * 64;
+    for (int tt = 0; tt < 2; ++tt) {
+      const int row = min(max(slot_rows[t * kTileRows + 16 * tt + li], 0), a.src_rows - 1);
+      x_row[tt] = (const bf16_t*)a.src + (int64_t)row * a.ld_src + 16 * kb + (int64_t)s0 * 64;
+    }
   }
   __syncthreads();
   for (int j = 0; j < 8;) {
@@ -295,72 +310,70 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
     if (g < 0) continue;
     const int r = class_rank(a.rank[g], a.rank_lo, RP);
     if (r <= 0) continue;  // adapter not live on this layer, or a group of another rank class
-    bool mine[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) mine[u] = 2 * wave + u >= lo && 2 * wave + u < hi;
-    const bool active = mine[0] || mine[1];  // wave-uniform
+    const bool active = wave >= lo && wave < hi;  // wave-uniform
     const bf16_t* W1 = group_weight<bf16_t>(a.w_shrink, a.w_shrink_base, a.shrink_group_stride, g) + (int64_t)s0 * 64;
-    // staging: piece p = tid + 256 i is columns 8 (p % 8) .. + 8 of rank index p / 8
+    // staging: piece p = tid + 512 i is columns 8 (p % 16) .. + 8 of rank index p / 16
     auto stage_load = [&](int s, uint4 (&wr)[NLD]) {
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
-        const int p = tid + 256 * i, n = p >> 3;
-        wr[i] = (n < r && s < ns) ? ld16(W1 + (int64_t)n * a.ld_shrink + (s << 6) + 8 * (p & 7)) : zero4();
+        const int p = tid + 512 * i, n = p >> 4, c = (s << 7) + 8 * (p & 15);
+        wr[i] = (n < r && c < (n64 << 6)) ? ld16(W1 + (int64_t)n * a.ld_shrink + c) : zero4();
       }
     };
     auto stage_store = [&](int buf, const uint4 (&wr)[NLD]) {
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
-        const int p = tid + 256 * i, n = p >> 3;
-        if (n < RP) st16(&wbuf[buf][n * WS + 8 * (p & 7)], wr[i]);
+        const int p = tid + 512 * i;
+        st16(&wbuf[buf][(p >> 4) * WS + 8 * (p & 15)], wr[i]);
       }
     };
     struct Step {
-      uint4 x0[2][2], x1[2][2];
+      uint4 x[2][2][2];  // [half of 64 columns][piece][16 rows]
     };
     auto issue = [&](int s, Step& X) {
-      const int c = min(s, ns - 1) << 6;  // requests past the slice repeat its last step and are not used
+      // (steps past the slice repeat its last one, a half past its end the half in front: requested and not used)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        X.x0[u][0] = ld16(xa[u] + c);
-        X.x1[u][0] = ld16(xa[u] + c + 8);
-        X.x0[u][1] = ld16(xb[u] + c);
-        X.x1[u][1] = ld16(xb[u] + c + 8);
+      for (int hf = 0; hf < 2; ++hf) {
+        const int c = min(2 * s + hf, n64 - 1) << 6;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) X.x[hf][p][tt] = ld16(x_row[tt] + c + 8 * p);
       }
     };
-    f32x4 acc[2][2][NB];
+    f32x4 acc[2][NB];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[u][tt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     uint4 wr[WD][NLD];
-    // (w_cur: the weights of step s + 1, w_next: where those of step s + WD go; one and the same for WD = 1)
+    // (w_cur: the weights of step s + 1, w_next: where those of step s + WD go)
     auto step = [&](int s, const Step& X, Step& Xnext, const uint4 (&w_cur)[NLD], uint4 (&w_next)[NLD]) {
       lds_barrier();  // block s is complete; the other buffer has been read by everyone
       stage_load(s + WD, w_next);
-      if (active) issue(s + S - 1, Xnext);
       if (active) {
+        issue(s + S - 1, Xnext);
         const bf16_t* wb = wbuf[s & 1] + li * WS + 16 * kb;
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const uint4 w0 = ld16(wb + 16 * nb * WS), w1 = ld16(wb + 16 * nb * WS + 8);
+        for (int hf = 0; hf < 2; ++hf) {
+          if (hf && 2 * s + 1 >= n64) break;
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
+          for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-              acc[u][tt][nb] = mfma16(X.x0[u][tt], w0, acc[u][tt][nb]);
-              acc[u][tt][nb] = mfma16(X.x1[u][tt], w1, acc[u][tt][nb]);
+            for (int p = 0; p < 2; ++p) {
+              const uint4 w = ld16(wb + 16 * nb * WS + 64 * hf + 8 * p);
+#pragma unroll
+              for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mfma16(X.x[hf][p][tt], w, acc[tt][nb]);
             }
+          __builtin_amdgcn_sched_barrier(0);  // (reading the weights further ahead costs registers: spills)
         }
       }
       stage_store((s + 1) & 1, w_cur);  // block s + 1 (zeros past the slice), visible behind the next barrier
     };
     Step T[S];
-    static_assert(S % WD == 0, "the loop's unrolling names the weight registers");
     stage_load(0, wr[0]);
-    if constexpr (WD > 1) stage_load(1, wr[1]);
+    stage_load(1, wr[1]);
+    if constexpr (WD > 2) stage_load(2, wr[2]);
     if (active) {
 #pragma unroll
       for (int i = 0; i < S - 1; ++i) issue(i, T[i]);
@@ -376,25 +389,20 @@ __device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_
       if (s + i < ns) step(s + i, T[i], T[(i + S - 1) % S], wr[(i + 1) % WD], wr[i % WD]);  // block-uniform
     lds_barrier();  // the next run's first block goes into buffer 0
     if (!active) continue;
+    float* out = a.hpart + ((int64_t)(t_first + wave) * a.kslices + ks) * (kTileRows * RP) + 4 * kb * RP + li;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (!mine[u]) continue;
-      float* out = a.hpart + ((int64_t)(t_first + 2 * wave + u) * a.kslices + ks) * (kTileRows * RP) + 4 * kb * RP + li;
+    for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) out[(16 * tt + v) * RP + 16 * nb] = acc[u][tt][nb][v];
-    }
+        for (int v = 0; v < 4; ++v) out[(16 * tt + v) * RP + 16 * nb] = acc[tt][nb][v];
   }
 }
 
 template <int NB>
-// (NB = 8: one block per CU, or the accumulators spill)
-__global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void k_shrink_quad(PassArgs a, const int32_t* __restrict__ tile_group,
-                                                     const int32_t* __restrict__ slot_rows, int max_tiles) {
-  shrink_quad_body<NB>(a, tile_group, slot_rows, max_tiles, blockIdx.x);
+__global__ __launch_bounds__(512) void k_shrink_oct(PassArgs a, const int32_t* __restrict__ tile_group,
+                                                    const int32_t* __restrict__ slot_rows, int max_tiles) {
+  shrink_oct_body<NB>(a, tile_group, slot_rows, max_tiles, blockIdx.x);
 }
 
 // Adds the slices of a split shrink in slice order and writes h (one block per tile).
@@ -465,7 +473,9 @@ __global__ __launch_bounds__(256) void k_shrink_finish(PassArgs a, bf16_t* __res
 // from the start of the wave.  (Used for padded rank 16; above that
 // k_expand_multi shares the weight block between tiles.)
 // ---------------------------------------------------------------------------
-template <int NB>
+// FIN: the slices of a split shrink are added here, by every wave for its tile (NB = 1), and the wave of the first
+// columns writes h: for launches of few tiles (see kFewFinishReads).  Same sums, same rounding as k_shrink_finish.
+template <int NB, bool FIN = false>
 __device__ __forceinline__ void expand_flat_body(const PassArgs& a, const bf16_t* __restrict__ hrow,
                                                  const int32_t* __restrict__ tile_group,
                                                  const int32_t* __restrict__ slot_rows,
@@ -499,9 +509,51 @@ __device__ __forceinline__ void expand_flat_body(const PassArgs& a, const bf16_t
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
       const int n0 = 32 * ks + 8 * kb;
-      hop[tt][ks] = n0 < RP ? ld16(hrow + (int64_t)(slot0 + 16 * tt + li) * RP + n0) : zero4();
+      if constexpr (!FIN) hop[tt][ks] = n0 < RP ? ld16(hrow + (int64_t)(slot0 + 16 * tt + li) * RP + n0) : zero4();
     }
   const int g = max(g_raw, 0);
+  if constexpr (FIN) {
+    static_assert(NB == 1, "one operand step");
+    const int r = g_raw < 0 ? 0 : class_rank(a.rank[g], a.rank_lo, RP);
+    const float sc = a.scale[g];
+    const bool first = item - nth * ngroups == 0;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const int slot = slot0 + 16 * tt + li;
+      const bool real = kb < 2 && r > 0 && slot_rows[slot] >= 0;
+      const float* p = a.hpart + (int64_t)tile_id * a.kslices * (kTileRows * RP) + (16 * tt + li) * RP + 8 * (kb & 1);
+      float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int k0 = 0; k0 < a.kslices; k0 += 4) {  // four slices are requested together and added in slice order
+        float4 v[4][2];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            v[k][q] = real && k0 + k < a.kslices
+                          ? *reinterpret_cast<const float4*>(p + (int64_t)(k0 + k) * (kTileRows * RP) + 4 * q)
+                          : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            sum[4 * q] += v[k][q].x;
+            sum[4 * q + 1] += v[k][q].y;
+            sum[4 * q + 2] += v[k][q].z;
+            sum[4 * q + 3] += v[k][q].w;
+          }
+      }
+      hop[tt][0] = real ? make_uint4(pack_bf16(sum[0] * sc, sum[1] * sc), pack_bf16(sum[2] * sc, sum[3] * sc),
+                                     pack_bf16(sum[4] * sc, sum[5] * sc), pack_bf16(sum[6] * sc, sum[7] * sc))
+                        : zero4();
+      if (first && kb < 2 && r > 0) {
+        st16(const_cast<bf16_t*>(hrow) + (int64_t)slot * RP + 8 * kb, hop[tt][0]);
+        const uint32_t w[4] = {hop[tt][0].x, hop[tt][0].y, hop[tt][0].z, hop[tt][0].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          ((bf16_t*)a.hT)[(int64_t)(8 * kb + i) * a.ldh + slot] = (bf16_t)(w[i >> 1] >> (16 * (i & 1)));
+      }
+    }
+  }
   const int rows[2][4] = {{r0.x, r0.y, r0.z, r0.w}, {r1.x, r1.y, r1.z, r1.w}};
   bool rok[2][4];
   bf16_t* yp[2][4];
@@ -553,12 +605,12 @@ __device__ __forceinline__ void expand_flat_body(const PassArgs& a, const bf16_t
   }
 }
 
-template <int NB>
+template <int NB, bool FIN>
 __global__ __launch_bounds__(256) void k_expand_mfma(PassArgs a, const bf16_t* __restrict__ hrow,
                                                      const int32_t* __restrict__ tile_group,
                                                      const int32_t* __restrict__ slot_rows,
                                                      const int32_t* __restrict__ tile_walk, int num_items) {
-  expand_flat_body<NB>(a, hrow, tile_group, slot_rows, tile_walk, num_items, blockIdx.x);
+  expand_flat_body<NB, FIN>(a, hrow, tile_group, slot_rows, tile_walk, num_items, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
