@@ -727,7 +727,7 @@ static int lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const v
     SegLayout L(d->rows, d->num_groups);
     SegView V(d->seg_ws, L);
     int rc = build_lists(P, d, (char*)ws + P.ws_core_total, V, L, (hipStream_t)stream);
-    if (rc == TK_OK && store_dx && dx)
+    if (rc == TK_OK && store_dx && dx && P.n > 1)  // (one class: the expand clears the rows of no live group)
       rc = launch_zero_rows(dx, lddx, d->in_features, d->dtype, d->rank, d->max_rank, d->map_rows, V, L,
                             (hipStream_t)stream);
     if (rc != TK_OK) return rc;

@@ -256,13 +256,24 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
   const int g = checked_group(tile_group[tile_id], a.tb);
   const int4 r0 = *reinterpret_cast<const int4*>(slot_rows + slot0 + 4 * kb);
   const int4 r1 = *reinterpret_cast<const int4*>(slot_rows + slot0 + 16 + 4 * kb);
-  if (g < 0) return;
-  const int r = class_rank(a.rank[g], a.rank_lo, RP);
-  if (r <= 0) return;
+  const int r = g < 0 ? 0 : class_rank(a.rank[g], a.rank_lo, RP);
   const int rows[2][4] = {{r0.x, r0.y, r0.z, r0.w}, {r1.x, r1.y, r1.z, r1.w}};
   const int c = (item - nth * ngroups) * (16 * E) + E * li;  // this lane's columns
   const int keep = min(E, a.width_dst - c);                  // <= 0: none
   T* dst = (T*)a.dst + c;
+  if (r <= 0) {
+    if (a.dst_store && !a.class_mode) {  // no live group: zeros (several classes: launch_zero_rows)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = checked_row(rows[tt][v], a.tb);
+          for (int q = 0; q < E && row >= 0; ++q)
+            if (q < keep) dst[(int64_t)row * a.ld_dst + q] = (T)0;
+        }
+    }
+    return;
+  }
   const T* W = group_weight<T>(a.w_expand, a.w_expand_base, a.expand_group_stride, g);
   const T* h = (const T*)a.hT + (int64_t)a.rpad * a.ldh + (int64_t)slot0 * RP;
   uint4 y[2][4];
@@ -330,7 +341,8 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
     }
 }
 
-// Zeros in the rows whose group is not live, next to an expand that writes the others instead of adding onto them.
+// Zeros in the rows whose group is not live, next to the expands of several rank classes that write the others instead
+// of adding onto them (with one class the expand does it).
 template <typename T>
 __global__ __launch_bounds__(256) void k_zero_rows(T* dst, int64_t ld, int width, const int32_t* __restrict__ rank,
                                                    int max_rank, TableBounds tb, const int32_t* __restrict__ tile_group,
@@ -812,8 +824,12 @@ int launch_convert_weights(const tk_lora_desc& d, void* stage, bool want_a, bool
 namespace {
 
 template <typename T, int NB>
-void launch_pass_any(const PassArgs& a, const SegView& seg, const SegLayout& L, int phases, hipStream_t s) {
+void launch_pass_any(const PassArgs& a0, const SegView& seg, const SegLayout& L, int phases, hipStream_t s) {
   constexpr int E = Piece<T>::E;
+  // A source of up to 1536 columns is walked by one block per tile: its waves take two or three times the steps (6.5 ->
+  // 8 us for 512 x 1024 in fp32), which costs less than the launch that would add the slices (4 us)
+  PassArgs a = a0;
+  if (a.kslices <= 3 && a.width_src <= 1536) a.kslices = 1;
   const int32_t* rows = seg.slot_table(a.map_rows);
   if (phases & 1) {
     // the slices of the split shrink's plan (its buffer holds kslices slices of every tile)

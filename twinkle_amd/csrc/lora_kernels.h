@@ -581,7 +581,17 @@ __device__ __forceinline__ void expand_flat_body(const PassArgs& a, const bf16_t
       const int wrow = a.expand_swizzled ? c0 + 16 * q + li : c0 + 8 * li + q;
       bq[q][ks] = n0 < r ? keep_first(ld16(W2 + (int64_t)wrow * a.ld_expand + n0), r - n0) : zero4();
     }
-  if (r <= 0) return;  // unused tile, or adapter not live on this layer (uniform over the wave)
+  if (r <= 0) {  // unused tile, or adapter not live on this layer (uniform over the wave)
+    if (a.dst_store && !a.class_mode) {  // (several classes: launch_zero_rows)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (checked_row(rows[tt][v], a.tb) >= 0)
+            st16_nt((bf16_t*)a.dst + (int64_t)rows[tt][v] * a.ld_dst + 8 * li + c0, zero4());
+    }
+    return;
+  }
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) {
     f32x4 d[8];
@@ -773,6 +783,19 @@ __global__ __launch_bounds__(256) void k_expand_multi(PassArgs a, const bf16_t* 
       }
     }
   };
+  // the rows of a tile that has no live group (one class: nobody else writes them)
+  auto zero_tile = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = checked_row(slot_rows[(tile0 + t) * kTileRows + 8 * kb + i], a.tb);
+      if (row >= 0) st16_nt(dst + (int64_t)row * a.ld_dst, zero4());
+    }
+  };
+  if constexpr (STORE && !CLS) {
+#pragma unroll
+    for (int t = 0; t < TPI; ++t)
+      if (t < nt && gt[t] < 0) zero_tile(t);
+  }
   // tiles past the last one of the table carry -1 and come last
   bool uniform = true;
 #pragma unroll
@@ -784,7 +807,11 @@ __global__ __launch_bounds__(256) void k_expand_multi(PassArgs a, const bf16_t* 
 #pragma unroll
     for (int t = 0; t < TPI; ++t) nv += gt[t] >= 0;
     load_weights(gt[0]);
-    if (r <= 0) return;  // adapter not live on this layer
+    if (r <= 0) {  // adapter not live on this layer
+      if constexpr (STORE && !CLS)
+        for (int t = 0; t < nv; ++t) zero_tile(t);
+      return;
+    }
     issue(0, A);
     for (int t = 0; t < nv; t += 2) {
       issue(t + 1 < nv ? t + 1 : nt, B);
@@ -799,7 +826,10 @@ __global__ __launch_bounds__(256) void k_expand_multi(PassArgs a, const bf16_t* 
   for (int t = 0; t < nt; ++t) {  // a group boundary inside the item: tile by tile
     if (gt[t] < 0) continue;
     load_weights(gt[t]);
-    if (r <= 0) continue;
+    if (r <= 0) {
+      if constexpr (STORE && !CLS) zero_tile(t);
+      continue;
+    }
     issue(t, A);
     consume(A);
   }

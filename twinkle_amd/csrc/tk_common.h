@@ -375,7 +375,8 @@ struct PassArgs {
   // groups whose rank is not in (rank_lo, rpad] are skipped (see class_rank); class_mode != 0 says that such groups
   // may exist, and kernels then look at the rank before they request a tile's rows
   int32_t rank_lo, class_mode;
-  // 1: rows are written (dst = h W2^T) instead of added onto; the rows of no live group are left to launch_zero_rows
+  // 1: rows are written (dst = h W2^T, zeros in the rows of no live group) instead of added onto; with class_mode
+  // those zeros are left to launch_zero_rows
   int32_t dst_store;
   WorkList wl_tiles, wl_pairs, wl_octs, wl_sets;  // class_mode: the items of this class (see WorkList)
   TableBounds tb;
