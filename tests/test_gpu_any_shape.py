@@ -158,3 +158,38 @@ def test_rank_128(dev, t, k, m, ranks):
 def test_few_tiles_and_slices(dev, t, k, m, ranks):
     from test_gpu_lora import _run
     _run(dev, torch.bfloat16, *_problem(t, k, m, len(ranks), max(ranks), ranks, seed=t + m))
+
+
+@pytest.mark.parametrize('k', [1001, 513, 1004])
+@pytest.mark.parametrize('t,m,ranks', [
+    (300, 256, [16, 5]),                            # padded rank 16: one class
+    (300, 640, [32, 20]),
+    (300, 384, [64, 33]),
+    (300, 256, [128, 100]),
+    (900, 640, [128, 64, 20, 8]),                   # every rank class
+])
+def test_dx_of_an_odd_width_behind_an_aligned_dy(dev, t, k, m, ranks):
+    """dy suits the MFMA row contraction, which can carry the transposed weight copies in blocks of 8 x 8 features; the
+    input width does not, so those copies have to reach its last columns some other way.  The workspace holds NaN."""
+    from twinkle_amd import lora_bwd_workspace_bytes
+    from twinkle_amd.ops import _lora_bwd
+    bf16 = torch.bfloat16
+    x, base, dy, a, b, ids, _, scales = _problem(t, k, m, len(ranks), max(ranks), ranks, seed=t + k)
+    xd, yd, dyd = (v.to(bf16).to(dev) for v in (x, base, dy))
+    ad, bd = [w.to(bf16).to(dev) for w in a], [w.to(bf16).to(dev) for w in b]
+    seg = build_segments(ids.to(torch.int32).to(dev), len(ranks), check=True)
+    groups = AdapterGroups(ad, bd, ranks, scales)
+    h = lora_fwd_(xd, yd, seg, groups)
+    f64 = lambda v: v.to(bf16).double()  # noqa: E731
+    _, dxo, dao, dbo = oracle.multi_lora_linear_grads(f64(x), f64(base), ids, [f64(w) for w in a], [f64(w) for w in b],
+                                                      ranks, scales, f64(dy))
+    for entry, start in (('tk_lora_bwd', 0.0), ('tk_lora_bwd_store', float('nan'))):
+        dxd = torch.full_like(xd, start)
+        ws = torch.full((lora_bwd_workspace_bytes(seg, groups),), 255, dtype=torch.uint8, device=dev)
+        ga, gb = [torch.zeros_like(w) for w in ad], [torch.zeros_like(w) for w in bd]
+        pa, pb = (torch.tensor([w.data_ptr() for w in g], dtype=torch.int64, device=dev) for g in (ga, gb))
+        _lora_bwd(entry, dyd, xd, h, dxd, pa, pb, seg, groups, workspace=ws)
+        assert max_rel_err(dxd, dxo) < TOL[bf16], entry
+        for g in range(len(ranks)):
+            assert max_rel_err(ga[g], dao[g]) < TOL[bf16], f'dA[{g}]'
+            assert max_rel_err(gb[g], dbo[g]) < TOL[bf16], f'dB[{g}]'

@@ -671,7 +671,9 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   do {
     bool wT_done = false;
     if (grad_B) {
-      if (!side && need_wT && mfma && wgrad_mfma_supported(gb) && d->out_features % 8 == 0) {
+      // (the copies are made in blocks of 8 x 8 features: an input width that ends inside one is left to
+      // launch_transpose_weights, or the last columns of dx would be products with rows nobody wrote)
+      if (!side && need_wT && mfma && wgrad_mfma_supported(gb) && d->out_features % 8 == 0 && d->in_features % 8 == 0) {
         gb.tr = tr;  // one stream: the MFMA launch also writes the transposed weight copies of the pass below
         wT_done = true;
       }
