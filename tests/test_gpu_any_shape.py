@@ -193,3 +193,25 @@ def test_dx_of_an_odd_width_behind_an_aligned_dy(dev, t, k, m, ranks):
         for g in range(len(ranks)):
             assert max_rel_err(ga[g], dao[g]) < TOL[bf16], f'dA[{g}]'
             assert max_rel_err(gb[g], dbo[g]) < TOL[bf16], f'dB[{g}]'
+
+
+@pytest.mark.parametrize('r,r2', [(65, 64), (71, 3), (100, 99), (124, 17), (127, 8)])
+def test_lora_b_as_columns_that_end_with_their_buffer(dev, r, r2):
+    """Above rank 64 adapters may lie at any element address: B_g = the last r columns of a buffer whose row stride the
+    MFMA kernels take.  The operand pieces of the last row then end with the buffer, also of a smaller rank."""
+    t, k, m = 300, 128, 256
+    x, base, dy, a, b, ids, _, scales = _problem(t, k, m, 2, r, [r, r2], seed=r)
+    bf16, f64 = torch.bfloat16, lambda v: v.to(torch.bfloat16).double()  # noqa: E731
+    ld = (r + 15) // 8 * 8
+    bd = []
+    for w in b:
+        wide = torch.full((m, ld), float('nan'), dtype=bf16, device=dev)
+        wide[:, ld - r:] = w.to(bf16).to(dev)
+        bd.append(wide[:, ld - r:])
+    groups = AdapterGroups([w.to(bf16).to(dev) for w in a], bd, [r, r2], scales)
+    seg = build_segments(ids.to(torch.int32).to(dev), 2, check=True)
+    yd = base.to(bf16).to(dev)
+    lora_fwd_(x.to(bf16).to(dev), yd, seg, groups)
+    yo, *_ = oracle.multi_lora_linear_grads(f64(x), f64(base), ids, [f64(w) for w in a], [f64(w) for w in b], [r, r2],
+                                            scales, f64(dy))
+    assert max_rel_err(yd, yo) < TOL[bf16]

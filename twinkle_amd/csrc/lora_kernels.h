@@ -737,9 +737,34 @@ __global__ __launch_bounds__(256) void k_expand_multi(PassArgs a, const bf16_t* 
   };
   uint4 bq[8][NKS];
   int r = 0;
+  // Above rank 64 adapters may lie at any element address: a piece that the rank cuts may then reach past the matrix's
+  // last row, behind which there need be nothing to read, so the rows q = 7 are read element by element.  (Copies inside
+  // a workspace, the only weights of the writing form, are aligned: there a piece ends where an aligned 16 bytes end.)
+  auto load_cut_weights = [&](const bf16_t* W2) {
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int n0 = 32 * ks + 8 * kb;
+      const bf16_t* p = W2 + (int64_t)(c0 + 8 * li) * a.ld_expand + n0;
+#pragma unroll
+      for (int q = 0; q < 7; ++q) bq[q][ks] = n0 < r ? keep_first(ld16(p + q * a.ld_expand), r - n0) : zero4();
+      uint64_t lo = 0, hi = 0;
+#pragma unroll 1
+      for (int i = min(r - n0, 8) - 1; i >= 0; --i) {
+        hi = (hi << 16) | (lo >> 48);
+        lo = (lo << 16) | p[7 * a.ld_expand + i];
+      }
+      bq[7][ks] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    }
+  };
   auto load_weights = [&](int g) {  // this wave's block of W2 for group g
     r = CLS ? class_rank(a.rank[g], a.rank_lo, RP) : min(a.rank[g], RP);
     const bf16_t* W2 = group_weight<bf16_t>(a.w_expand, a.w_expand_base, a.expand_group_stride, g);
+    if constexpr (NB == 8 && !STORE) {
+      if ((r & 7) && (reinterpret_cast<uintptr_t>(W2) & 15u) && c0 + 128 == a.width_dst) {  // (uniform over the wave)
+        load_cut_weights(W2);
+        return;
+      }
+    }
 #pragma unroll
     for (int q = 0; q < 8; ++q)
 #pragma unroll
