@@ -215,3 +215,22 @@ def test_lora_b_as_columns_that_end_with_their_buffer(dev, r, r2):
     yo, *_ = oracle.multi_lora_linear_grads(f64(x), f64(base), ids, [f64(w) for w in a], [f64(w) for w in b], [r, r2],
                                             scales, f64(dy))
     assert max_rel_err(yd, yo) < TOL[bf16]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_gradients_of_adapters_that_are_views_of_wider_buffers(dev, dtype):
+    """Adapters with a row stride of their own through autograd: their gradients are written at that stride."""
+    from twinkle_amd import multi_lora_delta
+    t, k, m, ranks = 200, 72, 136, [8, 5]
+    x, base, dy, a, b, ids, _, scales = _problem(t, k, m, 2, 8, ranks, seed=4)
+    ad, bd = ([_strided(w, dtype, dev, 3).detach().requires_grad_(True) for w in ws] for ws in (a, b))
+    y = multi_lora_delta(x.to(dtype).to(dev), base.to(dtype).to(dev), build_segments(ids.to(torch.int32).to(dev), 2),
+                         AdapterGroups(ad, bd, ranks, scales))
+    y.backward(dy.to(dtype).to(dev))
+    f64 = lambda v: v.to(dtype).double()  # noqa: E731
+    yo, _, dao, dbo = oracle.multi_lora_linear_grads(f64(x), f64(base), ids, [f64(w) for w in a], [f64(w) for w in b],
+                                                     ranks, scales, f64(dy))
+    assert max_rel_err(y.detach(), yo) < TOL[dtype]
+    for g, r in enumerate(ranks):
+        assert max_rel_err(ad[g].grad[:r], dao[g][:r]) < TOL[dtype] and max_rel_err(bd[g].grad[:, :r], dbo[g][:, :r]) < TOL[dtype]
+        assert torch.count_nonzero(ad[g].grad[r:]) == 0 and torch.count_nonzero(bd[g].grad[:, r:]) == 0

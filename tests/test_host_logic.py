@@ -585,3 +585,30 @@ def test_adapter_checkpoint_keys_with_linear_and_packed_expert_parameters(tmp_pa
     assert want.keys() == got.keys()
     for k in want:
         assert torch.equal(want[k], got[k]), k
+
+
+@pytest.mark.parametrize('pad', [0, 3])
+def test_gradient_arena_spans_strided_adapters(pad):
+    """Gradients are written at the tensors' own row strides: every row the kernels write lies inside its tensor's place
+    in the arena, no two overlap, and the views handed to autograd show them."""
+    from twinkle_amd import AdapterGroups
+    k, m, ranks = 24, 40, [8, 0, 5, 8]
+    a = [torch.zeros(8, k + pad)[:, :k] for _ in ranks]
+    b = [torch.zeros(m, 8 + pad)[:, pad:] for _ in ranks]
+    groups = AdapterGroups(a, b, ranks, [1.0] * 4)
+    for side, elems, rel, ld, width in (('a', groups.a_arena_elems, groups._grad_a_rel, k + pad, k),
+                                        ('b', groups.b_arena_elems, groups._grad_b_rel, 8 + pad, 8)):
+        arena = torch.zeros(elems)
+        views = groups.grad_views(arena, side)
+        for g, r in enumerate(ranks):
+            if r == 0:
+                assert views[g] is None
+                continue
+            rows, cols = (r, width) if side == 'a' else (m, r)
+            for i in range(rows):
+                at = int(rel[g]) // 4 + i * ld
+                assert at + cols <= elems
+                assert torch.count_nonzero(arena[at:at + cols]) == 0
+                arena[at:at + cols] = g + 1
+            block = views[g][:r] if side == 'a' else views[g][:, :r]
+            assert torch.equal(block, torch.full_like(block, g + 1))

@@ -130,8 +130,13 @@ class AdapterGroups:
         for t, keep in zip(tensors, live):
             offs.append(total if keep else 0)     # groups of rank 0 are never written: any offset will do
             if keep:
-                total += (t.numel() + 127) // 128 * 128
+                total += (AdapterGroups._extent(t) + 127) // 128 * 128
         return offs, total
+
+    @staticmethod
+    def _extent(t):
+        # the kernels write a gradient at its tensor's own strides (lda, ldb), so its place in the arena spans those
+        return t.numel() if t.is_contiguous() else 1 + sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
 
     def arena_plan(self):
         """``(needs_zeros, a_shape, b_shape)`` of the gradient arenas, worked out at the first backward.
@@ -155,7 +160,8 @@ class AdapterGroups:
                         blocks[j].add(o)
                 zeros = zeros or not whole or any(k and len(b) * d[0] * d[1] != z.numel()
                                                   for k, b, d, z in zip(live, blocks, dims, sizes))
-                alike = all(live) and sizes[0].numel() % 128 == 0 and all(z == sizes[0] for z in sizes)
+                alike = all(live) and sizes[0].numel() % 128 == 0 and all(z == sizes[0] for z in sizes) and \
+                    all(t.is_contiguous() for t in tensors)
                 shapes.append((len(sizes), *sizes[0]) if alike else None)
             self._arena_plan = (zeros, *shapes)
         return self._arena_plan
@@ -183,7 +189,9 @@ class AdapterGroups:
         alike = self.arena_plan()[1 if side == 'a' else 2]
         if alike is not None:
             return list(arena.view(alike).unbind(0))
-        return [arena[o:o + t.numel()].view(t.shape) if keep else None for t, o, keep in zip(tensors, offs, live)]
+        return [None if not keep else arena[o:o + t.numel()].view(t.shape) if t.is_contiguous() else
+                arena.as_strided(t.shape, t.stride(), arena.storage_offset() + o)
+                for t, o, keep in zip(tensors, offs, live)]
 
     def autograd_tensors(self) -> List[torch.Tensor]:
         """The tensors gradients are reported for: the masters where there are any, else the tensors read."""
