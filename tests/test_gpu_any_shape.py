@@ -111,6 +111,30 @@ def test_a_dx_that_is_written_equals_one_that_starts_at_zero(dev, dtype, t, k, m
     assert torch.count_nonzero(written[dead.to(dev)]) == 0
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('k,ranks', [(1, [8, 0]), (41, [8, 0]), (2053, [16, 0, 3]),        # one class: the expand clears
+                                     (41, [8, 0, 20]), (2053, [40, 8, 0]), (2048, [0, 0])])  # several, none
+def test_rows_of_no_adapter_are_cleared_up_to_their_ends(dev, dtype, k, ranks):
+    """The written dx as rows at odd element addresses with three elements between them: zeros in every column of the rows
+    of no live adapter (whole and cut pieces of 16 bytes, more than one block of columns) and nothing around them."""
+    from twinkle_amd.ops import _lora_bwd
+    t, m, n = 130, 24, len(ranks)
+    x, base, dy, a, b, ids, _, scales = _problem(t, k, m, n, max(max(ranks), 1), ranks, seed=k)
+    ids[::3] = -1
+    xd, yd, dyd = (v.to(dtype).to(dev) for v in (x, base, dy))
+    seg = build_segments(ids.to(torch.int32).to(dev), n)
+    groups = AdapterGroups([w.to(dtype).to(dev) for w in a], [w.to(dtype).to(dev) for w in b], ranks, scales)
+    h = lora_fwd_(xd, yd, seg, groups)
+    added = torch.zeros_like(xd)
+    written = _strided(torch.full((t, k), float('nan')), dtype, dev, 3)
+    _lora_bwd('tk_lora_bwd', dyd, xd, h, added, None, None, seg, groups)
+    _lora_bwd('tk_lora_bwd_store', dyd, xd, h, written, None, None, seg, groups)
+    assert torch.equal(added, written)
+    dead = (ids < 0) | (torch.tensor(ranks)[ids.clamp(0)] == 0)
+    assert torch.count_nonzero(written[dead.to(dev)]) == 0
+    assert torch.count_nonzero(written._base[:, 0]) == 0 and torch.count_nonzero(written._base[:, 1 + k:]) == 0
+
+
 @pytest.mark.parametrize('max_r,ranks', [(8, [8, 8, 8]), (8, [8, 4, 8]), (8, [8, 0, 8]), (24, [24, 24, 24])])
 def test_gradients_of_adapters_without_rows_are_zero(dev, max_r, ranks):
     """The gradient arena starts uninitialised where every live block is written: also the block of an adapter that no
