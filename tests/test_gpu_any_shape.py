@@ -175,6 +175,9 @@ def test_rank_128(dev, t, k, m, ranks):
     (1, 1024, 128, [16]),                           # one row, two slices
     (33, 1088, 256, [16, 5, 0]),                    # a last slice of one step, a dead adapter
     (300, 4096, 1024, [16, 8, 1]),                  # eight slices; dy in two
+    (24, 4096, 1024, [16, 8, 1]),                   # eight rows an adapter: the eight slices summed in the expand
+    (25, 4096, 1024, [16, 8, 1]),                   # ... and one more: before it
+    (24, 4672, 256, [16, 8, 1]),                    # ten slices
     (2500, 2048, 1152, [16, 16]),                   # few blocks for the shrink, too many readings for the expand
     (2304, 2112, 384, [64, 40]),                    # rank 64, eight waves: slices that end in half a step
     (2400, 1024, 512, [32, 20, 32]),                # ... and rank 32, runs of several groups in eight tiles

@@ -309,10 +309,20 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // sum of the slices, few against pair: 32 rows 7.0 / 9.1 us, 1024 8.7 / 10.1, 4096 14.4 / 15.7, 8192 21.0 / 20.2; 14336
 // columns: 1024 rows 16.9 / 18.0, 2048 21.5 / 21.5, 4096 33.1 / 30.6).
 constexpr int64_t kFewShrinkBlocks = 9 * 256;  // (tile, slice) pairs
-// The expand adds the slices itself up to 8192 readings of a tile's slice (2 KB each, from L2): a launch less, which is
-// what a small eager call is bound by (a decode step of 32 rows: 33 -> 30 us a pass).  On the GPU alone it is 0.5 us
-// faster at 32 rows x 4096 and slower from 256 rows on (by 0.5 us; 1.3 us at 1024).
-constexpr int64_t kFewFinishReads = 8192;
+// The expand of few tiles adds the slices itself: a launch less against every wave's reading of its tile's slices (2 KB
+// each, from L2; nothing is read for padding slots, so tiles of few rows are cheap).  GPU time of a forward with / without:
+//   up to 4 slices (2048 columns)  32 x 2048 -> 2048 9.7 / 10.9, 512 x 1024 -> 14336 13.9 / 14.8 (4700 readings),
+//                                  3072 x 2048 -> 2048 17.5 / 17.3 (6460), 2048 x 2048 -> 4096 18.6 / 17.5 (10370)
+//   8 slices, 4096 -> 4096         16 adapters: 32 rows 10.7 / 11.2, 128 11.1 / 11.6, 256 12.5 / 12.1;
+//                                  one adapter: 8 rows 10.5 / 10.7, 32 12.3 / 11.7 (a full tile)
+//   28 slices, 14336 -> 4096       4 adapters: 8 rows 14.7 / 13.2, 64 18.1 / 13.7 us
+// An eager call saves 1 to 2.5 us of host time besides (a decode step of 32 rows takes 30 us instead of 33; 256 rows of 16
+// adapters, eight slices, one after the other: 13.1 instead of 15.1), so there eight slices count as few at any row count.
+constexpr int64_t kFewFinishReads = 6400;
+inline bool finish_in_expand(const PassArgs& a, const SegLayout& L, hipStream_t s) {
+  if (a.kslices <= 1 || a.kslices > 8 || L.max_tiles * (a.width_dst >> 7) * a.kslices > kFewFinishReads) return false;
+  return a.kslices <= 4 || L.rows <= 8 * (int64_t)L.groups || !stream_is_capturing(s);
+}
 
 template <int NB>
 void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int phases, hipStream_t s) {
@@ -330,8 +340,7 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
       hipLaunchKernelGGL((k_shrink_pair<NB, NW>), dim3((unsigned)(ceil_div(L.max_tiles, 2) * a.kslices)),
                          dim3(NW * 64), 0, s, a, hrow, seg.tile_group, rows, (int)L.max_tiles);
   }
-  const bool fin = NB == 1 && (phases & 5) && (phases & 2) && a.dst && a.kslices > 1 && !a.class_mode &&
-                   L.max_tiles * (a.width_dst >> 7) * a.kslices <= kFewFinishReads;
+  const bool fin = NB == 1 && (phases & 5) && (phases & 2) && a.dst && !a.class_mode && finish_in_expand(a, L, s);
   if ((phases & 5) && a.kslices > 1 && !fin)
     hipLaunchKernelGGL((k_shrink_finish<NB>), dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group,
                        rows);
