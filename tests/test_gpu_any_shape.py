@@ -179,6 +179,8 @@ def test_rank_128(dev, t, k, m, ranks):
     (25, 4096, 1024, [16, 8, 1]),                   # ... and one more: before it
     (24, 4672, 256, [16, 8, 1]),                    # ten slices
     (2500, 2048, 1152, [16, 16]),                   # few blocks for the shrink, too many readings for the expand
+    (7100, 4096, 128, [16]),                        # the most blocks of the few-tile shrink (224 tiles x 8 slices)
+    (7105, 4096, 128, [16]),                        # one tile more: k_shrink_pair
     (2304, 2112, 384, [64, 40]),                    # rank 64, eight waves: slices that end in half a step
     (2400, 1024, 512, [32, 20, 32]),                # ... and rank 32, runs of several groups in eight tiles
 ])

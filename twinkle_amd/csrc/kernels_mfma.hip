@@ -305,10 +305,10 @@ __global__ __launch_bounds__(256) void k_dy_fused_multi(DyFusedJobs jobs, const 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Few tiles at padded rank 16.  k_shrink_few: up to nine waves per CU (16 adapters of rank 16, 4096 columns, with the
-// sum of the slices, few against pair: 32 rows 7.0 / 9.1 us, 1024 8.7 / 10.1, 4096 14.4 / 15.7, 8192 21.0 / 20.2; 14336
-// columns: 1024 rows 16.9 / 18.0, 2048 21.5 / 21.5, 4096 33.1 / 30.6).
-constexpr int64_t kFewShrinkBlocks = 9 * 256;  // (tile, slice) pairs
+// Few tiles at padded rank 16: k_shrink_few up to seven waves per CU.  Forward with few / pair, us (4096 columns unless
+// said): 1024 rows 13.5 / 14.8, 4096 (1160 blocks) 21.2 / 21.9, 6144 (1672) 23.9 / 24.4, 8192 (2184) 29.0 / 28.1, 12288
+// 36.4 / 34.9, 16 adapters; 12288 x 2048 (1572) 25.8 / 26.5; 14336 columns: 1024 rows 21.9 / 22.8, 2048 (1932) 27.7 / 26.5.
+constexpr int64_t kFewShrinkBlocks = 7 * 256;  // (tile, slice) pairs
 // The expand of few tiles adds the slices itself: a launch less against every wave's reading of its tile's slices (2 KB
 // each, from L2; nothing is read for padding slots, so tiles of few rows are cheap).  GPU time of a forward with / without:
 //   up to 4 slices (2048 columns)  32 x 2048 -> 2048 9.7 / 10.9, 512 x 1024 -> 14336 13.9 / 14.8 (4700 readings),
