@@ -33,6 +33,9 @@ def _strided(t, dtype, dev, pad):
     (300, 512, 256, [40, 64], 1),                    # whole widths at odd row starts
     (450, 513, 640, [128, 65, 100], 3),              # several slices of the source, the largest rank
     (1100, 1100, 72, [20, 128, 1, 0, 64], 0),        # ranks of every class in one call, one adapter not live
+    (600, 1025, 65, [128, 128], 1),                  # few tiles, fp32 and bf16: three slices of a wide step
+    (300, 1281, 64, [20], 1),                        # fp32: more than one slice
+    (6100, 641, 33, [128], 0),                       # many tiles: one block walks all slices
     (4700, 72, 1031, [24, 8], 0),                    # groups of several chunks
 ])
 def test_edges(dev, dtype, t, k, m, ranks, pad):
