@@ -189,7 +189,7 @@ def test_empty_and_huge_segments(dev, dtype):
 
 @pytest.mark.parametrize('dtype,t,k,m,max_r,ranks', [
     (torch.bfloat16, 3000, 256, 1024, 16, [16, 8, 16]),     # single pass over dy, several chunks per group
-    (torch.bfloat16, 1500, 256, 384, 64, [64, 20, 33]),     # separate kernels, two streams
+    (torch.bfloat16, 1500, 256, 384, 64, [64, 20, 33]),     # separate kernels (one stream at this size)
     (torch.float32, 700, 40, 24, 8, [8, 3, 5]),             # generic kernels
 ])
 def test_rows_without_an_adapter_keep_the_base_output(dev, dtype, t, k, m, max_r, ranks):
@@ -425,16 +425,21 @@ def test_custom_ops_match_direct_calls(dev):
     assert y1.float().sub(bf(base).float()).abs().max() > 0
 
 
-@pytest.mark.parametrize('max_r,ranks', [(16, [16, 7, 16]), (32, [32, 16, 24]), (64, [64, 16, 40])])
-def test_hip_graph_replay_matches_eager(dev, max_r, ranks):
+@pytest.mark.parametrize('max_r,ranks,t,k,m', [
+    (16, [16, 7, 16], 1200, 256, 1024), (32, [32, 16, 24], 1200, 256, 1024), (64, [64, 16, 40], 1200, 256, 1024),
+    (64, [64, 40, 50], 11000, 2048, 4096),                  # 128 MB of x and dy: a captured backward forks from there on
+    (128, [128, 100, 70], 8300, 2048, 2048),                # 64 MB at rank 65 to 128
+    (16, [16, 7, 16], 6800, 252, 1030),                     # 16 MB for odd widths in bf16
+])
+def test_hip_graph_replay_matches_eager(dev, max_r, ranks, t, k, m):
     """Segment build + forward + backward captured in a HIP graph and replayed: every replay equals the eager result.
 
-    Ranks 16 and 32 take the single-pass dy kernel; rank 64 takes the separate kernels, whose backward forks onto
-    the library's side stream and joins back (both must be capturable).  Eager work and synchronisations run
-    between the replays.
+    Ranks 16 and 32 take the single-pass dy kernel, the others the separate kernels: on one stream at the first
+    shape, forked onto the library's side stream and joined back at the larger and odd ones (all must be capturable).
+    Eager work and synchronisations run between the replays.
     """
     from twinkle_amd import lora_bwd_, lora_bwd_workspace_bytes, lora_fwd_, lora_h_bytes
-    t, k, m, n = 1200, 256, 1024, 3
+    n = 3
     x, base, dy, a, b, ids, _, scales = _problem(t, k, m, n, max_r, ranks, seed=21)
     bf = lambda v: v.bfloat16().to(dev)  # noqa: E731
     xd, dyd, based = bf(x), bf(dy), bf(base)
@@ -572,10 +577,11 @@ sys.exit(0 if worst < 2e-2 else 1)
 '''
 
 
-@pytest.mark.parametrize('env', [{'TK_FORCE_GENERIC': '1'}, {'TK_BWD_STREAMS': '0'}])
+@pytest.mark.parametrize('env', [{'TK_FORCE_GENERIC': '1'}, {'TK_BWD_STREAMS': '0'}, {'TK_BWD_STREAMS': '1'}])
 def test_environment_switches_in_a_child_process(dev, env):
-    """TK_FORCE_GENERIC=1 (every launch on the shape-agnostic kernels) and TK_BWD_STREAMS=0 (backward on the
-    caller's stream only) are read once per process, so each runs in a child: same bar against the oracle."""
+    """TK_FORCE_GENERIC=1 (every launch on the shape-agnostic kernels) and TK_BWD_STREAMS=0 / 1 (backward on the
+    caller's stream only / forked at every size) are read once per process, so each runs in a child: same bar against
+    the oracle."""
     import os
     import subprocess
     import sys
@@ -585,15 +591,41 @@ def test_environment_switches_in_a_child_process(dev, env):
     assert out.returncode == 0, out.stdout[-2000:] + out.stderr[-2000:]
 
 
-def test_two_host_threads_call_the_two_stream_backward(dev):
-    """Rank 32 at an output width of 384 takes the backward that forks onto the library's per-device side stream;
-    two host threads, each on its own stream with its own buffers, must get what they get alone (the kernels are
-    deterministic: bit-equal)."""
+_FORKED_CHILD = r'''
+import sys, torch
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests")
+import test_gpu_lora as T
+dev = torch.device("cuda:0")
+print("two threads", flush=True)
+T.test_two_host_threads_call_the_two_stream_backward(dev, 3000, 512, 384)
+print("graph replay", flush=True)
+T.test_hip_graph_replay_matches_eager(dev, 64, [64, 16, 40], 1200, 256, 1024)
+'''
+
+
+def test_every_backward_forked_in_a_child_process(dev):
+    """The fork's event lock under two threads and the fork under capture, at shapes the rule would leave on one stream:
+    whatever sizes the rule takes, these are on two (TK_BWD_STREAMS=1)."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, '-c', _FORKED_CHILD, root], env={**os.environ, 'TK_BWD_STREAMS': '1'},
+                         capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout[-2000:] + out.stderr[-2000:]
+
+
+@pytest.mark.parametrize('t,k,m', [(3000, 512, 384),       # one stream per call at this size
+                                   (9000, 1000, 1030)])    # odd widths in bf16 fork from 32 MB of x and dy on
+def test_two_host_threads_call_the_two_stream_backward(dev, t, k, m):
+    """Rank 32 at an output width that is no multiple of 512 takes the backward that can fork onto the library's
+    per-device side stream; two host threads, each on its own stream with its own buffers, must get what they get alone
+    (the kernels are deterministic: bit-equal)."""
     import threading
     dt = torch.bfloat16
 
     def make(seed):
-        t, k, m, n, max_r = 3000, 512, 384, 3, 32
+        n, max_r = 3, 32
         x, base, dy, a, b, ids, ranks, scales = _problem(t, k, m, n, max_r, [32, 20, 32], seed=seed)
         p = {'x': x.to(dt).to(dev), 'dy': dy.to(dt).to(dev), 'y0': base.to(dt).to(dev)}
         ad, bd = [v.to(dt).to(dev) for v in a], [v.to(dt).to(dev) for v in b]

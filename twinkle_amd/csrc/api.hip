@@ -69,7 +69,8 @@ bool force_generic() {
 // The backward pass has two independent chains that meet only at the end (dB needs dy and h; dX and
 // dA need the dy shrink), and no single kernel of either reaches the memory system's peak, so the
 // library runs them on two streams: the caller's and one of its own per device (default priority,
-// non-blocking), forked and joined with events.  TK_BWD_STREAMS=0 keeps everything on the caller's stream.
+// non-blocking), forked and joined with events, where that pays (see worth_forking).  TK_BWD_STREAMS=0 keeps everything
+// on the caller's stream, TK_BWD_STREAMS=1 forks at every size.
 struct SideStream {
   hipStream_t stream = nullptr;
   hipEvent_t fork = nullptr, mid = nullptr, join = nullptr;
@@ -77,15 +78,16 @@ struct SideStream {
   std::mutex use;  // held while a call enqueues its fork .. join sequence: the events are shared per device
 };
 
-// x and dy together below this: the backward stays on the caller's stream (see lora_bwd_class)
-constexpr int64_t kSideStreamBytes = 192ll << 20;
+// 0: never, 1: always, 2: by the rule
+int side_stream_mode() {
+  static const int mode = [] {
+    const char* e = getenv("TK_BWD_STREAMS");
+    return e && (e[0] == '0' || e[0] == '1') ? e[0] - '0' : 2;
+  }();
+  return mode;
+}
 
 SideStream* side_stream() {
-  static const bool enabled = [] {
-    const char* e = getenv("TK_BWD_STREAMS");
-    return !(e && e[0] == '0');
-  }();
-  if (!enabled) return nullptr;
   constexpr int kMaxDevices = 64;
   static SideStream side[kMaxDevices];
   static std::mutex mu;
@@ -102,6 +104,29 @@ SideStream* side_stream() {
     if (!ok) (void)hipGetLastError();
   }
   return x.state == 1 ? &x : nullptr;
+}
+
+// Whether a backward of `bytes` of x and dy runs its chains side by side.  Fork and join are six calls of the runtime,
+// about 40 us of host time, and two waits of about 2 us each on the GPU.  The lines lie where shuffled and packed rows both
+// gain (shuffled ones gain from less: their kernels wait more).  One stream / forked, us, 4096 -> 4096 unless said:
+//   eager, one call after the other
+//     rank 64 packed    64 MB 85 / 92, 128 MB 120 / 128, 256 MB 224 / 210; shuffled 128 MB 134 / 131;
+//                       4096 -> 14336 packed 158 MB 146 / 155
+//     rank 128 packed   96 MB 124 / 135, 128 MB 160 / 164, 156 MB 206 / 184; shuffled 96 MB 150 / 148, 128 MB 200 / 178
+//     fp32 rank 16      256 MB 167 / 166
+//     bf16 on the kernels for any shape   1000 -> 1500 rank 24: 20 MB 77 / 78, 39 MB 118 / 112; 4096 -> 4001 rank 64:
+//                       16 MB 81 / 82, 63 MB 155 / 139 (their launches are small and fill the chip badly)
+//   replay of a captured graph, which pays no host time
+//     rank 64 packed    96 MB 104 / 109, 128 MB 123 / 122, 156 MB 162 / 140; shuffled 128 MB 136 / 126; fp32 rank 16: 64 MB
+//                       66 / 70, 128 MB 96 / 89
+//     rank 128 packed   64 MB 120 / 115, 96 MB 127 / 130, 128 MB 164 / 155; shuffled 64 MB 152 / 134, 128 MB 203 / 176
+//     bf16 on the kernels for any shape   1000 -> 1500 rank 24: 10 MB 72 / 58; 4001 -> 4096 rank 16: 1 MB 38 / 48, 8 MB 54 / 58,
+//                       31 MB 74 / 71, 127 MB 166 / 138
+bool worth_forking(int64_t bytes, bool any_shape_bf16, int rpad, hipStream_t s) {
+  const int64_t mb = bytes >> 20;
+  if (mb >= (any_shape_bf16 ? 32 : rpad > 64 ? 144 : 192)) return true;
+  if (mb < (any_shape_bf16 ? 16 : rpad > 64 ? 64 : 128)) return false;
+  return stream_is_capturing(s);
 }
 
 // Several rank classes in one call (tk_lora_desc::rank_classes) are independent chains of launches over disjoint
@@ -652,11 +677,14 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   // Separate kernels.  Two chains that meet only at the end: dB (reads dy and h) runs on a side stream,
   // the dy shrink -> dX on the caller's; dA follows the shrink on the side stream, next to the expand.
   // Without a side stream everything runs in the same order on the caller's stream.
-  // Small problems stay on one stream: the fork and the join are six calls of the runtime (30 us of host time) and a wait
-  // on each side, more than two kernels of a few microseconds gain from running side by side.
   const int64_t bytes = d->rows * ((int64_t)d->in_features + d->out_features) * elt_bytes(d->dtype);
-  const bool large = bytes >= kSideStreamBytes;
-  SideStream* side = (grad_B && need_wT && may_fork && large) ? side_stream() : nullptr;
+  const bool any_shape_bf16 = d->dtype == TK_DTYPE_BF16 &&
+                              !(mfma && pass_mfma_supported(a) && (!grad_A || wgrad_mfma_supported(ga)) &&
+                                (!grad_B || wgrad_mfma_supported(gb)));
+  SideStream* side = nullptr;
+  if (grad_B && need_wT && may_fork && side_stream_mode() != 0 &&
+      (side_stream_mode() == 1 || worth_forking(bytes, any_shape_bf16, a.rpad, s)))
+    side = side_stream();
   hipStream_t s2 = side ? side->stream : s;
   // two host threads must not interleave their records and waits on the device's one set of events
   std::unique_lock<std::mutex> side_guard;

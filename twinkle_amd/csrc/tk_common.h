@@ -556,4 +556,14 @@ bool dy_fused_supported(const WgradArgs& a, int kslices);
 int launch_dy_fused(const WgradArgs& a, const void* const* lora_B, int64_t ldb, float* hpart, int kslices,
                     const SegView& seg, const SegLayout& L, hipStream_t s);
 
+// Whether `s` is being captured into a graph: such a call is replayed without the host time its launches cost here.
+inline bool stream_is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {  // (the default stream next to a capture elsewhere)
+    (void)hipGetLastError();
+    return false;
+  }
+  return status == hipStreamCaptureStatusActive;
+}
+
 }  // namespace tk

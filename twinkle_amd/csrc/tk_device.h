@@ -60,16 +60,6 @@ __device__ inline int work_item(const WorkList& wl, int i) {
   return i < *wl.count ? wl.ids[i] : -1;
 }
 
-// Whether `s` is being captured into a graph: such a call is replayed without the host time its launches cost here.
-inline bool stream_is_capturing(hipStream_t s) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &status) != hipSuccess) {  // (the default stream next to a capture elsewhere)
-    (void)hipGetLastError();
-    return false;
-  }
-  return status == hipStreamCaptureStatusActive;
-}
-
 inline int check_launch() { return hipGetLastError() == hipSuccess ? TK_OK : TK_ERR_LAUNCH; }
 
 }  // namespace tk
