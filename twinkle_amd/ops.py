@@ -147,20 +147,17 @@ class AdapterGroups:
         cost the host more than the launches of the backward (16 adapters: 95 us)."""
         if self._arena_plan is None:
             zeros, shapes = False, []
+            some = min(self.ranks) > 0 or [i for i, r in enumerate(self.ranks) if r > 0]
+            pick = (lambda v: v) if some is True else (lambda v: [v[i] for i in some])
             for tensors, live, index, offset, rank_dim, ld in (
-                    (self.a_tensors, self.a_live, self.a_index, self.a_offset, 0, self.lda),
-                    (self.b_tensors, self.b_live, self.b_index, self.b_offset, 1, self.ldb)):
-                sizes = [t.shape for t in tensors]
-                blocks = [set() for _ in sizes]       # offsets of the blocks that are written, per tensor
-                dims = [tuple(z[-2:]) for z in sizes]
-                whole = all(z[1] == ld for z in dims)
-                for r, j, o in zip(self.ranks, index, offset):
-                    if r > 0:
-                        whole = whole and r == dims[j][rank_dim]
-                        blocks[j].add(o)
-                zeros = zeros or not whole or any(k and len(b) * d[0] * d[1] != z.numel()
-                                                  for k, b, d, z in zip(live, blocks, dims, sizes))
-                alike = all(live) and sizes[0].numel() % 128 == 0 and all(z == sizes[0] for z in sizes) and \
+                    (self.a_tensors, self.a_live, self.a_index, self.a_offset, -2, self.lda),
+                    (self.b_tensors, self.b_live, self.b_index, self.b_offset, -1, self.ldb)):
+                index, sizes = pick(index), [t.shape for t in tensors]
+                # (sets of all groups at once: this runs at the first backward of every object, for 512 groups of experts too)
+                whole = all(r == sizes[j][rank_dim] and ld == sizes[j][-1] for r, j in set(zip(pick(self.ranks), index)))
+                there = sum(z[:-2].numel() if len(z) > 2 else 1 for z, keep in zip(sizes, live) if keep)
+                zeros = zeros or not whole or len(set(zip(index, pick(offset)))) != there
+                alike = all(live) and len(set(sizes)) == 1 and sizes[0].numel() % 128 == 0 and \
                     all(t.is_contiguous() for t in tensors)
                 shapes.append((len(sizes), *sizes[0]) if alike else None)
             self._arena_plan = (zeros, *shapes)
