@@ -852,8 +852,9 @@ void launch_pass_any(const PassArgs& a0, const SegView& seg, const SegLayout& L,
   // 64 equal, 1024 x 1500 rank 128 40.0 / 35.5.
   PassArgs a = a0;
   if (a.kslices <= 3 && a.width_src <= 1536) {
-    const bool some = L.max_tiles >= 96;  // tiles
-    const bool one = L.max_tiles >= 192 || (sizeof(T) == 4 ? NB <= 2 && (a.width_src <= 1280 || some) : NB <= 4 || some);
+    const int64_t tiles = L.live_tiles();
+    const bool some = tiles >= 96;
+    const bool one = tiles >= 192 || (sizeof(T) == 4 ? NB <= 2 && (a.width_src <= 1280 || some) : NB <= 4 || some);
     if (one) a.kslices = 1;
   }
   const int32_t* rows = seg.slot_table(a.map_rows);

@@ -308,6 +308,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Few tiles at padded rank 16: k_shrink_few up to seven waves per CU.  Forward with few / pair, us (4096 columns unless
 // said): 1024 rows 13.5 / 14.8, 4096 (1160 blocks) 21.2 / 21.9, 6144 (1672) 23.9 / 24.4, 8192 (2184) 29.0 / 28.1, 12288
 // 36.4 / 34.9, 16 adapters; 12288 x 2048 (1572) 25.8 / 26.5; 14336 columns: 1024 rows 21.9 / 22.8, 2048 (1932) 27.7 / 26.5.
+// (Tiles that may hold rows count: 256 rows of a decode step over 512 expert groups are 256, and the empty ones cost little.)
 constexpr int64_t kFewShrinkBlocks = 7 * 256;  // (tile, slice) pairs
 // The expand of few tiles adds the slices itself: a launch less against every wave's reading of its tile's slices (2 KB
 // each, from L2; nothing is read for padding slots, so tiles of few rows are cheap).  GPU time of a forward with / without:
@@ -333,7 +334,7 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
     if (NB > 1 && a.oct_steps > 0)  // see shrink_plan
       hipLaunchKernelGGL((k_shrink_oct<NB == 1 ? 2 : NB>), dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(512), 0, s,
                          a, seg.tile_group, rows, (int)L.max_tiles);
-    else if (NB == 1 && L.max_tiles * a.kslices <= kFewShrinkBlocks)
+    else if (NB == 1 && L.live_tiles() * a.kslices <= kFewShrinkBlocks)
       hipLaunchKernelGGL(k_shrink_few, dim3((unsigned)(L.max_tiles * a.kslices)), dim3(64), 0, s, a, hrow, seg.tile_group,
                          rows);
     else

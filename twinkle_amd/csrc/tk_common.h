@@ -82,6 +82,7 @@ struct SegLayout {
   int64_t chunk_tiles;   // tiles per weight-gradient chunk (chunk_tiles_for(rows))
   int64_t max_tiles, max_chunks, max_partials;
   int64_t slots;         // padded sorted length: 32 * max_tiles
+  int64_t live_tiles() const { return std::min(max_tiles, rows); }  // at most that many tiles hold a row
   // byte offsets from the workspace base
   int64_t off_inv, off_slot_row, off_slot_pos, off_offsets, off_tile_group, off_tile_order, off_set_order, off_round_moved, off_chunks,
       off_tile_first,
