@@ -163,6 +163,21 @@ def test_gradients_of_adapters_without_rows_are_zero(dev, max_r, ranks):
                     assert torch.count_nonzero(w.grad) == 0
 
 
+@pytest.mark.parametrize('ranks', [[8, 8, 8], [8, 4, 8]])    # one unbind per side, one view per tensor
+def test_a_gradient_keeps_its_side_alive_and_no_more(dev, ranks):
+    """The gradients of lora_A share one storage and those of lora_B another: a held gradient of one side does not keep the
+    other side's memory."""
+    from twinkle_amd import multi_lora_delta
+    x, base, dy, a, b, ids, _, scales = _problem(200, 128, 256, 3, 8, ranks, seed=6)
+    ad, bd = ([w.bfloat16().to(dev).requires_grad_(True) for w in ws] for ws in (a, b))
+    y = multi_lora_delta(x.bfloat16().to(dev), base.bfloat16().to(dev), build_segments(ids.to(torch.int32).to(dev), 3),
+                         AdapterGroups(ad, bd, ranks, scales))
+    grads = torch.autograd.grad(y, ad + bd, dy.bfloat16().to(dev))
+    for side, ws in ((grads[:3], ad), (grads[3:], bd)):
+        assert all(g.untyped_storage().nbytes() <= sum(2 * w.numel() + 512 for w in ws) for g in side)
+    assert grads[0].untyped_storage().data_ptr() != grads[3].untyped_storage().data_ptr()
+
+
 @pytest.mark.parametrize('t,k,m,ranks', [
     (2304, 2048, 1024, [128, 65]),                  # long groups: weights shared in LDS, chunks in pairs
     (2304, 1024, 512, [100, 128]),                  # the narrowest source of that kernel

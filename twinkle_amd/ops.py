@@ -114,9 +114,7 @@ class AdapterGroups:
         esz = a0.element_size()
         rel_a = [(self._a_arena_off[j] + o) * esz for j, o in zip(self.a_index, self.a_offset)]
         rel_b = [(self._b_arena_off[j] + o) * esz for j, o in zip(self.b_index, self.b_offset)]
-        both = self.a_arena_elems * esz               # one arena for both sides: B's starts where A's ends
-        rel = torch.tensor([rel_b, rel_a, [r + both for r in rel_b]], dtype=torch.int64, device=dev)
-        self._grad_b_rel, self._grad_a_rel, self._grad_rel = rel[0], rel[1], rel[1:]
+        self._grad_a_rel, self._grad_b_rel = torch.tensor([rel_a, rel_b], dtype=torch.int64, device=dev).unbind(0)
         self._arena_plan = None
         self._ptr_key = None
         self._size_cache = {}
@@ -185,7 +183,7 @@ class AdapterGroups:
             arena = arena.to(masters[0].dtype)        # one cast for the whole side; the views below share it
         alike = self.arena_plan()[1 if side == 'a' else 2]
         if alike is not None:
-            return list(arena.view(alike).unbind(0))
+            return list((arena if arena.dim() > 1 else arena.view(alike)).unbind(0))
         return [None if not keep else arena[o:o + t.numel()].view(t.shape) if t.is_contiguous() else
                 arena.as_strided(t.shape, t.stride(), arena.storage_offset() + o)
                 for t, o, keep in zip(tensors, offs, live)]
@@ -422,11 +420,13 @@ def _weight_grads(ctx_groups: AdapterGroups, needs_a: bool, needs_b: bool, devic
     groups = ctx_groups
     arena_a = arena_b = pa = pb = None
     if needs_a and needs_b:
-        na, nb = groups.a_arena_elems, groups.b_arena_elems
-        new = torch.zeros if groups.arena_plan()[0] or not rows else torch.empty
-        arena = new(na + nb, dtype=groups.weight_dtype, device=device)
-        arena_a, arena_b = arena.split_with_sizes((na, nb))
-        pa, pb = (groups._grad_rel + arena.data_ptr()).unbind(0)
+        # an arena per side, so that a gradient somebody holds keeps the others of its side alive and no more; both pointer
+        # tables by one launch
+        zeros, a_shape, b_shape = groups.arena_plan()
+        new = torch.zeros if zeros or not rows else torch.empty
+        arena_a = new(a_shape or groups.a_arena_elems, dtype=groups.weight_dtype, device=device)
+        arena_b = new(b_shape or groups.b_arena_elems, dtype=groups.weight_dtype, device=device)
+        pa, pb = torch._foreach_add([groups._grad_a_rel, groups._grad_b_rel], [arena_a.data_ptr(), arena_b.data_ptr()])
         return arena_a, arena_b, pa, pb
     if needs_a:
         arena_a = torch.zeros(groups.a_arena_elems, dtype=groups.weight_dtype, device=device)
