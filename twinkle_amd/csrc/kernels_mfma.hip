@@ -1,5 +1,6 @@
 // bf16 launches of the segmented LoRA pass (kernel templates: lora_kernels.h), and the bf16-only kernels:
 //
+//   k_shrink_few        h of few tiles at rank <= 16
 //   k_dy_fused<NB>      backward, rank <= 32: dB and the slices of dh from one pass over dy
 //   k_transpose_job     B^T, A^T copies for the backward shrink / expand
 //   *_multi             the same bodies for several projections in one launch
@@ -303,6 +304,22 @@ __global__ __launch_bounds__(256) void k_dy_fused_multi(DyFusedJobs jobs, const 
                    blockIdx.y, j.x_blocks);
 }
 
+// The shrink of few tiles at padded rank 16: one wave per (tile, slice) requests its whole slice, eight steps, at once.
+// There are too few blocks to cover latencies with each other, so the launch takes as long as one block, and that as
+// many memory latencies as it has batches (five with k_shrink_pair's).  Same products in the same order: same bits.
+__global__ __launch_bounds__(64) void k_shrink_few(PassArgs a, bf16_t* __restrict__ hrow,
+                                                   const int32_t* __restrict__ tile_group,
+                                                   const int32_t* __restrict__ slot_rows) {
+  __shared__ float part[1][kTileRows][17];
+  const int nth = blockIdx.x / a.kslices, ks = blockIdx.x - nth * a.kslices;
+  const int tile = checked_tile(work_item(a.wl_tiles, nth), a.tb);
+  if (tile < 0) return;
+  const int g = checked_group(tile_group[tile], a.tb);
+  if (g < 0) return;
+  const int tiles[1] = {tile};
+  shrink_tiles<1, 1, 1, kShrinkSteps>(a, hrow, slot_rows, tiles, g, ks, part);
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Few tiles at padded rank 16: k_shrink_few up to seven waves per CU.  Forward with few / pair, us (4096 columns unless
@@ -346,17 +363,10 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
     hipLaunchKernelGGL((k_shrink_finish<NB>), dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group,
                        rows);
   if (!a.dst || !(phases & 2)) return;
-  const int64_t ngroups = a.width_dst >> 7;
   if constexpr (NB > 1) {
-    constexpr int TPI = 4;
-    const int64_t blocks = ceil_div(L.max_tiles, TPI) * ceil_div(ngroups, 4);
-    const auto kernel = a.dst_store ? (a.wl_sets.ids ? k_expand_multi<NB, TPI, true, true> : k_expand_multi<NB, TPI, false, true>)
-                                    : (a.wl_sets.ids ? k_expand_multi<NB, TPI, true, false> : k_expand_multi<NB, TPI, false, false>);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, hrow, seg.tile_group, rows,
-                       seg.set_walk(a.map_rows), seg.header, seg.round_moved,
-                       (int)std::min<int64_t>(L.sort_blocks, 64), (int)L.max_tiles);
+    launch_expand_multi<NB>(a, hrow, seg, L, s);
   } else {
-    const int64_t items = L.max_tiles * ngroups;
+    const int64_t items = L.max_tiles * (a.width_dst >> 7);
     const auto kernel = fin ? k_expand_mfma<NB, true> : k_expand_mfma<NB, false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(items, 4)), dim3(256), 0, s, a, hrow, seg.tile_group, rows,
                        seg.tile_walk(a.map_rows), (int)items);
@@ -488,10 +498,10 @@ int launch_shrink_multi(const PassArgs* a, int n, const SegView& seg, const SegL
   PassJobs J{};
   for (int p = 0; p < n; ++p) J.p[p] = a[p];
   const int32_t* rows = seg.slot_table(a[0].map_rows);
-  const bool quad = a[0].oct_steps > 0;
-  const int items = (int)(ceil_div(L.max_tiles, quad ? 8 : 2) * a[0].kslices);
+  const bool oct = a[0].oct_steps > 0;
+  const int items = (int)(ceil_div(L.max_tiles, oct ? 8 : 2) * a[0].kslices);
   const dim3 grid((unsigned)(ceil_div(items, 8) * 8 * n));
-  if (quad) {  // the single-projection launch makes the same choice: same sums, same bits
+  if (oct) {  // the single-projection launch makes the same choice: same sums, same bits
     if (a[0].rpad <= 32)
       hipLaunchKernelGGL((k_shrink_oct_multi<2>), grid, dim3(512), 0, s, J, n, items, seg.tile_group, rows,
                          (int)L.max_tiles);

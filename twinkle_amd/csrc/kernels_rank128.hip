@@ -27,15 +27,7 @@ int launch_pass_rank128(const PassArgs& a, const SegView& seg, const SegLayout& 
   }
   if (((phases & 4) || ((phases & 1) && a.oct_steps > 0)) && a.kslices > 1)
     hipLaunchKernelGGL(k_shrink_finish<8>, dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group, rows);
-  if (a.dst && (phases & 2)) {
-    constexpr int TPI = 4;
-    const int64_t blocks = ceil_div(L.max_tiles, TPI) * ceil_div(a.width_dst >> 7, 4);
-    const auto kernel = a.dst_store ? (a.wl_sets.ids ? k_expand_multi<8, TPI, true, true> : k_expand_multi<8, TPI, false, true>)
-                                    : (a.wl_sets.ids ? k_expand_multi<8, TPI, true, false> : k_expand_multi<8, TPI, false, false>);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, hrow, seg.tile_group, rows,
-                       seg.set_walk(a.map_rows), seg.header, seg.round_moved, (int)std::min<int64_t>(L.sort_blocks, 64),
-                       (int)L.max_tiles);
-  }
+  if (a.dst && (phases & 2)) launch_expand_multi<8>(a, hrow, seg, L, s);
   return check_launch();
 }
 

@@ -1,5 +1,5 @@
 // Kernel templates of the segmented LoRA pass, bf16 on v_mfma_f32_16x16x32_bf16 (fp32 accumulate), instantiated by
-// kernels_mfma.hip.
+// kernels_mfma.hip (rank up to 64) and kernels_rank128.hip.
 //
 // All of these kernels stream activations from HBM: the matrix cores are used
 // because the vector ALUs could not keep up with 8 TB/s at these ranks, not
@@ -237,22 +237,6 @@ __global__ __launch_bounds__(NW * 64) void k_shrink_pair(PassArgs a, bf16_t* __r
                                                          const int32_t* __restrict__ tile_group,
                                                          const int32_t* __restrict__ slot_rows, int max_tiles) {
   shrink_pair_body<NB, NW>(a, hrow, tile_group, slot_rows, max_tiles, blockIdx.x);
-}
-
-// The shrink of few tiles at padded rank 16: one wave per (tile, slice) requests its whole slice, eight steps, at once.
-// There are too few blocks to cover latencies with each other, so the launch takes as long as one block, and that as
-// many memory latencies as it has batches (five with k_shrink_pair's).  Same products in the same order: same bits.
-__global__ __launch_bounds__(64) void k_shrink_few(PassArgs a, bf16_t* __restrict__ hrow,
-                                                   const int32_t* __restrict__ tile_group,
-                                                   const int32_t* __restrict__ slot_rows) {
-  __shared__ float part[1][kTileRows][17];
-  const int nth = blockIdx.x / a.kslices, ks = blockIdx.x - nth * a.kslices;
-  const int tile = checked_tile(work_item(a.wl_tiles, nth), a.tb);
-  if (tile < 0) return;
-  const int g = checked_group(tile_group[tile], a.tb);
-  if (g < 0) return;
-  const int tiles[1] = {tile};
-  shrink_tiles<1, 1, 1, kShrinkSteps>(a, hrow, slot_rows, tiles, g, ks, part);
 }
 
 // ---------------------------------------------------------------------------
@@ -1082,7 +1066,7 @@ __global__ __launch_bounds__(64) void k_wgrad_pipe(WgradArgs a, const ChunkInfo*
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient at padded rank 32 and 64: (chunk, 128 columns), two waves, each owning half of the rank
+// Weight gradient above rank 16: (chunk, 128 columns), two waves (four at padded rank 128), each owning half of the rank
 // indices and both needing every tile of the source (one wave with all of them would hold 64 or 128
 // accumulator registers next to its tiles in flight: measured 49 against 41 us at rank 32, one wave per SIMD
 // at rank 64).  Two independent readers of a tile drift apart and the later one misses the CU's cache
@@ -1231,6 +1215,18 @@ __global__ __launch_bounds__((NB == 8 ? 256 : 128) * PAIRS) void k_wgrad_coop(Wg
                                                               const int32_t* __restrict__ slot_rows) {
   wgrad_coop_body<NB, S, PAIRS>(a, chunks, slot_rows, blockIdx.x * PAIRS + (PAIRS > 1 ? threadIdx.x >> 7 : 0), blockIdx.y,
                                 gridDim.x * PAIRS);
+}
+
+// The expand above rank 16: written or added, one class or several.
+template <int NB>
+inline void launch_expand_multi(const PassArgs& a, const bf16_t* hrow, const SegView& seg, const SegLayout& L, hipStream_t s) {
+  constexpr int TPI = kSetTiles;
+  const int64_t blocks = ceil_div(L.max_tiles, TPI) * ceil_div(a.width_dst >> 7, 4);
+  const auto kernel = a.dst_store ? (a.wl_sets.ids ? k_expand_multi<NB, TPI, true, true> : k_expand_multi<NB, TPI, false, true>)
+                                  : (a.wl_sets.ids ? k_expand_multi<NB, TPI, true, false> : k_expand_multi<NB, TPI, false, false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, hrow, seg.tile_group, seg.slot_table(a.map_rows),
+                     seg.set_walk(a.map_rows), seg.header, seg.round_moved, (int)std::min<int64_t>(L.sort_blocks, 64),
+                     (int)L.max_tiles);
 }
 
 }  // namespace

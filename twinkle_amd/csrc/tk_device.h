@@ -38,8 +38,8 @@ __device__ inline ChunkInfo checked_chunk(ChunkInfo ci, const TableBounds& tb) {
   return ci;
 }
 
-// Weight-gradient launches at padded rank 64 take two consecutive chunks of a group as one work item
-// (WgradArgs::pair_chunks): their partial sums are 64 x width floats per chunk, written once and read once by the
+// Weight-gradient launches at padded rank 64 and 128 take two consecutive chunks of a group as one work item
+// (WgradArgs::pair_chunks): their partial sums are rpad x width floats per chunk, written once and read once by the
 // reduction, and half as many of them are worth more there than the parallelism of short chunks (config 5's q
 // projection: 40 partials of 1 MB per gradient).  Chunk `b` is taken by the block of the chunk `a` in front of it
 // when both belong to one group, b's partial slot is odd and the two are neighbours in slots and in tiles; the
