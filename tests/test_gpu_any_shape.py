@@ -200,6 +200,8 @@ def test_rank_128(dev, t, k, m, ranks):
     (2500, 2048, 1152, [16, 16]),                   # few blocks for the shrink, too many readings for the expand
     (7100, 4096, 128, [16]),                        # the most blocks of the few-tile shrink (224 tiles x 8 slices)
     (7105, 4096, 128, [16]),                        # one tile more: k_shrink_pair
+    (8200, 4096, 128, [64, 40]),                    # more sets of eight tiles than CUs: four waves
+    (6150, 4096, 128, [32, 20]),                    # ... at rank 32
     (2304, 2112, 384, [64, 40]),                    # rank 64, eight waves: slices that end in half a step
     (2400, 1024, 512, [32, 20, 32]),                # ... and rank 32, runs of several groups in eight tiles
 ])
@@ -282,3 +284,18 @@ def test_gradients_of_adapters_that_are_views_of_wider_buffers(dev, dtype):
     for g, r in enumerate(ranks):
         assert max_rel_err(ad[g].grad[:r], dao[g][:r]) < TOL[dtype] and max_rel_err(bd[g].grad[:, :r], dbo[g][:, :r]) < TOL[dtype]
         assert torch.count_nonzero(ad[g].grad[r:]) == 0 and torch.count_nonzero(bd[g].grad[:, r:]) == 0
+
+
+@pytest.mark.parametrize('t,r', [(6144, 32), (8192, 64)])
+def test_eight_and_four_waves_give_the_same_bits(dev, t, r):
+    """One row more than the most that k_shrink_oct takes goes through k_shrink_quad: the rows both have come out alike."""
+    x, base, _, a, b, _, ranks, scales = _problem(t + 1, 4096, 128, 2, r, [r, r - 9], seed=r)
+    ids = (torch.arange(t + 1) * 2 // t).clamp(max=1).to(torch.int32).to(dev)
+    bf16 = torch.bfloat16
+    groups = AdapterGroups([w.to(bf16).to(dev) for w in a], [w.to(bf16).to(dev) for w in b], ranks, scales)
+    xd, out = x.to(bf16).to(dev), []
+    for rows in (t, t + 1):
+        yd = base[:rows].to(bf16).to(dev)
+        lora_fwd_(xd[:rows], yd, build_segments(ids[:rows], 2), groups)
+        out.append(yd)
+    assert torch.equal(out[0], out[1][:t])

@@ -524,7 +524,7 @@ static PassArgs fwd_pass_args(const tk_lora_desc* d, const void* x, int64_t ldx,
   a.map_rows = d->map_rows;  a.rpad = rank_pad(d->max_rank);  a.src_rows = (int32_t)d->rows;
   a.hpart = (float*)((char*)h + round_up(2 * (int64_t)a.rpad * a.ldh * elt_bytes(d->dtype), 256));
   const ShrinkPlan plan = shrink_plan(d->rows, d->num_groups, d->in_features, a.rpad);
-  a.kslices = plan.kslices;  a.oct_steps = plan.oct_steps;
+  a.kslices = plan.kslices;  a.set_steps = plan.set_steps;  a.set_waves = plan.set_waves;
   return a;
 }
 
@@ -578,7 +578,7 @@ static BwdPlan bwd_plan(const tk_lora_desc* d, const BwdLayout& B, const void* d
   a.map_rows = d->map_rows;  a.rpad = (int32_t)B.rpad;  a.src_rows = (int32_t)d->rows;
   a.hpart = (float*)(w + B.off_hpart);
   const ShrinkPlan plan = shrink_plan(d->rows, d->num_groups, d->out_features, a.rpad);
-  a.kslices = plan.kslices;  a.oct_steps = plan.oct_steps;
+  a.kslices = plan.kslices;  a.set_steps = plan.set_steps;  a.set_waves = plan.set_waves;
   TransposeJob& tr = p.tr;
   tr.lora_A = d->lora_A;  tr.lda = d->lda;
   tr.lora_B = d->lora_B;  tr.ldb = d->ldb;

@@ -1,6 +1,7 @@
 // bf16 launches of the segmented LoRA pass (kernel templates: lora_kernels.h), and the bf16-only kernels:
 //
 //   k_shrink_few        h of few tiles at rank <= 16
+//   k_shrink_quad       h at rank 17 to 64 with many tiles
 //   k_dy_fused<NB>      backward, rank <= 32: dB and the slices of dh from one pass over dy
 //   k_transpose_job     B^T, A^T copies for the backward shrink / expand
 //   *_multi             the same bodies for several projections in one launch
@@ -304,6 +305,162 @@ __global__ __launch_bounds__(256) void k_dy_fused_multi(DyFusedJobs jobs, const 
                    blockIdx.y, j.x_blocks);
 }
 
+// ---------------------------------------------------------------------------
+// k_shrink_oct (lora_kernels.h) with four waves instead of eight: a block of four waves owns (eight consecutive tiles,
+// slice of columns), wave w takes tiles 2 w and 2 w + 1 through all steps of 64 columns, and the weight block of a step
+// (16 * NB x 64) is fetched once per block, 16 B per thread, into a double-buffered LDS tile.  Two such blocks fit a CU
+// where one of eight waves does (registers), and a block that waits leaves the other one running, which is what counts
+// once the chip is full (see oct_blocks).  Activations: two or three steps in registers per wave.
+// ---------------------------------------------------------------------------
+template <int NB>
+__device__ __forceinline__ void shrink_quad_body(const PassArgs& a, const int32_t* __restrict__ tile_group,
+                                                 const int32_t* __restrict__ slot_rows, int max_tiles, int item) {
+  constexpr int RP = 16 * NB;
+  constexpr int WS = 72;                    // row stride of a staged weight block in bf16 (144 B: conflict-free)
+  constexpr int NLD = (RP * 8 + 255) / 256;  // 16-byte pieces of a weight block per thread
+  constexpr int S = NB == 4 ? 2 : 3;  // steps of activations in registers (rank 64: the accumulators take the room)
+  __shared__ __attribute__((aligned(16))) bf16_t wbuf[2][RP * WS];
+  __shared__ int32_t gts[8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
+  const int nth = item / a.kslices, ks = item - nth * a.kslices;
+  const int set = work_item(a.wl_octs, nth);
+  if (set < 0) return;  // past the end of this rank class's list (uniform over the block)
+  const int t_first = set * 8;
+  if (tid < 8) gts[tid] = t_first + tid < max_tiles ? checked_group(tile_group[t_first + tid], a.tb) : -1;
+  const int nsteps = a.width_src >> 6;
+  const int s0 = ks * a.set_steps;
+  const int ns = min(a.set_steps, nsteps - s0);  // >= 1 for every slice
+  // this wave's two tiles
+  const bf16_t* src = (const bf16_t*)a.src;
+  const bf16_t *xa[2], *xb[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int t = min(t_first + 2 * wave + u, max_tiles - 1);
+    int ra = slot_rows[t * kTileRows + li], rb = slot_rows[t * kTileRows + 16 + li];
+    ra = min(max(ra, 0), a.src_rows - 1);
+    rb = min(max(rb, 0), a.src_rows - 1);
+    xa[u] = src + (int64_t)ra * a.ld_src + 16 * kb + (int64_t)s0 * 64;
+    xb[u] = src + (int64_t)rb * a.ld_src + 16 * kb + (int64_t)s0 * 64;
+  }
+  __syncthreads();
+  for (int j = 0; j < 8;) {
+    const int g = gts[j];
+    int e = j + 1;
+    while (e < 8 && gts[e] == g) ++e;
+    const int lo = j, hi = e;  // the run: tiles t_first + lo .. t_first + hi - 1, all of group g
+    j = e;
+    if (g < 0) continue;
+    const int r = class_rank(a.rank[g], a.rank_lo, RP);
+    if (r <= 0) continue;  // adapter not live on this layer, or a group of another rank class
+    bool mine[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) mine[u] = 2 * wave + u >= lo && 2 * wave + u < hi;
+    const bool active = mine[0] || mine[1];  // wave-uniform
+    const bf16_t* W1 = group_weight<bf16_t>(a.w_shrink, a.w_shrink_base, a.shrink_group_stride, g) + (int64_t)s0 * 64;
+    // staging: piece p = tid + 256 i is columns 8 (p % 8) .. + 8 of rank index p / 8
+    auto stage_load = [&](int s, uint4 (&wr)[NLD]) {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        const int p = tid + 256 * i, n = p >> 3;
+        wr[i] = (n < r && s < ns) ? ld16(W1 + (int64_t)n * a.ld_shrink + (s << 6) + 8 * (p & 7)) : zero4();
+      }
+    };
+    auto stage_store = [&](int buf, const uint4 (&wr)[NLD]) {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        const int p = tid + 256 * i, n = p >> 3;
+        if (n < RP) st16(&wbuf[buf][n * WS + 8 * (p & 7)], wr[i]);
+      }
+    };
+    struct Step {
+      uint4 x0[2][2], x1[2][2];
+    };
+    auto issue = [&](int s, Step& X) {
+      const int c = min(s, ns - 1) << 6;  // requests past the slice repeat its last step and are not used
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        X.x0[u][0] = ld16(xa[u] + c);
+        X.x1[u][0] = ld16(xa[u] + c + 8);
+        X.x0[u][1] = ld16(xb[u] + c);
+        X.x1[u][1] = ld16(xb[u] + c + 8);
+      }
+    };
+    f32x4 acc[2][2][NB];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[u][tt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 wr[NLD];
+    auto step = [&](int s, const Step& X, Step& Xnext) {
+      lds_barrier();  // block s is complete; the other buffer has been read by everyone
+      stage_load(s + 1, wr);
+      if (active) issue(s + S - 1, Xnext);
+      if (active) {
+        const bf16_t* wb = wbuf[s & 1] + li * WS + 16 * kb;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const uint4 w0 = ld16(wb + 16 * nb * WS), w1 = ld16(wb + 16 * nb * WS + 8);
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+              acc[u][tt][nb] = mfma16(X.x0[u][tt], w0, acc[u][tt][nb]);
+              acc[u][tt][nb] = mfma16(X.x1[u][tt], w1, acc[u][tt][nb]);
+            }
+        }
+      }
+      stage_store((s + 1) & 1, wr);  // block s + 1 (zeros past the slice), visible behind the next barrier
+    };
+    Step T[S];
+    stage_load(0, wr);
+    if (active) {
+#pragma unroll
+      for (int i = 0; i < S - 1; ++i) issue(i, T[i]);
+    }
+    stage_store(0, wr);
+    int s = 0;
+    for (; s + S <= ns; s += S) {
+#pragma unroll
+      for (int i = 0; i < S; ++i) step(s + i, T[i], T[(i + S - 1) % S]);
+    }
+#pragma unroll
+    for (int i = 0; i < S - 1; ++i)
+      if (s + i < ns) step(s + i, T[i], T[(i + S - 1) % S]);  // block-uniform
+    lds_barrier();  // the next run's first block goes into buffer 0
+    if (!active) continue;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (!mine[u]) continue;
+      float* out = a.hpart + ((int64_t)(t_first + 2 * wave + u) * a.kslices + ks) * (kTileRows * RP) + 4 * kb * RP + li;
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) out[(16 * tt + v) * RP + 16 * nb] = acc[u][tt][nb][v];
+    }
+  }
+}
+
+template <int NB>
+__global__ __launch_bounds__(256, 2) void k_shrink_quad(PassArgs a, const int32_t* __restrict__ tile_group,
+                                                     const int32_t* __restrict__ slot_rows, int max_tiles) {
+  shrink_quad_body<NB>(a, tile_group, slot_rows, max_tiles, blockIdx.x);
+}
+
+// The same for up to kMaxShared projections that read the same source (see shared_source_item).
+template <int NB>
+__global__ __launch_bounds__(256, 2) void k_shrink_quad_multi(PassJobs jobs, int nproj, int items,
+                                                           const int32_t* __restrict__ tile_group,
+                                                           const int32_t* __restrict__ slot_rows, int max_tiles) {
+  int p, item;
+  shared_source_item(blockIdx.x, nproj, p, item);
+  if (item >= items) return;
+  shrink_quad_body<NB>(jobs.p[p], tile_group, slot_rows, max_tiles, item);
+}
+
 // The shrink of few tiles at padded rank 16: one wave per (tile, slice) requests its whole slice, eight steps, at once.
 // There are too few blocks to cover latencies with each other, so the launch takes as long as one block, and that as
 // many memory latencies as it has batches (five with k_shrink_pair's).  Same products in the same order: same bits.
@@ -348,9 +505,10 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
   const int32_t* rows = seg.slot_table(a.map_rows);
   constexpr int NW = NB == 1 ? 1 : (NB == 2 ? 2 : 4);  // shrink_waves(16 * NB)
   if (phases & 1) {
-    if (NB > 1 && a.oct_steps > 0)  // see shrink_plan
-      hipLaunchKernelGGL((k_shrink_oct<NB == 1 ? 2 : NB>), dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(512), 0, s,
-                         a, seg.tile_group, rows, (int)L.max_tiles);
+    if (NB > 1 && a.set_steps > 0)  // see shrink_plan
+      hipLaunchKernelGGL((a.set_waves == 8 ? k_shrink_oct<NB == 1 ? 2 : NB> : k_shrink_quad<NB == 1 ? 2 : NB>),
+                         dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(64 * a.set_waves), 0, s, a,
+                         seg.tile_group, rows, (int)L.max_tiles);
     else if (NB == 1 && L.live_tiles() * a.kslices <= kFewShrinkBlocks)
       hipLaunchKernelGGL(k_shrink_few, dim3((unsigned)(L.max_tiles * a.kslices)), dim3(64), 0, s, a, hrow, seg.tile_group,
                          rows);
@@ -498,16 +656,13 @@ int launch_shrink_multi(const PassArgs* a, int n, const SegView& seg, const SegL
   PassJobs J{};
   for (int p = 0; p < n; ++p) J.p[p] = a[p];
   const int32_t* rows = seg.slot_table(a[0].map_rows);
-  const bool oct = a[0].oct_steps > 0;
-  const int items = (int)(ceil_div(L.max_tiles, oct ? 8 : 2) * a[0].kslices);
+  const bool set = a[0].set_steps > 0;
+  const int items = (int)(ceil_div(L.max_tiles, set ? 8 : 2) * a[0].kslices);
   const dim3 grid((unsigned)(ceil_div(items, 8) * 8 * n));
-  if (oct) {  // the single-projection launch makes the same choice: same sums, same bits
-    if (a[0].rpad <= 32)
-      hipLaunchKernelGGL((k_shrink_oct_multi<2>), grid, dim3(512), 0, s, J, n, items, seg.tile_group, rows,
-                         (int)L.max_tiles);
-    else
-      hipLaunchKernelGGL((k_shrink_oct_multi<4>), grid, dim3(512), 0, s, J, n, items, seg.tile_group, rows,
-                         (int)L.max_tiles);
+  if (set) {  // (same sums and same bits as the single-projection launch, whichever kernel either takes)
+    const auto kernel = a[0].set_waves == 8 ? (a[0].rpad <= 32 ? k_shrink_oct_multi<2> : k_shrink_oct_multi<4>)
+                                            : (a[0].rpad <= 32 ? k_shrink_quad_multi<2> : k_shrink_quad_multi<4>);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * a[0].set_waves), 0, s, J, n, items, seg.tile_group, rows, (int)L.max_tiles);
   } else if (a[0].rpad <= 32) {
     hipLaunchKernelGGL((k_shrink_pair_multi<2, 2>), grid, dim3(128), 0, s, J, n, items, seg.tile_group, rows,
                        (int)L.max_tiles);

@@ -17,7 +17,7 @@ int launch_pass_rank128(const PassArgs& a, const SegView& seg, const SegLayout& 
   if (phases & 1) {
     // weights shared in LDS where the plan asks for it; short groups and wide sources take the tile-by-tile kernel, whose
     // blocks of four waves do not wait for groups of eight tiles
-    if (a.oct_steps == 0) {
+    if (a.set_steps == 0) {
       const int rc = launch_pass_generic(a, seg, L, TK_DTYPE_BF16, 1, s);
       if (rc != TK_OK) return rc;
     } else {
@@ -25,7 +25,7 @@ int launch_pass_rank128(const PassArgs& a, const SegView& seg, const SegLayout& 
                          seg.tile_group, rows, (int)L.max_tiles);
     }
   }
-  if (((phases & 4) || ((phases & 1) && a.oct_steps > 0)) && a.kslices > 1)
+  if (((phases & 4) || ((phases & 1) && a.set_steps > 0)) && a.kslices > 1)
     hipLaunchKernelGGL(k_shrink_finish<8>, dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group, rows);
   if (a.dst && (phases & 2)) launch_expand_multi<8>(a, hrow, seg, L, s);
   return check_launch();

@@ -250,9 +250,10 @@ __global__ __launch_bounds__(NW * 64) void k_shrink_pair(PassArgs a, bf16_t* __r
 // overwritten one step after the barrier behind its last reader.  The eight tiles are taken in runs of equal group
 // (almost always one run); waves whose tile lies outside the run still help to stage the weights.  What bounds it is
 // memory latency: a wave keeps S - 1 steps (8 KB each: 256 contiguous bytes of 32 rows) in flight and the weights are
-// requested two steps ahead.  (Four waves of two tiles and 64 columns a step before, 128 bytes of a row at a time:
-// 6000 x 4096 at rank 64 28 against 20 us, 32768 x 4096 about 80 both, 3.5 TB/s of source.)  Every block leaves its sums as one slice of the split-shrink buffer (k_shrink_finish
-// follows); each entry is the sum of one wave's MFMA chain, so results do not depend on timing.
+// requested two steps ahead.  (k_shrink_quad in kernels_mfma.hip is the same with four waves of two tiles and 64 columns a
+// step: see oct_blocks for which is faster where.)  Every block leaves its sums as one slice of the split-shrink buffer
+// (k_shrink_finish follows); each entry is the sum of one wave's MFMA chain in column order, in either kernel, so results
+// do not depend on timing or on the choice.
 // ---------------------------------------------------------------------------
 template <int NB>
 __device__ __forceinline__ void shrink_oct_body(const PassArgs& a, const int32_t* __restrict__ tile_group,
@@ -271,8 +272,8 @@ __device__ __forceinline__ void shrink_oct_body(const PassArgs& a, const int32_t
   if (set < 0) return;  // past the end of this rank class's list (uniform over the block)
   const int t_first = set * 8;
   if (tid < 8) gts[tid] = t_first + tid < max_tiles ? checked_group(tile_group[t_first + tid], a.tb) : -1;
-  const int s0 = ks * a.oct_steps;                                 // in 64-column steps
-  const int n64 = min(a.oct_steps, (a.width_src >> 6) - s0);       // >= 1 for every slice
+  const int s0 = ks * a.set_steps;                                 // in 64-column steps
+  const int n64 = min(a.set_steps, (a.width_src >> 6) - s0);       // >= 1 for every slice
   const int ns = (n64 + 1) >> 1;                                   // steps of 128 columns, the last perhaps half
   // this wave's tile
   const bf16_t* x_row[2];

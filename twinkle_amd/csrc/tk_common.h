@@ -221,25 +221,35 @@ static inline int shrink_waves(int rpad) { return rpad <= 16 ? 1 : (rpad <= 32 ?
 static inline int shrink_kslices(int width, int rpad) {
   return (int)ceil_div(ceil_div(width, 64), (int64_t)kShrinkSteps * shrink_waves(rpad));
 }
-// Above rank 16, with long groups and a source of 1024 to 4096 columns, the shrink runs as k_shrink_oct: blocks of
-// (eight tiles, `steps` steps of 64 columns).  The slices are cut so that there are at most two blocks of eight waves
-// per CU (twice as many slices: 98 us against 77 for 32768 x 4096 at rank 64, their sums are written and read; half as
-// many: 81).  Wider sources stay with k_shrink_pair (24 adapters of rank 8 to 64, 32768 x 4096 -> 14336: the training
-// step takes 1037 us, with the wide dy on k_shrink_oct 1054).
-constexpr int kOctResident = 512;
+// Above rank 16, with long groups and a source of 1024 to 4096 columns, the shrink runs as k_shrink_oct or k_shrink_quad:
+// blocks of (eight tiles, `steps` steps of 64 columns), at most 512 of them (twice as many slices: 98 us against 77 for
+// 32768 x 4096 at rank 64, their sums are written and read; half as many: 81).  Wider sources stay with k_shrink_pair (24
+// adapters of rank 8 to 64, 32768 x 4096 -> 14336: the training step takes 1037 us, with the wide dy on k_shrink_oct 1054).
+constexpr int kSetBlocks = 512;
+// A CU holds one block of k_shrink_oct or two of k_shrink_quad (registers).  The eight waves read 256 contiguous bytes of a
+// row per step and are faster while every block has a CU of its own; past that they run in rounds.  Shrink with its slice
+// sums, eight adapters, oct / quad, us, rows packed and shuffled:
+//   rank 64   4096 x 4096 (128 blocks) 23 / 26, 25 / 33; 8192 x 4096 and 16384 x 2048 (256) 28 / 29, 33 / 36 and 27 / 28, 33 / 35
+//             12288 x 4096 (384) 46 / 40, 47 / 50; 16384 x 4096 (512) 52 / 47, 60 / 58; 32768 x 4096 79 / 76, 93 / 89
+//   rank 32   4096 x 4096 (128) 23 / 22, 24 / 28; 12288 x 2048 (192) 23 / 23, 24 / 28; 16384 x 2048 (256) 26 / 24, 32 / 28
+//             8192 x 4096 (256) 28 / 24, 33 / 30; 16384 x 4096 (512) 52 / 40, 58 / 48
+// Rank 128 has only the eight waves.
+static inline int64_t oct_blocks(int rpad) { return rpad <= 32 ? 192 : 256; }
 struct ShrinkPlan {
-  int kslices;     // slices per tile
-  int oct_steps;  // 0: k_shrink_pair; else steps per slice of k_shrink_oct
+  int kslices;    // slices per tile
+  int set_steps;  // 0: k_shrink_pair; else steps per slice of the kernels that own eight tiles
+  int set_waves;  // 8: k_shrink_oct, 4: k_shrink_quad
 };
 static inline ShrinkPlan shrink_plan(int64_t rows, int64_t groups, int width, int rpad) {
   const int nsteps = (int)ceil_div(width, 64);
   if (rpad <= 16 || nsteps < 16 || nsteps > 64 || rows < 8 * kTileRows * groups)
-    return ShrinkPlan{shrink_kslices(width, rpad), 0};
+    return ShrinkPlan{shrink_kslices(width, rpad), 0, 0};
   const int64_t sets = ceil_div(rows, 8 * kTileRows);
-  int ks = (int)std::min<int64_t>(kOctResident / sets, nsteps / 8);
+  int ks = (int)std::min<int64_t>(kSetBlocks / sets, nsteps / 8);
   ks = std::max(ks, 2);
   const int steps = (int)ceil_div(nsteps, ks);
-  return ShrinkPlan{(int)ceil_div(nsteps, steps), steps};  // no empty slice at the end
+  ks = (int)ceil_div(nsteps, steps);  // no empty slice at the end
+  return ShrinkPlan{ks, steps, rpad > 64 || sets * ks <= oct_blocks(rpad) ? 8 : 4};
 }
 static inline int64_t shrink_partial_bytes(int64_t rows, int64_t groups, int width, int rpad) {
   const int ks = std::max(shrink_kslices(width, rpad), shrink_plan(rows, groups, width, rpad).kslices);
@@ -369,7 +379,7 @@ struct PassArgs {
   int32_t src_rows;  // rows of src / dst (bound for speculative row addresses)
   float* hpart;          // partial sums of the split shrink, [tile][slice][32][rpad]
   int32_t kslices;       // blocks per tile of the MFMA shrink
-  int32_t oct_steps;    // 0: k_shrink_pair; else k_shrink_oct with this many 64-column steps per slice
+  int32_t set_steps;     // 0: k_shrink_pair; else k_shrink_oct / k_shrink_quad with this many 64-column steps per slice
   // the expand weight's rows are permuted inside every group of 128 (TransposeJob::swizzle_a): the row of
   // column c0 + 8 i + q lies at c0 + 16 q + i, so that the 16 rows one MFMA operand load touches are adjacent
   int32_t expand_swizzled;
@@ -381,6 +391,7 @@ struct PassArgs {
   int32_t dst_store;
   WorkList wl_tiles, wl_pairs, wl_octs, wl_sets;  // class_mode: the items of this class (see WorkList)
   TableBounds tb;
+  int32_t set_waves;  // with set_steps: 8 (k_shrink_oct) or 4 (k_shrink_quad), for the launcher
 };
 
 // Optional side job of a weight-gradient launch (bf16 MFMA path): the first `y_blocks` rows of the
