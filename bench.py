@@ -702,7 +702,9 @@ class StepHarness:
 
     def time_steps(self, steps, warmup, first=0):
         """Wall clock around exactly `steps` steps behind `warmup` untimed ones, device synchronised on both sides."""
+        import gc
         import torch
+        gc.collect()  # (33 ms in a process that has imported torch: due now, not in the middle of the timed steps)
         for i in range(warmup):
             self.step(first + i)
         torch.cuda.synchronize()
