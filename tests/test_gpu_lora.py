@@ -597,7 +597,7 @@ sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests")
 import test_gpu_lora as T
 dev = torch.device("cuda:0")
 print("two threads", flush=True)
-T.test_two_host_threads_call_the_two_stream_backward(dev, 3000, 512, 384)
+T.test_two_host_threads_call_the_two_stream_backward(dev, 3000, 512, 384, 32)
 print("graph replay", flush=True)
 T.test_hip_graph_replay_matches_eager(dev, 64, [64, 16, 40], 1200, 256, 1024)
 '''
@@ -615,18 +615,19 @@ def test_every_backward_forked_in_a_child_process(dev):
     assert out.returncode == 0, out.stdout[-2000:] + out.stderr[-2000:]
 
 
-@pytest.mark.parametrize('t,k,m', [(3000, 512, 384),       # one stream per call at this size
-                                   (9000, 1000, 1030)])    # odd widths in bf16 fork from 32 MB of x and dy on
-def test_two_host_threads_call_the_two_stream_backward(dev, t, k, m):
-    """Rank 32 at an output width that is no multiple of 512 takes the backward that can fork onto the library's
-    per-device side stream; two host threads, each on its own stream with its own buffers, must get what they get alone
-    (the kernels are deterministic: bit-equal)."""
+@pytest.mark.parametrize('t,k,m,r', [(3000, 512, 384, 32),       # one stream per call at this size
+                                     (9000, 1000, 1030, 32),     # odd widths in bf16 fork from 32 MB of x and dy on
+                                     (12288, 256, 128, 64)])     # many rows at rank 64
+def test_two_host_threads_call_the_two_stream_backward(dev, t, k, m, r):
+    """Rank 32 at an output width that is no multiple of 512, or rank 64, takes the backward that can fork onto the
+    library's per-device side stream; two host threads, each on its own stream with its own buffers, must get what they
+    get alone (the kernels are deterministic: bit-equal)."""
     import threading
     dt = torch.bfloat16
 
     def make(seed):
-        n, max_r = 3, 32
-        x, base, dy, a, b, ids, ranks, scales = _problem(t, k, m, n, max_r, [32, 20, 32], seed=seed)
+        n = 3
+        x, base, dy, a, b, ids, ranks, scales = _problem(t, k, m, n, r, [r, r - 12, r], seed=seed)
         p = {'x': x.to(dt).to(dev), 'dy': dy.to(dt).to(dev), 'y0': base.to(dt).to(dev)}
         ad, bd = [v.to(dt).to(dev) for v in a], [v.to(dt).to(dev) for v in b]
         p['seg'] = build_segments(ids.to(torch.int32).to(dev), n)

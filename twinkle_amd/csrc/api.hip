@@ -114,6 +114,9 @@ SideStream* side_stream() {
 //                       4096 -> 14336 packed 158 MB 146 / 155
 //     rank 128 packed   96 MB 124 / 135, 128 MB 160 / 164, 156 MB 206 / 184; shuffled 96 MB 150 / 148, 128 MB 200 / 178
 //     fp32 rank 16      256 MB 167 / 166
+//     many rows and a dy no wider than x, whose kernels alone leave the chip idle: rank 64 12288 x 4096 -> 1024 packed 137 /
+//                       127, 12288 x 2048 -> 512 109 / 105, 16384 x 4096 -> 1024 153 / 137, shuffled 172 / 148; 8192 x 4096 ->
+//                       1024 107 / 110; a wider one not: 16384 x 1024 -> 4096 132 / 139, shuffled 158 / 153; rank 128 alike
 //     bf16 on the kernels for any shape   1000 -> 1500 rank 24: 20 MB 77 / 78, 39 MB 118 / 112; 4096 -> 4001 rank 64:
 //                       16 MB 81 / 82, 63 MB 155 / 139 (their launches are small and fill the chip badly)
 //   replay of a captured graph, which pays no host time
@@ -122,10 +125,13 @@ SideStream* side_stream() {
 //     rank 128 packed   64 MB 120 / 115, 96 MB 127 / 130, 128 MB 164 / 155; shuffled 64 MB 152 / 134, 128 MB 203 / 176
 //     bf16 on the kernels for any shape   1000 -> 1500 rank 24: 10 MB 72 / 58; 4001 -> 4096 rank 16: 1 MB 38 / 48, 8 MB 54 / 58,
 //                       31 MB 74 / 71, 127 MB 166 / 138
-bool worth_forking(int64_t bytes, bool any_shape_bf16, int rpad, hipStream_t s) {
+//     highest of several rank classes, next to the others   ranks 16 and 64, 2048 x 2048 -> 1024 99 / 91; ranks 8 to 64, 16384
+//                       rows of it 159 / 138
+bool worth_forking(const tk_lora_desc& d, int64_t bytes, bool any_shape_bf16, int rpad, bool class_mode, hipStream_t s) {
   const int64_t mb = bytes >> 20;
   if (mb >= (any_shape_bf16 ? 32 : rpad > 64 ? 144 : 192)) return true;
-  if (mb < (any_shape_bf16 ? 16 : rpad > 64 ? 64 : 128)) return false;
+  if (d.dtype == TK_DTYPE_BF16 && rpad >= 64 && d.rows >= 12288 && d.in_features >= d.out_features) return true;
+  if (mb < (class_mode ? 0 : any_shape_bf16 ? 16 : rpad > 64 ? 64 : 128)) return false;
   return stream_is_capturing(s);
 }
 
@@ -681,10 +687,13 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   const bool any_shape_bf16 = d->dtype == TK_DTYPE_BF16 &&
                               !(mfma && pass_mfma_supported(a) && (!grad_A || wgrad_mfma_supported(ga)) &&
                                 (!grad_B || wgrad_mfma_supported(gb)));
-  SideStream* side = nullptr;
-  if (grad_B && need_wT && may_fork && side_stream_mode() != 0 &&
-      (side_stream_mode() == 1 || worth_forking(bytes, any_shape_bf16, a.rpad, s)))
-    side = side_stream();
+  // (asked for at the first backward that could fork, at whatever size: a stream made later, behind others of the program,
+  // may share a hardware queue with the caller's, and then nothing runs side by side)
+  SideStream* side = grad_B && need_wT && may_fork && side_stream_mode() != 0 ? side_stream() : nullptr;
+  if (side && side_stream_mode() != 1 && !worth_forking(*d, bytes, any_shape_bf16, a.rpad, class_mode != 0, s)) side = nullptr;
+  // next to the contraction of dB a block of eight waves waits for a CU of its own; with up to 1024 columns of dy that is
+  // most of its time (32768 x 4096 -> 1024 at rank 64: the backward takes 230 us, 258 with k_shrink_oct)
+  if (side && a.rpad <= 64 && a.set_waves == 8 && a.width_src <= 1024) a.set_waves = 4;
   hipStream_t s2 = side ? side->stream : s;
   // two host threads must not interleave their records and waits on the device's one set of events
   std::unique_lock<std::mutex> side_guard;

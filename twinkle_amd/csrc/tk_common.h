@@ -233,8 +233,9 @@ constexpr int kSetBlocks = 512;
 //             12288 x 4096 (384) 46 / 40, 47 / 50; 16384 x 4096 (512) 52 / 47, 60 / 58; 32768 x 4096 79 / 76, 93 / 89
 //   rank 32   4096 x 4096 (128) 23 / 22, 24 / 28; 12288 x 2048 (192) 23 / 23, 24 / 28; 16384 x 2048 (256) 26 / 24, 32 / 28
 //             8192 x 4096 (256) 28 / 24, 33 / 30; 16384 x 4096 (512) 52 / 40, 58 / 48
+//             one adapter, 256 to 2048 rows: the forward takes 32 / 30
 // Rank 128 has only the eight waves.
-static inline int64_t oct_blocks(int rpad) { return rpad <= 32 ? 192 : 256; }
+static inline int64_t oct_blocks(int rpad, int64_t groups) { return rpad > 32 ? 256 : groups > 1 ? 192 : 0; }
 struct ShrinkPlan {
   int kslices;    // slices per tile
   int set_steps;  // 0: k_shrink_pair; else steps per slice of the kernels that own eight tiles
@@ -249,7 +250,7 @@ static inline ShrinkPlan shrink_plan(int64_t rows, int64_t groups, int width, in
   ks = std::max(ks, 2);
   const int steps = (int)ceil_div(nsteps, ks);
   ks = (int)ceil_div(nsteps, steps);  // no empty slice at the end
-  return ShrinkPlan{ks, steps, rpad > 64 || sets * ks <= oct_blocks(rpad) ? 8 : 4};
+  return ShrinkPlan{ks, steps, rpad > 64 || sets * ks <= oct_blocks(rpad, groups) ? 8 : 4};
 }
 static inline int64_t shrink_partial_bytes(int64_t rows, int64_t groups, int width, int rpad) {
   const int ks = std::max(shrink_kslices(width, rpad), shrink_plan(rows, groups, width, rpad).kslices);
