@@ -123,8 +123,8 @@ SideStream* side_stream() {
 //     rank 64 packed    96 MB 104 / 109, 128 MB 123 / 122, 156 MB 162 / 140; shuffled 128 MB 136 / 126; fp32 rank 16: 64 MB
 //                       66 / 70, 128 MB 96 / 89
 //     rank 128 packed   64 MB 120 / 115, 96 MB 127 / 130, 128 MB 164 / 155; shuffled 64 MB 152 / 134, 128 MB 203 / 176
-//     bf16 on the kernels for any shape   1000 -> 1500 rank 24: 10 MB 72 / 58; 4001 -> 4096 rank 16: 1 MB 38 / 48, 8 MB 54 / 58,
-//                       31 MB 74 / 71, 127 MB 166 / 138
+//     bf16 on the kernels for any shape   1000 -> 1500 rank 24: 10 MB 72 / 58; 4001 -> 4096 rank 16: 1 MB 38 / 48, 8 MB
+//                       54 / 58, 31 MB 74 / 71, 127 MB 166 / 138
 //     highest of several rank classes, next to the others   ranks 16 and 64, 2048 x 2048 -> 1024 99 / 91; ranks 8 to 64, 16384
 //                       rows of it 159 / 138
 bool worth_forking(const tk_lora_desc& d, int64_t bytes, bool any_shape_bf16, int rpad, bool class_mode, hipStream_t s) {
