@@ -847,14 +847,15 @@ void launch_pass_any(const PassArgs& a0, const SegView& seg, const SegLayout& L,
   // launch that adds the slices and their way through memory.  Many tiles always: (one block / slices, us) fp32 8192 x 1536
   // rank 8 25 / 29, rank 128 68 / 83; bf16 32768 x 1000 rank 128 101 / 130.  Few tiles leave the chip idle meanwhile, so
   // there by the length of the steps, which grows with width and rank and is longer in fp32 (an eighth of the products per
-  // instruction): fp32 512 x 1024 rank 8 16.1 / 16.8, rank 32 x 1536 23.6 / 21.3 and at 3072 rows 26.1 / 27.8; 2048 x 1536
+  // instruction): fp32 512 x 1024 rank 8 16.1 / 16.8, 512 x 1536 rank 32 23.6 / 21.3 and at 3072 rows 26.1 / 27.8; 2048 x 1536
   // rank 64 37.6 / 28.9, rank 128 60.4 / 43.1, 4096 x 1024 rank 128 51.5 / 47.0; bf16 2048 x 1500 rank 32 22.7 / 24.2, rank
-  // 64 equal, 1024 x 1500 rank 128 40.0 / 35.5.
+  // 64 equal, 1024 x 1500 rank 128 40.0 / 35.5.  (fp32 512 x 1536 rank 8: 18.5 / 17.0 on the GPU, but a launch less of an eager
+  // pass that the host sets the pace of: 387 rows of 18 adapters 34 / 37.)
   PassArgs a = a0;
   if (a.kslices <= 3 && a.width_src <= 1536) {
     const int64_t tiles = L.live_tiles();
     const bool some = tiles >= 96;
-    const bool one = tiles >= 192 || (sizeof(T) == 4 ? NB <= 2 && (a.width_src <= 1280 || some) : NB <= 4 || some);
+    const bool one = tiles >= 192 || (sizeof(T) == 4 ? NB == 1 || (NB == 2 && (a.width_src <= 1280 || some)) : NB <= 4 || some);
     if (one) a.kslices = 1;
   }
   const int32_t* rows = seg.slot_table(a.map_rows);
