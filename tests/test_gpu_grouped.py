@@ -189,6 +189,61 @@ def test_register_staged_kernels_behind_the_switch(dev, monkeypatch, transposed)
     assert max_rel_err(grouped_linear_(xd, wd, seg, nt, groups=groups, h=h, map_rows=True), want) < 2e-2
 
 
+@pytest.mark.parametrize('max_r,ranks,sizes', [
+    (8, [8] * 12, 20),                    # a row block of eight groups, one 64-deep step of LoRA weights
+    (16, [16] * 12, 20),                  # two steps
+    (64, [64, 33, 0, 64, 7, 64], 40),     # a step per group
+    (16, [12, 5, 12], 70),                # ranks that end inside a piece
+    (24, [24, 8], 300),
+])
+@pytest.mark.parametrize('offset', [0, 3])   # elements the adapters start off a 16-byte boundary
+def test_lora_step_of_the_direct_kernel(dev, max_r, ranks, sizes, offset):
+    """Row blocks with several groups and steps, ranks that end inside a piece, matrices that are not 16-byte aligned, and
+    isolation: one tenant's B holds infinities, NaN and the largest values, which may reach its own rows only."""
+    e, nt, k, n = 2, len(ranks), 128, 256
+    expert = torch.arange(e).repeat_interleave(nt * sizes)
+    tenant = torch.arange(nt).repeat_interleave(sizes).repeat(e)
+    t = expert.numel()
+    g = torch.Generator().manual_seed(max_r + offset)
+    x = torch.randn(t, k, generator=g).bfloat16()
+    w = (torch.randn(e, n, k, generator=g) / k**0.5).bfloat16()
+    bad = nt - 1
+
+    def shifted(*shape, std):
+        flat = torch.empty(offset + shape[0] * shape[1] * shape[2], dtype=torch.bfloat16, device=dev)
+        v = flat[offset:].view(shape)
+        return v.copy_((torch.randn(*shape, generator=g) * std).bfloat16())
+
+    a = [shifted(e, max_r, k, std=k**-0.5) for _ in range(nt)]
+    b = [shifted(e, n, max_r, std=0.05) for _ in range(nt)]
+    b[bad].view(-1)[::3] = float('inf')
+    b[bad].view(-1)[1::3] = float('nan')
+    b[bad].view(-1)[2::3] = torch.finfo(torch.bfloat16).max
+    for v, r in zip(b, ranks):            # columns past a tenant's rank are nobody's: they may hold anything
+        v[..., r:] = float('nan')
+    idx = [i % nt for i in range(e * nt)]
+    groups = AdapterGroups(a, b, [ranks[i % nt] for i in range(e * nt)], [2.0] * (e * nt), a_index=idx,
+                           a_offset=[(i // nt) * max_r * k for i in range(e * nt)], b_index=idx,
+                           b_offset=[(i // nt) * n * max_r for i in range(e * nt)], rank_classes=False)
+    seg = build_segments((expert * nt + tenant).to(torch.int32).to(dev), e * nt)
+    xd, wd = x.to(dev), w.to(dev)
+    h = torch.empty(lora_h_bytes(seg, groups), dtype=torch.uint8, device=dev)
+    lora_shrink_(xd, seg, groups, h, map_rows=False)
+    got = grouped_linear_(xd, wd, seg, nt, groups=groups, h=h, map_rows=False).cpu()
+    want = _reference(x, w, expert)
+    own = tenant == bad
+    if ranks[bad] > 0:
+        assert not torch.isfinite(got[own]).all()
+    for ei in range(e):
+        for ti in range(nt):
+            rows = ((expert == ei) & (tenant == ti)).nonzero().flatten()
+            if ti != bad and ranks[ti] > 0:
+                r = ranks[ti]
+                want[rows] += 2.0 * (x[rows].double() @ a[ti][ei, :r].double().cpu().t()) @ b[ti][ei, :, :r].double().cpu().t()
+    # h and y are rounded to eight bits once each
+    assert max_rel_err(got[~own], want[~own]) < 1e-2
+
+
 def test_unsupported_shapes_are_refused(dev):
     e, nt, t = 2, 1, 64
     keys = torch.zeros(t, dtype=torch.int32, device=dev)

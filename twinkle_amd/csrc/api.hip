@@ -843,6 +843,7 @@ int tk_grouped_linear(const tk_grouped_desc* g, const tk_lora_desc* lora, const 
       return TK_ERR_INVALID;
     if (lora->max_rank > 64) return TK_ERR_UNSUPPORTED;
     a.rpad = rank_pad(lora->max_rank);
+    a.rshift = lora->max_rank <= 8 ? 3 : a.rpad == 16 ? 4 : a.rpad == 32 ? 5 : 6;
     tk_lora_desc staged;
     if (mixed_weights(*lora)) {
       // fp32 adapters: the epilogue multiplies with the bf16 copy of B, made in the tail of h like tk_lora_expand

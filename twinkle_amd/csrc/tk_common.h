@@ -493,10 +493,16 @@ int launch_expand_shared_wide(const SharedExpandArgs& a, int rpad, const SegView
 int launch_wgrad_coop_multi(const SharedWgradArgs& a, const SegView& seg, const SegLayout& L, hipStream_t s);
 
 // kernels_grouped.hip
-struct GroupedPlanEntry {  // a row block of the grouped GEMM: up to 4 consecutive tiles of one expert
+struct GroupedPlanEntry {  // a row block of the grouped GEMM: up to 8 consecutive tiles of one expert
   int32_t tile0, ntiles, expert;
   int32_t first, count;  // the expert's row blocks are the entries [first, first + count)
-  int32_t pad;
+  int32_t ngroups;       // distinct groups with a LoRA term among the tiles
+  int32_t pad[2];
+  int32_t pos[8];        // tile t: sorted position of its first row
+  int32_t cnt[8];        //         its rows
+  int32_t number[8];     //         its group's place among those, -1 without a LoRA term
+  int32_t rank[8];       // of the groups: live rank, matrix
+  const uint16_t* matrix[8];
 };
 struct GroupedArgs {
   const uint16_t* x;  int64_t ldx;                     // activations, rows reached through the slot table
@@ -507,6 +513,7 @@ struct GroupedArgs {
   // LoRA term (rpad = 0: none): y += h B_g^T with h[slot][rpad] as the shrink kernels leave it
   const void* const* lora_B;  int64_t ldb;
   const int32_t* rank;  int32_t rpad;
+  int32_t rshift;                                      // log2 of the rank indices a group takes of a step (3 .. 6)
   const uint16_t* hrow;
   TableBounds tb;
 };
