@@ -228,6 +228,21 @@ int tk_lora_bwd_store(const tk_lora_desc* desc, const void* dy_device, int64_t l
                       const void* h_device, void* dx_device, int64_t lddx, void* const* grad_A, void* const* grad_B,
                       int32_t accumulate, void* workspace_device, int64_t workspace_bytes, tk_stream_t stream);
 
+/* tk_lora_bwd (store_dx 0) or tk_lora_bwd_store (1) with the gradients of either matrix inside one buffer: group g's lies
+ * base_A + at_A[g] bytes in (at_A device array [G], laid out once; the base changes with every call's buffer).  A null
+ * table: those gradients are not wanted. */
+int tk_lora_bwd_into(const tk_lora_desc* desc, const void* dy_device, int64_t lddy, const void* x_device, int64_t ldx,
+                     const void* h_device, void* dx_device, int64_t lddx, int32_t store_dx, const int64_t* at_A,
+                     void* base_A, const int64_t* at_B, void* base_B, void* workspace_device, int64_t workspace_bytes,
+                     tk_stream_t stream);
+
+/* tk_lora_bwd_shared with gradients placed like those of tk_lora_bwd_into; tables and bases per projection (host arrays). */
+int tk_lora_bwd_shared_into(const tk_lora_desc* const* descs, int32_t n, const void* const* dy_device, const int64_t* lddy,
+                            const void* x_device, int64_t ldx, const void* const* h_device, void* dx_device, int64_t lddx,
+                            const int64_t* const* at_A, void* const* base_A, const int64_t* const* at_B,
+                            void* const* base_B, void* const* workspace_device, const int64_t* workspace_bytes,
+                            tk_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Multi-tenant optimizer step over adapter tensors (one launch set for all tenants).
  *

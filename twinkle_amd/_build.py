@@ -18,6 +18,26 @@ HIPCC_FLAGS = [
 ]
 
 
+# the autograd nodes of the plain path: a Python extension on torch's C++ interface, linked to the library above
+HOST_SOURCE = 'host_torch.cpp'
+HOST_PATH = os.path.join(os.path.dirname(CSRC), '_host.so')
+
+
+def _host_commands(obj: str):
+    import sysconfig
+
+    import torch
+    root = torch.__path__[0]
+    system = [os.path.join(root, 'include'), os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'),
+              '/opt/rocm/include', sysconfig.get_paths()['include']]
+    compile_ = ['g++', '-O2', '-std=c++17', '-fPIC', '-D__HIP_PLATFORM_AMD__', '-DUSE_ROCM',
+                f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+                *[a for d in system for a in ('-isystem', d)], '-I', INCLUDE, '-c', os.path.join(CSRC, HOST_SOURCE), '-o', obj]
+    link = ['g++', '-shared', obj, '-o', HOST_PATH, '-L', os.path.join(root, 'lib'), '-ltorch_python', '-ltorch',
+            '-ltorch_cpu', '-lc10', '-lc10_hip', '-L', CSRC, '-ltwinkle_amd', '-Wl,-rpath,$ORIGIN/csrc']
+    return compile_, link
+
+
 def build_library(verbose: bool = False) -> str:
     """Compile every HIP source (side by side) and link ``csrc/libtwinkle_amd.so``; returns its path."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
@@ -25,7 +45,7 @@ def build_library(verbose: bool = False) -> str:
     def run(cmd) -> str:
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
-            raise RuntimeError('hipcc failed:\n' + ' '.join(cmd) + '\n' + proc.stdout + proc.stderr)
+            raise RuntimeError('compiling failed:\n' + ' '.join(cmd) + '\n' + proc.stdout + proc.stderr)
         return proc.stderr
 
     with tempfile.TemporaryDirectory() as tmp:
@@ -33,8 +53,10 @@ def build_library(verbose: bool = False) -> str:
         compiles = [[hipcc, *HIPCC_FLAGS, '-I', INCLUDE, '-I', CSRC, '-c', os.path.join(CSRC, s), '-o', o]
                     for s, o in zip(SOURCES, objects)]
         with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
-            notes = list(pool.map(run, compiles))
+            host_compile, host_link = _host_commands(os.path.join(tmp, 'host_torch.o'))
+            notes = list(pool.map(run, [*compiles, host_compile]))
         notes.append(run([hipcc, '--offload-arch=gfx950', '-shared', *objects, '-o', LIB_PATH]))
+        notes.append(run(host_link))
     if verbose:
         print('\n'.join(n for n in notes if n))
     return LIB_PATH

@@ -12,7 +12,9 @@ from ctypes import POINTER, Structure, c_char_p, c_float, c_int32, c_int64, c_vo
 
 import torch  # noqa: F401  (must come first: brings in the HIP runtime the library binds to)
 
-from ._build import LIB_PATH
+from torch.autograd import forward_ad
+
+from ._build import HOST_PATH, LIB_PATH
 
 TK_OK = 0
 TK_ERR_INVALID = -1
@@ -96,10 +98,14 @@ EXPORTS = {
                               c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
     'tk_lora_bwd_store': (c_int32, [POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                     c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
+    'tk_lora_bwd_into': (c_int32, [POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
+                                   c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     # arrays indexed by projection are host arrays: pointers to descriptors / device pointers / strides
     'tk_lora_fwd_shared': (c_int32, [c_void_p, c_int32, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     'tk_lora_bwd_shared': (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
                                      c_int64, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
+    'tk_lora_bwd_shared_into': (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
+                                          c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     'tk_grouped_linear_workspace_bytes': (c_int64, [POINTER(GroupedDesc)]),
     'tk_grouped_linear': (c_int32, [POINTER(GroupedDesc), POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64,
                                     c_void_p, c_void_p, c_int64, c_void_p]),
@@ -136,6 +142,25 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The autograd nodes of the plain path (csrc/host_torch.cpp), ``None`` where a call has to take the Python one whatever
+    its tensors are: under a tracing compiler and inside forward-mode differentiation."""
+    global _host
+    if torch.compiler.is_dynamo_compiling() or forward_ad._current_level >= 0:
+        return None
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f'{HOST_PATH} is missing: build it with `python -m twinkle_amd._build` '
+                               '(or __graft_entry__.build()); there is no fallback path')
+        from . import _host as module
+        _host = module
+    return _host
 
 
 def check(code: int, what: str) -> None:

@@ -534,6 +534,13 @@ static PassArgs fwd_pass_args(const tk_lora_desc* d, const void* x, int64_t ldx,
   return a;
 }
 
+// Where the weight gradients go: group g's at table[g] + base (either table null: those are not wanted).
+struct GradTables {
+  void* const* A;
+  void* const* B;
+  uint64_t base_A, base_B;
+};
+
 // Everything the backward of one projection needs, carved from its workspace.
 struct BwdPlan {
   WgradArgs ga{}, gb{};  // dA[n][k] = sum_rows dh[row][n] x[row][k];  dB[m][n] = sum_rows dy[row][m] h[row][n]
@@ -545,8 +552,9 @@ struct BwdPlan {
 };
 
 static BwdPlan bwd_plan(const tk_lora_desc* d, const BwdLayout& B, const void* dy, int64_t lddy, const void* x,
-                        int64_t ldx, const void* h, void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B,
-                        int32_t accumulate, void* ws, int rank_lo = 0, int class_mode = 0) {
+                        int64_t ldx, const void* h, void* dx, int64_t lddx, const GradTables& grads, int32_t accumulate,
+                        void* ws, int rank_lo = 0, int class_mode = 0) {
+  void* const *grad_A = grads.A, *const *grad_B = grads.B;
   BwdPlan p;
   p.ga.rank_lo = p.gb.rank_lo = p.a.rank_lo = p.tr.rank_lo = rank_lo;
   p.a.class_mode = class_mode;
@@ -560,7 +568,7 @@ static BwdPlan bwd_plan(const tk_lora_desc* d, const BwdLayout& B, const void* d
     g.src = dy;  g.ld_src = lddy;
     g.hT = h;    g.ldh = B.ldh;
     g.partial = (float*)(w + B.off_part_b);
-    g.grad = grad_B;  g.ld_grad = d->ldb;
+    g.grad = grad_B;  g.grad_base = grads.base_B;  g.ld_grad = d->ldb;
     g.rank = d->rank;  g.width = d->out_features;  g.transposed = 1;
     g.accumulate = accumulate;  g.map_rows = d->map_rows;  g.rpad = (int32_t)B.rpad;
   }
@@ -569,7 +577,7 @@ static BwdPlan bwd_plan(const tk_lora_desc* d, const BwdLayout& B, const void* d
     g.src = x;  g.ld_src = ldx;
     g.hT = p.dh;  g.ldh = B.ldh;
     g.partial = (float*)(w + B.off_part_a);
-    g.grad = grad_A;  g.ld_grad = d->lda;
+    g.grad = grad_A;  g.grad_base = grads.base_A;  g.ld_grad = d->lda;
     g.rank = d->rank;  g.width = d->in_features;  g.transposed = 0;
     g.accumulate = accumulate;  g.map_rows = d->map_rows;  g.rpad = (int32_t)B.rpad;
   }
@@ -647,15 +655,16 @@ int tk_lora_expand(const tk_lora_desc* d, const void* h, void* y, int64_t ldy, t
 
 // The backward of the groups of one rank class (d: the class's descriptor; every group when there is one class).
 static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, const void* dy, int64_t lddy,
-                          const void* x, int64_t ldx, const void* h, void* dx, int64_t lddx, void* const* grad_A,
-                          void* const* grad_B, int32_t accumulate, bool store_dx, void* ws, hipStream_t s, bool may_fork) {
+                          const void* x, int64_t ldx, const void* h, void* dx, int64_t lddx, const GradTables& grads,
+                          int32_t accumulate, bool store_dx, void* ws, hipStream_t s, bool may_fork) {
+  void* const *grad_A = grads.A, *const *grad_B = grads.B;
   const int rank_lo = P.rc[c].lo, class_mode = P.n > 1;
   BwdLayout B(*d);
   SegLayout L(d->rows, d->num_groups);
   SegView V(d->seg_ws, L);
   int rc;
   const bool need_wT = dx || grad_A;
-  BwdPlan plan = bwd_plan(d, B, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate, ws, rank_lo, class_mode);
+  BwdPlan plan = bwd_plan(d, B, dy, lddy, x, ldx, h, dx, lddx, grads, accumulate, ws, rank_lo, class_mode);
   use_lists(P, c, L, &plan.a, &plan.ga, &plan.gb);
   plan.a.dst_store = store_dx ? 1 : 0;
   WgradArgs &ga = plan.ga, &gb = plan.gb;
@@ -746,8 +755,8 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
 }
 
 static int lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
-                    void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, bool store_dx,
-                    void* ws, int64_t ws_bytes, tk_stream_t stream) {
+                    void* dx, int64_t lddx, const GradTables& grads, int32_t accumulate, bool store_dx, void* ws,
+                    int64_t ws_bytes, tk_stream_t stream) {
   if (!desc_ok(d)) return TK_ERR_INVALID;
   if (d->rows == 0 || (d->max_rank == 0 && !(store_dx && dx))) return TK_OK;
   if (d->max_rank == 0) {  // every row is written: zeros
@@ -758,8 +767,8 @@ static int lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const v
   }
   if (!dy || lddy < d->out_features || !ws) return TK_ERR_INVALID;
   if (dx && lddx < d->in_features) return TK_ERR_INVALID;
-  if (grad_A && (!x || ldx < d->in_features)) return TK_ERR_INVALID;
-  if (grad_B && !h) return TK_ERR_INVALID;
+  if (grads.A && (!x || ldx < d->in_features)) return TK_ERR_INVALID;
+  if (grads.B && !h) return TK_ERR_INVALID;
   ClassPlan P = class_plan(d);
   if (ws_bytes < P.ws_total) return TK_ERR_WORKSPACE;
   {
@@ -775,21 +784,29 @@ static int lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const v
   // workspace; of h (one layout, written by the forward at the largest padded rank) it reads the rank-major copy,
   // whose row stride does not depend on the padded rank, up to its own padded rank.
   return for_each_class(P.n, (hipStream_t)stream, [&](int c, hipStream_t cs, bool forked) {
-    return lora_bwd_class(&P.d[c], P, c, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate,
-                          store_dx, (char*)ws + P.ws_off[c], cs, !forked);
+    return lora_bwd_class(&P.d[c], P, c, dy, lddy, x, ldx, h, dx, lddx, grads, accumulate, store_dx,
+                          (char*)ws + P.ws_off[c], cs, !forked);
   });
 }
 
 int tk_lora_bwd(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
                 void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, void* ws,
                 int64_t ws_bytes, tk_stream_t stream) {
-  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate, false, ws, ws_bytes, stream);
+  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, {grad_A, grad_B, 0, 0}, accumulate, false, ws, ws_bytes, stream);
 }
 
 int tk_lora_bwd_store(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
                       void* dx, int64_t lddx, void* const* grad_A, void* const* grad_B, int32_t accumulate, void* ws,
                       int64_t ws_bytes, tk_stream_t stream) {
-  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, grad_A, grad_B, accumulate, true, ws, ws_bytes, stream);
+  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, {grad_A, grad_B, 0, 0}, accumulate, true, ws, ws_bytes, stream);
+}
+
+int tk_lora_bwd_into(const tk_lora_desc* d, const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* h,
+                     void* dx, int64_t lddx, int32_t store_dx, const int64_t* at_A, void* base_A, const int64_t* at_B,
+                     void* base_B, void* ws, int64_t ws_bytes, tk_stream_t stream) {
+  if ((at_A && !base_A) || (at_B && !base_B)) return TK_ERR_INVALID;
+  const GradTables grads{(void* const*)at_A, (void* const*)at_B, (uint64_t)base_A, (uint64_t)base_B};
+  return lora_bwd(d, dy, lddy, x, ldx, h, dx, lddx, grads, 0, store_dx != 0, ws, ws_bytes, stream);
 }
 
 // ---- packed experts: grouped base GEMM (+ LoRA term) ---------------------------------------------------------------
@@ -1004,13 +1021,13 @@ int tk_lora_fwd_shared(const tk_lora_desc* const* descs_in, int32_t n, const voi
   return launch_pass_multi(a, n, V, L, 4 | 2, s);
 }
 
-int tk_lora_bwd_shared(const tk_lora_desc* const* descs_in, int32_t n, const void* const* dy, const int64_t* lddy,
-                       const void* x, int64_t ldx, const void* const* h, void* dx, int64_t lddx,
-                       void* const* const* grad_A, void* const* const* grad_B, int32_t accumulate, void* const* ws,
-                       const int64_t* ws_bytes, tk_stream_t stream) {
+static int lora_bwd_shared(const tk_lora_desc* const* descs_in, int32_t n, const void* const* dy, const int64_t* lddy,
+                           const void* x, int64_t ldx, const void* const* h, void* dx, int64_t lddx,
+                           const GradTables* grads, int32_t accumulate, void* const* ws, const int64_t* ws_bytes,
+                           tk_stream_t stream) {
   const SingleClassDescs local(descs_in, n);
   const tk_lora_desc* const* descs = descs_in ? local.p : nullptr;
-  if (!shared_descs_ok(descs, n) || !dy || !lddy || !h || !grad_A || !grad_B || !ws || !ws_bytes) return TK_ERR_INVALID;
+  if (!shared_descs_ok(descs, n) || !dy || !lddy || !h || !ws || !ws_bytes) return TK_ERR_INVALID;
   const tk_lora_desc* d0 = descs[0];
   if (d0->rows == 0) return TK_OK;
   if (!x || ldx < d0->in_features || !dx || lddx < d0->in_features) return TK_ERR_INVALID;
@@ -1021,14 +1038,14 @@ int tk_lora_bwd_shared(const tk_lora_desc* const* descs_in, int32_t n, const voi
   bool fast = shared_fast_path(descs, n);
   for (int p = 0; p < n; ++p) {
     const tk_lora_desc* d = descs[p];
-    if (!dy[p] || lddy[p] < d->out_features || !h[p] || !grad_A[p] || !grad_B[p] || !ws[p]) return TK_ERR_INVALID;
+    if (!dy[p] || lddy[p] < d->out_features || !h[p] || !grads[p].A || !grads[p].B || !ws[p]) return TK_ERR_INVALID;
     BwdLayout B(*d);
     if (ws_bytes[p] < B.total) return TK_ERR_WORKSPACE;
     if (d->max_rank == 0) {
       fast = false;
       continue;
     }
-    plan[p] = bwd_plan(d, B, dy[p], lddy[p], x, ldx, h[p], dx, lddx, grad_A[p], grad_B[p], accumulate, ws[p]);
+    plan[p] = bwd_plan(d, B, dy[p], lddy[p], x, ldx, h[p], dx, lddx, grads[p], accumulate, ws[p]);
     fast = fast && pass_mfma_supported(plan[p].a) && dy_fused_supported(plan[p].gb, plan[p].a.kslices) &&
            wgrad_mfma_supported(plan[p].ga);
   }
@@ -1077,8 +1094,8 @@ int tk_lora_bwd_shared(const tk_lora_desc* const* descs_in, int32_t n, const voi
       return launch_wgrad_reduce_multi(red, 2 * n, V, L, s);
     }
     for (int p = 0; p < n; ++p)
-      if ((rc = tk_lora_bwd(descs[p], dy[p], lddy[p], x, ldx, h[p], dx, lddx, grad_A[p], grad_B[p], accumulate, ws[p],
-                            ws_bytes[p], stream)) != TK_OK)
+      if ((rc = lora_bwd(descs[p], dy[p], lddy[p], x, ldx, h[p], dx, lddx, grads[p], accumulate, false, ws[p], ws_bytes[p],
+                         stream)) != TK_OK)
         return rc;
     return TK_OK;
   }
@@ -1112,6 +1129,29 @@ int tk_lora_bwd_shared(const tk_lora_desc* const* descs_in, int32_t n, const voi
   if ((rc = launch_expand_shared(ea, V, L, s)) != TK_OK) return rc;  // dx += sum_p dh_p A_p
   if ((rc = launch_wgrad_shared(wa, V, L, s)) != TK_OK) return rc;   // dA_p for all p, x read once
   return launch_wgrad_reduce_multi(red, 2 * n, V, L, s);
+}
+
+int tk_lora_bwd_shared(const tk_lora_desc* const* descs, int32_t n, const void* const* dy, const int64_t* lddy, const void* x,
+                       int64_t ldx, const void* const* h, void* dx, int64_t lddx, void* const* const* grad_A,
+                       void* const* const* grad_B, int32_t accumulate, void* const* ws, const int64_t* ws_bytes,
+                       tk_stream_t stream) {
+  if (!grad_A || !grad_B || n < 1 || n > TK_MAX_SHARED) return TK_ERR_INVALID;
+  GradTables grads[TK_MAX_SHARED] = {};
+  for (int p = 0; p < n; ++p) grads[p] = GradTables{grad_A[p], grad_B[p], 0, 0};
+  return lora_bwd_shared(descs, n, dy, lddy, x, ldx, h, dx, lddx, grads, accumulate, ws, ws_bytes, stream);
+}
+
+int tk_lora_bwd_shared_into(const tk_lora_desc* const* descs, int32_t n, const void* const* dy, const int64_t* lddy,
+                            const void* x, int64_t ldx, const void* const* h, void* dx, int64_t lddx,
+                            const int64_t* const* at_A, void* const* base_A, const int64_t* const* at_B, void* const* base_B,
+                            void* const* ws, const int64_t* ws_bytes, tk_stream_t stream) {
+  if (!at_A || !base_A || !at_B || !base_B || n < 1 || n > TK_MAX_SHARED) return TK_ERR_INVALID;
+  GradTables grads[TK_MAX_SHARED] = {};
+  for (int p = 0; p < n; ++p) {
+    if (!base_A[p] || !base_B[p]) return TK_ERR_INVALID;
+    grads[p] = GradTables{(void* const*)at_A[p], (void* const*)at_B[p], (uint64_t)base_A[p], (uint64_t)base_B[p]};
+  }
+  return lora_bwd_shared(descs, n, dy, lddy, x, ldx, h, dx, lddx, grads, 0, ws, ws_bytes, stream);
 }
 
 int64_t tk_opt_workspace_bytes(int32_t num_tensors, int64_t max_numel) {

@@ -379,7 +379,7 @@ __device__ inline void store_grad(const WgradArgs& a, int g, int n, int c, float
     store_grad<float>(a, g, n, c, v);
     return;
   }
-  T* gp = (T*)a.grad[g];
+  T* gp = grad_of<T>(a, g);
   T* o = a.transposed ? gp + (int64_t)c * a.ld_grad + n : gp + (int64_t)n * a.ld_grad + c;
   if (a.accumulate) v += to_f32(*o);
   from_f32(v, o);
@@ -551,7 +551,7 @@ __device__ __forceinline__ void wgrad_reduce_body(const WgradArgs& a, int n0, co
   const int nlive = PAIRED && nchunk > 0 ? live_partials(nchunk, pf) : nchunk;  // (no chunks: zeros are written)
   auto slot = [&](int m) { return PAIRED ? live_partial(m, pf) : m; };
   const int64_t stride = partial_slot_floats(a.rpad, a.width);
-  T* const gt = (T*)a.grad[g];
+  T* const gt = grad_of<T>(a, g);
   if (a.transposed && (a.ld_grad & (sizeof(T) == 2 ? 7 : 3)) == 0 && (reinterpret_cast<uintptr_t>(gt) & 15u) == 0 &&
       (r & 7) == 0) {
     // A transposed gradient ([width][r], dB) whose rows are whole 16-byte pieces.  With a thread per column and an
@@ -644,7 +644,7 @@ __device__ __forceinline__ void wgrad_reduce_body(const WgradArgs& a, int n0, co
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] += v[j][i];
   }
-  T* gp = (T*)a.grad[g];
+  T* gp = grad_of<T>(a, g);
   if (sizeof(T) == 2 && a.transposed && n0 + 8 <= r && (a.ld_grad & 7) == 0 &&
       (reinterpret_cast<uintptr_t>(gp) & 15u) == 0) {
     uint4* o = reinterpret_cast<uint4*>(gp + (int64_t)c * a.ld_grad + n0);

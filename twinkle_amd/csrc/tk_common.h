@@ -416,7 +416,8 @@ struct WgradArgs {
   const void* src;  int64_t ld_src;   // x | dy
   const void* hT;   int64_t ldh;      // dh | h
   float* partial;                     // [max_partials][width / 128][rpad][128], see partial_index
-  void* const* grad;                  // device array [G]
+  void* const* grad;                  // device array [G], counted from grad_base
+  uint64_t grad_base;
   int64_t ld_grad;
   const int32_t* rank;
   int32_t width;       // K | M

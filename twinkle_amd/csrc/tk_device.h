@@ -26,6 +26,12 @@ __device__ inline const T* group_weight(const void* const* ptrs, const void* bas
   return ptrs ? (const T*)ptrs[g] : (const T*)base + (int64_t)g * stride;
 }
 
+// Gradient of group g: the table's entries are addresses, or places in the buffer at grad_base.
+template <typename T>
+__device__ inline T* grad_of(const WgradArgs& a, int g) {
+  return reinterpret_cast<T*>(reinterpret_cast<uint64_t>(a.grad[g]) + a.grad_base);
+}
+
 // Entries of the segment table before they are used as indices (see TableBounds).
 __device__ inline int checked_group(int g, const TableBounds& tb) { return (unsigned)g < (unsigned)tb.groups ? g : -1; }
 __device__ inline int checked_row(int r, const TableBounds& tb) { return (unsigned)r < (unsigned)tb.rows ? r : -1; }

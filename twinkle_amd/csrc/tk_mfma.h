@@ -149,7 +149,7 @@ __device__ inline void wgrad_store(const f32x4 (&acc)[8][NB], float* lds, const 
     return;
   }
   if (a.grad_f32) {  // fp32 gradients next to bf16 activations: the same two walks with fp32 stores
-    float* gf = (float*)a.grad[g];
+    float* gf = grad_of<float>(a, g);
     const bool vecf = (reinterpret_cast<uintptr_t>(gf) & 15u) == 0 && (a.ld_grad & 3) == 0;
     if (!a.transposed) {
 #pragma unroll
@@ -176,7 +176,7 @@ __device__ inline void wgrad_store(const f32x4 (&acc)[8][NB], float* lds, const 
     }
     return;
   }
-  bf16_t* gp = (bf16_t*)a.grad[g];
+  bf16_t* gp = grad_of<bf16_t>(a, g);
   const bool vec = (reinterpret_cast<uintptr_t>(gp) & 15u) == 0 && (a.ld_grad & 7) == 0;
   if (!a.transposed) {
     // grad[n][c0 + c]: four rows of 128 columns per step

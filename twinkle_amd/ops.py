@@ -116,6 +116,7 @@ class AdapterGroups:
         rel_b = [(self._b_arena_off[j] + o) * esz for j, o in zip(self.b_index, self.b_offset)]
         self._grad_a_rel, self._grad_b_rel = torch.tensor([rel_a, rel_b], dtype=torch.int64, device=dev).unbind(0)
         self._arena_plan = None
+        self._host = None
         self._ptr_key = None
         self._size_cache = {}
         self._desc_template = self._desc_key = None
@@ -160,6 +161,25 @@ class AdapterGroups:
                 shapes.append((len(sizes), *sizes[0]) if alike else None)
             self._arena_plan = (zeros, *shapes)
         return self._arena_plan
+
+    def host_groups(self):
+        """This object as the C++ nodes know it; ``None`` with master weights, which only the Python nodes serve."""
+        if self._host is None and self.master_a is None:
+            self.refresh()
+            sides = (('a', self.a_tensors, self.a_index, self.a_offset, self.a_live, self._a_arena_off, self.a_arena_elems,
+                      self._grad_a_rel, self.a_ptrs),
+                     ('b', self.b_tensors, self.b_index, self.b_offset, self.b_live, self._b_arena_off, self.b_arena_elems,
+                      self._grad_b_rel, self.b_ptrs))
+            names = ('tensors', 'index', 'offset', 'live', 'at', 'elems', 'grads_at', 'pointers')
+            fields = {f'{side[0]}_{name}': value for side in sides for name, value in zip(names, side[1:])}
+            self._host = _lib.host().make_groups(dict(
+                fields, rank=self.rank_dev, scale=self.scale_dev, in_features=self.in_features,
+                out_features=self.out_features, max_rank=self.max_rank, dtype=_lib.dtype_code(self.dtype), lda=self.lda,
+                ldb=self.ldb, weights_f32=int(self.weights_f32), rank_classes=self.rank_classes))
+            self._host_plan = False
+        if not self._host_plan and self._host is not None and torch.is_grad_enabled():
+            self._host.zeros, self._host_plan = self.arena_plan()[0], True
+        return self._host
 
     def refresh(self) -> None:
         """Rebuild the device pointer arrays if a parameter's storage moved."""
@@ -587,12 +607,29 @@ def grouped_experts_linear(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTa
 def multi_lora_delta(x: torch.Tensor, base_out: torch.Tensor, seg: SegmentTable, groups: AdapterGroups,
                      map_rows: bool = True) -> torch.Tensor:
     """``base_out`` with every adapter's LoRA term added to its own rows (in place, differentiable)."""
+    host = _lib.host()
+    handle = groups.host_groups() if host is not None else None
+    if handle is not None:
+        out = host.delta(x, base_out, seg.workspace, seg.rows, seg.num_groups, handle, bool(map_rows))
+        if out is not None:
+            return out
     return _LoraDelta.apply(x, base_out, seg, groups, map_rows, *groups.autograd_tensors())
+
+
+def _host_linear(x, weights, biases, seg, groups_list, map_rows):
+    host = _lib.host()
+    handles = [g.host_groups() for g in groups_list] if host is not None else [None]
+    if None in handles:
+        return None
+    return host.linear(x, weights, biases, seg.workspace, seg.rows, seg.num_groups, handles, bool(map_rows))
 
 
 def multi_lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], seg: SegmentTable,
                       groups: AdapterGroups, map_rows: bool = True) -> torch.Tensor:
     """``F.linear(x, weight, bias)`` plus the segmented LoRA update as one autograd node."""
+    out = _host_linear(x, (weight,), (bias,), seg, (groups,), map_rows)
+    if out is not None:
+        return out[0]
     return _LoraLinear.apply(x, weight, bias, seg, groups, map_rows, *groups.autograd_tensors())
 
 
@@ -736,6 +773,9 @@ def multi_lora_linear_shared(x: torch.Tensor, weights: Sequence[torch.Tensor],
                              groups_list: Sequence[AdapterGroups], map_rows: bool = True) -> Tuple[torch.Tensor, ...]:
     """:func:`multi_lora_linear` for projections that read the same ``x``: ``F.linear(x, weights[p], biases[p])``
     plus the segmented LoRA update of ``groups_list[p]``, all projections in one autograd node."""
+    out = _host_linear(x, weights, biases, seg, groups_list, map_rows)
+    if out is not None:
+        return tuple(out)
     has_bias = tuple(b is not None for b in biases)
     dummies = [b if b is not None else x.new_zeros(0) for b in biases]
     lora = []

@@ -94,16 +94,21 @@ def build_segments(keys: torch.Tensor, num_groups: int, num_tokens: Optional[int
     num_tokens = rows if num_tokens is None else num_tokens
     if num_tokens and rows % num_tokens:
         raise ValueError(f'rows ({rows}) must be a multiple of num_tokens ({num_tokens})')
-    lib = _lib.load()
-    nbytes = lib.tk_segment_workspace_bytes(rows, num_groups)
-    _lib.check(nbytes, 'tk_segment_workspace_bytes')
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
-    perm = torch.empty(rows, dtype=torch.int64, device=keys.device) if want_perm else None
-    offsets = torch.empty(num_groups + 1, dtype=torch.int64, device=keys.device) if want_offsets else None
-    code = lib.tk_segment_build(keys.data_ptr() if rows else None, _lib.TK_KEY_I32 if keys.dtype == torch.int32 else
-                                _lib.TK_KEY_I64, rows, num_groups, perm.data_ptr() if want_perm else None,
-                                offsets.data_ptr() if want_offsets else None, ws.data_ptr(), nbytes, _lib.stream_ptr())
-    _lib.check(code, 'tk_segment_build')
+    host = _lib.host()
+    built = host.segment_build(keys, num_groups, want_perm, want_offsets) if host is not None else None
+    if built is not None:
+        ws, perm, offsets = built
+    else:
+        lib = _lib.load()
+        nbytes = lib.tk_segment_workspace_bytes(rows, num_groups)
+        _lib.check(nbytes, 'tk_segment_workspace_bytes')
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
+        perm = torch.empty(rows, dtype=torch.int64, device=keys.device) if want_perm else None
+        offsets = torch.empty(num_groups + 1, dtype=torch.int64, device=keys.device) if want_offsets else None
+        code = lib.tk_segment_build(keys.data_ptr() if rows else None, _lib.TK_KEY_I32 if keys.dtype == torch.int32 else
+                                    _lib.TK_KEY_I64, rows, num_groups, perm.data_ptr() if want_perm else None,
+                                    offsets.data_ptr() if want_offsets else None, ws.data_ptr(), nbytes, _lib.stream_ptr())
+        _lib.check(code, 'tk_segment_build')
     table = SegmentTable(rows, num_groups, num_tokens, ws, perm, offsets)
     if check:
         bad = table.bad_keys()
