@@ -180,3 +180,39 @@ def test_the_host_side_check_sees_a_changed_entry(dev):
         assert code == _lib.TK_ERR_INVALID and check.value > 0
         failed.add(check.value)
     assert failed == {1, 6}
+
+
+@pytest.mark.parametrize('rows', [1, 63, 64, 65, 1000, 1024, 1025, 2047, 2048, 2049])
+@pytest.mark.parametrize('groups', [1, 2, 63, 64, 65, 511, 512, 1022, 1023, 1024])
+@pytest.mark.parametrize('dtype', [torch.int32, torch.int64])
+def test_builder_of_small_batches(dev, rows, groups, dtype):
+    """The one-block builder at the edges of its rounds, groups and counts, and the builders past them: order and offsets
+    of the oracle, every array of the table consistent; and, where the builders compute it, the tiles and the sets of four
+    in the order of their first row."""
+    g = torch.Generator().manual_seed(rows * 2000 + groups)
+    keys = torch.randint(-1, groups + 1, (rows,), generator=g)
+    keys[torch.rand(rows, generator=g) < 0.5] = groups // 2      # one long group among short ones
+    seg = build_segments(keys.to(dtype).to(dev), groups)
+    seg.validate()
+    own = (keys >= 0) & (keys < groups)
+    bucket = torch.where(own, keys, torch.full_like(keys, groups))
+    perm, _, offsets = oracle.segment_build_sort(bucket, groups + 1)
+    assert torch.equal(seg.perm.cpu(), perm) and torch.equal(seg.offsets.cpu(), offsets[:groups + 1])
+    assert seg.bad_keys() == int((~own).sum())
+    if groups > 63 or rows > 32768:
+        return
+    table = seg.workspace.cpu().view(torch.int32)
+    tiles = -(-rows // 32) + groups + 1
+
+    def pad(n):
+        return -(-4 * n // 256) * 64
+
+    at = 64 + pad(rows + 64) + 2 * pad(32 * tiles) + pad(groups + 2) + pad(tiles + 1)
+    slot_row = table[64 + pad(rows + 64):][:32 * tiles].view(tiles, 32)
+    counts = torch.bincount(bucket, minlength=groups + 1)
+    real = int(((counts[:groups] + 31) // 32).sum())
+    first = slot_row[:real, 0]
+    assert torch.equal(table[at:at + real].long(), torch.argsort(first))
+    at += pad(tiles + 1)
+    sets = -(-real // 4)
+    assert torch.equal(table[at:at + sets].long(), torch.argsort(first[::4]))

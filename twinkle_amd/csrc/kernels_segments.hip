@@ -2,7 +2,7 @@
 // gather / scatter-back kernels that use its table.  Integer work, HBM-light:
 // the table is built once per batch and read by every LoRA layer.
 //
-// Small inputs take one launch (k_seg_one, below).  General pipeline (three
+// Small inputs take one launch (k_seg_small and k_seg_one, below).  General pipeline (three
 // launches, no host synchronisation anywhere):
 //   k_seg_hist    one wave per 512 rows: per-key counts by bit-sliced ballots
 //                 (no contended atomics) -> hist[block][group]
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(64) void k_seg_scatter(const KeyT* __restrict__ key
 // (lane % 16, rows of 65 words: equal keys of different lanes fall into different banks).  The
 // block's own 512 rows are ranked by its first 8 waves, one 64-row round each: rank inside the round
 // from bit-sliced ballots, rounds before it from a small per-round table.  All threads then fill
-// the block's share of the tile / chunk tables.  Integer adds only: the result does not depend on
+// the block's share of the tile / chunk tables (a tile's entries by eight threads: one thread a tile, writing its padding slot
+// by slot, cost 1 us).  Integer adds only: the result does not depend on
 // the order in which the adds land.
 // ---------------------------------------------------------------------------
 constexpr int kOneGroups = 64;
@@ -505,22 +506,26 @@ __global__ __launch_bounds__(kOneWaves * 64) void k_seg_one(const KeyT* __restri
   const int real_tiles = tfirst[groups - 1];  // the tiles of the rows without a group come after them
   // spread over the blocks: entry i belongs to thread i / sort_blocks of block i % sort_blocks
   const int stride = sort_blocks * kOneWaves * 64;
-  for (int i = tid * sort_blocks + blk; i < max_tiles; i += stride) {
+  for (int at = tid * sort_blocks + blk; at < 8 * max_tiles; at += stride) {  // eight threads a tile, four slots each
+    const int i = at >> 3, j = 4 * (at & 7);
     int g = -1, pos0 = 0, valid = 0;
     if (i < num_tiles) {
       g = group_of(tfirst, groups, i);
       pos0 = offs[g] + (i - tfirst[g]) * kTileRows;  // sorted position of the tile's first slot
       valid = min(kTileRows, offs[g + 1] - pos0);      // padding is at the end of a group's last tile
     }
-    V.tile_group[i] = g == groups - 1 ? -1 : g;
-    if (i >= real_tiles) V.tile_order[i] = i;  // nothing to do in these: they stay where they are, after the others
-    if (i >= real_tiles && i % kSetTiles == 0) V.set_order[i / kSetTiles] = i / kSetTiles;
-    int4* sp = reinterpret_cast<int4*>(V.slot_pos + (int64_t)i * kTileRows);
-#pragma unroll
-    for (int j = 0; j < kTileRows; j += 4)
-      sp[j / 4] = make_int4(j < valid ? pos0 + j : -1, j + 1 < valid ? pos0 + j + 1 : -1,
-                            j + 2 < valid ? pos0 + j + 2 : -1, j + 3 < valid ? pos0 + j + 3 : -1);
-    for (int j = valid; j < kTileRows; ++j) V.slot_row[(int64_t)i * kTileRows + j] = -1;
+    if (j == 0) {
+      V.tile_group[i] = g == groups - 1 ? -1 : g;
+      if (i >= real_tiles) V.tile_order[i] = i;  // nothing to do in these: they stay where they are, after the others
+      if (i >= real_tiles && i % kSetTiles == 0) V.set_order[i / kSetTiles] = i / kSetTiles;
+    }
+    *reinterpret_cast<int4*>(V.slot_pos + (int64_t)i * kTileRows + j) =
+        make_int4(j < valid ? pos0 + j : -1, j + 1 < valid ? pos0 + j + 1 : -1, j + 2 < valid ? pos0 + j + 2 : -1,
+                  j + 3 < valid ? pos0 + j + 3 : -1);
+    if (j >= valid)
+      *reinterpret_cast<int4*>(V.slot_row + (int64_t)i * kTileRows + j) = make_int4(-1, -1, -1, -1);
+    else
+      for (int q = max(valid - j, 0); q < 4; ++q) V.slot_row[(int64_t)i * kTileRows + j + q] = -1;
   }
   for (int i = tid * sort_blocks + blk; i < max_chunks; i += stride) {
     ChunkInfo c{-1, 0, 0, -1};
@@ -534,6 +539,199 @@ __global__ __launch_bounds__(kOneWaves * 64) void k_seg_one(const KeyT* __restri
       c.partial = (cfirst[g + 1] - cfirst[g] > 1 && g != groups - 1) ? pfirst[g] + j : -1;
     }
     V.chunks[i] = c;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// One block for a batch of at most kSmallRounds * 64 rows (a decode step, a small batch, also over the groups of many experts):
+// every row is in the block, so counts per 64-row round, their prefix over rounds and groups, and the sweep order of the tiles
+// (the rows that open a tile, counted) need no second look at the keys.  Bound by latency: a chain of one load, six barriers
+// and one round of stores, and by fetching its own instructions.
+// Replayed in a graph: 32 rows of 16 groups 8.1 us (k_seg_one) -> 5.2, 256 rows of 512 groups 22 (three launches) -> 6.8.
+// ---------------------------------------------------------------------------
+constexpr int kSmallRounds = 32;
+constexpr int kSmallGroups = 1024;        // buckets
+constexpr int kSmallCounts = 18 * 1024;   // rounds x buckets (36 KB of LDS)
+constexpr int kSmallWaves = 16;
+
+template <typename KeyT>
+__global__ __launch_bounds__(kSmallWaves * 64) void k_seg_small(const KeyT* __restrict__ keys, int rows, int groups, int key_bits,
+                                                                int rounds, int max_tiles, int max_chunks, int chunk_tiles,
+                                                                int sweep, SegView V, int64_t* __restrict__ perm_out,
+                                                                int64_t* __restrict__ offsets_out) {
+  extern __shared__ uint32_t cnt_words[];  // rows of each group in each round, then those ahead of the round
+  uint16_t* cnt = reinterpret_cast<uint16_t*>(cnt_words);
+  __shared__ int32_t offs[kSmallGroups + 1], tfirst[kSmallGroups + 1], cfirst[kSmallGroups + 1], pfirst[kSmallGroups + 1];
+  __shared__ int16_t tile_of[kSmallRounds * 2 + kSmallGroups], chunk_of[kSmallRounds + kSmallGroups];
+  __shared__ unsigned long long wave_sums[kSmallWaves];
+  __shared__ uint16_t opened[2][kSmallRounds];  // tiles / sets opened by the rows of a round
+  __shared__ int bad_s[kSmallWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int key[2], rank[2], bad = 0;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int f = (wave + u * kSmallWaves) * 64 + lane;
+    key[u] = f < rows ? load_key(keys, f, groups, &bad) : -1;
+  }
+  for (int i = tid; i < (rounds * groups + 1) / 2; i += kSmallWaves * 64) cnt_words[i] = 0;
+  __syncthreads();
+#pragma unroll 1
+  for (int u = 0; u < 2; ++u) {
+    const int round = wave + u * kSmallWaves;
+    if (round >= rounds) break;
+    const int k = u ? key[1] : key[0];
+    const unsigned long long same = same_key_lanes(k >= 0, max(k, 0), key_bits);
+    const int r = __popcll(same & ((1ull << lane) - 1ull));  // rows with equal keys keep their lane order
+    if (k >= 0 && r == 0) cnt[round * groups + k] = (uint16_t)__popcll(same);
+    if (u) rank[1] = r; else rank[0] = r;
+  }
+  {
+    const int n = __popcll(__ballot(bad > 0)) + __popcll(__ballot(bad > 1));
+    if (lane == 0) bad_s[wave] = n;
+  }
+  __syncthreads();
+  // thread g: its group's rows ahead of every round, then all groups' firsts by one scan of four 16-bit counts at a time
+  int count = 0;
+  if (tid < groups)
+    for (int r = 0; r < rounds; ++r) {
+      const int c = cnt[r * groups + tid];
+      cnt[r * groups + tid] = (uint16_t)count;
+      count += c;
+    }
+  const int ntile = (count + kTileRows - 1) / kTileRows, nchunk = (ntile + chunk_tiles - 1) / chunk_tiles;
+  const int npart = (nchunk > 1 && tid != groups - 1) ? nchunk : 0;
+  const unsigned long long v = (unsigned long long)count | (unsigned long long)ntile << 16 | (unsigned long long)nchunk << 32 |
+                               (unsigned long long)npart << 48;
+  unsigned long long incl = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned long long o = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += o;
+  }
+  if (lane == 63) wave_sums[wave] = incl;
+  __syncthreads();
+  unsigned long long ahead = 0, total = 0;
+  for (int w = 0; w < kSmallWaves; ++w) {
+    if (w < wave) ahead += wave_sums[w];
+    total += wave_sums[w];
+  }
+  const unsigned long long excl = tid < groups ? ahead + incl - v : total;
+  auto part = [](unsigned long long x, int i) { return (int)((x >> (16 * i)) & 0xffff); };
+  if (tid <= groups) {  // (entry `groups`: the totals; a block of exactly `groups` threads writes it below)
+    offs[tid] = part(excl, 0);
+    tfirst[tid] = part(excl, 1);
+    cfirst[tid] = part(excl, 2);
+    pfirst[tid] = part(excl, 3);
+  }
+  if (tid == 0) {
+    offs[groups] = part(total, 0);
+    tfirst[groups] = part(total, 1);
+    cfirst[groups] = part(total, 2);
+    pfirst[groups] = part(total, 3);
+  }
+  if (tid < groups) {
+    for (int j = 0; j < ntile; ++j) tile_of[part(excl, 1) + j] = (int16_t)tid;
+    for (int j = 0; j < nchunk; ++j) chunk_of[part(excl, 2) + j] = (int16_t)tid;
+  }
+  __syncthreads();
+  for (int g = tid; g <= groups; g += kSmallWaves * 64) {
+    V.offsets[g] = offs[g];
+    V.tile_first[g] = tfirst[g];
+    V.chunk_first[g] = cfirst[g];
+    V.partial_first[g] = pfirst[g];
+    if (offsets_out && g < groups) offsets_out[g] = offs[g];
+  }
+  const int num_tiles = tfirst[groups], num_chunks = cfirst[groups], real_tiles = tfirst[groups - 1];
+  if (tid == 0) {
+    int bad_total = 0;
+    for (int w = 0; w < kSmallWaves; ++w) bad_total += bad_s[w];
+    SegHeader* hdr = V.header;
+    hdr->magic = kSegMagic;
+    hdr->rows = rows;
+    hdr->groups = groups - 1;
+    hdr->num_tiles = num_tiles;
+    hdr->num_chunks = num_chunks;
+    hdr->num_partials = pfirst[groups];
+    hdr->bad_keys = bad_total;
+    hdr->identity_order = sweep ? 0 : 1;
+  }
+  int opens = 0;  // bits 0, 1: this lane's row of round wave + 16 u opens a tile; bits 2, 3: and a set
+#pragma unroll 1
+  for (int u = 0; u < 2; ++u) {
+    const int round = wave + u * kSmallWaves, f = round * 64 + lane, k = u ? key[1] : key[0];
+    if (round >= rounds) break;
+    bool moved = false, tile = false, set = false;
+    if (k >= 0) {
+      const int in_group = cnt[round * groups + k] + (u ? rank[1] : rank[0]);
+      const int pos = offs[k] + in_group, slot = tfirst[k] * kTileRows + in_group;
+      moved = pos != f;
+      V.inv[f] = pos;
+      if (perm_out) perm_out[pos] = f;
+      V.slot_row[slot] = f;
+      tile = k != groups - 1 && (in_group & (kTileRows - 1)) == 0;
+      set = tile && (slot / kTileRows) % kSetTiles == 0;
+    }
+    if (!sweep) continue;
+    const unsigned long long m = __ballot(moved), t = __ballot(tile), s = __ballot(set);
+    opens |= (int)tile << u | (int)set << (2 + u);
+    if (lane == 0) {
+      V.round_moved[round] = m != 0ull;
+      opened[0][round] = (uint16_t)__popcll(t);
+      opened[1][round] = (uint16_t)__popcll(s);
+    }
+  }
+  // per-tile entries (8 threads a tile, four slots each) and chunks; a tile that no group owns stays where it is in the orders
+  for (int i = tid; i < 8 * max_tiles; i += kSmallWaves * 64) {
+    const int tile = i >> 3, j = 4 * (i & 7);
+    int g = -1, pos0 = 0, valid = 0;
+    if (tile < num_tiles) {
+      g = tile_of[tile];
+      pos0 = offs[g] + (tile - tfirst[g]) * kTileRows;
+      valid = min(kTileRows, offs[g + 1] - pos0);
+    }
+    if (j == 0) {
+      V.tile_group[tile] = g == groups - 1 ? -1 : g;
+      if (!sweep || tile >= real_tiles) {
+        V.tile_order[tile] = tile;
+        if (tile % kSetTiles == 0) V.set_order[tile / kSetTiles] = tile / kSetTiles;
+      }
+    }
+    *reinterpret_cast<int4*>(V.slot_pos + (int64_t)tile * kTileRows + j) =
+        make_int4(j < valid ? pos0 + j : -1, j + 1 < valid ? pos0 + j + 1 : -1, j + 2 < valid ? pos0 + j + 2 : -1,
+                  j + 3 < valid ? pos0 + j + 3 : -1);
+    if (j >= valid)
+      *reinterpret_cast<int4*>(V.slot_row + (int64_t)tile * kTileRows + j) = make_int4(-1, -1, -1, -1);
+    else
+      for (int q = max(valid - j, 0); q < 4; ++q) V.slot_row[(int64_t)tile * kTileRows + j + q] = -1;
+  }
+  for (int i = tid; i < max_chunks; i += kSmallWaves * 64) {
+    ChunkInfo c{-1, 0, 0, -1};
+    if (i < num_chunks) {
+      const int g = chunk_of[i], j = i - cfirst[g], tiles = tfirst[g + 1] - tfirst[g];
+      c.group = g == groups - 1 ? -1 : g;
+      c.tile0 = tfirst[g] + j * chunk_tiles;
+      c.ntiles = min(chunk_tiles, tiles - j * chunk_tiles);
+      c.partial = (cfirst[g + 1] - cfirst[g] > 1 && g != groups - 1) ? pfirst[g] + j : -1;
+    }
+    V.chunks[i] = c;
+  }
+  if (!sweep) return;
+  __syncthreads();
+#pragma unroll 1
+  for (int u = 0; u < 2; ++u) {
+    const int round = wave + u * kSmallWaves, k = u ? key[1] : key[0];
+    if (round >= rounds) break;
+    const bool tile = (opens >> u) & 1, set = (opens >> (2 + u)) & 1;
+    const unsigned long long t = __ballot(tile), s = __ballot(set);
+    if (!tile) continue;
+    int place = __popcll(t & ((1ull << lane) - 1ull)), set_place = __popcll(s & ((1ull << lane) - 1ull));
+    for (int r = 0; r < round; ++r) {
+      place += opened[0][r];
+      set_place += opened[1][r];
+    }
+    const int id = tfirst[k] + (cnt[round * groups + k] + (u ? rank[1] : rank[0])) / kTileRows;
+    V.tile_order[place] = id;
+    if (set) V.set_order[set_place] = id / kSetTiles;
   }
 }
 
@@ -707,6 +905,23 @@ int launch_segment_build(const void* keys, int key_dtype, int64_t rows, int32_t 
   const size_t lds = sizeof(int32_t) * (size_t)groups;
   int key_bits = 0;
   while ((1 << key_bits) < groups) ++key_bits;
+  const int rounds = (int)ceil_div(rows, 64);
+  // (up to 64 groups k_seg_one's blocks share the rows: 1024 rows of 16 groups 6.3 here, 7.0 there, 2048 rows 8.5 / 7.1; past
+  // them three launches are the other choice: 2048 rows of 256 groups 8.7 / 24)
+  if (rows > 0 && rounds <= (groups <= kOneGroups ? kSmallRounds / 2 : kSmallRounds) && groups <= kSmallGroups &&
+      rounds * groups <= kSmallCounts) {
+    const size_t counts = (size_t)round_up(2 * (int64_t)rounds * groups, 4);
+    const int sweep = groups <= kOneGroups;  // as the other builders: beyond that the tiles keep the table's order
+    if (key_dtype == TK_KEY_I32)
+      hipLaunchKernelGGL(k_seg_small<int32_t>, dim3(1), dim3(kSmallWaves * 64), counts, s, (const int32_t*)keys, (int)rows,
+                         groups, key_bits, rounds, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, sweep, V, perm_out,
+                         offsets_out);
+    else
+      hipLaunchKernelGGL(k_seg_small<int64_t>, dim3(1), dim3(kSmallWaves * 64), counts, s, (const int64_t*)keys, (int)rows,
+                         groups, key_bits, rounds, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, sweep, V, perm_out,
+                         offsets_out);
+    return check_launch();
+  }
   if (groups <= kOneGroups && nblk <= kOneBlocks) {
     if (key_dtype == TK_KEY_I32)
       hipLaunchKernelGGL(k_seg_one<int32_t>, dim3(nblk), dim3(kOneWaves * 64), 0, s, (const int32_t*)keys, (int)rows,
