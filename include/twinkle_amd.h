@@ -122,6 +122,20 @@ int tk_unpermute_weight_grad(const void* dout_device, int64_t ld_dout, const voi
                              float* dw_device, const void* seg_ws_device, int64_t rows, int64_t num_tokens,
                              int32_t width, int32_t num_groups, int32_t dtype, tk_stream_t stream);
 
+/* Both gradients of tk_unpermute_rows with weights from one look at each row: grad_rows as tk_permute_rows with weights
+ * writes it, dw as above (fp32 when dw_f32, else in `dtype`).  At most TK_UNPERMUTE_BWD_TOP_K rows a token. */
+#define TK_UNPERMUTE_BWD_TOP_K 32
+int tk_unpermute_bwd(const void* dout_device, int64_t ld_dout, const void* rows_device, int64_t ld_rows,
+                     void* grad_rows_device, int64_t ld_grad, const void* weights_device, void* dw_device, int32_t dw_f32,
+                     const void* seg_ws_device, int64_t rows, int64_t num_tokens, int32_t width, int32_t num_groups,
+                     int32_t dtype, tk_stream_t stream);
+
+/* Keys of top-k routed rows: keys[k * num_tokens + t] = selected[t * stride_t + k * stride_k] * num_tenants + tenant[t], 32-bit
+ * arithmetic; selected and tenant (null: 0) int32 or int64 (TK_KEY_*). */
+int tk_topk_keys(const void* selected_device, int32_t sel_dtype, int64_t stride_t, int64_t stride_k,
+                 const void* tenant_device, int32_t tenant_dtype, int32_t* keys_device, int64_t num_tokens, int32_t top_k,
+                 int32_t num_tenants, tk_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Segmented LoRA linear.
  *

@@ -216,3 +216,37 @@ def test_builder_of_small_batches(dev, rows, groups, dtype):
     at += pad(tiles + 1)
     sets = -(-real // 4)
     assert torch.equal(table[at:at + sets].long(), torch.argsort(first[::4]))
+
+
+@pytest.mark.parametrize('dtype,wdtype', [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                          (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize('t,k,h', [(1, 1, 8), (37, 3, 40), (50, 8, 2056), (20, 32, 100), (9, 5, 33)])
+def test_both_gradients_of_the_weighted_unpermute(dev, dtype, wdtype, t, k, h):
+    """One kernel for both against the launches for one of them (rows: same bits; weights: 32-bit sums of h products in
+    another order, then the type's rounding), widths off the 16-byte pieces among them."""
+    g = torch.Generator().manual_seed(t + h)
+    seg = build_segments(torch.randint(0, 7, (t * k,), generator=g, dtype=torch.int32).to(dev), 7, num_tokens=t)
+    rows = torch.randn(t * k, h, generator=g).to(dev, dtype).requires_grad_(True)
+    w = torch.rand(t, k, generator=g).to(dev, wdtype).requires_grad_(True)
+    dy = torch.randn(t, h, generator=g).to(dev, dtype)
+    both = torch.autograd.grad(unpermute(rows, w, seg), [rows, w], dy)
+    only_rows, = torch.autograd.grad(unpermute(rows, w.detach(), seg), [rows], dy)
+    only_w, = torch.autograd.grad(unpermute(rows.detach(), w, seg), [w], dy)
+    assert torch.equal(both[0], only_rows) and both[1].dtype == only_w.dtype
+    scale = (dy.float().norm() * rows.detach().float().norm() / t).item()
+    ulp = 2**-8 if wdtype == torch.bfloat16 else 2**-24 * h
+    assert (both[1].float() - only_w.float()).abs().max().item() <= 2 * ulp * scale
+
+
+@pytest.mark.parametrize('dtype', [torch.int32, torch.int64])
+@pytest.mark.parametrize('tenant_dtype', [None, torch.int32, torch.int64])
+@pytest.mark.parametrize('t,k', [(0, 4), (1, 1), (300, 1), (77, 8)])
+def test_keys_of_routed_rows(dev, dtype, tenant_dtype, t, k):
+    g = torch.Generator().manual_seed(t)
+    wide = torch.randint(-2, 600, (t, 2 * k), generator=g).to(dtype)
+    for sel in (wide[:, :k], wide[:, ::2], wide[:, :k].t().contiguous().t()):
+        tenant = None if tenant_dtype is None else torch.randint(0, 5, (t,), generator=g).to(tenant_dtype)
+        want = flat_keys_from_topk(sel, tenant, 5)              # on the CPU: torch operations
+        layout = torch.empty_strided(sel.shape, sel.stride(), dtype=dtype, device=dev).copy_(sel)
+        got = flat_keys_from_topk(layout, tenant.to(dev) if tenant is not None else None, 5)
+        assert got.dtype == want.dtype and got.is_contiguous() and torch.equal(got.cpu(), want)

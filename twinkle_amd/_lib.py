@@ -29,6 +29,7 @@ TK_KEY_I32 = 0
 TK_KEY_I64 = 1
 TK_TILE_ROWS = 32
 TK_CHUNK_ROWS = 128
+TK_UNPERMUTE_BWD_TOP_K = 32
 TK_MAX_GROUPS = 16384
 TK_MAX_RANK = 128
 
@@ -98,6 +99,10 @@ EXPORTS = {
                               c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
     'tk_lora_bwd_store': (c_int32, [POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                     c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
+    'tk_unpermute_bwd': (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int32,
+                                   c_void_p, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p]),
+    'tk_topk_keys': (c_int32, [c_void_p, c_int32, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_int64, c_int32, c_int32,
+                               c_void_p]),
     'tk_lora_bwd_into': (c_int32, [POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                    c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     # arrays indexed by projection are host arrays: pointers to descriptors / device pointers / strides

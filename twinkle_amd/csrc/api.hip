@@ -434,6 +434,29 @@ int tk_unpermute_weight_grad(const void* dout, int64_t ld_dout, const void* rows
                                 dtype, (hipStream_t)stream);
 }
 
+int tk_unpermute_bwd(const void* dout, int64_t ld_dout, const void* rows_p, int64_t ld_rows, void* grad_rows, int64_t ld_grad,
+                     const void* weights, void* dw, int32_t dw_f32, const void* seg_ws, int64_t rows, int64_t num_tokens,
+                     int32_t width, int32_t num_groups, int32_t dtype, tk_stream_t stream) {
+  if (!rows_args_ok(dout, rows_p, seg_ws, rows, num_tokens, width, num_groups, dtype) ||
+      (rows > 0 && (!grad_rows || !weights || !dw)))
+    return TK_ERR_INVALID;
+  if (ld_dout < width || ld_rows < width || ld_grad < width) return TK_ERR_INVALID;
+  if (rows > num_tokens * TK_UNPERMUTE_BWD_TOP_K) return TK_ERR_UNSUPPORTED;
+  return launch_unpermute_bwd(dout, ld_dout, rows_p, ld_rows, grad_rows, ld_grad, weights, dw, dw_f32, seg_ws, rows, num_tokens,
+                              width, num_groups, dtype, (hipStream_t)stream);
+}
+
+int tk_topk_keys(const void* selected, int32_t sel_dtype, int64_t stride_t, int64_t stride_k, const void* tenant,
+                 int32_t tenant_dtype, int32_t* keys, int64_t num_tokens, int32_t top_k, int32_t num_tenants,
+                 tk_stream_t stream) {
+  auto type_ok = [](int32_t t) { return t == TK_KEY_I32 || t == TK_KEY_I64; };
+  if (num_tokens < 0 || top_k < 0 || num_tokens * top_k >= (1ll << 31) || !type_ok(sel_dtype) || (tenant && !type_ok(tenant_dtype)))
+    return TK_ERR_INVALID;
+  if (num_tokens * top_k > 0 && (!selected || !keys)) return TK_ERR_INVALID;
+  return launch_topk_keys(selected, sel_dtype, stride_t, stride_k, tenant, tenant_dtype, keys, num_tokens, top_k, num_tenants,
+                          (hipStream_t)stream);
+}
+
 // what the size queries need of a descriptor: shapes and dtype, no pointers
 static bool desc_shape_ok(const tk_lora_desc* d) {
   return d && d->rows >= 0 && d->num_groups > 0 && d->num_groups <= TK_MAX_GROUPS && d->max_rank >= 0 &&

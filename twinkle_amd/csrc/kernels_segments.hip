@@ -14,6 +14,7 @@
 //   k_seg_scatter one wave per 512 rows: stable rank inside the wave by
 //                 bit-sliced ballots, cursor per group in LDS -> inv, slot_row
 #include <initializer_list>
+#include <type_traits>
 
 #include "tk_device.h"
 
@@ -784,6 +785,8 @@ __global__ __launch_bounds__(1024) void k_class_lists(ClassListArgs p, ClassList
   if (tid == 0) ((int32_t*)p.base[c])[which] = running;
 }
 
+constexpr int kUnpermuteTopK = TK_UNPERMUTE_BWD_TOP_K;
+
 // 16 bytes of a row: the unit the row movers below load and store when width, strides and pointers allow
 // (V = 8 bf16 / 4 fp32 elements), else V = 1.  The arithmetic per element and the order of every sum are the
 // same for both.
@@ -879,6 +882,61 @@ __global__ __launch_bounds__(64) void k_unpermute_wgrad(const T* __restrict__ do
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
   if (threadIdx.x == 0) dw[(int64_t)t * top_k + k] = acc;
+}
+
+// Both gradients of the weighted unpermute from one look at each row: grad_rows[pos(k, t)] = dout[t] * w[t, k] and
+// dw[t, k] = <dout[t], rows[pos(k, t)]>.  A block owns a token, whose dout stays in its cache over the top_k rows.  Bound by
+// memory: rows read and grad_rows written once (as two launches dout crossed the caches twice as often and the rows' reads had
+// no writes next to them: 65536 rows of 2048, 166 us; here 104).
+template <typename T, int V, typename W>
+__global__ __launch_bounds__(256) void k_unpermute_bwd(const T* __restrict__ dout, int64_t ld_dout, const T* __restrict__ rows_,
+                                                       int64_t ld_rows, T* __restrict__ grad, int64_t ld_grad,
+                                                       const T* __restrict__ w, W* __restrict__ dw,
+                                                       const int32_t* __restrict__ inv, int tokens, int top_k, int width) {
+  __shared__ float sums[kUnpermuteTopK][4];
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const RowVec<T, V>* d = reinterpret_cast<const RowVec<T, V>*>(dout + (int64_t)t * ld_dout);
+#pragma unroll 2
+  for (int k = 0; k < top_k; ++k) {
+    const int j = inv[(int64_t)k * tokens + t];
+    float acc = 0.f;
+    if ((unsigned)j < (unsigned)(tokens * top_k)) {  // (a position outside the table's rows: no row, no gradient)
+      const RowVec<T, V>* r = reinterpret_cast<const RowVec<T, V>*>(rows_ + (int64_t)j * ld_rows);
+      RowVec<T, V>* g = reinterpret_cast<RowVec<T, V>*>(grad + (int64_t)j * ld_grad);
+      const float wt = to_f32(w[(int64_t)t * top_k + k]);
+      for (int c = threadIdx.x; c < width / V; c += 256) {
+        RowVec<T, V> x = d[c];
+        const RowVec<T, V> y = r[c];
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          acc += to_f32(x.v[i]) * to_f32(y.v[i]);
+          from_f32(to_f32(x.v[i]) * wt, &x.v[i]);
+        }
+        g[c] = x;
+      }
+    }
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s, 64);
+    if (lane == 0) sums[k][wave] = acc;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < top_k) {
+    const float* s = sums[threadIdx.x];
+    from_f32((s[0] + s[1]) + (s[2] + s[3]), &dw[(int64_t)t * top_k + threadIdx.x]);
+  }
+}
+
+// keys[k T + t] = selected[t, k] * num_tenants + tenant[t], in 32 bits
+template <typename S, typename N>
+__global__ __launch_bounds__(256) void k_topk_keys(const S* __restrict__ selected, int64_t stride_t, int64_t stride_k,
+                                                   const N* __restrict__ tenant, int32_t* __restrict__ keys, int tokens,
+                                                   int64_t rows, int num_tenants) {
+  const int64_t f = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (f >= rows) return;
+  const int64_t t = f % tokens, k = f / tokens;
+  uint32_t key = (uint32_t)selected[t * stride_t + k * stride_k] * (uint32_t)num_tenants;
+  if (tenant) key += (uint32_t)tenant[t];
+  keys[f] = (int32_t)key;
 }
 
 // whether rows of `width` elements at these strides and addresses can move in 16-byte pieces
@@ -1030,6 +1088,48 @@ int launch_unpermute_wgrad(const void* dout, int64_t ld_dout, const void* rows_,
     TK_ROW_MOVER(k_unpermute_wgrad, uint16_t, rows_vectorise<uint16_t>(width, {ld_dout, ld_rows}, {dout, rows_}), grid,
                  block, (const uint16_t*)dout, ld_dout, (const uint16_t*)rows_, ld_rows, dw, V.inv, (int)tokens, top_k,
                  width);
+  return check_launch();
+}
+
+int launch_unpermute_bwd(const void* dout, int64_t ld_dout, const void* rows_, int64_t ld_rows, void* grad, int64_t ld_grad,
+                         const void* w, void* dw, int dw_f32, const void* ws, int64_t rows, int64_t tokens, int32_t width,
+                         int32_t groups, int dtype, hipStream_t s) {
+  if (rows == 0) return TK_OK;
+  SegLayout L(rows, groups);
+  SegView V(ws, L);
+  const int top_k = (int)(rows / tokens);
+  const dim3 grid((unsigned)tokens), block(256);
+  auto launch = [&](auto vec, auto element, auto weight) {
+    using T = decltype(element);
+    using W = decltype(weight);
+    hipLaunchKernelGGL((k_unpermute_bwd<T, decltype(vec)::value, W>), grid, block, 0, s, (const T*)dout, ld_dout,
+                       (const T*)rows_, ld_rows, (T*)grad, ld_grad, (const T*)w, (W*)dw, V.inv, (int)tokens, top_k, width);
+  };
+  using std::integral_constant;
+  if (dtype == TK_DTYPE_F32) {
+    if (rows_vectorise<float>(width, {ld_dout, ld_rows, ld_grad}, {dout, rows_, grad})) launch(integral_constant<int, 4>{}, float{}, float{});
+    else launch(integral_constant<int, 1>{}, float{}, float{});
+  } else {
+    const bool vec = rows_vectorise<uint16_t>(width, {ld_dout, ld_rows, ld_grad}, {dout, rows_, grad});
+    if (vec && dw_f32) launch(integral_constant<int, 8>{}, uint16_t{}, float{});
+    else if (vec) launch(integral_constant<int, 8>{}, uint16_t{}, uint16_t{});
+    else if (dw_f32) launch(integral_constant<int, 1>{}, uint16_t{}, float{});
+    else launch(integral_constant<int, 1>{}, uint16_t{}, uint16_t{});
+  }
+  return check_launch();
+}
+
+int launch_topk_keys(const void* selected, int sel_dtype, int64_t stride_t, int64_t stride_k, const void* tenant,
+                     int tenant_dtype, int32_t* keys, int64_t tokens, int32_t top_k, int32_t num_tenants, hipStream_t s) {
+  const int64_t rows = tokens * top_k;
+  if (rows == 0) return TK_OK;
+  const dim3 grid((unsigned)ceil_div(rows, 256)), block(256);
+  auto launch = [&](auto sel, auto ten) {
+    hipLaunchKernelGGL((k_topk_keys<decltype(sel), decltype(ten)>), grid, block, 0, s, (const decltype(sel)*)selected, stride_t,
+                       stride_k, (const decltype(ten)*)tenant, keys, (int)tokens, rows, num_tenants);
+  };
+  if (sel_dtype == TK_KEY_I32) tenant_dtype == TK_KEY_I32 ? launch(int32_t{}, int32_t{}) : launch(int32_t{}, int64_t{});
+  else tenant_dtype == TK_KEY_I32 ? launch(int64_t{}, int32_t{}) : launch(int64_t{}, int64_t{});
   return check_launch();
 }
 

@@ -533,6 +533,11 @@ int launch_class_lists(const int32_t* rank, int n, const RankClass* rc, void* co
                        const SegView& seg, const SegLayout& L, hipStream_t s);
 int launch_segment_build(const void* keys, int key_dtype, int64_t rows, int32_t groups, int64_t* perm_out,
                          int64_t* offsets_out, void* ws, hipStream_t s);
+int launch_unpermute_bwd(const void* dout, int64_t ld_dout, const void* rows_, int64_t ld_rows, void* grad, int64_t ld_grad,
+                         const void* w, void* dw, int dw_f32, const void* ws, int64_t rows, int64_t tokens, int32_t width,
+                         int32_t groups, int dtype, hipStream_t s);
+int launch_topk_keys(const void* selected, int sel_dtype, int64_t stride_t, int64_t stride_k, const void* tenant,
+                     int tenant_dtype, int32_t* keys, int64_t tokens, int32_t top_k, int32_t num_tenants, hipStream_t s);
 int launch_permute(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, const void* w, const void* ws,
                    int64_t rows, int64_t tokens, int32_t width, int32_t groups, int dtype, hipStream_t s);
 int launch_unpermute(const void* rows_, int64_t ld_rows, void* out, int64_t ld_out, const void* w, const void* ws,

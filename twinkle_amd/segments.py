@@ -117,11 +117,32 @@ def build_segments(keys: torch.Tensor, num_groups: int, num_tokens: Optional[int
     return table
 
 
+def _keys_on_gpu(selected: torch.Tensor, tenant: Optional[torch.Tensor]) -> bool:
+    """Plain GPU tensors one launch makes the keys of (torch's three to five cost more than the table behind them)."""
+    def plain(t, dim):
+        return (type(t) is torch.Tensor and t.is_cuda and t.dim() == dim and t.dtype in (torch.int32, torch.int64) and
+                t.device == selected.device)
+
+    return (plain(selected, 2) and selected.numel() < 2**31 and _lib.host() is not None and
+            not torch._C._are_functorch_transforms_active() and
+            (tenant is None or (plain(tenant, 1) and tenant.is_contiguous() and tenant.shape[0] == selected.shape[0])))
+
+
 def flat_keys_from_topk(selected: torch.Tensor, tenant: Optional[torch.Tensor] = None,
                         num_tenants: int = 1) -> torch.Tensor:
     """Keys ``expert * num_tenants + tenant[t]`` in the reference's row order ``f = k * T + t``."""
     if selected.dim() == 1:
         selected = selected[:, None]
+    if _keys_on_gpu(selected, tenant):
+        tokens, top_k = selected.shape
+        keys = torch.empty(tokens * top_k, dtype=torch.int32, device=selected.device)
+        key_type = {torch.int32: _lib.TK_KEY_I32, torch.int64: _lib.TK_KEY_I64}
+        code = _lib.load().tk_topk_keys(selected.data_ptr(), key_type[selected.dtype], selected.stride(0), selected.stride(1),
+                                        tenant.data_ptr() if tenant is not None else None,
+                                        key_type[tenant.dtype] if tenant is not None else 0, keys.data_ptr(), tokens, top_k,
+                                        int(num_tenants), _lib.stream_ptr())
+        _lib.check(code, 'tk_topk_keys')
+        return keys
     keys = selected.to(torch.int32) * num_tenants
     if tenant is not None:
         keys = keys + tenant.to(torch.int32)[:, None]
@@ -206,6 +227,17 @@ class _Unpermute(torch.autograd.Function):
         rows, weights = ctx.saved_tensors
         seg = ctx.seg
         grad_out = grad_out.contiguous()
+        if weights is not None and all(ctx.needs_input_grad[:2]) and seg.top_k <= _lib.TK_UNPERMUTE_BWD_TOP_K:
+            w = weights.to(rows.dtype).contiguous()
+            grad_rows = torch.empty(seg.rows, rows.shape[1], dtype=rows.dtype, device=rows.device)
+            same = weights.dtype == rows.dtype
+            dw = torch.empty(seg.num_tokens, seg.top_k, dtype=weights.dtype if same else torch.float32, device=rows.device)
+            code = _lib.load().tk_unpermute_bwd(
+                grad_out.data_ptr(), grad_out.stride(0), rows.data_ptr(), rows.stride(0), grad_rows.data_ptr(),
+                grad_rows.stride(0), w.data_ptr(), dw.data_ptr(), 0 if same else 1, seg.workspace.data_ptr(), seg.rows,
+                seg.num_tokens, rows.shape[1], seg.num_groups, _lib.dtype_code(rows.dtype), _lib.stream_ptr())
+            _lib.check(code, 'tk_unpermute_bwd')
+            return grad_rows, dw.to(weights.dtype), None
         grad_rows = _gather_rows(grad_out, weights, seg) if ctx.needs_input_grad[0] else None
         grad_w = None
         if weights is not None and ctx.needs_input_grad[1]:
