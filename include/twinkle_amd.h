@@ -82,6 +82,12 @@ int64_t tk_segment_workspace_bytes(int64_t rows, int32_t num_groups);
 int tk_segment_build(const void* keys_device, int32_t key_dtype, int64_t rows, int32_t num_groups,
                      int64_t* perm_out_device, int64_t* offsets_out_device, void* seg_ws_device,
                      int64_t seg_ws_bytes, tk_stream_t stream);
+/* The table of top-k routed rows for calls that read the tokens themselves (the *_tokens calls, num_tokens in
+ * tk_grouped_linear_bwd) instead of a permuted copy: row f = k * num_tokens + t of the table stands for token t, i.e. its row
+ * entries hold f mod num_tokens.  Positions, groups, and the inverse that tk_unpermute_rows uses are those of
+ * tk_segment_build; calls with map_rows = 1 and tk_permute_rows have no use for it, and tk_segment_validate refuses it. */
+int tk_segment_build_tokens(const void* keys_device, int32_t key_dtype, int64_t rows, int32_t num_groups, int64_t num_tokens,
+                            void* seg_ws_device, int64_t seg_ws_bytes, tk_stream_t stream);
 /* Synchronises the stream and copies one counter back: number of out-of-range keys. */
 int tk_segment_bad_keys(const void* seg_ws_device, tk_stream_t stream, int64_t* count_out_host);
 
@@ -122,8 +128,9 @@ int tk_unpermute_weight_grad(const void* dout_device, int64_t ld_dout, const voi
                              float* dw_device, const void* seg_ws_device, int64_t rows, int64_t num_tokens,
                              int32_t width, int32_t num_groups, int32_t dtype, tk_stream_t stream);
 
-/* Both gradients of tk_unpermute_rows with weights from one look at each row: grad_rows as tk_permute_rows with weights
- * writes it, dw as above (fp32 when dw_f32, else in `dtype`).  At most TK_UNPERMUTE_BWD_TOP_K rows a token. */
+/* Both gradients of tk_unpermute_rows from one look at each row: grad_rows as tk_permute_rows (with or without weights)
+ * writes it, dw as above (fp32 when dw_f32, else in `dtype`), for at most TK_UNPERMUTE_BWD_TOP_K rows a token.  dw null: not
+ * wanted, rows are not read.  Needs the table's positions only (also a table of tk_segment_build_tokens). */
 #define TK_UNPERMUTE_BWD_TOP_K 32
 int tk_unpermute_bwd(const void* dout_device, int64_t ld_dout, const void* rows_device, int64_t ld_rows,
                      void* grad_rows_device, int64_t ld_grad, const void* weights_device, void* dw_device, int32_t dw_f32,
@@ -370,6 +377,23 @@ int64_t tk_grouped_linear_workspace_bytes(const tk_grouped_desc* desc);
 int tk_grouped_linear(const tk_grouped_desc* desc, const tk_lora_desc* lora, const void* x_device, int64_t ldx,
                       void* y_device, int64_t ldy, const void* h_device, void* workspace_device,
                       int64_t workspace_bytes, tk_stream_t stream);
+
+/* tk_lora_shrink and tk_grouped_linear (layout 0, map_rows 0) with x = the tokens [num_tokens][in_features], each read by the
+ * rows of the table that stand for it (tk_segment_build_tokens); y and h as before. */
+int tk_lora_shrink_tokens(const tk_lora_desc* desc, const void* x_device, int64_t ldx, int64_t num_tokens, void* h_device,
+                          tk_stream_t stream);
+int tk_grouped_linear_tokens(const tk_grouped_desc* desc, const tk_lora_desc* lora, const void* x_device, int64_t ldx,
+                             int64_t num_tokens, void* y_device, int64_t ldy, const void* h_device, void* workspace_device,
+                             int64_t workspace_bytes, tk_stream_t stream);
+/* The backward of tk_grouped_linear with the LoRA term on frozen weights (map_rows 0): dx[row] = dy[row] W_e +
+ * scale_g (dy[row] B_g) A_g, written (null: not wanted), and the adapters' gradients as tk_lora_bwd_into places them.  `desc`
+ * is the layout-1 description (in_features = width of dy), `lora` the forward's; x as the forward read it: rows in segment
+ * order, or the tokens (num_tokens > 0; dx still has a row per row of the table).  lora_ws: tk_lora_bwd_workspace_bytes. */
+int tk_grouped_linear_bwd(const tk_grouped_desc* desc, const tk_lora_desc* lora, const void* dy_device, int64_t lddy,
+                          const void* x_device, int64_t ldx, int64_t num_tokens, const void* h_device, void* dx_device,
+                          int64_t lddx, const int64_t* at_A, void* base_A, const int64_t* at_B, void* base_B,
+                          void* gemm_ws_device, int64_t gemm_ws_bytes, void* lora_ws_device, int64_t lora_ws_bytes,
+                          tk_stream_t stream);
 
 /* ---- gated activation of the packed experts --------------------------------------------------------------
  *

@@ -1,0 +1,118 @@
+"""Packed experts on the tokens themselves (no permuted copy), and the backward whose GEMM takes the LoRA part of dx along:
+against the same block put together from permute, experts and unpermute, and against float64."""
+import pytest
+import torch
+
+from twinkle_amd import LoraConfig, build_segments, flat_keys_from_topk, permute, unpermute
+from twinkle_amd.expert_lora import ExpertLoraSlots, experts_forward, moe_experts_block
+
+pytestmark = pytest.mark.gpu
+
+
+class _Experts(torch.nn.Module):
+
+    def __init__(self, gate_up, down):
+        super().__init__()
+        self.gate_up_proj = torch.nn.Parameter(gate_up, requires_grad=False)
+        self.down_proj = torch.nn.Parameter(down, requires_grad=False)
+        self.act_fn = torch.nn.functional.silu
+
+
+def _problem(dev, t, e, k, hidden, inter, ranks, max_r, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    mod = _Experts((torch.randn(e, 2 * inter, hidden, generator=g) / hidden**0.5).bfloat16().to(dev),
+                   (torch.randn(e, hidden, inter, generator=g) / inter**0.5).bfloat16().to(dev))
+    slots = [ExpertLoraSlots(e, fin, fout, max_loras=len(ranks), max_r=max_r, dtype=torch.bfloat16, device=dev)
+             for fin, fout in ((hidden, 2 * inter), (inter, hidden))]
+    names = [f'lora_{j}' if r else None for j, r in enumerate(ranks)]
+    params = []
+    for s in slots:
+        for name, r in zip(names, ranks):
+            if name is None:
+                continue
+            s.configure_slot(name, LoraConfig(r=r, lora_alpha=2 * r))
+            for p, std in ((s.lora_A[name], s.in_features**-0.5), (s.lora_B[name], 0.1)):
+                with torch.no_grad():
+                    p.copy_((torch.randn(p.shape, generator=g) * std).bfloat16())
+                params.append(p)
+    sel = torch.topk(torch.randn(t, e, generator=g), k).indices.to(dev)
+    w = torch.rand(t, k, generator=g).bfloat16().to(dev).requires_grad_(True)
+    tenant = torch.randint(0, len(ranks), (t,), generator=g, dtype=torch.int32).to(dev)
+    x = torch.randn(t, hidden, generator=g).bfloat16().to(dev).requires_grad_(True)
+    dy = torch.randn(t, hidden, generator=g).bfloat16().to(dev)
+    return mod, slots, names, params, sel, w, tenant, x, dy
+
+
+def _exact(mod, slots, names, sel, w, tenant, x):
+    """float64, expert by expert and tenant by tenant, on merged weights."""
+    out = torch.zeros_like(x)
+    gate_up, down = mod.gate_up_proj.double(), mod.down_proj.double()
+    for e in range(gate_up.shape[0]):
+        for n, name in enumerate(names):
+            hit = ((sel == e) & (tenant == n)[:, None]).nonzero()
+            if not len(hit):
+                continue
+            t, k = hit.unbind(1)
+            ws = [gate_up[e], down[e]]
+            if name is not None:
+                for i, s in enumerate(slots):
+                    r = s.r[name]
+                    ws[i] = ws[i] + s.scaling[name] * s.lora_B[name][e, :, :r].double() @ s.lora_A[name][e, :r].double()
+            gu = x[t] @ ws[0].t()
+            gate, up = gu.chunk(2, -1)
+            out = out.index_add(0, t, (torch.nn.functional.silu(gate) * up) @ ws[1].t() * w[t, k, None])
+    return out
+
+
+@pytest.mark.parametrize('t,e,k,hidden,inter,ranks,max_r', [
+    (1, 4, 2, 128, 128, (8,), 8),                       # one token
+    (37, 8, 3, 256, 128, (8, 8), 8),                    # widths that the 256-wide kernel takes in one direction only
+    (300, 4, 4, 256, 256, (8, 5, 8), 8),                # rows of every expert, tenants of two and three tiles
+    (700, 6, 2, 512, 256, (16, 0, 12), 16),             # a tenant without adapters
+    (900, 3, 2, 256, 512, (64, 64), 64),                # a LoRA step per group
+    (500, 4, 2, 256, 256, (8, 64), 64),                 # two rank classes: the LoRA part of dx in a pass of its own
+    (2000, 2, 1, 256, 256, (32,) * 6, 32),              # several LoRA steps in a row block, top 1
+])
+def test_block_on_tokens(dev, t, e, k, hidden, inter, ranks, max_r):
+    mod, slots, names, params, sel, w, tenant, x, dy = _problem(dev, t, e, k, hidden, inter, ranks, max_r)
+    inputs = [x, w, *params]
+    out = moe_experts_block(x, sel, w, tenant, mod, names, *slots)
+    got = [out.detach(), *torch.autograd.grad(out, inputs, dy)]
+    with torch.no_grad():
+        assert torch.equal(moe_experts_block(x, sel, w, tenant, mod, names, *slots), got[0])
+    # the same block put together from its parts: the same products, so the same bits forward
+    nt = len(names)
+    seg = build_segments(flat_keys_from_topk(sel, tenant if nt > 1 else None, nt), e * nt, num_tokens=t)
+    rows, _ = permute(x, seg)
+    ref = unpermute(experts_forward(mod, rows, seg, names, *slots), w, seg)
+    assert torch.equal(ref, got[0])
+    want = [ref.detach(), *torch.autograd.grad(ref, inputs, dy)]
+    exact_in = [v.detach().double().requires_grad_(True) for v in (x, w)]
+    exact_out = _exact(mod, slots, names, sel, exact_in[1], tenant, exact_in[0])
+    exact = [exact_out, *torch.autograd.grad(exact_out, exact_in, dy.double())]
+    for i, (p, q) in enumerate(zip(got, want)):
+        if i < 3:          # outputs and the gradients of x and the routing weights: bf16 intermediates, four products in a row
+            scale = exact[i].abs().max().item()
+            assert (p.double() - exact[i]).abs().max().item() < 2e-2 * scale, i
+        scale = q.double().abs().max().item()
+        assert (p.double() - q.double()).abs().max().item() <= 2e-2 * scale, i
+
+
+def test_strided_tokens_and_frozen_adapters(dev):
+    mod, slots, names, params, sel, w, tenant, x, dy = _problem(dev, 200, 4, 2, 256, 256, (8, 8), 8)
+    wide = torch.randn(200, 512, device=dev).bfloat16()
+    wide[:, :256] = x.detach()
+    view = wide[:, :256].requires_grad_(True)
+    base = moe_experts_block(x, sel, w, tenant, mod, names, *slots)
+    assert torch.equal(moe_experts_block(view, sel, w, tenant, mod, names, *slots), base)
+    want, = torch.autograd.grad(base, [x], dy, retain_graph=True)
+    for p in params:
+        p.requires_grad_(False)
+    only_x, = torch.autograd.grad(moe_experts_block(view, sel, w, tenant, mod, names, *slots), [view], dy)
+    assert torch.equal(only_x, want)
+    fixed, = torch.autograd.grad(moe_experts_block(view, sel, w.detach(), tenant, mod, names, *slots), [view], dy)
+    assert torch.equal(fixed, want)              # routing weights that need no gradient
+    # rows whose address no 16-byte load takes: the permuted copy
+    off = torch.randn(200, 257, device=dev).bfloat16()
+    off[:, 1:] = x.detach()
+    assert torch.equal(moe_experts_block(off[:, 1:], sel, w, tenant, mod, names, *slots), base)

@@ -233,6 +233,10 @@ def test_both_gradients_of_the_weighted_unpermute(dev, dtype, wdtype, t, k, h):
     only_rows, = torch.autograd.grad(unpermute(rows, w.detach(), seg), [rows], dy)
     only_w, = torch.autograd.grad(unpermute(rows.detach(), w, seg), [w], dy)
     assert torch.equal(both[0], only_rows) and both[1].dtype == only_w.dtype
+    perm = seg.perm                                   # rows: the token's dy, scaled in fp32 and rounded once
+    want = (dy[perm % t].float() * w.detach().to(dtype).t().reshape(-1)[perm, None].float()).to(dtype)
+    assert torch.equal(only_rows, want)
+    assert torch.equal(torch.autograd.grad(unpermute(rows, None, seg), [rows], dy)[0], dy[perm % t])
     scale = (dy.float().norm() * rows.detach().float().norm() / t).item()
     ulp = 2**-8 if wdtype == torch.bfloat16 else 2**-24 * h
     assert (both[1].float() - only_w.float()).abs().max().item() <= 2 * ulp * scale

@@ -99,6 +99,13 @@ EXPORTS = {
                               c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
     'tk_lora_bwd_store': (c_int32, [POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                     c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
+    'tk_segment_build_tokens': (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_int64, c_void_p, c_int64, c_void_p]),
+    'tk_lora_shrink_tokens': (c_int32, [POINTER(LoraDesc), c_void_p, c_int64, c_int64, c_void_p, c_void_p]),
+    'tk_grouped_linear_tokens': (c_int32, [POINTER(GroupedDesc), POINTER(LoraDesc), c_void_p, c_int64, c_int64, c_void_p,
+                                           c_int64, c_void_p, c_void_p, c_int64, c_void_p]),
+    'tk_grouped_linear_bwd': (c_int32, [POINTER(GroupedDesc), POINTER(LoraDesc), c_void_p, c_int64, c_void_p, c_int64, c_int64,
+                                        c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                        c_void_p, c_int64, c_void_p]),
     'tk_unpermute_bwd': (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int32,
                                    c_void_p, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p]),
     'tk_topk_keys': (c_int32, [c_void_p, c_int32, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_int64, c_int32, c_int32,

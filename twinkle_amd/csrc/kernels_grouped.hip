@@ -143,7 +143,8 @@ __global__ __launch_bounds__(256) void k_grouped_plan(GroupedArgs a, SegView V, 
 template <int NKS, int BIG, int TR>
 __global__ __launch_bounds__(BIG ? 512 : 256) __attribute__((amdgpu_waves_per_eu(2))) void k_grouped_gemm(
     GroupedArgs a, const GroupedPlanEntry* __restrict__ plan, const int32_t* __restrict__ nblocks,
-    const int32_t* __restrict__ tile_group, const int32_t* __restrict__ slot_rows, int nsplit, int cpi) {
+    const int32_t* __restrict__ tile_group, const int32_t* __restrict__ slot_rows, const int32_t* __restrict__ y_rows,
+    int nsplit, int cpi) {
   constexpr int THREADS = BIG ? 512 : 256, WN = BIG ? 4 : 2, RB = BIG ? 8 : 4, CB = 4;
   constexpr int BM = 2 * 16 * RB, BN = WN * 16 * CB;  // 128 x 128 or 256 x 256
   constexpr int LROWS = THREADS / 8;                   // rows moved per pass of the block's loads
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(BIG ? 512 : 256) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int r = 16 * RB * wm + 16 * rb + li;
-    out_row[rb] = r < live ? checked_row(slot_rows[slot0 + r], a.tb) : -1;
+    out_row[rb] = r < live ? checked_row(y_rows[slot0 + r], a.tb) : -1;
   }
   const bf16_t* wbase = a.w + (int64_t)pe.expert * a.w_stride;
   const int nk = a.K / kGBK;
@@ -500,7 +501,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
   };
   // byte offsets of the wave's four x rows (rows past the end of a tile hold some row of x: their sums are never stored)
   auto x_rows = [&](const GroupedPlanEntry* pe, int (&row)[4]) __attribute__((always_inline)) {
-    if (a.map_rows) {
+    if (a.x_map) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) row[i] = wave < pe->ntiles ? slot_rows[(pe->tile0 + wave) * kTileRows + 8 * i + lrow] : 0;
     } else {
@@ -828,6 +829,14 @@ bool grouped_gemm_supported(const GroupedArgs& a) {
   return true;
 }
 
+bool grouped_gemm_direct(const GroupedArgs& a) {
+  // (TK_GROUPED_DIRECT=0 in the environment keeps the register-staged kernels in use: an A/B switch, read per call)
+  const char* env_direct = getenv("TK_GROUPED_DIRECT");
+  return TK_GROUPED_DL && !(env_direct && env_direct[0] == '0') && (int64_t)a.src_rows * a.ldx * 2 < (1ll << 32) &&
+         (int64_t)(a.w_rows_are_inputs ? a.K : a.N) * a.ldw * 2 < (1ll << 32) && a.ldy % 8 == 0 &&
+         (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0;  // (16-byte stores)
+}
+
 // upper bound of the row blocks, for either block size (workspace sizing)
 int64_t grouped_plan_entries(const SegLayout& L, int64_t experts) { return ceil_div(L.max_tiles, 4) + experts; }
 
@@ -839,19 +848,15 @@ int launch_grouped_gemm(const GroupedArgs& a, int experts, int nt, GroupedPlanEn
   // 8-wave kernel serves the transposing form and the rest, except with the LoRA term on small experts (its epilogue
   // has no registers to spare: measured at 512 rows per expert, 4 waves are then 5 % faster).
   const int nks = a.rpad == 0 ? 0 : (a.rpad <= 32 ? 1 : 2);
-  // (TK_GROUPED_DIRECT=0 in the environment keeps the register-staged kernels in use: an A/B switch, read per call)
-  const char* env_direct = getenv("TK_GROUPED_DIRECT");
-  const bool direct = TK_GROUPED_DL && !(env_direct && env_direct[0] == '0') &&
-                      (int64_t)a.src_rows * a.ldx * 2 < (1ll << 32) &&
-                      (int64_t)(a.w_rows_are_inputs ? a.K : a.N) * a.ldw * 2 < (1ll << 32) &&
-                      a.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0;  // (16-byte stores)
+  const bool direct = grouped_gemm_direct(a);
   const bool big =
       TK_GROUPED_BIG && a.N % 256 == 0 && (nks == 0 || direct || L.rows >= (int64_t)1024 * experts);
   const int ptiles = big ? 8 : 4, bn = big ? 256 : 128;
   const int max_entries = (int)(ceil_div(L.max_tiles, ptiles) + experts);
   hipLaunchKernelGGL(k_grouped_plan, dim3((unsigned)ceil_div(max_entries, kPlanBlock)), dim3(256), 0, s, a, seg, experts, nt,
                      plan, nblocks, max_entries, ptiles);
-  const int32_t* rows = seg.slot_table(a.map_rows);
+  const int32_t* y_rows = seg.slot_table(a.map_rows);
+  const int32_t* rows = a.x_map ? seg.slot_row : y_rows;
   const int ncb = a.N / bn;
   if (big && direct) {
     const dim3 blocks((unsigned)std::min<int64_t>(round_up((int64_t)max_entries * ncb, 8), kGroupedBlocks));
@@ -879,13 +884,13 @@ int launch_grouped_gemm(const GroupedArgs& a, int experts, int nt, GroupedPlanEn
   const dim3 grid((unsigned)((int64_t)max_entries * nsplit));
 #define TK_LAUNCH_GROUPED(NKS, BIG)                                                                                  \
   hipLaunchKernelGGL((k_grouped_gemm<NKS, BIG, 0>), grid, dim3(BIG ? 512 : 256), 0, s, a, plan, nblocks, seg.tile_group, \
-                     rows, nsplit, cpi)
+                     rows, y_rows, nsplit, cpi)
   if (a.w_rows_are_inputs) {  // never with the LoRA term (the caller checks)
     if (big)
-      hipLaunchKernelGGL((k_grouped_gemm<0, 1, 1>), grid, dim3(512), 0, s, a, plan, nblocks, seg.tile_group, rows, nsplit,
+      hipLaunchKernelGGL((k_grouped_gemm<0, 1, 1>), grid, dim3(512), 0, s, a, plan, nblocks, seg.tile_group, rows, y_rows, nsplit,
                          cpi);
     else
-      hipLaunchKernelGGL((k_grouped_gemm<0, 0, 1>), grid, dim3(256), 0, s, a, plan, nblocks, seg.tile_group, rows, nsplit,
+      hipLaunchKernelGGL((k_grouped_gemm<0, 0, 1>), grid, dim3(256), 0, s, a, plan, nblocks, seg.tile_group, rows, y_rows, nsplit,
                          cpi);
   } else if (big) {
     if (nks == 0) TK_LAUNCH_GROUPED(0, 1);

@@ -69,6 +69,9 @@ __device__ inline void load_keys8(const KeyT* keys, int64_t f0, int64_t rows, bo
   for (int j = 0; j < 8; ++j) out[j] = f0 + j < rows ? load_key(keys, f0 + j, buckets, bad) : -1;
 }
 
+// What a row's slot holds: the row, or the token it belongs to (top-k routing: row k * tokens + t).
+__device__ inline int32_t slot_entry(int row, int tokens) { return tokens > 0 ? row % tokens : row; }
+
 // lanes of this wave that are valid and hold the same key as the calling lane
 __device__ inline unsigned long long same_key_lanes(bool valid, int key, int key_bits) {
   unsigned long long same = __ballot(valid);
@@ -265,7 +268,7 @@ __device__ inline void seg_fill_tables(const SegView& V, int groups, int max_til
 template <typename KeyT>
 __global__ __launch_bounds__(64) void k_seg_scatter(const KeyT* __restrict__ keys, int rows, int groups, int key_bits,
                                                     SegView V, int64_t* __restrict__ perm_out, int sort_blocks,
-                                                    int max_tiles, int max_chunks, int chunk_tiles) {
+                                                    int max_tiles, int max_chunks, int chunk_tiles, int tokens) {
   extern __shared__ int32_t cursor[];
   const int lane = threadIdx.x;
   const int blk = blockIdx.x;
@@ -301,7 +304,7 @@ __global__ __launch_bounds__(64) void k_seg_scatter(const KeyT* __restrict__ key
       V.inv[f] = pos;
       if (perm_out) perm_out[pos] = f;
       // padded slot = 32 * first tile of the group + position inside the group
-      V.slot_row[V.tile_first[key] * kTileRows + (pos - V.offsets[key])] = (int32_t)f;
+      V.slot_row[V.tile_first[key] * kTileRows + (pos - V.offsets[key])] = slot_entry((int)f, tokens);
     }
   }
 }
@@ -328,7 +331,7 @@ constexpr int kOneBatch = kOneBlocks / kOneWaves;  // sort blocks whose keys a w
 template <typename KeyT>
 __global__ __launch_bounds__(kOneWaves * 64) void k_seg_one(const KeyT* __restrict__ keys, int rows, int groups,
                                                             int key_bits, int sort_blocks, int max_tiles,
-                                                            int max_chunks, int chunk_tiles, SegView V,
+                                                            int max_chunks, int chunk_tiles, int tokens, SegView V,
                                                             int64_t* __restrict__ perm_out,
                                                             int64_t* __restrict__ offsets_out) {
   __shared__ int32_t cnt[2][kOneSubs][kOneGroups + 1];  // keys ahead of this block / in it and after it
@@ -465,7 +468,7 @@ __global__ __launch_bounds__(kOneWaves * 64) void k_seg_one(const KeyT* __restri
       V.inv[f] = pos;
       if (perm_out) perm_out[pos] = f;
       // padded slot = 32 * first tile of the group + position inside the group
-      V.slot_row[tfirst[mine] * kTileRows + in_group] = (int32_t)f;
+      V.slot_row[tfirst[mine] * kTileRows + in_group] = slot_entry((int)f, tokens);
     }
     // Sweep order of the tiles.  The row that opens a tile (position inside its group a multiple of 32) knows how
     // many tiles open before it: for every group, the rows of that group ahead of this row, in units of 32, rounded
@@ -558,7 +561,7 @@ constexpr int kSmallWaves = 16;
 template <typename KeyT>
 __global__ __launch_bounds__(kSmallWaves * 64) void k_seg_small(const KeyT* __restrict__ keys, int rows, int groups, int key_bits,
                                                                 int rounds, int max_tiles, int max_chunks, int chunk_tiles,
-                                                                int sweep, SegView V, int64_t* __restrict__ perm_out,
+                                                                int sweep, int tokens, SegView V, int64_t* __restrict__ perm_out,
                                                                 int64_t* __restrict__ offsets_out) {
   extern __shared__ uint32_t cnt_words[];  // rows of each group in each round, then those ahead of the round
   uint16_t* cnt = reinterpret_cast<uint16_t*>(cnt_words);
@@ -668,7 +671,7 @@ __global__ __launch_bounds__(kSmallWaves * 64) void k_seg_small(const KeyT* __re
       moved = pos != f;
       V.inv[f] = pos;
       if (perm_out) perm_out[pos] = f;
-      V.slot_row[slot] = f;
+      V.slot_row[slot] = slot_entry(f, tokens);
       tile = k != groups - 1 && (in_group & (kTileRows - 1)) == 0;
       set = tile && (slot / kTileRows) % kSetTiles == 0;
     }
@@ -884,8 +887,8 @@ __global__ __launch_bounds__(64) void k_unpermute_wgrad(const T* __restrict__ do
   if (threadIdx.x == 0) dw[(int64_t)t * top_k + k] = acc;
 }
 
-// Both gradients of the weighted unpermute from one look at each row: grad_rows[pos(k, t)] = dout[t] * w[t, k] and
-// dw[t, k] = <dout[t], rows[pos(k, t)]>.  A block owns a token, whose dout stays in its cache over the top_k rows.  Bound by
+// Both gradients of the weighted unpermute from one look at each row: grad_rows[pos(k, t)] = dout[t] * w[t, k] (w null: 1) and,
+// unless dw is null, dw[t, k] = <dout[t], rows[pos(k, t)]>.  A block owns a token, whose dout stays in its cache over the top_k rows.  Bound by
 // memory: rows read and grad_rows written once (as two launches dout crossed the caches twice as often and the rows' reads had
 // no writes next to them: 65536 rows of 2048, 166 us; here 104).
 template <typename T, int V, typename W>
@@ -903,9 +906,17 @@ __global__ __launch_bounds__(256) void k_unpermute_bwd(const T* __restrict__ dou
     if ((unsigned)j < (unsigned)(tokens * top_k)) {  // (a position outside the table's rows: no row, no gradient)
       const RowVec<T, V>* r = reinterpret_cast<const RowVec<T, V>*>(rows_ + (int64_t)j * ld_rows);
       RowVec<T, V>* g = reinterpret_cast<RowVec<T, V>*>(grad + (int64_t)j * ld_grad);
-      const float wt = to_f32(w[(int64_t)t * top_k + k]);
+      const float wt = w ? to_f32(w[(int64_t)t * top_k + k]) : 1.f;
       for (int c = threadIdx.x; c < width / V; c += 256) {
         RowVec<T, V> x = d[c];
+        if (!dw) {
+          if (w) {
+#pragma unroll
+            for (int i = 0; i < V; ++i) from_f32(to_f32(x.v[i]) * wt, &x.v[i]);
+          }
+          g[c] = x;
+          continue;
+        }
         const RowVec<T, V> y = r[c];
 #pragma unroll
         for (int i = 0; i < V; ++i) {
@@ -917,10 +928,10 @@ __global__ __launch_bounds__(256) void k_unpermute_bwd(const T* __restrict__ dou
     }
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s, 64);
-    if (lane == 0) sums[k][wave] = acc;
+    if (dw && lane == 0) sums[k][wave] = acc;
   }
   __syncthreads();
-  if ((int)threadIdx.x < top_k) {
+  if (dw && (int)threadIdx.x < top_k) {
     const float* s = sums[threadIdx.x];
     from_f32((s[0] + s[1]) + (s[2] + s[3]), &dw[(int64_t)t * top_k + threadIdx.x]);
   }
@@ -954,7 +965,7 @@ inline bool rows_vectorise(int width, std::initializer_list<int64_t> lds, std::i
 }  // namespace
 
 int launch_segment_build(const void* keys, int key_dtype, int64_t rows, int32_t groups, int64_t* perm_out,
-                         int64_t* offsets_out, void* ws, hipStream_t s) {
+                         int64_t* offsets_out, void* ws, int tokens, hipStream_t s) {
   SegLayout L(rows, groups);
   SegView V(ws, L);
   const int nblk = (int)L.sort_blocks;
@@ -972,22 +983,24 @@ int launch_segment_build(const void* keys, int key_dtype, int64_t rows, int32_t 
     const int sweep = groups <= kOneGroups;  // as the other builders: beyond that the tiles keep the table's order
     if (key_dtype == TK_KEY_I32)
       hipLaunchKernelGGL(k_seg_small<int32_t>, dim3(1), dim3(kSmallWaves * 64), counts, s, (const int32_t*)keys, (int)rows,
-                         groups, key_bits, rounds, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, sweep, V, perm_out,
+                         groups, key_bits, rounds, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, sweep, tokens, V,
+                         perm_out,
                          offsets_out);
     else
       hipLaunchKernelGGL(k_seg_small<int64_t>, dim3(1), dim3(kSmallWaves * 64), counts, s, (const int64_t*)keys, (int)rows,
-                         groups, key_bits, rounds, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, sweep, V, perm_out,
+                         groups, key_bits, rounds, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, sweep, tokens, V,
+                         perm_out,
                          offsets_out);
     return check_launch();
   }
   if (groups <= kOneGroups && nblk <= kOneBlocks) {
     if (key_dtype == TK_KEY_I32)
       hipLaunchKernelGGL(k_seg_one<int32_t>, dim3(nblk), dim3(kOneWaves * 64), 0, s, (const int32_t*)keys, (int)rows,
-                         groups, key_bits, nblk, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, V, perm_out,
+                         groups, key_bits, nblk, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, tokens, V, perm_out,
                          offsets_out);
     else
       hipLaunchKernelGGL(k_seg_one<int64_t>, dim3(nblk), dim3(kOneWaves * 64), 0, s, (const int64_t*)keys, (int)rows,
-                         groups, key_bits, nblk, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, V, perm_out,
+                         groups, key_bits, nblk, (int)L.max_tiles, (int)L.max_chunks, (int)L.chunk_tiles, tokens, V, perm_out,
                          offsets_out);
     return check_launch();
   }
@@ -1004,11 +1017,11 @@ int launch_segment_build(const void* keys, int key_dtype, int64_t rows, int32_t 
   if (key_dtype == TK_KEY_I32)
     hipLaunchKernelGGL(k_seg_scatter<int32_t>, dim3(nblk + fill_blocks), dim3(64), lds, s, (const int32_t*)keys,
                        (int)rows, groups, key_bits, V, perm_out, nblk, (int)L.max_tiles, (int)L.max_chunks,
-                       (int)L.chunk_tiles);
+                       (int)L.chunk_tiles, tokens);
   else
     hipLaunchKernelGGL(k_seg_scatter<int64_t>, dim3(nblk + fill_blocks), dim3(64), lds, s, (const int64_t*)keys,
                        (int)rows, groups, key_bits, V, perm_out, nblk, (int)L.max_tiles, (int)L.max_chunks,
-                       (int)L.chunk_tiles);
+                       (int)L.chunk_tiles, tokens);
   return check_launch();
 }
 

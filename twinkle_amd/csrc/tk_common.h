@@ -508,9 +508,10 @@ struct GroupedPlanEntry {  // a row block of the grouped GEMM: up to 8 consecuti
 struct GroupedArgs {
   const uint16_t* x;  int64_t ldx;                     // activations, rows reached through the slot table
   const uint16_t* w;  int64_t w_stride, ldw;           // packed weights: expert e at w + e * w_stride, [N][K]
-  int32_t w_rows_are_inputs;                           // ... or [K][N]: y = x W (no LoRA term then)
+  int32_t w_rows_are_inputs;                           // ... or [K][N]: y = x W (LoRA term: lora_B holds A_g [r][N])
   uint16_t* y;        int64_t ldy;
   int32_t K, N, src_rows, map_rows;
+  int32_t x_map;                                       // x's src_rows rows are reached through slot_row whatever map_rows says of y
   // LoRA term (rpad = 0: none): y += h B_g^T with h[slot][rpad] as the shrink kernels leave it
   const void* const* lora_B;  int64_t ldb;
   const int32_t* rank;  int32_t rpad;
@@ -519,6 +520,7 @@ struct GroupedArgs {
   TableBounds tb;
 };
 bool grouped_gemm_supported(const GroupedArgs& a);
+bool grouped_gemm_direct(const GroupedArgs& a);  // k_grouped_gemm_dl takes it: the only kernel with a LoRA term for [K][N] weights
 int64_t grouped_plan_entries(const SegLayout& L, int64_t experts);
 int launch_grouped_gemm(const GroupedArgs& a, int experts, int nt, GroupedPlanEntry* plan, int32_t* nblocks,
                         const SegView& seg, const SegLayout& L, hipStream_t s);
@@ -532,7 +534,7 @@ int launch_swiglu(const void* gate_up, int64_t ld_in, const void* dout, int64_t 
 int launch_class_lists(const int32_t* rank, int n, const RankClass* rc, void* const* lists, int map_rows,
                        const SegView& seg, const SegLayout& L, hipStream_t s);
 int launch_segment_build(const void* keys, int key_dtype, int64_t rows, int32_t groups, int64_t* perm_out,
-                         int64_t* offsets_out, void* ws, hipStream_t s);
+                         int64_t* offsets_out, void* ws, int tokens, hipStream_t s);
 int launch_unpermute_bwd(const void* dout, int64_t ld_dout, const void* rows_, int64_t ld_rows, void* grad, int64_t ld_grad,
                          const void* w, void* dw, int dw_f32, const void* ws, int64_t rows, int64_t tokens, int32_t width,
                          int32_t groups, int dtype, hipStream_t s);

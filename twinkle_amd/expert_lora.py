@@ -456,11 +456,24 @@ def moe_experts_block(hidden_states: torch.Tensor, selected_experts: torch.Tenso
     weighted unpermute (the single-rank part of the reference's patched block forward,
     moe/expert_parallel.py:253-255 and moe/ep_utils.py:99-149, :280-287).  ``tenant [T]`` gives every token's
     index into ``tenant_slots`` (``None``: one tenant)."""
-    from .segments import build_segments, flat_keys_from_topk, permute, unpermute
+    from .segments import build_segments, build_token_segments, flat_keys_from_topk, permute, unpermute
     nt = len(tenant_slots)
     experts = experts_mod.gate_up_proj.shape[0]
     tokens = hidden_states.shape[0]
     keys = flat_keys_from_topk(selected_experts, tenant if nt > 1 else None, nt)
+    gate_up, down, x = experts_mod.gate_up_proj, experts_mod.down_proj, hidden_states
+    if (x.is_cuda and keys.is_cuda and keys.numel() and grouped_gemm_applies(gate_up, x) and grouped_gemm_applies(down, x) and
+            x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0):
+        # the first GEMM reads the tokens where they are: their permuted copy would be written once and read three times
+        from .ops import grouped_experts_linear
+        seg = build_token_segments(keys, experts * nt, tokens)
+        gate_up_out = grouped_experts_linear(x, gate_up, seg, nt,
+                                             gate_up_slots.groups(tenant_slots) if gate_up_slots is not None else None,
+                                             tokens=True)
+        hidden = _gated_activation(experts_mod, gate_up_out).contiguous()
+        out_rows = grouped_experts_linear(hidden, down, seg, nt,
+                                          down_slots.groups(tenant_slots) if down_slots is not None else None)
+        return unpermute(out_rows, routing_weights.to(x.dtype), seg)
     seg = build_segments(keys, experts * nt, num_tokens=tokens)
     rows, _ = permute(hidden_states, seg)
     out_rows = experts_forward(experts_mod, rows, seg, tenant_slots, gate_up_slots, down_slots)

@@ -14,7 +14,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from .segments import SegmentTable
+from .segments import SegmentTable, _scatter_rows
 
 
 class AdapterGroups:
@@ -409,19 +409,10 @@ def grouped_linear_(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTable, gr
     if y is None:
         y = torch.empty(seg.rows, out_f, dtype=x.dtype, device=x.device)
     _check_rows(y, 'y', seg.rows, out_f, weight.dtype)
-    g = _lib.GroupedDesc()
-    g.rows, g.num_groups, g.groups_per_expert = seg.rows, seg.num_groups, groups_per_expert
-    g.in_features, g.out_features = in_f, out_f
-    g.dtype = _lib.dtype_code(weight.dtype)
-    g.map_rows = 1 if map_rows else 0
-    g.seg_ws = seg.workspace.data_ptr()
-    g.weight, g.weight_stride, g.ldw = weight.data_ptr(), weight.stride(0), weight.stride(1)
-    g.weight_layout = 1 if transposed else 0
+    g = _grouped_desc(seg, groups_per_expert, weight, in_f, out_f, map_rows, transposed)
     lib = _lib.load()
     if workspace is None:
-        n = lib.tk_grouped_linear_workspace_bytes(ctypes.byref(g))
-        _lib.check(n, 'tk_grouped_linear_workspace_bytes')
-        workspace = torch.empty(n, dtype=torch.uint8, device=x.device)
+        workspace = _grouped_workspace(g, x.device)
     d = None
     if groups is not None:
         if h is None:
@@ -434,6 +425,46 @@ def grouped_linear_(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTable, gr
                                  _lib.stream_ptr())
     _lib.check(code, 'tk_grouped_linear')
     return y
+
+
+def _grouped_desc(seg, groups_per_expert, weight, in_f, out_f, map_rows, transposed) -> _lib.GroupedDesc:
+    g = _lib.GroupedDesc()
+    g.rows, g.num_groups, g.groups_per_expert = seg.rows, seg.num_groups, groups_per_expert
+    g.in_features, g.out_features = in_f, out_f
+    g.dtype = _lib.dtype_code(weight.dtype)
+    g.map_rows = 1 if map_rows else 0
+    g.seg_ws = seg.workspace.data_ptr()
+    g.weight, g.weight_stride, g.ldw = weight.data_ptr(), weight.stride(0), weight.stride(1)
+    g.weight_layout = 1 if transposed else 0
+    return g
+
+
+def _grouped_workspace(g: _lib.GroupedDesc, device) -> torch.Tensor:
+    n = _lib.load().tk_grouped_linear_workspace_bytes(ctypes.byref(g))
+    _lib.check(n, 'tk_grouped_linear_workspace_bytes')
+    return torch.empty(n, dtype=torch.uint8, device=device)
+
+
+def _grouped_from_tokens(tokens, weight, seg, groups_per_expert, groups):
+    """``(y, h)`` of the grouped linear on the tokens a :func:`build_token_segments` table's rows stand for."""
+    experts, out_f, in_f = weight.shape
+    _check_rows(tokens, 'tokens', seg.num_tokens, in_f, weight.dtype)
+    lib, h, d = _lib.load(), None, None
+    if groups is not None:
+        if groups.num_groups != seg.num_groups or groups.in_features != in_f or groups.out_features != out_f:
+            raise ValueError('adapters and weights describe different layers')
+        d = ctypes.byref(_desc(seg, groups, False))
+        h = torch.empty(lora_h_bytes(seg, groups), dtype=torch.uint8, device=tokens.device)
+        _lib.check(lib.tk_lora_shrink_tokens(d, tokens.data_ptr(), tokens.stride(0), seg.num_tokens, h.data_ptr(),
+                                             _lib.stream_ptr()), 'tk_lora_shrink_tokens')
+    y = torch.empty(seg.rows, out_f, dtype=weight.dtype, device=tokens.device)
+    g = _grouped_desc(seg, groups_per_expert, weight, in_f, out_f, False, False)
+    ws = _grouped_workspace(g, tokens.device)
+    code = lib.tk_grouped_linear_tokens(ctypes.byref(g), d, tokens.data_ptr(), tokens.stride(0), seg.num_tokens, y.data_ptr(),
+                                        y.stride(0), h.data_ptr() if h is not None else None, ws.data_ptr(), ws.numel(),
+                                        _lib.stream_ptr())
+    _lib.check(code, 'tk_grouped_linear_tokens')
+    return y, h
 
 
 def _weight_grads(ctx_groups: AdapterGroups, needs_a: bool, needs_b: bool, device, rows: int):
@@ -556,52 +587,78 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
 
 
 class _GroupedExpertsLinear(torch.autograd.Function):
-    """Frozen packed expert weights and the (expert, tenant) LoRA terms as one node on rows in segment order.
+    """Frozen packed expert weights and the (expert, tenant) LoRA terms as one node on rows in segment order, or (``tokens``) on
+    the tokens whose rows those are, which saves the permuted copy of them.
 
-    Forward: shrink, then the grouped GEMM with the LoRA term in its epilogue.  Backward: the grouped GEMM in its
-    transposing form on the same weights gives the base part of ``dx``; the segmented backward adds the LoRA part
-    onto it in place and yields the adapters' gradients.  The weights get no gradient (the reference freezes them)."""
+    Forward: shrink, then the grouped GEMM with the LoRA term as one of its steps.  Backward: dh and dB from dy, then the
+    grouped GEMM in its transposing form on the same weights gives dx, the LoRA part as one of its steps again, then dA; the
+    tokens' gradient is the sum over their rows.  The weights get no gradient (the reference freezes them)."""
 
     @staticmethod
-    def forward(ctx, x, weight, seg, groups_per_expert, groups, *weights):
+    def forward(ctx, x, weight, seg, groups_per_expert, groups, tokens, *weights):
         h = None
-        if groups is not None:
-            h = torch.empty(lora_h_bytes(seg, groups), dtype=torch.uint8, device=x.device)
-            lora_shrink_(x, seg, groups, h, map_rows=False)
-        y = grouped_linear_(x, weight, seg, groups_per_expert, groups=groups, h=h, map_rows=False)
+        if tokens:
+            y, h = _grouped_from_tokens(x, weight, seg, groups_per_expert, groups)
+        else:
+            if groups is not None:
+                h = torch.empty(lora_h_bytes(seg, groups), dtype=torch.uint8, device=x.device)
+                lora_shrink_(x, seg, groups, h, map_rows=False)
+            y = grouped_linear_(x, weight, seg, groups_per_expert, groups=groups, h=h, map_rows=False)
         ctx.save_for_backward(x, weight, h)
-        ctx.seg, ctx.groups, ctx.groups_per_expert = seg, groups, groups_per_expert
+        ctx.seg, ctx.groups, ctx.groups_per_expert, ctx.tokens = seg, groups, groups_per_expert, tokens
         return y
 
     @staticmethod
     def backward(ctx, dy):
         x, weight, h = ctx.saved_tensors
-        seg, groups = ctx.seg, ctx.groups
+        seg, groups, per_expert = ctx.seg, ctx.groups, ctx.groups_per_expert
         dy = dy.contiguous()
         needs_dx = ctx.needs_input_grad[0]
-        dx = grouped_linear_(dy, weight, seg, ctx.groups_per_expert, map_rows=False, transposed=True) \
-            if needs_dx else None
+
+        def of_tokens(dx):
+            return _scatter_rows(dx, None, seg) if dx is not None and ctx.tokens else dx
+
         if groups is None:
-            return (dx, None, None, None, None)
+            dx = grouped_linear_(dy, weight, seg, per_expert, map_rows=False, transposed=True) if needs_dx else None
+            return (of_tokens(dx), None, None, None, None, None)
         na, nb = len(groups.a_tensors), len(groups.b_tensors)
-        needs_a = any(ctx.needs_input_grad[5:5 + na])
-        needs_b = any(ctx.needs_input_grad[5 + na:5 + na + nb])
-        arena_a, arena_b, pa, pb = _weight_grads(groups, needs_a, needs_b, dy.device, seg.rows)
+        needs_a = any(ctx.needs_input_grad[6:6 + na])
+        needs_b = any(ctx.needs_input_grad[6 + na:6 + na + nb])
+        out_f, in_f = weight.shape[1:]
+        _check_rows(dy, 'dy', seg.rows, out_f, groups.dtype)
+        dx = torch.empty(seg.rows, in_f, dtype=dy.dtype, device=dy.device) if needs_dx else None
+        arenas = [None, None]
+        for i, (needed, elems) in enumerate(((needs_a, groups.a_arena_elems), (needs_b, groups.b_arena_elems))):
+            if needed:
+                new = torch.zeros if groups.arena_plan()[0] or not seg.rows else torch.empty
+                arenas[i] = new(elems, dtype=groups.weight_dtype, device=dy.device)
         if needs_dx or needs_a or needs_b:
-            lora_bwd_(dy, x, h, dx, pa, pb, seg, groups, False, accumulate=False)
-        ga = groups.grad_views(arena_a, 'a') if needs_a else [None] * na
-        gb = groups.grad_views(arena_b, 'b') if needs_b else [None] * nb
-        return (dx, None, None, None, None, *ga, *gb)
+            g = _grouped_desc(seg, per_expert, weight, out_f, in_f, False, True)
+            ws = _grouped_workspace(g, dy.device)
+            lora_ws = torch.empty(lora_bwd_workspace_bytes(seg, groups), dtype=torch.uint8, device=dy.device)
+            at = (groups._grad_a_rel, groups._grad_b_rel)
+            places = [p for t, arena in zip(at, arenas) for p in
+                      ((t.data_ptr(), arena.data_ptr()) if arena is not None and arena.numel() else (None, None))]
+            code = _lib.load().tk_grouped_linear_bwd(
+                ctypes.byref(g), ctypes.byref(_desc(seg, groups, False)), dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0),
+                seg.num_tokens if ctx.tokens else 0, h.data_ptr(), dx.data_ptr() if dx is not None else None,
+                dx.stride(0) if dx is not None else 0, *places, ws.data_ptr(), ws.numel(), lora_ws.data_ptr(), lora_ws.numel(),
+                _lib.stream_ptr())
+            _lib.check(code, 'tk_grouped_linear_bwd')
+        ga = groups.grad_views(arenas[0], 'a') if needs_a else [None] * na
+        gb = groups.grad_views(arenas[1], 'b') if needs_b else [None] * nb
+        return (of_tokens(dx), None, None, None, None, None, *ga, *gb)
 
 
 def grouped_experts_linear(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTable, groups_per_expert: int,
-                           groups: Optional[AdapterGroups] = None) -> torch.Tensor:
+                           groups: Optional[AdapterGroups] = None, tokens: bool = False) -> torch.Tensor:
     """``y = x W_e^T`` plus every (expert, tenant) group's LoRA term, for rows in segment order; differentiable in
-    ``x`` and the adapters, not in the frozen ``weight [E, out, in]`` (both widths multiples of 128)."""
+    ``x`` and the adapters, not in the frozen ``weight [E, out, in]`` (both widths multiples of 128).  ``tokens``: ``x`` holds
+    the tokens ``[seg.num_tokens, in]`` that the rows of a :func:`build_token_segments` table stand for."""
     extra = groups.autograd_tensors() if groups is not None else []
     if groups is not None:
         groups.sync_masters()
-    return _GroupedExpertsLinear.apply(x, weight, seg, groups_per_expert, groups, *extra)
+    return _GroupedExpertsLinear.apply(x, weight, seg, groups_per_expert, groups, tokens, *extra)
 
 
 def multi_lora_delta(x: torch.Tensor, base_out: torch.Tensor, seg: SegmentTable, groups: AdapterGroups,

@@ -36,6 +36,7 @@ class SegmentTable:
         self.workspace = workspace
         self.perm = perm
         self.offsets = offsets
+        self.of_tokens = False    # built by build_token_segments
 
     @property
     def device(self):
@@ -117,6 +118,22 @@ def build_segments(keys: torch.Tensor, num_groups: int, num_tokens: Optional[int
     return table
 
 
+def build_token_segments(keys: torch.Tensor, num_groups: int, num_tokens: int) -> SegmentTable:
+    """The table of top-k routed rows for kernels that read the tokens themselves (``tk_segment_build_tokens``): for
+    :func:`twinkle_amd.ops.grouped_experts_linear` with ``tokens`` and :func:`unpermute`, nothing else.  ``keys`` as
+    :func:`flat_keys_from_topk` makes them."""
+    lib, rows = _lib.load(), keys.numel()
+    nbytes = lib.tk_segment_workspace_bytes(rows, num_groups)
+    _lib.check(nbytes, 'tk_segment_workspace_bytes')
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
+    code = lib.tk_segment_build_tokens(keys.data_ptr(), _lib.TK_KEY_I32 if keys.dtype == torch.int32 else _lib.TK_KEY_I64, rows,
+                                       num_groups, num_tokens, ws.data_ptr(), nbytes, _lib.stream_ptr())
+    _lib.check(code, 'tk_segment_build_tokens')
+    table = SegmentTable(rows, num_groups, num_tokens, ws, None, None)
+    table.of_tokens = True
+    return table
+
+
 def _keys_on_gpu(selected: torch.Tensor, tenant: Optional[torch.Tensor]) -> bool:
     """Plain GPU tensors one launch makes the keys of (torch's three to five cost more than the table behind them)."""
     def plain(t, dim):
@@ -186,6 +203,8 @@ def _check_2d(t: torch.Tensor, name: str):
 
 def _gather_rows(src, weights, seg):
     _check_2d(src, 'tokens')
+    if seg.of_tokens:
+        raise ValueError('a table of tokens does not say which row a slot holds')
     out = torch.empty(seg.rows, src.shape[1], dtype=src.dtype, device=src.device)
     if weights is not None:
         weights = weights.to(src.dtype).contiguous()
@@ -227,19 +246,22 @@ class _Unpermute(torch.autograd.Function):
         rows, weights = ctx.saved_tensors
         seg = ctx.seg
         grad_out = grad_out.contiguous()
-        if weights is not None and all(ctx.needs_input_grad[:2]) and seg.top_k <= _lib.TK_UNPERMUTE_BWD_TOP_K:
-            w = weights.to(rows.dtype).contiguous()
+        grad_rows = grad_w = None
+        if ctx.needs_input_grad[0]:
+            w = weights.to(rows.dtype).contiguous() if weights is not None else None
             grad_rows = torch.empty(seg.rows, rows.shape[1], dtype=rows.dtype, device=rows.device)
-            same = weights.dtype == rows.dtype
-            dw = torch.empty(seg.num_tokens, seg.top_k, dtype=weights.dtype if same else torch.float32, device=rows.device)
+            dw = None
+            if weights is not None and ctx.needs_input_grad[1] and seg.top_k <= _lib.TK_UNPERMUTE_BWD_TOP_K:
+                kind = weights.dtype if weights.dtype == rows.dtype else torch.float32
+                dw = torch.empty(seg.num_tokens, seg.top_k, dtype=kind, device=rows.device)
             code = _lib.load().tk_unpermute_bwd(
                 grad_out.data_ptr(), grad_out.stride(0), rows.data_ptr(), rows.stride(0), grad_rows.data_ptr(),
-                grad_rows.stride(0), w.data_ptr(), dw.data_ptr(), 0 if same else 1, seg.workspace.data_ptr(), seg.rows,
-                seg.num_tokens, rows.shape[1], seg.num_groups, _lib.dtype_code(rows.dtype), _lib.stream_ptr())
+                grad_rows.stride(0), w.data_ptr() if w is not None else None, dw.data_ptr() if dw is not None else None,
+                1 if dw is not None and dw.dtype == torch.float32 else 0, seg.workspace.data_ptr(), seg.rows, seg.num_tokens,
+                rows.shape[1], seg.num_groups, _lib.dtype_code(rows.dtype), _lib.stream_ptr())
             _lib.check(code, 'tk_unpermute_bwd')
-            return grad_rows, dw.to(weights.dtype), None
-        grad_rows = _gather_rows(grad_out, weights, seg) if ctx.needs_input_grad[0] else None
-        grad_w = None
+            if dw is not None:
+                return grad_rows, dw.to(weights.dtype), None
         if weights is not None and ctx.needs_input_grad[1]:
             dw = torch.empty(seg.num_tokens, seg.top_k, dtype=torch.float32, device=rows.device)
             lib = _lib.load()
