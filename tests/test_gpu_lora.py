@@ -713,3 +713,31 @@ def test_backward_with_a_subset_of_the_outputs(dev, max_r, ranks):
                 assert max_rel_err(gb[g], full[2][g].double().cpu()) < 1e-2, want
             else:
                 assert torch.count_nonzero(gb[g]) == 0
+
+
+@pytest.mark.parametrize('rank', [17, 32, 40, 64, 100, 128])
+@pytest.mark.parametrize('rows,groups,width', [(256, 1, 1024), (257, 1, 1088), (600, 2, 1024), (1023, 3, 4096), (2100, 8, 2048)])
+@pytest.mark.parametrize('offset', [0, 4])
+def test_shrink_by_sets_of_eight_tiles(dev, rank, rows, groups, width, offset):
+    """The shrink that loads straight into LDS: sets that straddle groups, the last set and the last slice short, slices of
+    steps off its unrolling, ranks that end inside a load, lora_A off its 16-byte alignment, rows of no adapter."""
+    g = torch.Generator().manual_seed(rank + rows)
+    a = []
+    for _ in range(groups):
+        flat = torch.empty(offset + rank * width, dtype=torch.bfloat16, device=dev)
+        a.append(flat[offset:].view(rank, width).copy_(torch.randn(rank, width, generator=g) / width**0.5))
+    out = 128
+    b = [torch.zeros(out, 128, dtype=torch.bfloat16, device=dev) for _ in range(groups)]
+    for v in b:
+        v[:, :128].copy_(torch.eye(128))                    # y = h, rank index by rank index
+    ids = torch.randint(-1, groups, (rows,), generator=g, dtype=torch.int32)
+    x = torch.randn(rows, width + 8, generator=g).bfloat16().to(dev)[:, :width]
+    y = torch.zeros(rows, out, dtype=torch.bfloat16, device=dev)
+    groups_ = AdapterGroups(a, b, [rank] * groups, [1.0] * groups)
+    lora_fwd_(x, y, build_segments(ids.to(dev), groups), groups_)
+    want = torch.zeros(rows, out, dtype=torch.float64)
+    for i in range(groups):
+        m = ids == i
+        want[m, :rank] = x[m.to(dev)].double().cpu() @ a[i].double().cpu().t()
+    # sums of `width` products in fp32, h rounded to eight bits; y holds h
+    assert max_rel_err(y, want) < 2**-8 + 1e-5

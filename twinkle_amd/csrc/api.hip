@@ -765,9 +765,13 @@ static int lora_bwd_class(const tk_lora_desc* d, const ClassPlan& P, int c, cons
   // may share a hardware queue with the caller's, and then nothing runs side by side)
   SideStream* side = grad_B && need_wT && may_fork && side_stream_mode() != 0 ? side_stream() : nullptr;
   if (side && side_stream_mode() != 1 && !worth_forking(*d, bytes, any_shape_bf16, a.rpad, class_mode != 0, s)) side = nullptr;
-  // next to the contraction of dB a block of eight waves waits for a CU of its own; with up to 1024 columns of dy that is
-  // most of its time (32768 x 4096 -> 1024 at rank 64: the backward takes 230 us, 258 with k_shrink_oct)
-  if (side && a.rpad <= 64 && a.set_waves == 8 && a.width_src <= 1024) a.set_waves = 4;
+  // next to the contraction of dB a block of eight waves waits for a CU of its own; with up to 1024 columns of dy and a block
+  // for most CUs that is most of its time (rank 64, 32768 x 4096 -> 1024, 256 blocks: the backward takes 242 us, 263 with
+  // k_shrink_dl; 12288 rows, 96 blocks: 133 and 124)
+  if (side && a.rpad <= 64 && a.set_steps > 0 && a.width_src <= 1024 && ceil_div(d->rows, 8 * kTileRows) * a.kslices > 192) {
+    a.set_waves = 4;
+    a.set_narrow = 1;
+  }
   hipStream_t s2 = side ? side->stream : s;
   // two host threads must not interleave their records and waits on the device's one set of events
   std::unique_lock<std::mutex> side_guard;

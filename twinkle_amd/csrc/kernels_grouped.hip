@@ -370,35 +370,6 @@ __global__ __launch_bounds__(BIG ? 512 : 256) __attribute__((amdgpu_waves_per_eu
 // products before them run.  A tile multiplies with the piece of its own group only, picked out of the weight tile, so
 // what another tenant's adapter holds (infinities, NaN) never meets its rows.
 // ---------------------------------------------------------------------------
-// Wait until at most YOUNGER of the wave's loads are in flight (they complete in order) and its LDS reads are done,
-// then the block barrier.  Written out: the fences of __syncthreads() make the compiler wait for every load in
-// flight, the look-ahead ones included.
-template <int YOUNGER>
-__device__ __forceinline__ void loads_landed_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(0x0070 | YOUNGER);  // vmcnt(YOUNGER), at most 15, lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
-__device__ __forceinline__ void load16_to_lds(const bf16_t* base, uint32_t byte_offset, bf16_t* window) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void*)(reinterpret_cast<const char*>(base) + byte_offset),
-      (__attribute__((address_space(3))) void*)window, 16, 0, 0);
-}
-
-// The same with a buffer descriptor: per-lane offset in a 32-bit register, the step's offset in a scalar one, nothing past
-// `bytes`.
-typedef __amdgpu_buffer_rsrc_t Buffer;
-__device__ __forceinline__ Buffer buffer_of(const void* p, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)min(bytes, (int64_t)0xffffffff), 0x00020000);
-}
-__device__ __forceinline__ void buffer16_to_lds(Buffer b, uint32_t lane_offset, uint32_t offset, bf16_t* window) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void*)window, 16, (int)lane_offset,
-                                           (int)offset, 0, 0);
-}
-
 // 64 bits per lane from LDS, transposed among 16 lanes (ds_read_b64_tr_b16): with M[p][e] the four 16-bit elements
 // e that lane p of a group of 16 points at, lane l receives M[4 e + (l >> 2)][l & 3], e = 0..3.
 __device__ __forceinline__ uint2 lds_read_transposed(const char* p) {
@@ -413,9 +384,6 @@ __device__ __forceinline__ int here(int v) {
   asm volatile("" : "+v"(v));
   return v;
 }
-
-// what the LoRA step multiplies with past a group's rank
-__device__ __attribute__((aligned(16))) uint32_t grouped_zeros[4];
 
 // TR = 1: the weight rows are input features (y = x W, the backward of TR = 0 on the same memory).  The weight
 // tile of a step is then 64 rows of 256 outputs, 512 bytes a row, and lies in LDS as it lies in memory (a wave-wide
@@ -608,7 +576,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
         const bf16_t* src = TR ? p + (int64_t)(2 * i) * a.ldb + 8 * (chunk ^ ((i & 1) << 2)) : p + (int64_t)(8 * i) * a.ldb;
         bf16_t* to = TR ? Bs + (8 * wave + 2 * i) * BN : Bs + window + 8 * i * kGBK;
         if (!slow) {
-          load16_to_lds(live ? src : reinterpret_cast<const bf16_t*>(grouped_zeros), 0u, to);
+          load16_to_lds(live ? src : reinterpret_cast<const bf16_t*>(kernel_zeros), 0u, to);
         } else {
           const int keep = !live ? 0 : TR ? 8 : min(lora_r - n0, 8);
 #pragma unroll 1

@@ -505,7 +505,10 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
   const int32_t* rows = seg.slot_table(a.map_rows);
   constexpr int NW = NB == 1 ? 1 : (NB == 2 ? 2 : 4);  // shrink_waves(16 * NB)
   if (phases & 1) {
-    if (NB > 1 && a.set_steps > 0)  // see shrink_plan
+    if (NB > 1 && a.set_steps > 0 && shrink_dl_applies(a))
+      hipLaunchKernelGGL((k_shrink_dl<NB == 1 ? 2 : NB>), dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(512), 0,
+                         s, a, seg.tile_group, rows, (int)L.max_tiles);
+    else if (NB > 1 && a.set_steps > 0)  // see shrink_plan
       hipLaunchKernelGGL((a.set_waves == 8 ? k_shrink_oct<NB == 1 ? 2 : NB> : k_shrink_quad<NB == 1 ? 2 : NB>),
                          dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(64 * a.set_waves), 0, s, a,
                          seg.tile_group, rows, (int)L.max_tiles);

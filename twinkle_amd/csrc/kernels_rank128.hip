@@ -2,7 +2,7 @@
 //
 // What bounds these kernels is the memory system, as at the lower ranks; the rank costs registers (accumulators and the
 // weight block of the expand) and L2 reads of weights.  8192 rows x 4096 columns, four adapters, us, against the kernels
-// for any shape (kernels_generic.hip): shrink 64 + 14 -> 38 + 11 (the slices hold half as many bytes as the source),
+// for any shape (kernels_generic.hip): shrink 64 + 14 -> 30 + 11 (the slices hold half as many bytes as the source),
 // expand 84 -> 49 (2.7 TB/s of y; 31 where it only writes), row contraction 94 -> 35 (chunks in pairs and one reader per
 // tile), its reduction 36 -> 22.
 #include <algorithm>
@@ -20,6 +20,9 @@ int launch_pass_rank128(const PassArgs& a, const SegView& seg, const SegLayout& 
     if (a.set_steps == 0) {
       const int rc = launch_pass_generic(a, seg, L, TK_DTYPE_BF16, 1, s);
       if (rc != TK_OK) return rc;
+    } else if (shrink_dl_applies(a)) {
+      hipLaunchKernelGGL(k_shrink_dl<8>, dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(512), 0, s, a,
+                         seg.tile_group, rows, (int)L.max_tiles);
     } else {
       hipLaunchKernelGGL(k_shrink_oct<8>, dim3((unsigned)(ceil_div(L.max_tiles, 8) * a.kslices)), dim3(512), 0, s, a,
                          seg.tile_group, rows, (int)L.max_tiles);

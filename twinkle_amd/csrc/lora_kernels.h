@@ -7,7 +7,7 @@
 // wave-wide load covers whole 128-byte lines and every activation byte crosses
 // HBM once per pass.
 //
-//   k_shrink_pair / k_shrink_oct / k_shrink_finish    h = scale * x A^T (split over column slices when x is wide)
+//   k_shrink_pair / k_shrink_dl / k_shrink_oct / k_shrink_finish    h = scale * x A^T (split over column slices when x is wide)
 //   k_expand_mfma / k_expand_multi                     y += h B^T in place (rank <= 16 / above)
 //   k_wgrad_pipe / k_wgrad_coop                        dA, dB: contraction over the rows of a chunk (rank <= 16 / above)
 //   transpose_weights_job                              B^T, A^T copies for the backward shrink / expand
@@ -22,6 +22,8 @@
 #pragma once
 
 #include <algorithm>
+
+#include <type_traits>
 
 #include "tk_mfma.h"
 
@@ -388,6 +390,146 @@ __global__ __launch_bounds__(512) void k_shrink_oct(PassArgs a, const int32_t* _
                                                     const int32_t* __restrict__ slot_rows, int max_tiles) {
   shrink_oct_body<NB>(a, tile_group, slot_rows, max_tiles, blockIdx.x);
 }
+
+// ---------------------------------------------------------------------------
+// The same work as k_shrink_oct, item by item and sum by sum, with the operands going from memory straight into LDS: no
+// registers hold loads in flight, so three stages of 64 columns (x 32 KB, weights RP x 128 B) are on their way per CU where
+// the registers held one or two steps, which is what the time of a step was.  A wave's tile goes through a window of its own
+// (no barrier for it), the weights are shared: one barrier a step, behind a wait for the wave's loads of that step; the
+// stage read before it takes the loads two steps ahead.  Rows of 128 B, 16-byte chunk c of row r at position c ^ (r & 7): a
+// load covers whole lines, an operand read eight different bank groups.
+// Source under 4 GB (32-bit row offsets); the weights of a matrix that is not 16-byte aligned go through registers.
+// Shrink with its slice sums, eight adapters, oct or quad / here, us: rank 128 8192 x 4096 49.6 / 39.3, 32768 x 4096 126 /
+// 104; rank 64 8192 x 4096 32.6 / 28.2, 32768 x 4096 86 / 76; rank 32 8192 x 4096 28.7 / 23.6, 2048 x 1024 20.1 / 14.1: faster
+// at every size from 2048 x 1024 to 32768 x 4096, rows packed or shuffled.
+// ---------------------------------------------------------------------------
+template <int NB>
+__device__ __forceinline__ void shrink_dl_body(const PassArgs& a, const int32_t* __restrict__ tile_group,
+                                               const int32_t* __restrict__ slot_rows, int max_tiles, int item) {
+  constexpr int RP = 16 * NB, NW = NB > 4 ? NB / 4 : 1;  // NW: weight loads of a wave per step (8 rank indices each)
+  __shared__ __attribute__((aligned(1024))) bf16_t X0[256 * 64], X1[256 * 64], X2[256 * 64];
+  __shared__ __attribute__((aligned(1024))) bf16_t W0[RP * 64], W1[RP * 64], W2[RP * 64];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kb = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nth = item / a.kslices, ks = item - nth * a.kslices;
+  const int set = work_item(a.wl_octs, nth);
+  if (set < 0) return;  // past the end of this rank class's list (uniform over the block)
+  const int t_first = set * 8;
+  const int my_tile = t_first + (lane & 7);
+  const int gts = my_tile < max_tiles ? checked_group(tile_group[my_tile], a.tb) : -1;  // lane j: group of tile j
+  const int s0 = ks * a.set_steps;
+  const int ns = min(a.set_steps, (a.width_src >> 6) - s0);  // >= 1 for every slice
+  const int lrow = lane >> 3, chunk = (lane & 7) ^ lrow;
+  uint32_t xoff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = min(t_first + wave, max_tiles - 1);
+    const int row = min(max(slot_rows[t * kTileRows + 8 * i + lrow], 0), a.src_rows - 1);
+    xoff[i] = (uint32_t)row * (uint32_t)(a.ld_src * 2) + (uint32_t)(s0 * 128 + chunk * 16);
+  }
+  const int64_t xbytes = ((int64_t)(a.src_rows - 1) * a.ld_src + a.width_src) * 2;
+  const uint32_t rd = (uint32_t)((2 * kb) ^ (li & 7)) * 16u;  // this lane's chunk 2 kb of a row; chunk 2 kb + 1: ^ 16
+  for (int j = 0; j < 8;) {
+    const int g = __builtin_amdgcn_readlane(gts, j);
+    int e = j + 1;
+    while (e < 8 && __builtin_amdgcn_readlane(gts, e) == g) ++e;
+    const int lo = j, hi = e;  // the run: tiles t_first + lo .. t_first + hi - 1, all of group g
+    j = e;
+    if (g < 0) continue;
+    const int r = class_rank(a.rank[g], a.rank_lo, RP);
+    if (r <= 0) continue;  // adapter not live on this layer, or a group of another rank class
+    const bool active = wave >= lo && wave < hi;
+    const bf16_t* W = group_weight<bf16_t>(a.w_shrink, a.w_shrink_base, a.shrink_group_stride, g) + (int64_t)s0 * 64;
+    const bf16_t* wp[NW];
+    uint32_t wlive[NW];
+    int wrow[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      wrow[i] = 8 * (NB >= 4 ? wave + 8 * i : wave & (2 * NB - 1));  // (rank 32: two waves bring the same rows)
+      const int n = wrow[i] + lrow;
+      wlive[i] = n < r ? ~0u : 0u;
+      wp[i] = n < r ? W + (int64_t)n * a.ld_shrink + 8 * chunk : reinterpret_cast<const bf16_t*>(kernel_zeros);
+    }
+    auto fetch_x = [&](int s, bf16_t* X) __attribute__((always_inline)) {
+      const Buffer xbuf = buffer_of(a.src, active && s < ns ? xbytes : 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) buffer16_to_lds(xbuf, xoff[i], (uint32_t)s * 128u, X + (32 * wave + 8 * i) * 64);
+    };
+    auto fetch_w = [&](int s, bf16_t* Ws, auto direct) __attribute__((always_inline)) {
+      const uint32_t at = (uint32_t)min(s, ns - 1) * 128u;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        if constexpr (decltype(direct)::value) {
+          load16_to_lds(wp[i], at & wlive[i], Ws + wrow[i] * 64);
+        } else {
+          st16(Ws + wrow[i] * 64 + 8 * lane,
+               ld16(reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(wp[i]) + (at & wlive[i]))));
+        }
+      }
+    };
+    f32x4 acc[2][NB];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const bf16_t* X, const bf16_t* Ws) __attribute__((always_inline)) {
+      const char* xr = reinterpret_cast<const char*>(X) + (32 * wave + li) * 128;
+      const char* wr = reinterpret_cast<const char*>(Ws) + li * 128;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const uint32_t at = rd ^ (16u * p);
+        uint4 fx[2], fw[NB];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) fx[tt] = *reinterpret_cast<const uint4*>(xr + 2048 * tt + at);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) fw[nb] = *reinterpret_cast<const uint4*>(wr + 2048 * nb + at);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mfma16(fw[nb], fx[tt], acc[tt][nb]);
+      }
+    };
+    auto run = [&](auto direct) __attribute__((always_inline)) {
+      fetch_x(0, X0);
+      fetch_w(0, W0, direct);
+      fetch_x(1, X1);
+      fetch_w(1, W1, direct);
+      auto step = [&](int s, const bf16_t* X, const bf16_t* Ws, bf16_t* Xn, bf16_t* Wn) __attribute__((always_inline)) {
+        if constexpr (decltype(direct)::value) loads_landed_barrier<4 + NW>();
+        else loads_landed_barrier<4>();  // (the younger step's weights have been waited for on their way)
+        fetch_x(s + 2, Xn);
+        fetch_w(s + 2, Wn, direct);
+        if (active && s < ns) compute(X, Ws);
+      };
+      for (int s = 0; s < ns; s += 3) {
+        step(s, X0, W0, X2, W2);
+        step(s + 1, X1, W1, X0, W0);
+        step(s + 2, X2, W2, X1, W1);
+      }
+    };
+    if ((reinterpret_cast<uintptr_t>(W) & 15u) == 0) run(std::integral_constant<bool, true>{});
+    else run(std::integral_constant<bool, false>{});
+    if (active) {
+      float* out = a.hpart + ((int64_t)(t_first + wave) * a.kslices + ks) * (kTileRows * RP) + li * RP + 4 * kb;
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          *reinterpret_cast<float4*>(out + 16 * tt * RP + 16 * nb) =
+              make_float4(acc[tt][nb][0], acc[tt][nb][1], acc[tt][nb][2], acc[tt][nb][3]);
+    }
+    loads_landed_barrier<0>();  // the stages are the next run's, or the next block's
+  }
+}
+
+template <int NB>
+__global__ __launch_bounds__(512) void k_shrink_dl(PassArgs a, const int32_t* __restrict__ tile_group,
+                                                   const int32_t* __restrict__ slot_rows, int max_tiles) {
+  shrink_dl_body<NB>(a, tile_group, slot_rows, max_tiles, blockIdx.x);
+}
+
+// whether k_shrink_dl runs: sources of 32-bit offsets, and see set_narrow
+inline bool shrink_dl_applies(const PassArgs& a) { return !a.set_narrow && ((int64_t)a.src_rows * a.ld_src) * 2 < (1ll << 32); }
 
 // Adds the slices of a split shrink in slice order and writes h (one block per tile).
 template <int NB>

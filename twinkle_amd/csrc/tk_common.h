@@ -221,7 +221,8 @@ static inline int shrink_waves(int rpad) { return rpad <= 16 ? 1 : (rpad <= 32 ?
 static inline int shrink_kslices(int width, int rpad) {
   return (int)ceil_div(ceil_div(width, 64), (int64_t)kShrinkSteps * shrink_waves(rpad));
 }
-// Above rank 16, with long groups and a source of 1024 to 4096 columns, the shrink runs as k_shrink_oct or k_shrink_quad:
+// Above rank 16, with long groups and a source of 1024 to 4096 columns, the shrink runs as k_shrink_dl, and where that does not
+// apply (sources of 4 GB, several projections of one input, set_narrow) as k_shrink_oct or k_shrink_quad:
 // blocks of (eight tiles, `steps` steps of 64 columns), at most 512 of them (twice as many slices: 98 us against 77 for
 // 32768 x 4096 at rank 64, their sums are written and read; half as many: 81).  Wider sources stay with k_shrink_pair (24
 // adapters of rank 8 to 64, 32768 x 4096 -> 14336: the training step takes 1037 us, with the wide dy on k_shrink_oct 1054).
@@ -392,7 +393,8 @@ struct PassArgs {
   int32_t dst_store;
   WorkList wl_tiles, wl_pairs, wl_octs, wl_sets;  // class_mode: the items of this class (see WorkList)
   TableBounds tb;
-  int32_t set_waves;  // with set_steps: 8 (k_shrink_oct) or 4 (k_shrink_quad), for the launcher
+  int32_t set_waves;  // with set_steps, where k_shrink_dl does not run: 8 (k_shrink_oct) or 4 (k_shrink_quad), for the launcher
+  int32_t set_narrow;  // blocks of four waves wanted: k_shrink_quad instead of k_shrink_dl
 };
 
 // Optional side job of a weight-gradient launch (bf16 MFMA path): the first `y_blocks` rows of the

@@ -55,6 +55,38 @@ __device__ inline void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Wait until at most YOUNGER of the wave's loads are in flight (they complete in order) and its LDS reads are done,
+// then the block barrier.  Written out: the fences of __syncthreads() make the compiler wait for every load in
+// flight, the look-ahead ones included.
+template <int YOUNGER>
+__device__ __forceinline__ void loads_landed_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0070 | YOUNGER);  // vmcnt(YOUNGER), at most 15, lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void load16_to_lds(const bf16_t* base, uint32_t byte_offset, bf16_t* window) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)(reinterpret_cast<const char*>(base) + byte_offset),
+      (__attribute__((address_space(3))) void*)window, 16, 0, 0);
+}
+
+// The same with a buffer descriptor: per-lane offset in a 32-bit register, the step's offset in a scalar one, nothing past
+// `bytes`.
+typedef __amdgpu_buffer_rsrc_t Buffer;
+__device__ __forceinline__ Buffer buffer_of(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)min(bytes, (int64_t)0xffffffff), 0x00020000);
+}
+__device__ __forceinline__ void buffer16_to_lds(Buffer b, uint32_t lane_offset, uint32_t offset, bf16_t* window) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void*)window, 16, (int)lane_offset,
+                                           (int)offset, 0, 0);
+}
+
+// what a load straight into LDS fetches in the place of something that is not there
+__device__ __attribute__((aligned(16))) uint32_t kernel_zeros[4];
+
 // keep the first `keep` (0..8) bf16 elements of a quad, zero the rest
 __device__ inline uint4 keep_first(uint4 v, int keep) {
   if (keep >= 8) return v;
