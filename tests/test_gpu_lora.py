@@ -101,6 +101,20 @@ def test_small_shapes(dev, dtype, t, k, m, n, max_r, ranks):
     _run(dev, dtype, *_problem(t, k, m, n, max_r, ranks, seed=t))
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('k,m,max_r,ranks', [
+    (3, 7, 8, [3, 8]),             # rows shorter than a piece of 16 bytes (bf16)
+    (4, 8, 8, [4, 8]),             # one piece
+    (9, 13, 24, [24, 8]),          # a piece and a bit; every piece but the first is moved back into its row
+    (127, 129, 100, [100, 9]),     # a column either side of a wave's block (bf16); ranks that end inside a piece
+    (63, 65, 12, [12, 5]),         # ... (fp32)
+    (515, 1031, 24, [24, 17]),     # whole blocks of four waves and a cut one behind
+    (1601, 517, 40, [40, 33]),     # several slices of the shrink, the last one cut
+])
+def test_widths_and_ranks_that_end_inside_a_piece(dev, dtype, k, m, max_r, ranks):
+    _run(dev, dtype, *_problem(203, k, m, len(ranks), max_r, ranks, seed=k + m))
+
+
 @pytest.mark.parametrize('t,k,m,n,max_r,ranks', [
     (33, 40, 24, 3, 8, [2, 8, 5]),                 # odd widths: generic kernels
     (257, 128, 256, 4, 16, [16, 8, 16, 1]),

@@ -57,6 +57,23 @@ __device__ inline uint4 ld_piece(const T* p, int keep) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// A piece cut by the end of its row, without a load per element: it is loaded as the last E elements of the row (column
+// min(c, width - E)) and this drops the `drop` = c - that column elements in front, zeros behind.  drop >= E: all zeros.
+// The one wave at the end of a row set the pace of its whole launch while it loaded element by element: bf16, 3001 x 1000
+// and x 1500 at rank 24, shrink 10.7 -> 8.5 us, expand 15.5 -> 10.6, row contraction 20.0 -> 9.3 (means of the two widths).
+// Rows, or in the expand ranks, shorter than a piece have nothing to move back into and keep the loads with a guard each.
+template <typename T>
+__device__ inline uint4 drop_front(const uint4& v, int drop) {
+  constexpr int H = 8 / (int)sizeof(T);  // elements of half a piece
+  uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+  if (drop >= H) { lo = hi; hi = 0; }
+  const int bits = (drop & (H - 1)) * 8 * (int)sizeof(T);
+  lo = (lo >> bits) | ((hi << 1) << (63 - bits));
+  hi >>= bits;
+  if (drop >= 2 * H) lo = hi = 0;
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
 __device__ inline float part_f32(const uint4& v, int i) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
   return __uint_as_float(w[i]);
@@ -159,22 +176,43 @@ __global__ __launch_bounds__(256) void k_shrink_any(PassArgs a, int slice_cols, 
 #pragma unroll
           for (int p = 0; p < 2; ++p) acc[tt][nb] = mma_piece<T>(x[j][tt][p], w[j][nb][p], acc[tt][nb]);
   }
-  for (; c < k1; c += 4 * STEP) {  // the steps left, the last of them perhaps cut by the width
-    const int cc = c + 2 * E * kb;
-    uint4 x[2][2];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) x[tt][p] = ld_piece(xr[tt] + cc + p * E, k1 - cc - p * E);
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+  // The steps left, the last of them perhaps cut by the width (a slice ends at a whole step or there): the two pieces of
+  // a lane are moved back into the row and shifted.
+  auto steps_left = [&](auto cut) {
+    for (; c < k1; c += 4 * STEP) {
+      const int cc = c + 2 * E * kb;
+      uint4 x[2][2], w[NB][2];
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        const uint4 w = ld_piece(wr[nb] + cc + p * E, k1 - cc - p * E);
+        const int col = cut ? min(cc + p * E, a.width_src - E) : cc + p * E, keep = k1 - cc - p * E;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mma_piece<T>(x[tt][p], w, acc[tt][nb]);
+        for (int tt = 0; tt < 2; ++tt) x[tt][p] = cut ? ld_piece(xr[tt] + col) : ld_piece(xr[tt] + col, keep);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) w[nb][p] = cut ? ld_piece(wr[nb] + col) : ld_piece(wr[nb] + col, keep);
       }
-  }
+      if constexpr (cut) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + STEP > k1) {  // (uniform)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const int drop = max(0, cc + p * E - (a.width_src - E));
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) x[tt][p] = drop_front<T>(x[tt][p], drop);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) w[nb][p] = drop_front<T>(w[nb][p], drop);
+          }
+        }
+      }
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mma_piece<T>(x[tt][p], w[nb][p], acc[tt][nb]);
+    }
+  };
+  if (a.width_src >= E) steps_left(std::true_type{});
+  else steps_left(std::false_type{});  // (a row shorter than a piece)
   const float sc = a.scale[g];
 #pragma unroll
   for (int b = 0; b < NB; b += NBS) {
@@ -289,15 +327,19 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
   for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
     for (int q = 0; q < E; ++q) d[tt][q] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // whole: every lane has its E columns and the rank is whole pieces, so that nothing is guarded (rows of padding
-  // slots read row 0, rank indices past the rank read index 0 and are zeroed)
-  auto body = [&](auto whole) {
+  // 2, whole: every lane has its E columns and the rank is whole pieces, so that nothing is guarded (rows of padding
+  // slots read row 0, rank indices past the rank read index 0 and are zeroed).  1, cut: the pieces at the end of the
+  // width or the rank are moved back into their row and shifted, columns past the width read the last one's weights.
+  // 0: a row or a rank shorter than a piece, an element at a time.
+  const int back = c - min(c, a.width_dst - E);
+  auto body = [&](auto form) {
+    constexpr bool whole = form == 2, cut = form == 1;
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const T* row = dst + (int64_t)max(checked_row(rows[tt][v], a.tb), 0) * a.ld_dst;
-        y[tt][v] = a.dst_store ? zero4() : (whole ? ld_piece_nt(row) : ld_piece(row, keep));
+        y[tt][v] = a.dst_store ? zero4() : (whole ? ld_piece_nt(row) : (cut ? ld_piece_nt(row - back) : ld_piece(row, keep)));
       }
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -310,6 +352,8 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
       for (int q = 0; q < E; ++q) {
         if constexpr (whole) {
           w[q] = ld_piece(W + (int64_t)(c + q) * a.ld_expand + (n0 < r ? n0 : 0));
+        } else if constexpr (cut) {
+          w[q] = ld_piece(W + (int64_t)min(c + q, a.width_dst - 1) * a.ld_expand + min(n0, r - E));
         } else {
           w[q] = q < keep ? ld_piece(W + (int64_t)(c + q) * a.ld_expand + n0, r - n0) : zero4();
         }
@@ -318,13 +362,21 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
 #pragma unroll
       for (int q = 0; q < E; ++q) {
         if (whole && n0 >= r) w[q] = zero4();
+        if constexpr (cut) w[q] = drop_front<T>(w[q], max(0, n0 - (r - E)));
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) d[tt][q] = mma_piece<T>(hop[tt], w[q], d[tt][q]);
       }
     }
+    if constexpr (cut) {
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) y[tt][v] = drop_front<T>(y[tt][v], back);
+    }
   };
-  if ((c - E * li) + 16 * E <= a.width_dst && r % E == 0) body(std::true_type{});
-  else body(std::false_type{});
+  if ((c - E * li) + 16 * E <= a.width_dst && r % E == 0) body(std::integral_constant<int, 2>{});
+  else if (a.width_dst >= E && r >= E) body(std::integral_constant<int, 1>{});
+  else body(std::integral_constant<int, 0>{});
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
@@ -420,7 +472,10 @@ __global__ __launch_bounds__(256) void k_wgrad_any(WgradArgs a, const ChunkInfo*
   if (c0 >= a.width) return;  // (no barrier follows)
   const int c = c0 + E * li;
   const int keep = min(E, a.width - c);  // <= 0: none
-  const T* src = (const T*)a.src + c;
+  // lanes past the width's last whole piece load that piece and shift it (drop_front), unless a row is shorter than one
+  const bool wide = a.width >= E;
+  const int drop = wide ? max(0, c - (a.width - E)) : 0;
+  const T* src = (const T*)a.src + (c - drop);
   const T* hT = (const T*)a.hT + (int64_t)(nb0 + li) * a.ldh + (int64_t)ci.tile0 * kTileRows + 8 * kb;
   const bool full = c0 + CW <= a.width;  // every lane has its E columns (uniform over the wave)
   struct Tile {
@@ -432,7 +487,7 @@ __global__ __launch_bounds__(256) void k_wgrad_any(WgradArgs a, const ChunkInfo*
     const int4 rb = *reinterpret_cast<const int4*>(rows_s + t * kTileRows + 8 * kb + 4);
     const int rows[8] = {ra.x, ra.y, ra.z, ra.w, rb.x, rb.y, rb.z, rb.w};
     t_.live = 0;
-    if (full) {
+    if (wide) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) t_.x[i] = ld_piece(src + (int64_t)max(rows[i], 0) * a.ld_src);
     } else {
@@ -455,6 +510,10 @@ __global__ __launch_bounds__(256) void k_wgrad_any(WgradArgs a, const ChunkInfo*
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       if (!((t_.live >> i) & 1u)) t_.x[i] = zero4();
+    if (!full) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t_.x[i] = drop_front<T>(t_.x[i], drop);
+    }
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
