@@ -1,4 +1,5 @@
-"""Builds the gfx950 shared library in-tree with hipcc (no torch C++ ABI involved)."""
+"""Builds the gfx950 shared library in-tree with hipcc (no torch C++ ABI involved) and, next to it, the Python extension
+with the autograd nodes of the plain path (``_host``: g++ on torch's C++ interface)."""
 from __future__ import annotations
 
 import os
