@@ -101,6 +101,16 @@ def test_small_shapes(dev, dtype, t, k, m, n, max_r, ranks):
     _run(dev, dtype, *_problem(t, k, m, n, max_r, ranks, seed=t))
 
 
+@pytest.mark.parametrize('t,k,max_r,ranks', [
+    (97, 18432, 64, [64, 20, 0]),    # more slices than are requested together; a rank that ends inside a block's 32
+    (33, 9216, 32, [17, 32]),        # one block of rank indices a tile, a tile with one row
+    (600, 4096, 128, [128, 65]),     # four of them
+    (520, 2048, 128, [33, 128]),     # rank classes: other launches' tiles are left alone
+])
+def test_sums_of_shrink_slices_above_rank_16(dev, t, k, max_r, ranks):
+    _run(dev, torch.bfloat16, *_problem(t, k, 128, len(ranks), max_r, ranks, seed=k + t))
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize('k,m,max_r,ranks', [
     (3, 7, 8, [3, 8]),             # rows shorter than a piece of 16 bytes (bf16)

@@ -521,7 +521,7 @@ void launch_pass(const PassArgs& a, const SegView& seg, const SegLayout& L, int 
   }
   const bool fin = NB == 1 && (phases & 5) && (phases & 2) && a.dst && !a.class_mode && finish_in_expand(a, L, s);
   if ((phases & 5) && a.kslices > 1 && !fin)
-    hipLaunchKernelGGL((k_shrink_finish<NB>), dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group,
+    hipLaunchKernelGGL((k_shrink_finish<NB>), shrink_finish_grid<NB>(L), dim3(256), 0, s, a, hrow, seg.tile_group,
                        rows);
   if (!a.dst || !(phases & 2)) return;
   if constexpr (NB > 1) {
@@ -677,10 +677,10 @@ int launch_shrink_multi(const PassArgs* a, int n, const SegView& seg, const SegL
     for (int p = 0; p < n; ++p) {
       bf16_t* hrow = (bf16_t*)a[p].hT + (int64_t)a[p].rpad * a[p].ldh;
       if (a[0].rpad <= 32)
-        hipLaunchKernelGGL(k_shrink_finish<2>, dim3((unsigned)L.max_tiles), dim3(256), 0, s, a[p], hrow,
+        hipLaunchKernelGGL(k_shrink_finish<2>, shrink_finish_grid<2>(L), dim3(256), 0, s, a[p], hrow,
                            seg.tile_group, rows);
       else
-        hipLaunchKernelGGL(k_shrink_finish<4>, dim3((unsigned)L.max_tiles), dim3(256), 0, s, a[p], hrow,
+        hipLaunchKernelGGL(k_shrink_finish<4>, shrink_finish_grid<4>(L), dim3(256), 0, s, a[p], hrow,
                            seg.tile_group, rows);
     }
   }

@@ -29,7 +29,7 @@ int launch_pass_rank128(const PassArgs& a, const SegView& seg, const SegLayout& 
     }
   }
   if (((phases & 4) || ((phases & 1) && a.set_steps > 0)) && a.kslices > 1)
-    hipLaunchKernelGGL(k_shrink_finish<8>, dim3((unsigned)L.max_tiles), dim3(256), 0, s, a, hrow, seg.tile_group, rows);
+    hipLaunchKernelGGL(k_shrink_finish<8>, shrink_finish_grid<8>(L), dim3(256), 0, s, a, hrow, seg.tile_group, rows);
   if (a.dst && (phases & 2)) launch_expand_multi<8>(a, hrow, seg, L, s);
   return check_launch();
 }

@@ -581,12 +581,67 @@ __device__ __forceinline__ void shrink_finish_body(const PassArgs& a, bf16_t* __
   shrink_epilogue<RP, 256>(&part[0][0], 1, a, hrow, slot0, cnt, sc);
 }
 
+// The same above rank 16: a block takes 32 of a tile's rank indices (blockIdx.y), a thread four of them of one slot, so that
+// eight 16-byte loads are in flight per thread, there are RP / 32 blocks for a tile and h leaves in 8-byte pieces.
+// Bound by the latency of those loads and their number per CU.  One block per tile with 4-byte loads before, us: rank 128,
+// 8192 rows, 8 slices (33 MB) 11.5 -> 8.4; rank 64, 32768 rows 10.3 -> 9.2, 6000 rows 6.4 -> 5.0.
+template <int NB>
+__device__ __forceinline__ void shrink_finish_wide(const PassArgs& a, bf16_t* __restrict__ hrow,
+                                                   const int32_t* __restrict__ tile_group,
+                                                   const int32_t* __restrict__ slot_rows) {
+  constexpr int RP = 16 * NB;
+  __shared__ __attribute__((aligned(16))) bf16_t turn[32][kTileRows + 4];  // [rank index][slot]
+  const int tile_id = checked_tile(work_item(a.wl_tiles, blockIdx.x), a.tb);
+  if (tile_id < 0) return;
+  const int slot0 = tile_id * kTileRows, n0 = 32 * blockIdx.y, tid = threadIdx.x;
+  const int g = checked_group(tile_group[tile_id], a.tb);
+  if (a.class_mode && (g < 0 || class_rank(a.rank[g], a.rank_lo, RP) <= 0)) return;
+  const int my_row = slot_rows[slot0 + (tid & 31)];
+  const int slot = tid >> 3, n = 4 * (tid & 7);
+  const float* p = a.hpart + (int64_t)tile_id * a.kslices * (kTileRows * RP) + slot * RP + n0 + n;
+  float sum[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < a.kslices; k0 += 8) {
+    float4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      v[k] = k0 + k < a.kslices ? *reinterpret_cast<const float4*>(p + (int64_t)(k0 + k) * (kTileRows * RP))
+                                : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      sum[0] += v[k].x;
+      sum[1] += v[k].y;
+      sum[2] += v[k].z;
+      sum[3] += v[k].w;
+    }
+  }
+  const int gg = max(g, 0);
+  const int rk = class_rank(a.rank[gg], a.rank_lo, RP);
+  const float sc = a.scale[gg];
+  if (g < 0 || rk <= 0) return;  // (uniform over the block, like the returns above)
+  const int cnt = __popcll(__ballot(my_row >= 0) & 0xffffffffull);  // padding is at the end of a tile
+  uint2 o = make_uint2(0u, 0u);
+  if (slot < cnt) o = make_uint2(pack_bf16(sum[0] * sc, sum[1] * sc), pack_bf16(sum[2] * sc, sum[3] * sc));
+  *reinterpret_cast<uint2*>(hrow + (int64_t)(slot0 + slot) * RP + n0 + n) = o;
+  turn[n][slot] = (bf16_t)(o.x & 0xffffu);
+  turn[n + 1][slot] = (bf16_t)(o.x >> 16);
+  turn[n + 2][slot] = (bf16_t)(o.y & 0xffffu);
+  turn[n + 3][slot] = (bf16_t)(o.y >> 16);
+  __syncthreads();
+  const int rn = tid >> 3, s4 = 4 * (tid & 7);
+  *reinterpret_cast<uint2*>((bf16_t*)a.hT + (int64_t)(n0 + rn) * a.ldh + slot0 + s4) =
+      *reinterpret_cast<const uint2*>(&turn[rn][s4]);
+}
+
 template <int NB>
 __global__ __launch_bounds__(256) void k_shrink_finish(PassArgs a, bf16_t* __restrict__ hrow,
                                                        const int32_t* __restrict__ tile_group,
                                                        const int32_t* __restrict__ slot_rows) {
-  shrink_finish_body<NB>(a, hrow, tile_group, slot_rows, blockIdx.x);
+  if constexpr (NB == 1) shrink_finish_body<NB>(a, hrow, tile_group, slot_rows, blockIdx.x);
+  else shrink_finish_wide<NB>(a, hrow, tile_group, slot_rows);
 }
+
+template <int NB>
+inline dim3 shrink_finish_grid(const SegLayout& L) { return dim3((unsigned)L.max_tiles, (unsigned)std::max(NB / 2, 1)); }
 
 // ---------------------------------------------------------------------------
 // Expand: dst[row(slot)][c] += sum_n h[slot][n] * W2_g[c][n], read-modify-write
