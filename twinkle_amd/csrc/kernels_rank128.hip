@@ -2,7 +2,7 @@
 //
 // What bounds these kernels is the memory system, as at the lower ranks; the rank costs registers (accumulators and the
 // weight block of the expand) and L2 reads of weights.  8192 rows x 4096 columns, four adapters, us, against the kernels
-// for any shape (kernels_generic.hip): shrink 64 + 14 -> 30 + 11 (the slices hold half as many bytes as the source),
+// for any shape (kernels_generic.hip): shrink 64 + 14 -> 29 + 8 (the slices hold half as many bytes as the source),
 // expand 84 -> 49 (2.7 TB/s of y; 31 where it only writes), row contraction 94 -> 35 (chunks in pairs and one reader per
 // tile), its reduction 36 -> 22.
 #include <algorithm>
