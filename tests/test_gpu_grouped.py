@@ -244,6 +244,57 @@ def test_lora_step_of_the_direct_kernel(dev, max_r, ranks, sizes, offset):
     assert max_rel_err(got[~own], want[~own]) < 1e-2
 
 
+@pytest.mark.parametrize('n,ptiles', [(128, 4), (256, 8)])   # tiles of a row block: by the width of the kernel's block
+@pytest.mark.parametrize('e,nt,most', [(1, 1, 40), (3, 5, 90), (40, 6, 70)])   # one entry; a few; several blocks of entries
+def test_plan_entries(dev, e, nt, most, n, ptiles):
+    """The row blocks as the GEMM reads them from its workspace: rows of every tile, the groups with a LoRA term numbered in
+    the order of their tiles, their ranks and the addresses of their matrices, all of them in every entry."""
+    g = torch.Generator().manual_seed(e)
+    counts = torch.randint(0, most + 1, (e * nt,), generator=g)
+    counts[0] = most
+    keys = torch.repeat_interleave(torch.arange(e * nt, dtype=torch.int32), counts).to(dev)
+    seg = build_segments(keys, e * nt)
+    k, max_r = 64, 16
+    ranks = [(16, 0, 5, 9, 16, 1)[i % nt] for i in range(e * nt)]
+    a = torch.zeros(e * nt, max_r, k, dtype=torch.bfloat16, device=dev)
+    b = torch.zeros(e * nt, n, max_r, dtype=torch.bfloat16, device=dev)
+    groups = AdapterGroups(list(a), list(b), ranks, [1.0] * (e * nt), rank_classes=False)
+    t = seg.rows
+    x = torch.zeros(t, k, dtype=torch.bfloat16, device=dev)
+    w = torch.zeros(e, n, k, dtype=torch.bfloat16, device=dev)
+    h = torch.zeros(lora_h_bytes(seg, groups), dtype=torch.uint8, device=dev)
+    lora_shrink_(x, seg, groups, h, map_rows=False)
+    size = 224
+    ws = torch.full((256 + 256 + size * ((t + 31) // 32 + e * nt + 1 + e),), 0x5a, dtype=torch.uint8, device=dev)
+    grouped_linear_(x, w, seg, nt, groups=groups, h=h, map_rows=False, workspace=ws)
+    raw = ws.cpu()
+    entries = int(raw[:4].view(torch.int32))
+    want, tile, pos = [], 0, 0
+    for ei in range(e):
+        tiles = []                                    # of the expert: (group, first position, rows)
+        for gi in range(ei * nt, ei * nt + nt):
+            left = int(counts[gi])
+            while left > 0:
+                tiles.append((gi, pos, min(left, 32)))
+                pos, left = pos + min(left, 32), left - 32
+        blocks = -(-len(tiles) // ptiles)
+        per = -(-len(tiles) // blocks) if blocks else 1
+        for i in range(0, len(tiles), per):
+            want.append((tile + i, ei, tiles[i:i + per]))
+        tile += len(tiles)
+    assert entries == len(want)
+    for i, (tile0, expert, tiles) in enumerate(want):
+        one = raw[256 + size * i:256 + size * (i + 1)]
+        ints, matrices = one[:160].view(torch.int32).tolist(), one[160:].view(torch.int64).tolist()
+        pos, cnt, number, rank = (ints[8 + 8 * j:16 + 8 * j] for j in range(4))
+        live = list(dict.fromkeys(gi for gi, _, _ in tiles if ranks[gi] > 0))
+        assert ints[:3] == [tile0, len(tiles), expert] and ints[5] == len(live)
+        assert [(p, c) for p, c in zip(pos, cnt)][:len(tiles)] == [(p, c) for _, p, c in tiles]
+        assert number[:len(tiles)] == [live.index(gi) if gi in live else -1 for gi, _, _ in tiles]
+        assert rank[:len(live)] == [ranks[gi] for gi in live]
+        assert matrices[:len(live)] == [b[gi].data_ptr() for gi in live]
+
+
 def test_unsupported_shapes_are_refused(dev):
     e, nt, t = 2, 1, 64
     keys = torch.zeros(t, dtype=torch.int32, device=dev)

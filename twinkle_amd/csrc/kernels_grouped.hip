@@ -101,10 +101,10 @@ __global__ __launch_bounds__(256) void k_grouped_plan(GroupedArgs a, SegView V, 
   // thread = (entry, tile of the entry): group, first position and live rows of the tile; the distinct groups of a block
   // that carry a LoRA term are numbered in the order of its tiles (the eight threads of an entry are neighbours in a wave)
   const int i = tid >> 3, t = tid & 7;
-  if (base + i >= total) return;
+  const bool entry = base + i < total;
   GroupedPlanEntry& m = mine[i];
-  const bool have = t < m.ntiles;
-  const int tile = m.tile0 + t;  // (tile0 + ntiles <= max_tiles)
+  const bool have = entry && t < m.ntiles;
+  const int tile = have ? m.tile0 + t : 0;  // (tile0 + ntiles <= max_tiles)
   const int g = have ? checked_group(V.tile_group[tile], a.tb) : -1;
   const int row0 = have ? V.slot_pos[(int64_t)tile * kTileRows] : 0;
   const int end = g >= 0 ? V.offsets[g + 1] : 0;
@@ -114,20 +114,29 @@ __global__ __launch_bounds__(256) void k_grouped_plan(GroupedArgs a, SegView V, 
   const bool opens = lora && (t == 0 || before != g);
   const unsigned mask = (unsigned)(__ballot(opens) >> (threadIdx.x & 56)) & 0xffu;
   const int number = __popc(mask & ((2u << t) - 1u)) - 1;
-  m.pos[t] = pos;
-  m.cnt[t] = row0 >= 0 ? min(max(min(end, a.tb.rows) - pos, 0), kTileRows) : 0;
-  m.number[t] = lora ? number : -1;
-  if (opens) {
-    m.rank[number] = min(a.rank[g], a.rpad);
-    m.matrix[number] = (const bf16_t*)a.lora_B[g];
+  if (entry) {
+    m.pos[t] = pos;
+    m.cnt[t] = row0 >= 0 ? min(max(min(end, a.tb.rows) - pos, 0), kTileRows) : 0;
+    m.number[t] = lora ? number : -1;
+    if (opens) {
+      m.rank[number] = min(a.rank[g], a.rpad);
+      m.matrix[number] = (const bf16_t*)a.lora_B[g];
+    }
+    if (t == 0) m.ngroups = __popc(mask);
   }
-  if (t == 0) m.ngroups = __popc(mask);
-  __builtin_amdgcn_wave_barrier();
-  // (an entry's eight threads wrote it and now move it out together)
+  // An entry's eight threads wrote it and now move it out together: a block barrier, which orders the LDS accesses of
+  // different threads (a wave barrier does not), and words copied as bytes (the entry holds pointers, and a load of another
+  // type may move ahead of their stores).
+  __syncthreads();
+  if (!entry) return;
   constexpr int kWords = sizeof(GroupedPlanEntry) / 4;
-  const int32_t* from = reinterpret_cast<const int32_t*>(&m);
-  int32_t* to = reinterpret_cast<int32_t*>(&plan[base + i]);
-  for (int w = t; w < kWords; w += 8) to[w] = from[w];
+  const char* from = reinterpret_cast<const char*>(&m);
+  char* to = reinterpret_cast<char*>(&plan[base + i]);
+  for (int w = t; w < kWords; w += 8) {
+    int32_t word;
+    __builtin_memcpy(&word, from + 4 * w, 4);
+    __builtin_memcpy(to + 4 * w, &word, 4);
+  }
 }
 
 // NKS: MFMA steps of the LoRA term (0: none; 1: padded rank 16 or 32; 2: padded rank 64)
