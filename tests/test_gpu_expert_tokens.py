@@ -3,8 +3,10 @@ against the same block put together from permute, experts and unpermute, and aga
 import pytest
 import torch
 
-from twinkle_amd import LoraConfig, build_segments, flat_keys_from_topk, permute, unpermute
+from twinkle_amd import AdapterGroups, LoraConfig, build_segments, flat_keys_from_topk, permute, unpermute
 from twinkle_amd.expert_lora import ExpertLoraSlots, experts_forward, moe_experts_block
+from twinkle_amd.ops import grouped_experts_linear
+from twinkle_amd.segments import build_token_segments
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +118,44 @@ def test_strided_tokens_and_frozen_adapters(dev):
     off = torch.randn(200, 257, device=dev).bfloat16()
     off[:, 1:] = x.detach()
     assert torch.equal(moe_experts_block(off[:, 1:], sel, w, tenant, mod, names, *slots), base)
+
+
+def test_weights_tables_and_adapters_that_do_not_fit_are_refused(dev):
+    """Before anything is launched: with fewer experts than the table names the kernels would read past the weights."""
+    e, nt, t, k, n = 4, 2, 60, 128, 256
+    bf16 = torch.bfloat16
+    sel = torch.randint(0, e, (t, 2), generator=torch.Generator().manual_seed(0)).to(dev)
+    tenant = torch.zeros(t, dtype=torch.int32, device=dev)
+    keys = flat_keys_from_topk(sel, tenant, nt)
+    seg = build_token_segments(keys, e * nt, t)
+    x, w = torch.zeros(t, k, dtype=bf16, device=dev), torch.zeros(e, n, k, dtype=bf16, device=dev)
+
+    def adapters(kk=k, nn=n, g=e * nt, dtype=bf16):
+        return AdapterGroups([torch.zeros(8, kk, dtype=dtype, device=dev)], [torch.zeros(nn, 8, dtype=dtype, device=dev)], [8] * g,
+                             [1.0] * g, a_index=[0] * g, b_index=[0] * g)
+
+    assert grouped_experts_linear(x, w, seg, nt, adapters(), tokens=True).shape == (2 * t, n)
+    for args in ((x, w[:2], seg, nt), (x, w, seg, 1), (x, w.transpose(1, 2), seg, nt), (x, w.float(), seg, nt), (x, w[0], seg, nt),
+                 (x, w, build_segments(keys, e * nt, num_tokens=t), nt), (x[:-1], w, seg, nt),
+                 (x, w, seg, nt, adapters(dtype=torch.float32)), (x, w, seg, nt, adapters(kk=256)),
+                 (x, w, seg, nt, adapters(nn=128)), (x, w, seg, nt, adapters(g=e))):
+        with pytest.raises(ValueError):
+            grouped_experts_linear(*args, tokens=True)
+    for args in ((x, w.cpu(), seg, nt), (x.cpu(), w, seg, nt)):
+        with pytest.raises(RuntimeError):
+            grouped_experts_linear(*args, tokens=True)
+    # slots of another type than the experts, through the block itself
+    mod = _Experts(torch.zeros(e, 2 * k, k, dtype=bf16, device=dev), torch.zeros(e, k, k, dtype=bf16, device=dev))
+    slots = [ExpertLoraSlots(e, k, out, max_loras=1, max_r=8, dtype=torch.float32, device=dev) for out in (2 * k, k)]
+    for s in slots:
+        s.configure_slot('lora_0', LoraConfig(r=8, lora_alpha=8))
+    with pytest.raises(ValueError):
+        moe_experts_block(x, sel, torch.ones(t, 2, dtype=bf16, device=dev), None, mod, ['lora_0'], *slots)
+    wide = torch.zeros(2 * t, 3, dtype=torch.int32, device=dev)
+    wide[:, 1] = keys
+    assert torch.equal(build_token_segments(wide[:, 1], e * nt, t).workspace[:32], seg.workspace[:32])
+    for bad in ((keys.float(), e * nt, t), (keys, 0, t), (keys, e * nt, 0), (keys, e * nt, t - 1), (keys[:0], e * nt, t)):
+        with pytest.raises(ValueError):
+            build_token_segments(*bad)
+    with pytest.raises(RuntimeError):
+        build_token_segments(keys.cpu(), e * nt, t)

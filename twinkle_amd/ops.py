@@ -394,17 +394,11 @@ def grouped_linear_(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTable, gr
     (expert, tenant) groups is added on the accumulators, from ``h`` as :func:`lora_shrink_` left it.
     ``transposed=True`` computes ``y[row] = x[row] @ weight[e]`` instead (``weight [E, in, out]``): the backward of
     the plain call on the same weights."""
-    if not (x.is_cuda and weight.is_cuda):
-        raise RuntimeError('x and weight must live on the GPU: this path has no CPU implementation')
-    if weight.dim() != 3 or weight.stride(2) != 1 or weight.dtype != x.dtype:
-        raise ValueError('weight must be [experts, out, in] with unit inner stride and the dtype of x')
     if transposed and groups is not None:
         raise ValueError('the LoRA term goes with the plain call, not with transposed=True')
-    experts, out_f, in_f = weight.shape
+    out_f, in_f = _grouped_widths(x, weight, seg, groups_per_expert, groups)
     if transposed:
         out_f, in_f = in_f, out_f
-    if seg.num_groups != experts * groups_per_expert:
-        raise ValueError(f'segment table has {seg.num_groups} groups, weights give {experts} x {groups_per_expert}')
     _check_rows(x, 'x', seg.rows, in_f, weight.dtype)
     if y is None:
         y = torch.empty(seg.rows, out_f, dtype=x.dtype, device=x.device)
@@ -417,14 +411,28 @@ def grouped_linear_(x: torch.Tensor, weight: torch.Tensor, seg: SegmentTable, gr
     if groups is not None:
         if h is None:
             raise ValueError('the LoRA term needs the h that lora_shrink_ wrote')
-        if groups.num_groups != seg.num_groups or groups.in_features != in_f or groups.out_features != out_f:
-            raise ValueError('adapters and weights describe different layers')
         d = ctypes.byref(_desc(seg, groups, map_rows))
     code = lib.tk_grouped_linear(ctypes.byref(g), d, x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0),
                                  h.data_ptr() if h is not None else None, workspace.data_ptr(), workspace.numel(),
                                  _lib.stream_ptr())
     _lib.check(code, 'tk_grouped_linear')
     return y
+
+
+def _grouped_widths(x, weight, seg, groups_per_expert, groups):
+    """``(out, in)`` of packed weights that fit the input, the table and the adapters: the kernels derive the number of
+    experts from the table and take the adapters' type for that of the input."""
+    if not (x.is_cuda and weight.is_cuda):
+        raise RuntimeError('x and weight must live on the GPU: this path has no CPU implementation')
+    if weight.dim() != 3 or weight.stride(2) != 1 or weight.dtype != x.dtype:
+        raise ValueError('weight must be [experts, out, in] with unit inner stride and the dtype of x')
+    experts, out_f, in_f = weight.shape
+    if seg.num_groups != experts * groups_per_expert:
+        raise ValueError(f'segment table has {seg.num_groups} groups, weights give {experts} x {groups_per_expert}')
+    if groups is not None and (groups.num_groups != seg.num_groups or groups.in_features != in_f or
+                               groups.out_features != out_f or groups.dtype != weight.dtype):
+        raise ValueError('adapters and weights describe different layers')
+    return out_f, in_f
 
 
 def _grouped_desc(seg, groups_per_expert, weight, in_f, out_f, map_rows, transposed) -> _lib.GroupedDesc:
@@ -447,12 +455,12 @@ def _grouped_workspace(g: _lib.GroupedDesc, device) -> torch.Tensor:
 
 def _grouped_from_tokens(tokens, weight, seg, groups_per_expert, groups):
     """``(y, h)`` of the grouped linear on the tokens a :func:`build_token_segments` table's rows stand for."""
-    experts, out_f, in_f = weight.shape
+    if not seg.of_tokens:
+        raise ValueError('the tokens go with a table of tokens (build_token_segments)')
+    out_f, in_f = _grouped_widths(tokens, weight, seg, groups_per_expert, groups)
     _check_rows(tokens, 'tokens', seg.num_tokens, in_f, weight.dtype)
     lib, h, d = _lib.load(), None, None
     if groups is not None:
-        if groups.num_groups != seg.num_groups or groups.in_features != in_f or groups.out_features != out_f:
-            raise ValueError('adapters and weights describe different layers')
         d = ctypes.byref(_desc(seg, groups, False))
         h = torch.empty(lora_h_bytes(seg, groups), dtype=torch.uint8, device=tokens.device)
         _lib.check(lib.tk_lora_shrink_tokens(d, tokens.data_ptr(), tokens.stride(0), seg.num_tokens, h.data_ptr(),

@@ -77,6 +77,16 @@ def validate_segment_table(seg: SegmentTable) -> None:
     seg.validate()
 
 
+def _checked_keys(keys: torch.Tensor, num_groups: int, name: str) -> torch.Tensor:
+    if not keys.is_cuda:
+        raise RuntimeError(f'{name} needs keys on the GPU: this path has no CPU implementation')
+    if keys.dtype not in (torch.int32, torch.int64):
+        raise ValueError(f'keys must be int32 or int64, got {keys.dtype}')
+    if num_groups <= 0:
+        raise ValueError('num_groups must be positive')
+    return keys.reshape(-1).contiguous()
+
+
 def build_segments(keys: torch.Tensor, num_groups: int, num_tokens: Optional[int] = None, want_perm: bool = True,
                    want_offsets: bool = True, check: bool = False) -> SegmentTable:
     """Group flat rows by ``keys`` (int32 or int64, on the GPU), stably.
@@ -84,13 +94,7 @@ def build_segments(keys: torch.Tensor, num_groups: int, num_tokens: Optional[int
     ``check=True`` raises ``ValueError`` for keys outside ``[0, num_groups)``
     (costs a device synchronisation; an index error in the reference).
     """
-    if not keys.is_cuda:
-        raise RuntimeError('build_segments needs keys on the GPU: this path has no CPU implementation')
-    if keys.dtype not in (torch.int32, torch.int64):
-        raise ValueError(f'keys must be int32 or int64, got {keys.dtype}')
-    if num_groups <= 0:
-        raise ValueError('num_groups must be positive')
-    keys = keys.reshape(-1).contiguous()
+    keys = _checked_keys(keys, num_groups, 'build_segments')
     rows = keys.numel()
     num_tokens = rows if num_tokens is None else num_tokens
     if num_tokens and rows % num_tokens:
@@ -122,7 +126,10 @@ def build_token_segments(keys: torch.Tensor, num_groups: int, num_tokens: int) -
     """The table of top-k routed rows for kernels that read the tokens themselves (``tk_segment_build_tokens``): for
     :func:`twinkle_amd.ops.grouped_experts_linear` with ``tokens`` and :func:`unpermute`, nothing else.  ``keys`` as
     :func:`flat_keys_from_topk` makes them."""
+    keys = _checked_keys(keys, num_groups, 'build_token_segments')
     lib, rows = _lib.load(), keys.numel()
+    if num_tokens <= 0 or rows == 0 or rows % num_tokens:
+        raise ValueError(f'rows ({rows}) must be a positive multiple of num_tokens ({num_tokens})')
     nbytes = lib.tk_segment_workspace_bytes(rows, num_groups)
     _lib.check(nbytes, 'tk_segment_workspace_bytes')
     ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
