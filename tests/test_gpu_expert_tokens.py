@@ -3,7 +3,7 @@ against the same block put together from permute, experts and unpermute, and aga
 import pytest
 import torch
 
-from twinkle_amd import AdapterGroups, LoraConfig, build_segments, flat_keys_from_topk, permute, unpermute
+from twinkle_amd import AdapterGroups, LoraConfig, build_segments, flat_keys_from_topk, ops, permute, unpermute
 from twinkle_amd.expert_lora import ExpertLoraSlots, experts_forward, moe_experts_block
 from twinkle_amd.ops import grouped_experts_linear
 from twinkle_amd.segments import build_token_segments
@@ -159,3 +159,27 @@ def test_weights_tables_and_adapters_that_do_not_fit_are_refused(dev):
             build_token_segments(*bad)
     with pytest.raises(RuntimeError):
         build_token_segments(keys.cpu(), e * nt, t)
+
+
+def test_a_table_of_tokens_maps_no_rows(dev):
+    """Its slots hold tokens: whatever updates rows through them is refused, rows in segment order are as with any table."""
+    e, t, k, n = 4, 70, 128, 256
+    g = torch.Generator().manual_seed(1)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dev, torch.bfloat16)  # noqa: E731
+    keys = flat_keys_from_topk(torch.randint(0, e, (t, 2), generator=g).to(dev))
+    seg, rows = build_token_segments(keys, e, t), build_segments(keys, e, num_tokens=t)
+    groups = AdapterGroups([rand(8, k) for _ in range(e)], [rand(n, 8) for _ in range(e)], [8] * e, [1.0] * e)
+    x, y, w = rand(2 * t, k), rand(2 * t, n), rand(n, k)
+    for w_ in groups.a_tensors:
+        w_.requires_grad_(True)
+    h = torch.empty(ops.lora_h_bytes(seg, groups), dtype=torch.uint8, device=dev)
+    for call in (lambda: ops.multi_lora_delta(x, y.clone(), seg, groups), lambda: ops.multi_lora_linear(x, w, None, seg, groups),
+                 lambda: ops.multi_lora_delta_shared(x, [y.clone()], seg, [groups]),
+                 lambda: ops.multi_lora_linear_shared(x, [w, w], [None, None], seg, [groups, groups]),
+                 lambda: ops.lora_fwd_(x, y.clone(), seg, groups), lambda: ops.lora_shrink_(x, seg, groups, h),
+                 lambda: ops.grouped_linear_(x, w.expand(e, n, k).contiguous(), seg, 1, map_rows=True), lambda: permute(x[:t], seg)):
+        with pytest.raises(ValueError):
+            call()
+    got, want = (ops.multi_lora_delta(x, y.clone(), s, groups, map_rows=False) for s in (seg, rows))
+    assert torch.equal(got, want)
+    assert torch.equal(torch.autograd.grad(got, groups.a_tensors[0], y)[0], torch.autograd.grad(want, groups.a_tensors[0], y)[0])

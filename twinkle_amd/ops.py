@@ -221,6 +221,16 @@ class AdapterGroups:
                 torch._foreach_copy_(self.a_tensors + self.b_tensors, self.master_a + self.master_b)
 
 
+def _row_map(seg: SegmentTable, map_rows: bool) -> int:
+    """1 where rows are reached through the table.  A table of tokens has no such map: its slots hold tokens, of which several
+    rows are made, and every kernel that updates rows through it would update the wrong ones."""
+    if not map_rows:
+        return 0
+    if seg.of_tokens:
+        raise ValueError('a table of tokens does not say which row a slot holds: map_rows=False')
+    return 1
+
+
 def _desc(seg: SegmentTable, groups: AdapterGroups, map_rows: bool) -> _lib.LoraDesc:
     groups.refresh()
     # a fresh struct per call (callers keep several alive at once), copied from a template that holds everything
@@ -244,7 +254,7 @@ def _desc(seg: SegmentTable, groups: AdapterGroups, map_rows: bool) -> _lib.Lora
         groups._desc_template, groups._desc_key = template, groups._ptr_key
     d = _lib.LoraDesc.from_buffer_copy(template)
     d.rows = seg.rows
-    d.map_rows = 1 if map_rows else 0
+    d.map_rows = _row_map(seg, map_rows)
     d.seg_ws = seg.workspace.data_ptr()
     return d
 
@@ -265,7 +275,7 @@ def _cached_size(seg: SegmentTable, groups: AdapterGroups, which: str) -> int:
     key = (which, seg.rows)
     n = groups._size_cache.get(key)
     if n is None:
-        n = getattr(_lib.load(), which)(ctypes.byref(_desc(seg, groups, True)))
+        n = getattr(_lib.load(), which)(ctypes.byref(_desc(seg, groups, False)))
         _lib.check(n, which)
         if len(groups._size_cache) > 64:
             groups._size_cache.clear()
@@ -290,7 +300,7 @@ def lora_h_saved_bytes(seg: SegmentTable, groups: AdapterGroups) -> int:
     key = ('h_saved', seg.rows)
     n = groups._size_cache.get(key)
     if n is None:
-        d = _desc(seg, groups, True)
+        d = _desc(seg, groups, False)
         d.weights_f32 = 0
         n = _lib.load().tk_lora_h_bytes(ctypes.byref(d))
         _lib.check(n, 'tk_lora_h_bytes')
@@ -440,7 +450,7 @@ def _grouped_desc(seg, groups_per_expert, weight, in_f, out_f, map_rows, transpo
     g.rows, g.num_groups, g.groups_per_expert = seg.rows, seg.num_groups, groups_per_expert
     g.in_features, g.out_features = in_f, out_f
     g.dtype = _lib.dtype_code(weight.dtype)
-    g.map_rows = 1 if map_rows else 0
+    g.map_rows = _row_map(seg, map_rows)
     g.seg_ws = seg.workspace.data_ptr()
     g.weight, g.weight_stride, g.ldw = weight.data_ptr(), weight.stride(0), weight.stride(1)
     g.weight_layout = 1 if transposed else 0
@@ -675,7 +685,7 @@ def multi_lora_delta(x: torch.Tensor, base_out: torch.Tensor, seg: SegmentTable,
     host = _lib.host()
     handle = groups.host_groups() if host is not None else None
     if handle is not None:
-        out = host.delta(x, base_out, seg.workspace, seg.rows, seg.num_groups, handle, bool(map_rows))
+        out = host.delta(x, base_out, seg.workspace, seg.rows, seg.num_groups, handle, bool(_row_map(seg, map_rows)))
         if out is not None:
             return out
     return _LoraDelta.apply(x, base_out, seg, groups, map_rows, *groups.autograd_tensors())
@@ -686,7 +696,7 @@ def _host_linear(x, weights, biases, seg, groups_list, map_rows):
     handles = [g.host_groups() for g in groups_list] if host is not None else [None]
     if None in handles:
         return None
-    return host.linear(x, weights, biases, seg.workspace, seg.rows, seg.num_groups, handles, bool(map_rows))
+    return host.linear(x, weights, biases, seg.workspace, seg.rows, seg.num_groups, handles, bool(_row_map(seg, map_rows)))
 
 
 def multi_lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], seg: SegmentTable,
