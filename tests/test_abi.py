@@ -161,6 +161,29 @@ def test_entry_points_reject_malformed_arguments_on_the_host():
     g.weight_layout = 0
     g.rows, g.weight_stride = 0, 256 * 128
     assert lib.tk_grouped_linear(gref, None, None, 128, None, 256, None, None, 0, None) == _lib.TK_OK  # nothing to do
+    # packed experts on tokens, and their backward in one call (out and in of the transposing product swapped)
+    d.rows, d.in_features, d.out_features, d.num_groups, d.dtype, d.lda, d.map_rows = 64, 256, 128, 4, 1, 256, 0
+    g.rows, g.weight_layout, g.ldw = 64, 1, 256
+
+    def experts_bwd(tokens=0, dx=P, at_a=P, base_a=P):
+        return lib.tk_grouped_linear_bwd(gref, ref, P, 128, P, 256, tokens, P, dx, 256, at_a, base_a, P, P, P, need, P, 16, None)
+
+    for dx in (P, None):
+        for per_expert in (0, -1, 3):                                                         # 4 groups
+            g.groups_per_expert = per_expert
+            assert experts_bwd(dx=dx) == bad
+    g.groups_per_expert = 2
+    assert experts_bwd() == small and experts_bwd(dx=None) == small                           # the LoRA workspace of 16 bytes
+    assert experts_bwd(tokens=-1) == bad and experts_bwd(tokens=65) == bad
+    assert experts_bwd(base_a=None) == bad
+    g.weight_layout = 0
+    assert experts_bwd() == bad
+    assert lib.tk_grouped_linear_tokens(gref, None, P, 128, 0, P, 256, None, P, need, None) == bad    # no tokens
+    assert lib.tk_lora_shrink_tokens(ref, P, 256, 65, P, None) == bad                         # more tokens than rows
+    assert lib.tk_segment_build_tokens(P, 0, 64, 4, 63, P, 1 << 20, None) == bad              # rows not k * tokens
+    assert lib.tk_topk_keys(P, 0, 2, 1, None, 0, P, 1 << 62, 4, 1, None) == bad               # rows past 64 bits
+    assert lib.tk_topk_keys(P, 5, 2, 1, None, 0, P, 32, 2, 1, None) == bad                    # unknown key type
+    assert lib.tk_unpermute_bwd(P, 64, P, 64, P, 64, None, P, 0, P, 64, 64, 64, 4, 1, None) == bad    # dw without weights
     # gated activation
     assert lib.tk_swiglu_fwd(P, 32, P, 16, -1, 16, 1, None) == bad                            # negative rows
     assert lib.tk_swiglu_fwd(P, 31, P, 16, 4, 16, 1, None) == bad                             # ld below 2 * inter

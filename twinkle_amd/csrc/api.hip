@@ -457,7 +457,8 @@ int tk_topk_keys(const void* selected, int32_t sel_dtype, int64_t stride_t, int6
                  int32_t tenant_dtype, int32_t* keys, int64_t num_tokens, int32_t top_k, int32_t num_tenants,
                  tk_stream_t stream) {
   auto type_ok = [](int32_t t) { return t == TK_KEY_I32 || t == TK_KEY_I64; };
-  if (num_tokens < 0 || top_k < 0 || num_tokens * top_k >= (1ll << 31) || !type_ok(sel_dtype) || (tenant && !type_ok(tenant_dtype)))
+  if (num_tokens < 0 || top_k < 0 || num_tokens >= (1ll << 31) || num_tokens * top_k >= (1ll << 31) || !type_ok(sel_dtype) ||
+      (tenant && !type_ok(tenant_dtype)))
     return TK_ERR_INVALID;
   if (num_tokens * top_k > 0 && (!selected || !keys)) return TK_ERR_INVALID;
   return launch_topk_keys(selected, sel_dtype, stride_t, stride_k, tenant, tenant_dtype, keys, num_tokens, top_k, num_tenants,
@@ -985,7 +986,7 @@ int tk_grouped_linear_bwd(const tk_grouped_desc* g, const tk_lora_desc* lora, co
                           int64_t ldx, int64_t num_tokens, const void* h, void* dx, int64_t lddx, const int64_t* at_A,
                           void* base_A, const int64_t* at_B, void* base_B, void* gemm_ws, int64_t gemm_ws_bytes,
                           void* lora_ws, int64_t lora_ws_bytes, tk_stream_t stream) {
-  if (!g || !desc_ok(lora) || g->weight_layout != 1 || g->map_rows || lora->map_rows) return TK_ERR_INVALID;
+  if (!grouped_desc_ok(g) || !desc_ok(lora) || g->weight_layout != 1 || g->map_rows || lora->map_rows) return TK_ERR_INVALID;
   if (lora->rows != g->rows || lora->num_groups != g->num_groups || lora->out_features != g->in_features ||
       lora->in_features != g->out_features || lora->dtype != g->dtype || lora->seg_ws != g->seg_ws)
     return TK_ERR_INVALID;
