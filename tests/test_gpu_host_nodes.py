@@ -159,3 +159,34 @@ def test_threads(dev):
         th.join()
     for r in results:
         _same(r, want)
+
+
+@pytest.mark.parametrize('n', [0, 1, 2])     # delta, linear, shared linear
+def test_master_weights_take_the_python_node(dev, n):
+    """fp32 masters of bf16 compute copies: the gradients are the masters', in their type, and the copies' values but for it."""
+    parts = [_problem(dev, ranks=(16, 16, 5), seed=p) for p in range(max(n, 1))]
+    seg, x, base = parts[0][1], parts[0][2].requires_grad_(True), parts[0][3]
+    dy = torch.randn(base.shape, generator=torch.Generator().manual_seed(5)).to(dev, base.dtype)
+    ws = [(torch.randn(384, 512, generator=torch.Generator().manual_seed(p)) / 20).to(dev, base.dtype) for p in range(n)]
+    masters = [([w.detach().float().requires_grad_(True) for w in a], [w.detach().float().requires_grad_(True) for w in b])
+               for *_, a, b in parts]
+    groups = [AdapterGroups([w.detach() for w in p[4]], [w.detach() for w in p[5]], [16, 16, 5], [2.0] * 3, master_a=m[0],
+                            master_b=m[1]) for p, m in zip(parts, masters)]
+
+    def call(gs):
+        if n == 0:
+            return [multi_lora_delta(x, base.clone(), seg, gs[0])]
+        if n == 1:
+            return [ops.multi_lora_linear(x, ws[0], None, seg, gs[0])]
+        return list(ops.multi_lora_linear_shared(x, ws, [None] * n, seg, gs))
+
+    def run(gs, weights):
+        ys = call(gs)
+        return [*[y.detach() for y in ys], *torch.autograd.grad(ys, [x, *weights], [dy] * len(ys))]
+
+    got = run(groups, [w for m in masters for side in m for w in side])
+    want = run([p[0] for p in parts], [w for p in parts for side in p[4:] for w in side])
+    k = len(want) - sum(len(p[4]) + len(p[5]) for p in parts)
+    _same(got[:k], want[:k])
+    for p, q in zip(got[k:], want[k:]):
+        assert p.dtype == torch.float32 and torch.equal(p, q.float())

@@ -612,3 +612,13 @@ def test_gradient_arena_spans_strided_adapters(pad):
                 arena[at:at + cols] = g + 1
             block = views[g][:r] if side == 'a' else views[g][:, :r]
             assert torch.equal(block, torch.full_like(block, g + 1))
+
+
+def test_master_weights_have_no_handle_of_the_cpp_nodes():
+    from twinkle_amd import AdapterGroups
+    a, b = [torch.zeros(8, 16, dtype=torch.bfloat16)], [torch.zeros(32, 8, dtype=torch.bfloat16)]
+    groups = AdapterGroups(a, b, [8], [1.0], master_a=[t.float() for t in a], master_b=[t.float() for t in b])
+    for _ in range(2):
+        assert groups.host_groups() is None
+    with torch.no_grad():
+        assert groups.host_groups() is None

@@ -116,7 +116,7 @@ class AdapterGroups:
         rel_b = [(self._b_arena_off[j] + o) * esz for j, o in zip(self.b_index, self.b_offset)]
         self._grad_a_rel, self._grad_b_rel = torch.tensor([rel_a, rel_b], dtype=torch.int64, device=dev).unbind(0)
         self._arena_plan = None
-        self._host = None
+        self._host, self._host_plan = None, False
         self._ptr_key = None
         self._size_cache = {}
         self._desc_template = self._desc_key = None
@@ -164,7 +164,9 @@ class AdapterGroups:
 
     def host_groups(self):
         """This object as the C++ nodes know it; ``None`` with master weights, which only the Python nodes serve."""
-        if self._host is None and self.master_a is None:
+        if self.master_a is not None:
+            return None
+        if self._host is None:
             self.refresh()
             sides = (('a', self.a_tensors, self.a_index, self.a_offset, self.a_live, self._a_arena_off, self.a_arena_elems,
                       self._grad_a_rel, self.a_ptrs),
@@ -176,8 +178,7 @@ class AdapterGroups:
                 fields, rank=self.rank_dev, scale=self.scale_dev, in_features=self.in_features,
                 out_features=self.out_features, max_rank=self.max_rank, dtype=_lib.dtype_code(self.dtype), lda=self.lda,
                 ldb=self.ldb, weights_f32=int(self.weights_f32), rank_classes=self.rank_classes))
-            self._host_plan = False
-        if not self._host_plan and self._host is not None and torch.is_grad_enabled():
+        if not self._host_plan and torch.is_grad_enabled():
             self._host.zeros, self._host_plan = self.arena_plan()[0], True
         return self._host
 
