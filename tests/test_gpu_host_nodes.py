@@ -190,3 +190,19 @@ def test_master_weights_take_the_python_node(dev, n):
     _same(got[:k], want[:k])
     for p, q in zip(got[k:], want[k:]):
         assert p.dtype == torch.float32 and torch.equal(p, q.float())
+
+
+def test_calls_the_library_refuses_raise_the_same_errors(dev):
+    """Rows on top of each other pass every check on shapes; the library refuses their stride."""
+    groups, seg, x, base, a, b = _problem(dev)
+    w = torch.zeros(384, 512, dtype=x.dtype, device=dev)
+    flat, out = x[:1].expand(x.shape), base[:1].expand(base.shape)
+    calls = [lambda: multi_lora_delta(flat, base.clone(), seg, groups), lambda: multi_lora_delta(x, out, seg, groups),
+             lambda: ops.multi_lora_linear(flat, w, None, seg, groups),
+             lambda: ops.multi_lora_linear_shared(flat, [w, w], [None, None], seg, [groups, groups]),
+             lambda: ops._LoraDelta.apply(flat, base.clone(), seg, groups, True, *groups.autograd_tensors())]
+    for call in calls:
+        with pytest.raises(ValueError, match='invalid'):
+            call()
+    with torch.no_grad(), pytest.raises(ValueError, match='invalid'):
+        calls[0]()

@@ -26,8 +26,12 @@ using torch::autograd::variable_list;
 
 namespace {
 
+// (the exception types of _lib.check)
 void check(int64_t code, const char* what) {
-  TORCH_CHECK(code >= 0, what, ": ", tk_error_string((int)code), " (", code, ")");
+  if (code >= 0) return;
+  if (code == TK_ERR_INVALID || code == TK_ERR_UNSUPPORTED)
+    TORCH_CHECK_VALUE(false, what, ": ", tk_error_string((int)code), " (", code, ")");
+  TORCH_CHECK(false, what, ": ", tk_error_string((int)code), " (", code, ")");
 }
 tk_stream_t stream() { return (tk_stream_t)c10::hip::getCurrentHIPStream().stream(); }
 
