@@ -206,3 +206,35 @@ def test_calls_the_library_refuses_raise_the_same_errors(dev):
             call()
     with torch.no_grad(), pytest.raises(ValueError, match='invalid'):
         calls[0]()
+
+
+class _Tagged(torch.Tensor):
+    """A subclass of the kind that has a ``__torch_function__`` and no dispatch key."""
+
+
+@pytest.mark.parametrize('which', ['x', 'weight', 'bias', 'adapters', 'base'])
+def test_tensor_subclasses_take_the_python_node(dev, which, monkeypatch):
+    groups, seg, x, base, a, b = _problem(dev, ranks=(16, 16, 5))
+    made = {'x': x, 'base': base, 'weight': (torch.randn(384, 512, generator=torch.Generator().manual_seed(1)) / 20),
+            'bias': torch.zeros(384)}
+    made = {k: v.to(dev, torch.bfloat16) for k, v in made.items()}
+    if which == 'adapters':
+        groups = AdapterGroups([w.detach().as_subclass(_Tagged).requires_grad_(True) for w in a], b, [16, 16, 5], [2.0] * 3)
+    else:
+        made[which] = made[which].as_subclass(_Tagged)
+    x, base, w, bias = made['x'].requires_grad_(True), made['base'], made['weight'], made['bias']
+    taken = []
+    for name in ('_LoraDelta', '_LoraLinear', '_LoraLinearShared'):
+        node = getattr(ops, name)
+        monkeypatch.setattr(node, 'apply', lambda *args, node=node, apply=node.apply: taken.append(node) or apply(*args))
+    ys = [multi_lora_delta(x, base.clone(), seg, groups), ops.multi_lora_linear(x, w, bias, seg, groups),
+          ops.multi_lora_linear_shared(x, [w, w], [bias, None], seg, [groups, groups])[0]]
+    want = {'x': (True, True, True), 'base': (True, False, False), 'adapters': (True, True, True)}.get(which, (False, True, True))
+    assert [n in taken for n in (ops._LoraDelta, ops._LoraLinear, ops._LoraLinearShared)] == list(want)
+    kept = {'x': (1, 2), 'weight': (1, 2), 'bias': (1, 2), 'base': (0,), 'adapters': ()}[which]
+    assert [type(y) is _Tagged for y in ys] == [i in kept for i in range(3)]
+
+
+def test_keys_of_a_subclass(dev):
+    keys = torch.arange(40, dtype=torch.int32, device=dev) % 4
+    assert torch.equal(build_segments(keys.as_subclass(_Tagged), 4).offsets, build_segments(keys, 4).offsets)

@@ -57,6 +57,10 @@ bool plain_rows(const Tensor& t, int64_t rows, int64_t width, at::ScalarType dty
   return plain(t) && t.dim() == 2 && t.size(0) == rows && t.size(1) == width && t.stride(1) == 1 && t.scalar_type() == dtype;
 }
 
+// A tensor as Python holds it; undefined for a subclass, also one without a dispatch key of its own (__torch_function__ only),
+// and for what is no tensor at all.
+Tensor exact(py::handle h) { return THPVariable_CheckExact(h.ptr()) ? THPVariable_Unpack(h.ptr()) : Tensor(); }
+
 // One side (lora_A or lora_B) of an AdapterGroups object.
 struct Side {
   std::vector<Tensor> tensors;
@@ -377,8 +381,9 @@ bool wants_grad(const Groups& g) {
 }
 
 // ops.py::multi_lora_delta
-std::optional<Tensor> delta(const Tensor& x, const Tensor& y, const Tensor& seg, int64_t rows, int64_t num_groups,
+std::optional<Tensor> delta(py::handle x_, py::handle y_, const Tensor& seg, int64_t rows, int64_t num_groups,
                             const GroupsPtr& g, bool map_rows) {
+  const Tensor x = exact(x_), y = exact(y_);
   if (!plain_mode() || num_groups != g->base.num_groups || !plain(seg) ||
       !plain_rows(x, rows, g->base.in_features, g->dtype) || !plain_rows(y, rows, g->base.out_features, g->dtype) ||
       !plain_weights(*g))
@@ -397,33 +402,38 @@ std::optional<Tensor> delta(const Tensor& x, const Tensor& y, const Tensor& seg,
 }
 
 // ops.py::multi_lora_linear (one projection) and multi_lora_linear_shared
-std::optional<variable_list> linear(const Tensor& x, const std::vector<Tensor>& weights,
-                                    const std::vector<std::optional<Tensor>>& biases, const Tensor& seg, int64_t rows,
-                                    int64_t num_groups, const std::vector<GroupsPtr>& groups, bool map_rows) {
+std::optional<variable_list> linear(py::handle x_, const std::vector<py::object>& weights, const std::vector<py::object>& biases,
+                                    const Tensor& seg, int64_t rows, int64_t num_groups, const std::vector<GroupsPtr>& groups,
+                                    bool map_rows) {
   const size_t n = groups.size();
-  if (!plain_mode() || n < 1 || n > TK_MAX_SHARED || weights.size() != n || biases.size() != n || !plain(seg) || !at::GradMode::is_enabled())
+  const Tensor x = exact(x_);
+  if (!plain_mode() || n < 1 || n > TK_MAX_SHARED || weights.size() != n || biases.size() != n || !plain(x) || !plain(seg) ||
+      !at::GradMode::is_enabled())
     return std::nullopt;
   variable_list inputs{x};
   const CallPtr call = make_call(seg, rows, map_rows);
   bool grad = x.requires_grad();
+  variable_list given;  // the biases there are
   for (size_t p = 0; p < n; ++p) {
     const Groups& g = *groups[p];
+    const Tensor weight = exact(weights[p]);
     if (num_groups != g.base.num_groups || !plain_rows(x, rows, g.base.in_features, g.dtype) ||
-        !plain_rows(weights[p], g.base.out_features, g.base.in_features, g.dtype) || !plain_weights(g) ||
+        !plain_rows(weight, g.base.out_features, g.base.in_features, g.dtype) || !plain_weights(g) ||
         (n > 1 && (g.a.elems == 0 || g.b.elems == 0)))
       return std::nullopt;
-    if (biases[p] && !(plain(*biases[p]) && biases[p]->dim() == 1 && biases[p]->size(0) == g.base.out_features &&
-                       biases[p]->scalar_type() == g.dtype))
+    inputs.push_back(weight);
+    grad = grad || weight.requires_grad() || wants_grad(g);
+    call->has_bias.push_back(!biases[p].is_none());
+    if (biases[p].is_none()) continue;
+    const Tensor bias = exact(biases[p]);
+    if (!(plain(bias) && bias.dim() == 1 && bias.size(0) == g.base.out_features && bias.scalar_type() == g.dtype))
       return std::nullopt;
-    inputs.push_back(weights[p]);
-    grad = grad || weights[p].requires_grad() || (biases[p] && biases[p]->requires_grad()) || wants_grad(g);
+    given.push_back(bias);
+    grad = grad || bias.requires_grad();
   }
   // (autocast, which lifts its key from the excluded ones, would run the base GEMM in a type of its own)
   if (!grad || !c10::impl::tls_local_dispatch_key_set().excluded_.has(DispatchKey::AutocastCUDA)) return std::nullopt;
-  for (size_t p = 0; p < n; ++p) {
-    call->has_bias.push_back(biases[p].has_value());
-    if (biases[p]) inputs.push_back(*biases[p]);
-  }
+  inputs.insert(inputs.end(), given.begin(), given.end());
   for (size_t p = 0; p < n; ++p)
     for (const Side* s : {&groups[p]->a, &groups[p]->b}) inputs.insert(inputs.end(), s->tensors.begin(), s->tensors.end());
   call->groups = groups;
@@ -432,12 +442,13 @@ std::optional<variable_list> linear(const Tensor& x, const std::vector<Tensor>& 
 }
 
 // segments.py::build_segments: workspace, permutation, offsets
-std::optional<std::tuple<Tensor, std::optional<Tensor>, std::optional<Tensor>>> segment_build(const Tensor& keys,
-                                                                                               int64_t num_groups,
+std::optional<std::tuple<Tensor, std::optional<Tensor>, std::optional<Tensor>>> segment_build(py::handle keys_, int64_t num_groups,
                                                                                                bool want_perm,
                                                                                                bool want_offsets) {
+  const Tensor keys = exact(keys_);
+  if (!plain_mode() || !plain(keys)) return std::nullopt;
   const bool i32 = keys.scalar_type() == at::kInt;
-  if (!plain_mode() || !plain(keys) || !(i32 || keys.scalar_type() == at::kLong) || !keys.is_contiguous() || num_groups <= 0 ||
+  if (!(i32 || keys.scalar_type() == at::kLong) || !keys.is_contiguous() || num_groups <= 0 ||
       num_groups > TK_MAX_GROUPS)
     return std::nullopt;
   const int64_t rows = keys.numel(), n = tk_segment_workspace_bytes(rows, (int32_t)num_groups);

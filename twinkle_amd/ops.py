@@ -163,10 +163,13 @@ class AdapterGroups:
         return self._arena_plan
 
     def host_groups(self):
-        """This object as the C++ nodes know it; ``None`` with master weights, which only the Python nodes serve."""
+        """This object as the C++ nodes know it; ``None`` with master weights or adapters of a tensor subclass, which only the
+        Python nodes serve."""
         if self.master_a is not None:
             return None
         if self._host is None:
+            if any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in self.a_tensors + self.b_tensors):
+                return None
             self.refresh()
             sides = (('a', self.a_tensors, self.a_index, self.a_offset, self.a_live, self._a_arena_off, self.a_arena_elems,
                       self._grad_a_rel, self.a_ptrs),
