@@ -238,3 +238,14 @@ def test_tensor_subclasses_take_the_python_node(dev, which, monkeypatch):
 def test_keys_of_a_subclass(dev):
     keys = torch.arange(40, dtype=torch.int32, device=dev) % 4
     assert torch.equal(build_segments(keys.as_subclass(_Tagged), 4).offsets, build_segments(keys, 4).offsets)
+
+
+def test_linear_without_autograd_lays_nothing_out(dev):
+    groups, seg, x, base, a, b = _problem(dev)
+    w = torch.zeros(384, 512, dtype=x.dtype, device=dev)
+    with torch.no_grad():
+        ops.multi_lora_linear(x, w, None, seg, groups)
+        ops.multi_lora_linear_shared(x, [w, w], [None, None], seg, [groups, groups])
+    assert groups._host is None
+    ops.multi_lora_linear(x, w, None, seg, groups)
+    assert groups._host is not None

@@ -407,6 +407,8 @@ std::optional<variable_list> linear(py::handle x_, const std::vector<py::object>
                                     bool map_rows) {
   const size_t n = groups.size();
   const Tensor x = exact(x_);
+  // (autocast, which lifts its key from the excluded ones, would run the base GEMM in a type of its own)
+  if (!c10::impl::tls_local_dispatch_key_set().excluded_.has(DispatchKey::AutocastCUDA)) return std::nullopt;
   if (!plain_mode() || n < 1 || n > TK_MAX_SHARED || weights.size() != n || biases.size() != n || !plain(x) || !plain(seg) ||
       !at::GradMode::is_enabled())
     return std::nullopt;
@@ -431,8 +433,7 @@ std::optional<variable_list> linear(py::handle x_, const std::vector<py::object>
     given.push_back(bias);
     grad = grad || bias.requires_grad();
   }
-  // (autocast, which lifts its key from the excluded ones, would run the base GEMM in a type of its own)
-  if (!grad || !c10::impl::tls_local_dispatch_key_set().excluded_.has(DispatchKey::AutocastCUDA)) return std::nullopt;
+  if (!grad) return std::nullopt;
   inputs.insert(inputs.end(), given.begin(), given.end());
   for (size_t p = 0; p < n; ++p)
     for (const Side* s : {&groups[p]->a, &groups[p]->b}) inputs.insert(inputs.end(), s->tensors.begin(), s->tensors.end());

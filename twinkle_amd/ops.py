@@ -696,6 +696,8 @@ def multi_lora_delta(x: torch.Tensor, base_out: torch.Tensor, seg: SegmentTable,
 
 
 def _host_linear(x, weights, biases, seg, groups_list, map_rows):
+    if not torch.is_grad_enabled():     # (these nodes are for autograd: nothing is laid out for a call that has none)
+        return None
     host = _lib.host()
     handles = [g.host_groups() for g in groups_list] if host is not None else [None]
     if None in handles:
