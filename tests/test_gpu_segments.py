@@ -5,7 +5,7 @@ import torch
 import oracle
 from conftest import max_rel_err
 from twinkle_amd import build_segments, flat_keys_from_topk, packed_cu_seqlens, permute, unpermute
-from twinkle_amd import workloads
+from twinkle_amd import _lib, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -216,6 +216,29 @@ def test_builder_of_small_batches(dev, rows, groups, dtype):
     at += pad(tiles + 1)
     sets = -(-real // 4)
     assert torch.equal(table[at:at + sets].long(), torch.argsort(first[::4]))
+
+
+@pytest.mark.parametrize('rows', [1, 32, 64, 65, 512, 513, 1000, 1024, 1025, 1600, 4000])
+def test_moved_rounds_of_a_workspace_that_held_something(dev, rows):
+    """A byte for each of the eight rounds of every sort block, whatever the workspace held: set where a row of the round
+    moved.  One-block builder up to 1024 rows, several blocks above."""
+    lib, groups = _lib.load(), 4
+    tiles = -(-rows // 32) + groups + 1
+    at = sum(-(-n // 256) * 256 for n in (256, 4 * (rows + 64), 128 * tiles, 128 * tiles, 4 * (groups + 2), 4 * (tiles + 1),
+                                          4 * (tiles + 1), 4 * (tiles // 4 + 2)))
+    rounds, blocks = -(-rows // 64), -(-rows // 512)
+    in_order = torch.arange(rows, dtype=torch.int32) * groups // rows
+    swapped = in_order.clone()
+    swapped[-1], swapped[0] = in_order[0], in_order[-1]
+    for keys in (in_order, swapped):
+        n = lib.tk_segment_workspace_bytes(rows, groups)
+        ws = torch.full((n,), 0x5a, dtype=torch.uint8, device=dev)
+        on_gpu = keys.to(dev)
+        assert lib.tk_segment_build(on_gpu.data_ptr(), _lib.TK_KEY_I32, rows, groups, None, None, ws.data_ptr(), n,
+                                    _lib.stream_ptr()) == _lib.TK_OK
+        moved = torch.argsort(torch.argsort(keys, stable=True)) != torch.arange(rows)
+        want = [bool(moved[64 * r:64 * r + 64].any()) if r < rounds else False for r in range(8 * blocks)]
+        assert ws[at:at + 8 * blocks].cpu().ne(0).tolist() == want
 
 
 @pytest.mark.parametrize('dtype,wdtype', [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),

@@ -684,6 +684,8 @@ __global__ __launch_bounds__(kSmallWaves * 64) void k_seg_small(const KeyT* __re
       opened[1][round] = (uint16_t)__popcll(s);
     }
   }
+  // (the consumers look at whole sort blocks: no row of the rounds that the last one lacks has moved)
+  if (sweep && rounds + tid < (rounds + kKeysPerLane - 1) / kKeysPerLane * kKeysPerLane) V.round_moved[rounds + tid] = 0;
   // per-tile entries (8 threads a tile, four slots each) and chunks; a tile that no group owns stays where it is in the orders
   for (int i = tid; i < 8 * max_tiles; i += kSmallWaves * 64) {
     const int tile = i >> 3, j = 4 * (i & 7);

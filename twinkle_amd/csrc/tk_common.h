@@ -134,8 +134,8 @@ struct SegView {  // typed device pointers into a segment workspace
   int32_t* set_order;
   // [64 sort blocks][8 rounds of 64 rows]  one byte per round of the single-launch builder: non-zero when the sort
   // moved a row of the round (its sorted position differs from its row number).  All zero for the rounds of a build
-  // <=> the keys came in order <=> tile_order and set_order are the identity.  Bytes of rounds past the last row of
-  // the current build are stale.
+  // <=> the keys came in order <=> tile_order and set_order are the identity.  The last sort block's rounds past the last
+  // row hold zero; bytes of sort blocks past it are stale.
   uint8_t* round_moved;
   ChunkInfo* chunks;       // [max_chunks]
   int32_t* tile_first;     // [G + 2]  first tile of each group
