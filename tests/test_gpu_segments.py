@@ -6,6 +6,7 @@ import oracle
 from conftest import max_rel_err
 from twinkle_amd import build_segments, flat_keys_from_topk, packed_cu_seqlens, permute, unpermute
 from twinkle_amd import _lib, workloads
+from twinkle_amd.segments import _keys_on_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -277,3 +278,27 @@ def test_keys_of_routed_rows(dev, dtype, tenant_dtype, t, k):
         layout = torch.empty_strided(sel.shape, sel.stride(), dtype=dtype, device=dev).copy_(sel)
         got = flat_keys_from_topk(layout, tenant.to(dev) if tenant is not None else None, 5)
         assert got.dtype == want.dtype and got.is_contiguous() and torch.equal(got.cpu(), want)
+
+
+def test_keys_of_routed_rows_while_the_call_is_recorded(dev):
+    """Tracers and dispatch modes see torch operations: a launch of our own would leave no trace of how the keys came about."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+    sel, other = (torch.randint(0, 9, (50, 4), generator=torch.Generator().manual_seed(i)).to(dev) for i in range(2))
+    tenant = torch.randint(0, 3, (50,), generator=torch.Generator().manual_seed(5), dtype=torch.int32).to(dev)
+    want = flat_keys_from_topk(other, tenant, 3)
+    assert _keys_on_gpu(other, tenant)                       # outside of all that: one launch
+    for traced in (make_fx(lambda s, t: flat_keys_from_topk(s, t, 3))(sel, tenant),
+                   torch.jit.trace(lambda s, t: flat_keys_from_topk(s, t, 3), (sel, tenant))):
+        assert torch.equal(traced(other, tenant), want)
+
+    class Seen(TorchDispatchMode):
+        ops = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        assert torch.equal(flat_keys_from_topk(other, tenant, 3), want)
+    assert torch.ops.aten.mul.Tensor in Seen.ops

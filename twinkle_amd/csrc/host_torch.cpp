@@ -469,6 +469,7 @@ std::optional<std::tuple<Tensor, std::optional<Tensor>, std::optional<Tensor>>> 
 
 PYBIND11_MODULE(_host, m) {
   py::class_<Groups, GroupsPtr>(m, "Groups").def_readwrite("zeros", &Groups::zeros);
+  m.def("plain_mode", &plain_mode);
   m.def("make_groups", &make_groups);
   m.def("delta", &delta);
   m.def("linear", &linear);

@@ -142,14 +142,17 @@ def build_token_segments(keys: torch.Tensor, num_groups: int, num_tokens: int) -
 
 
 def _keys_on_gpu(selected: torch.Tensor, tenant: Optional[torch.Tensor]) -> bool:
-    """Plain GPU tensors one launch makes the keys of (torch's three to five cost more than the table behind them)."""
+    """Plain GPU tensors one launch makes the keys of (torch's three to five cost more than the table behind them), on the
+    current device and with nobody watching the operations: tracers, dispatch modes and transforms see torch's."""
     def plain(t, dim):
         return (type(t) is torch.Tensor and t.is_cuda and t.dim() == dim and t.dtype in (torch.int32, torch.int64) and
                 t.device == selected.device)
 
-    return (plain(selected, 2) and selected.numel() < 2**31 and _lib.host() is not None and
-            not torch._C._are_functorch_transforms_active() and
-            (tenant is None or (plain(tenant, 1) and tenant.is_contiguous() and tenant.shape[0] == selected.shape[0])))
+    if not (plain(selected, 2) and selected.numel() < 2**31 and
+            (tenant is None or (plain(tenant, 1) and tenant.is_contiguous() and tenant.shape[0] == selected.shape[0]))):
+        return False
+    host = _lib.host()
+    return host is not None and host.plain_mode() and selected.get_device() == torch._C._cuda_getDevice()
 
 
 def flat_keys_from_topk(selected: torch.Tensor, tenant: Optional[torch.Tensor] = None,
