@@ -249,3 +249,14 @@ def test_linear_without_autograd_lays_nothing_out(dev):
     assert groups._host is None
     ops.multi_lora_linear(x, w, None, seg, groups)
     assert groups._host is not None
+
+
+def test_inference_tensors_are_updated_in_their_mode_only(dev):
+    groups, seg, x, base, a, b = _problem(dev)
+    with torch.inference_mode():
+        y = base.clone()
+    for mode in (torch.no_grad, torch.enable_grad):
+        with mode(), pytest.raises(RuntimeError, match='Inplace update to inference tensor'):
+            multi_lora_delta(x, y, seg, groups)
+    with torch.inference_mode():
+        assert multi_lora_delta(x, y, seg, groups) is y

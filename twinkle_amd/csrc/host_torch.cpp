@@ -384,6 +384,8 @@ bool wants_grad(const Groups& g) {
 std::optional<Tensor> delta(py::handle x_, py::handle y_, const Tensor& seg, int64_t rows, int64_t num_groups,
                             const GroupsPtr& g, bool map_rows) {
   const Tensor x = exact(x_), y = exact(y_);
+  // (an inference tensor is not updated outside of that mode: the Python node says so)
+  if (y.defined() && y.is_inference() && !c10::InferenceMode::is_enabled()) return std::nullopt;
   if (!plain_mode() || num_groups != g->base.num_groups || !plain(seg) ||
       !plain_rows(x, rows, g->base.in_features, g->dtype) || !plain_rows(y, rows, g->base.out_features, g->dtype) ||
       !plain_weights(*g))
