@@ -177,42 +177,52 @@ __global__ __launch_bounds__(256) void k_shrink_any(PassArgs a, int slice_cols, 
           for (int p = 0; p < 2; ++p) acc[tt][nb] = mma_piece<T>(x[j][tt][p], w[j][nb][p], acc[tt][nb]);
   }
   // The steps left, the last of them perhaps cut by the width (a slice ends at a whole step or there): the two pieces of
-  // a lane are moved back into the row and shifted.
-  auto steps_left = [&](auto cut) {
-    for (; c < k1; c += 4 * STEP) {
-      const int cc = c + 2 * E * kb;
-      uint4 x[2][2], w[NB][2];
+  // a lane are moved back into the row and shifted, unless a row is shorter than a piece.  One loop for both: with a loop
+  // each the compiler kept a second set of accumulators, and at rank 128 one wave per SIMD where two fit (8192 x 4096 fp32
+  // at rank 128, forward 294 us against 274).  Not unrolled and laid out as the rare case: fp32 at rank 96 to 112, 300 x
+  // 4096, shrink 60 us otherwise, 53 so, although its whole steps never come here.
+  const bool wide = a.width_src >= E;
+#pragma clang loop unroll(disable)
+  for (; __builtin_expect(c < k1, 0); c += 4 * STEP) {
+    const int cc = c + 2 * E * kb;
+    uint4 x[2][2], w[NB][2];
+    if (wide) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        const int col = cut ? min(cc + p * E, a.width_src - E) : cc + p * E, keep = k1 - cc - p * E;
+        const int col = min(cc + p * E, a.width_src - E);
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) x[tt][p] = cut ? ld_piece(xr[tt] + col) : ld_piece(xr[tt] + col, keep);
+        for (int tt = 0; tt < 2; ++tt) x[tt][p] = ld_piece(xr[tt] + col);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) w[nb][p] = cut ? ld_piece(wr[nb] + col) : ld_piece(wr[nb] + col, keep);
+        for (int nb = 0; nb < NB; ++nb) w[nb][p] = ld_piece(wr[nb] + col);
       }
-      if constexpr (cut) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (c + STEP > k1) {  // (uniform)
+    } else {
 #pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const int drop = max(0, cc + p * E - (a.width_src - E));
+      for (int p = 0; p < 2; ++p) {
+        const int col = cc + p * E, keep = k1 - col;
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) x[tt][p] = drop_front<T>(x[tt][p], drop);
+        for (int tt = 0; tt < 2; ++tt) x[tt][p] = ld_piece(xr[tt] + col, keep);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) w[nb][p] = drop_front<T>(w[nb][p], drop);
-          }
-        }
+        for (int nb = 0; nb < NB; ++nb) w[nb][p] = ld_piece(wr[nb] + col, keep);
       }
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-          for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mma_piece<T>(x[tt][p], w[nb][p], acc[tt][nb]);
     }
-  };
-  if (a.width_src >= E) steps_left(std::true_type{});
-  else steps_left(std::false_type{});  // (a row shorter than a piece)
+    __builtin_amdgcn_sched_barrier(0);
+    if (wide && c + STEP > k1) {  // (uniform)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int drop = max(0, cc + p * E - (a.width_src - E));
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) x[tt][p] = drop_front<T>(x[tt][p], drop);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) w[nb][p] = drop_front<T>(w[nb][p], drop);
+      }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) acc[tt][nb] = mma_piece<T>(x[tt][p], w[nb][p], acc[tt][nb]);
+  }
   const float sc = a.scale[g];
 #pragma unroll
   for (int b = 0; b < NB; b += NBS) {
