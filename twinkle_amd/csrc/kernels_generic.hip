@@ -341,7 +341,11 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
   // slots read row 0, rank indices past the rank read index 0 and are zeroed).  1, cut: the pieces at the end of the
   // width or the rank are moved back into their row and shifted, columns past the width read the last one's weights.
   // 0: a row or a rank shorter than a piece, an element at a time.
+  // Cut pieces go through the caches and are shifted only where something is cut off: rows off the 16-byte pieces share
+  // their lines with the items beside them (8192 x 4001 fp32 at rank 13, us: an element at a time 64, non-temporal 75, so
+  // 59; bf16 71 / 56 / 46; 4096 columns, where only the rank is cut, fp32 54 / 58 / 49).
   const int back = c - min(c, a.width_dst - E);
+  const bool columns = (c - E * li) + 16 * E <= a.width_dst;  // every lane has its E columns (uniform over the wave)
   auto body = [&](auto form) {
     constexpr bool whole = form == 2, cut = form == 1;
 #pragma unroll
@@ -349,7 +353,7 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const T* row = dst + (int64_t)max(checked_row(rows[tt][v], a.tb), 0) * a.ld_dst;
-        y[tt][v] = a.dst_store ? zero4() : (whole ? ld_piece_nt(row) : (cut ? ld_piece_nt(row - back) : ld_piece(row, keep)));
+        y[tt][v] = a.dst_store ? zero4() : (whole ? ld_piece_nt(row) : (cut ? ld_piece(row - back) : ld_piece(row, keep)));
       }
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -372,19 +376,23 @@ __global__ __launch_bounds__(256) void k_expand_any(PassArgs a, const int32_t* _
 #pragma unroll
       for (int q = 0; q < E; ++q) {
         if (whole && n0 >= r) w[q] = zero4();
-        if constexpr (cut) w[q] = drop_front<T>(w[q], max(0, n0 - (r - E)));
+        if constexpr (cut) {
+          if (4 * E * (ks + 1) > r) w[q] = drop_front<T>(w[q], max(0, n0 - (r - E)));  // (uniform over the block)
+        }
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) d[tt][q] = mma_piece<T>(hop[tt], w[q], d[tt][q]);
       }
     }
     if constexpr (cut) {
+      if (!columns) {
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) y[tt][v] = drop_front<T>(y[tt][v], back);
+          for (int v = 0; v < 4; ++v) y[tt][v] = drop_front<T>(y[tt][v], back);
+      }
     }
   };
-  if ((c - E * li) + 16 * E <= a.width_dst && r % E == 0) body(std::integral_constant<int, 2>{});
+  if (columns && r % E == 0) body(std::integral_constant<int, 2>{});
   else if (a.width_dst >= E && r >= E) body(std::integral_constant<int, 1>{});
   else body(std::integral_constant<int, 0>{});
 #pragma unroll
