@@ -129,9 +129,8 @@ int tk_unpermute_weight_grad(const void* dout_device, int64_t ld_dout, const voi
                              int32_t width, int32_t num_groups, int32_t dtype, tk_stream_t stream);
 
 /* Both gradients of tk_unpermute_rows from one look at each row: grad_rows as tk_permute_rows (with or without weights)
- * writes it, dw as above (fp32 when dw_f32, else in `dtype`), for at most TK_UNPERMUTE_BWD_TOP_K rows a token.  dw null: not
- * wanted, rows are not read.  Needs the table's positions only (also a table of tk_segment_build_tokens). */
-#define TK_UNPERMUTE_BWD_TOP_K 32
+ * writes it, dw as above (fp32 when dw_f32, else in `dtype`).  dw null: not wanted, rows are not read.  Needs the table's
+ * positions only (also a table of tk_segment_build_tokens). */
 int tk_unpermute_bwd(const void* dout_device, int64_t ld_dout, const void* rows_device, int64_t ld_rows,
                      void* grad_rows_device, int64_t ld_grad, const void* weights_device, void* dw_device, int32_t dw_f32,
                      const void* seg_ws_device, int64_t rows, int64_t num_tokens, int32_t width, int32_t num_groups,

@@ -266,6 +266,25 @@ def test_both_gradients_of_the_weighted_unpermute(dev, dtype, wdtype, t, k, h):
     assert (both[1].float() - only_w.float()).abs().max().item() <= 2 * ulp * scale
 
 
+@pytest.mark.parametrize('dtype,wdtype', [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                          (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize('t,k,h', [(5, 33, 24), (3, 70, 520), (7, 3, 4096), (2, 5, 4104), (6, 2, 4608), (3, 3, 517), (4, 1, 1024)])
+def test_gradients_of_the_unpermute_are_those_of_separate_launches(dev, dtype, wdtype, t, k, h):
+    """Any number of rows a token, rows of less and of more than 512 pieces, ends of them inside a step: a wave sums a row as
+    the launch for the weights alone does, so the same bits."""
+    g = torch.Generator().manual_seed(t + h)
+    seg = build_segments(torch.randint(-1, 7, (t * k,), generator=g, dtype=torch.int32).to(dev), 7, num_tokens=t)
+    rows = torch.randn(t * k, h, generator=g).to(dev, dtype).requires_grad_(True)
+    w = torch.rand(t, k, generator=g).to(dev, wdtype).requires_grad_(True)
+    dy = torch.randn(t, h, generator=g).to(dev, dtype)
+    both = torch.autograd.grad(unpermute(rows, w, seg), [rows, w], dy)
+    assert torch.equal(both[1], torch.autograd.grad(unpermute(rows.detach(), w, seg), [w], dy)[0])
+    perm = seg.perm
+    want = (dy[perm % t].float() * w.detach().to(dtype).t().reshape(-1)[perm, None].float()).to(dtype)
+    assert torch.equal(both[0], want)
+    assert torch.equal(torch.autograd.grad(unpermute(rows, w.detach(), seg), [rows], dy)[0], want)
+
+
 @pytest.mark.parametrize('dtype', [torch.int32, torch.int64])
 @pytest.mark.parametrize('tenant_dtype', [None, torch.int32, torch.int64])
 @pytest.mark.parametrize('t,k', [(0, 4), (1, 1), (300, 1), (77, 8)])

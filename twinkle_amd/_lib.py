@@ -29,7 +29,6 @@ TK_KEY_I32 = 0
 TK_KEY_I64 = 1
 TK_TILE_ROWS = 32
 TK_CHUNK_ROWS = 128
-TK_UNPERMUTE_BWD_TOP_K = 32
 TK_MAX_GROUPS = 16384
 TK_MAX_RANK = 128
 

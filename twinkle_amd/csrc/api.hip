@@ -448,7 +448,6 @@ int tk_unpermute_bwd(const void* dout, int64_t ld_dout, const void* rows_p, int6
   if (!rows_args_ok(dout, grad_rows, seg_ws, rows, num_tokens, width, num_groups, dtype) || (dw && (!rows_p || !weights)))
     return TK_ERR_INVALID;
   if (ld_dout < width || (dw && ld_rows < width) || ld_grad < width) return TK_ERR_INVALID;
-  if (dw && rows > num_tokens * TK_UNPERMUTE_BWD_TOP_K) return TK_ERR_UNSUPPORTED;
   return launch_unpermute_bwd(dout, ld_dout, rows_p, ld_rows, grad_rows, ld_grad, weights, dw, dw_f32, seg_ws, rows, num_tokens,
                               width, num_groups, dtype, (hipStream_t)stream);
 }

@@ -790,8 +790,6 @@ __global__ __launch_bounds__(1024) void k_class_lists(ClassListArgs p, ClassList
   if (tid == 0) ((int32_t*)p.base[c])[which] = running;
 }
 
-constexpr int kUnpermuteTopK = TK_UNPERMUTE_BWD_TOP_K;
-
 // 16 bytes of a row: the unit the row movers below load and store when width, strides and pointers allow
 // (V = 8 bf16 / 4 fp32 elements), else V = 1.  The arithmetic per element and the order of every sum are the
 // same for both.
@@ -890,52 +888,59 @@ __global__ __launch_bounds__(64) void k_unpermute_wgrad(const T* __restrict__ do
 }
 
 // Both gradients of the weighted unpermute from one look at each row: grad_rows[pos(k, t)] = dout[t] * w[t, k] (w null: 1) and,
-// unless dw is null, dw[t, k] = <dout[t], rows[pos(k, t)]>.  A block owns a token, whose dout stays in its cache over the top_k rows.  Bound by
-// memory: rows read and grad_rows written once (as two launches dout crossed the caches twice as often and the rows' reads had
-// no writes next to them: 65536 rows of 2048, 166 us; here 104).
-template <typename T, int V, typename W>
+// with DW, dw[t, k] = <dout[t], rows[pos(k, t)]>.  A wave owns a row, the waves of a block neighbouring rows of a token, whose
+// dout they find in the CU's cache; the sums are those of k_unpermute_wgrad, term by term.  Bound by memory: rows read and
+// grad_rows written once.  WIDE (512 pieces of a row and more: eight steps of the wave): no guards but in the last step.
+// bf16, us, two launches / a block of four waves per token, one row after the other / here: 8192 tokens, top 8, 2048 wide
+// 157 / 125 / 119 (rows alone 80 / 78 / 53), 128 wide 38 / 43 / 23; 64 tokens, top 32, 512 wide 7.7 / 27 / 4.2; one token, top
+// 32, 7168 wide 11.7 / 72 / 8.6; 8192 tokens, top 1, 2048 wide 26.6 / 18.2 / 18.7.
+template <typename T, int V, typename W, bool DW, bool WIDE>
 __global__ __launch_bounds__(256) void k_unpermute_bwd(const T* __restrict__ dout, int64_t ld_dout, const T* __restrict__ rows_,
                                                        int64_t ld_rows, T* __restrict__ grad, int64_t ld_grad,
                                                        const T* __restrict__ w, W* __restrict__ dw,
                                                        const int32_t* __restrict__ inv, int tokens, int top_k, int width) {
-  __shared__ float sums[kUnpermuteTopK][4];
-  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const RowVec<T, V>* d = reinterpret_cast<const RowVec<T, V>*>(dout + (int64_t)t * ld_dout);
-#pragma unroll 2
-  for (int k = 0; k < top_k; ++k) {
-    const int j = inv[(int64_t)k * tokens + t];
-    float acc = 0.f;
-    if ((unsigned)j < (unsigned)(tokens * top_k)) {  // (a position outside the table's rows: no row, no gradient)
-      const RowVec<T, V>* r = reinterpret_cast<const RowVec<T, V>*>(rows_ + (int64_t)j * ld_rows);
-      RowVec<T, V>* g = reinterpret_cast<RowVec<T, V>*>(grad + (int64_t)j * ld_grad);
-      const float wt = w ? to_f32(w[(int64_t)t * top_k + k]) : 1.f;
-      for (int c = threadIdx.x; c < width / V; c += 256) {
-        RowVec<T, V> x = d[c];
-        if (!dw) {
-          if (w) {
+  const int lane = threadIdx.x & 63;
+  const unsigned i = blockIdx.x * 4u + (threadIdx.x >> 6);  // (rows < 2^31)
+  if (i >= (unsigned)(tokens * top_k)) return;
+  const int t = (int)(i / (unsigned)top_k), k = (int)(i - (unsigned)t * (unsigned)top_k);
+  const int j = inv[(int64_t)k * tokens + t];
+  float acc = 0.f;
+  if ((unsigned)j < (unsigned)(tokens * top_k)) {  // (a position outside the table's rows: no row, no gradient)
+    const RowVec<T, V>* d = reinterpret_cast<const RowVec<T, V>*>(dout + (int64_t)t * ld_dout);
+    const RowVec<T, V>* r = reinterpret_cast<const RowVec<T, V>*>(rows_ + (int64_t)j * ld_rows);
+    RowVec<T, V>* g = reinterpret_cast<RowVec<T, V>*>(grad + (int64_t)j * ld_grad);
+    const float wt = w ? to_f32(w[i]) : 1.f;
+    const int n = width / V;
+    // pieces c and c + 64: requested together, then scaled, added up and stored
+    auto two = [&](int c, auto guarded) __attribute__((always_inline)) {
+      constexpr bool G = decltype(guarded)::value;
+      RowVec<T, V> x[2], y[2];
 #pragma unroll
-            for (int i = 0; i < V; ++i) from_f32(to_f32(x.v[i]) * wt, &x.v[i]);
-          }
-          g[c] = x;
-          continue;
-        }
-        const RowVec<T, V> y = r[c];
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-          acc += to_f32(x.v[i]) * to_f32(y.v[i]);
-          from_f32(to_f32(x.v[i]) * wt, &x.v[i]);
-        }
-        g[c] = x;
+      for (int u = 0; u < 2; ++u) {
+        if (G && c + 64 * u >= n) continue;
+        x[u] = d[c + 64 * u];
+        if constexpr (DW) y[u] = r[c + 64 * u];
       }
-    }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (G && c + 64 * u >= n) break;
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          if constexpr (DW) acc += to_f32(x[u].v[q]) * to_f32(y[u].v[q]);
+          if (w) from_f32(to_f32(x[u].v[q]) * wt, &x[u].v[q]);
+        }
+        g[c + 64 * u] = x[u];
+      }
+    };
+    int c = lane;
+    if constexpr (WIDE)
+      for (; c + 64 < n; c += 128) two(c, std::false_type{});
+    for (; c < n; c += 128) two(c, std::true_type{});
+  }
+  if constexpr (DW) {
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s, 64);
-    if (dw && lane == 0) sums[k][wave] = acc;
-  }
-  __syncthreads();
-  if (dw && (int)threadIdx.x < top_k) {
-    const float* s = sums[threadIdx.x];
-    from_f32((s[0] + s[1]) + (s[2] + s[3]), &dw[(int64_t)t * top_k + threadIdx.x]);
+    if (lane == 0) from_f32(acc, &dw[i]);
   }
 }
 
@@ -1111,14 +1116,20 @@ int launch_unpermute_bwd(const void* dout, int64_t ld_dout, const void* rows_, i
                          int32_t groups, int dtype, hipStream_t s) {
   if (rows == 0) return TK_OK;
   SegLayout L(rows, groups);
-  SegView V(ws, L);
+  const SegView view(ws, L);
   const int top_k = (int)(rows / tokens);
-  const dim3 grid((unsigned)tokens), block(256);
+  const dim3 grid((unsigned)ceil_div(rows, 4)), block(256);
   auto launch = [&](auto vec, auto element, auto weight) {
     using T = decltype(element);
     using W = decltype(weight);
-    hipLaunchKernelGGL((k_unpermute_bwd<T, decltype(vec)::value, W>), grid, block, 0, s, (const T*)dout, ld_dout,
-                       (const T*)rows_, ld_rows, (T*)grad, ld_grad, (const T*)w, (W*)dw, V.inv, (int)tokens, top_k, width);
+    constexpr int V = decltype(vec)::value;
+    auto with = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, s, (const T*)dout, ld_dout, (const T*)rows_, ld_rows, (T*)grad, ld_grad,
+                         (const T*)w, (W*)dw, view.inv, (int)tokens, top_k, width);
+    };
+    const bool wide = width / V >= 512;
+    if (dw) with(wide ? k_unpermute_bwd<T, V, W, true, true> : k_unpermute_bwd<T, V, W, true, false>);
+    else with(wide ? k_unpermute_bwd<T, V, W, false, true> : k_unpermute_bwd<T, V, W, false, false>);
   };
   using std::integral_constant;
   if (dtype == TK_DTYPE_F32) {

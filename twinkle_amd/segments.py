@@ -261,7 +261,7 @@ class _Unpermute(torch.autograd.Function):
             w = weights.to(rows.dtype).contiguous() if weights is not None else None
             grad_rows = torch.empty(seg.rows, rows.shape[1], dtype=rows.dtype, device=rows.device)
             dw = None
-            if weights is not None and ctx.needs_input_grad[1] and seg.top_k <= _lib.TK_UNPERMUTE_BWD_TOP_K:
+            if weights is not None and ctx.needs_input_grad[1]:
                 kind = weights.dtype if weights.dtype == rows.dtype else torch.float32
                 dw = torch.empty(seg.num_tokens, seg.top_k, dtype=kind, device=rows.device)
             code = _lib.load().tk_unpermute_bwd(
