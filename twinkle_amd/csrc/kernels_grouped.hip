@@ -539,7 +539,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
     const bool more = it_next >= 0;
     int nb_next, drawn = 0;
     if (more && tid == 0) drawn = atomicAdd(tickets + xcd, 1);  // (used behind the products)
-    const GroupedPlanEntry* pe_next = entry_of(more ? it_next : 0, &nb_next);
+    const GroupedPlanEntry* pe_next = entry_of(more ? it_next : it, &nb_next);
     const int ntiles = min(pe->ntiles, 8), slot0 = pe->tile0 * kTileRows, ngroups = min(pe->ngroups, 8);
 
     // LoRA: this lane's group of step l (its matrix and live rank)
@@ -705,6 +705,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
       }
       x_offsets(pe_next, row_next);
       weights_of(pe_next, nb_next);
+      if (!more) xbytes_now = wbytes = 0;  // nothing follows: the same count of loads, which bring nothing
       fetch_x(0, As0);
       fetch_w(0, Bs0);
       __builtin_amdgcn_sched_barrier(0);
@@ -757,42 +758,50 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
         }
       }
     }
-    const int nb_now = nb;
-    const GroupedPlanEntry* pe_now = pe;
+    auto store = [&]() __attribute__((always_inline)) {
+      // lane holds y[slot 16 (2 rb + wm) + li][nb BN + 16 CB wn + 16 cb + 4 kb + v], v = 0..3.  Column blocks 2 c and 2 c + 1
+      // exchange between neighbouring kb, so that a lane has eight consecutive columns and a store covers 64 bytes of 16 rows.
+      const int ln = here(lane), i = 16 * wm + (ln & 15), chunk = ((ln >> 4) & 1) * 2 + (ln >> 5);
+      bf16_t* y0 = a.y + nb * BN + 16 * CB * wn + 8 * chunk;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        if (rb >= ntiles) break;
+        int row;
+        if (a.map_rows) row = checked_row(slot_rows[slot0 + kTileRows * rb + i], a.tb);
+        else row = i < pe->cnt[rb] ? pe->pos[rb] + i : -1;
+        uint4 out[CB / 2];
+#pragma unroll
+        for (int c = 0; c < CB / 2; ++c) {
+          const f32x4 u = acc[rb][2 * c], v = acc[rb][2 * c + 1];
+          const auto lo = __builtin_amdgcn_permlane16_swap(pack_bf16(u[0], u[1]), pack_bf16(v[0], v[1]), false, false);
+          const auto hi = __builtin_amdgcn_permlane16_swap(pack_bf16(u[2], u[3]), pack_bf16(v[2], v[3]), false, false);
+          out[c] = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+        }
+        if (row < 0) continue;
+        bf16_t* yp = y0 + (int64_t)row * a.ldy;
+#pragma unroll
+        for (int c = 0; c < CB / 2; ++c) st16(yp + 32 * c, out[c]);
+      }
+    };
     loads_landed_barrier<4 + WP>();
+    // A block's last item: no tiles behind it, and its stores are the last thing it does.  (It fetched the first tiles of any
+    // item before and waited for them and its stores: 160 KB a block.  us, forward with the LoRA term, then and now, and what
+    // the kernel with one block per item took: 1024 rows of 128 experts 768 -> 2048 102.6 / 97.0 / 109.2, 65536 rows
+    // 2048 -> 512 186.7 / 186.7 / 204.5; one item per block, 16 rows of 8 experts 2048 -> 1536 33.9 / 33.3 / 32.0.)
+    if (!more) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): no load may land in LDS that belongs to the next block
+      store();
+      return;
+    }
     fetch_w(1, Bs1);
     fetch_x(1, As1);
     fetch_w(2, Bs2);
-
-    // lane holds y[slot 16 (2 rb + wm) + li][nb BN + 16 CB wn + 16 cb + 4 kb + v], v = 0..3.  Column blocks 2 c and 2 c + 1
-    // exchange between neighbouring kb, so that a lane has eight consecutive columns and a store covers 64 bytes of 16 rows.
-    const int ln = here(lane), i = 16 * wm + (ln & 15), chunk = ((ln >> 4) & 1) * 2 + (ln >> 5);
-    bf16_t* y0 = a.y + nb_now * BN + 16 * CB * wn + 8 * chunk;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      if (rb >= ntiles) break;
-      int row;
-      if (a.map_rows) row = checked_row(slot_rows[slot0 + kTileRows * rb + i], a.tb);
-      else row = i < pe_now->cnt[rb] ? pe_now->pos[rb] + i : -1;
-      uint4 out[CB / 2];
-#pragma unroll
-      for (int c = 0; c < CB / 2; ++c) {
-        const f32x4 u = acc[rb][2 * c], v = acc[rb][2 * c + 1];
-        const auto lo = __builtin_amdgcn_permlane16_swap(pack_bf16(u[0], u[1]), pack_bf16(v[0], v[1]), false, false);
-        const auto hi = __builtin_amdgcn_permlane16_swap(pack_bf16(u[2], u[3]), pack_bf16(v[2], v[3]), false, false);
-        out[c] = make_uint4(lo[0], hi[0], lo[1], hi[1]);
-      }
-      if (row < 0) continue;
-      bf16_t* yp = y0 + (int64_t)row * a.ldy;
-#pragma unroll
-      for (int c = 0; c < CB / 2; ++c) st16(yp + 32 * c, out[c]);
-    }
-    if (!more) break;  // (with the tiles of an item that does not follow still on their way)
+    store();
+    it = it_next;
     it_next = item_of(k_after);
     pe = pe_next;
     nb = nb_next;
   }
-  loads_landed_barrier<0>();  // no load may land in LDS that belongs to the next block
 }
 
 }  // namespace
