@@ -45,8 +45,9 @@ def _problem(dev, t, e, k, hidden, inter, ranks, max_r, seed=0):
     return mod, slots, names, params, sel, w, tenant, x, dy
 
 
-def _exact(mod, slots, names, sel, w, tenant, x):
-    """float64, expert by expert and tenant by tenant, on merged weights."""
+def _exact(mod, slots, names, sel, w, tenant, x, params):
+    """float64, expert by expert and tenant by tenant, on merged weights (``params``: the adapters, as ``_problem`` lists them)."""
+    live = [name for name in names if name is not None]
     out = torch.zeros_like(x)
     gate_up, down = mod.gate_up_proj.double(), mod.down_proj.double()
     for e in range(gate_up.shape[0]):
@@ -58,8 +59,8 @@ def _exact(mod, slots, names, sel, w, tenant, x):
             ws = [gate_up[e], down[e]]
             if name is not None:
                 for i, s in enumerate(slots):
-                    r = s.r[name]
-                    ws[i] = ws[i] + s.scaling[name] * s.lora_B[name][e, :, :r].double() @ s.lora_A[name][e, :r].double()
+                    r, at = s.r[name], 2 * (i * len(live) + live.index(name))
+                    ws[i] = ws[i] + s.scaling[name] * params[at + 1][e, :, :r] @ params[at][e, :r]
             gu = x[t] @ ws[0].t()
             gate, up = gu.chunk(2, -1)
             out = out.index_add(0, t, (torch.nn.functional.silu(gate) * up) @ ws[1].t() * w[t, k, None])
@@ -89,13 +90,13 @@ def test_block_on_tokens(dev, t, e, k, hidden, inter, ranks, max_r):
     ref = unpermute(experts_forward(mod, rows, seg, names, *slots), w, seg)
     assert torch.equal(ref, got[0])
     want = [ref.detach(), *torch.autograd.grad(ref, inputs, dy)]
-    exact_in = [v.detach().double().requires_grad_(True) for v in (x, w)]
-    exact_out = _exact(mod, slots, names, sel, exact_in[1], tenant, exact_in[0])
+    exact_in = [v.detach().double().requires_grad_(True) for v in inputs]
+    exact_out = _exact(mod, slots, names, sel, exact_in[1], tenant, exact_in[0], exact_in[2:])
     exact = [exact_out, *torch.autograd.grad(exact_out, exact_in, dy.double())]
     for i, (p, q) in enumerate(zip(got, want)):
-        if i < 3:          # outputs and the gradients of x and the routing weights: bf16 intermediates, four products in a row
-            scale = exact[i].abs().max().item()
-            assert (p.double() - exact[i]).abs().max().item() < 2e-2 * scale, i
+        # bf16 intermediates, four products in a row; the two paths share the backward's kernels, so that one is not enough
+        scale = exact[i].abs().max().item()
+        assert (p.double() - exact[i]).abs().max().item() <= 2e-2 * scale, i
         scale = q.double().abs().max().item()
         assert (p.double() - q.double()).abs().max().item() <= 2e-2 * scale, i
 

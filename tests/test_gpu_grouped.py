@@ -6,6 +6,7 @@ import torch
 import oracle
 from conftest import max_rel_err
 from twinkle_amd import AdapterGroups, build_segments, grouped_linear_, lora_h_bytes, lora_shrink_
+from twinkle_amd.ops import grouped_experts_linear
 
 pytestmark = pytest.mark.gpu
 
@@ -242,6 +243,69 @@ def test_lora_step_of_the_direct_kernel(dev, max_r, ranks, sizes, offset):
                 want[rows] += 2.0 * (x[rows].double() @ a[ti][ei, :r].double().cpu().t()) @ b[ti][ei, :, :r].double().cpu().t()
     # h and y are rounded to eight bits once each
     assert max_rel_err(got[~own], want[~own]) < 1e-2
+
+
+@pytest.mark.parametrize('max_r,ranks,sizes', [
+    (8, [8] * 12, 20),                    # as above: eight groups in a row block
+    (16, [16] * 12, 20),
+    (64, [64, 33, 0, 64, 7, 64], 40),
+    (16, [12, 5, 12], 70),
+    (24, [24, 8], 300),
+])
+@pytest.mark.parametrize('offset', [0, 3])
+def test_lora_step_of_the_transposing_kernel(dev, max_r, ranks, sizes, offset):
+    """The backward of packed experts, whose GEMM takes the LoRA part of dx along: dx and the adapters' gradients against
+    float64, with matrices that are not 16-byte aligned, and isolation: one tenant's A holds infinities, NaN and the largest
+    values, which may reach its own rows and gradients only."""
+    e, nt, k, n = 2, len(ranks), 256, 128
+    expert = torch.arange(e).repeat_interleave(nt * sizes)
+    tenant = torch.arange(nt).repeat_interleave(sizes).repeat(e)
+    t = expert.numel()
+    g = torch.Generator().manual_seed(max_r + offset + 50)
+    x = torch.randn(t, k, generator=g).bfloat16()
+    dy = torch.randn(t, n, generator=g).bfloat16()
+    w = (torch.randn(e, n, k, generator=g) / k**0.5).bfloat16()
+    bad = nt - 1
+
+    def shifted(*shape, std):
+        flat = torch.empty(offset + shape[0] * shape[1] * shape[2], dtype=torch.bfloat16, device=dev)
+        return flat[offset:].view(shape).copy_((torch.randn(*shape, generator=g) * std).bfloat16())
+
+    a = [shifted(e, max_r, k, std=k**-0.5) for _ in range(nt)]
+    b = [shifted(e, n, max_r, std=0.05) for _ in range(nt)]
+    a[bad].view(-1)[::3] = float('inf')
+    a[bad].view(-1)[1::3] = float('nan')
+    a[bad].view(-1)[2::3] = torch.finfo(torch.bfloat16).max
+    for va, vb, r in zip(a, b, ranks):    # rank indices past a tenant's rank are nobody's: they may hold anything
+        va[:, r:] = float('nan')
+        vb[..., r:] = float('nan')
+    idx = [i % nt for i in range(e * nt)]
+    params = [v.requires_grad_(True) for v in (*a, *b)]
+    groups = AdapterGroups(a, b, [ranks[i % nt] for i in range(e * nt)], [2.0] * (e * nt), a_index=idx,
+                           a_offset=[(i // nt) * max_r * k for i in range(e * nt)], b_index=idx,
+                           b_offset=[(i // nt) * n * max_r for i in range(e * nt)], rank_classes=False)
+    seg = build_segments((expert * nt + tenant).to(torch.int32).to(dev), e * nt)
+    xd = x.to(dev).requires_grad_(True)
+    y = grouped_experts_linear(xd, w.to(dev), seg, nt, groups)
+    dx, *grads = torch.autograd.grad(y, [xd, *params], dy.to(dev), allow_unused=True)
+    dx, want = dx.cpu(), _reference(dy, w.transpose(1, 2).contiguous(), expert)
+    own = tenant == bad
+    if ranks[bad] > 0:
+        assert not torch.isfinite(dx[own]).all()
+    for ti, r in enumerate(ranks):
+        if ti == bad or r == 0:
+            continue
+        want_a, want_b = torch.zeros(e, r, k, dtype=torch.double), torch.zeros(e, n, r, dtype=torch.double)
+        for ei in range(e):
+            rows = ((expert == ei) & (tenant == ti)).nonzero().flatten()
+            ae, be = a[ti][ei, :r].detach().double().cpu(), b[ti][ei, :, :r].detach().double().cpu()
+            dh, xs = 2.0 * dy[rows].double() @ be, x[rows].double()
+            want[rows] += dh @ ae
+            want_a[ei], want_b[ei] = dh.t() @ xs, 2.0 * dy[rows].double().t() @ (xs @ ae.t())
+        # h or dh, then the gradient itself, are rounded to eight bits once each
+        assert max_rel_err(grads[ti][:, :r].cpu(), want_a) < 1e-2
+        assert max_rel_err(grads[nt + ti][..., :r].cpu(), want_b) < 1e-2
+    assert max_rel_err(dx[~own], want[~own]) < 1e-2
 
 
 @pytest.mark.parametrize('n,ptiles', [(128, 4), (256, 8)])   # tiles of a row block: by the width of the kernel's block
