@@ -829,9 +829,9 @@ int64_t grouped_plan_entries(const SegLayout& L, int64_t experts) { return ceil_
 int launch_grouped_gemm(const GroupedArgs& a, int experts, int nt, GroupedPlanEntry* plan, int32_t* nblocks,
                         const SegView& seg, const SegLayout& L, hipStream_t s) {
   if (L.rows == 0) return TK_OK;
-  // The 8-wave variants win wherever they apply.  The forward form loads its tiles straight into LDS
-  // (k_grouped_gemm_dl: 32-bit row offsets, so x and one expert's weights must span less than 4 GB); the older
-  // 8-wave kernel serves the transposing form and the rest, except with the LoRA term on small experts (its epilogue
+  // The 8-wave variants win wherever they apply.  Both weight layouts load their tiles straight into LDS
+  // (k_grouped_gemm_dl: 32-bit row offsets, so x and one expert's weights must span less than 4 GB); what that kernel does
+  // not take runs on the 8 waves of k_grouped_gemm, except with the LoRA term on small experts (its epilogue
   // has no registers to spare: measured at 512 rows per expert, 4 waves are then 5 % faster).
   const int nks = a.rpad == 0 ? 0 : (a.rpad <= 32 ? 1 : 2);
   const bool direct = grouped_gemm_direct(a);

@@ -223,9 +223,11 @@ static inline int shrink_kslices(int width, int rpad) {
 }
 // Above rank 16, with long groups and a source of 1024 to 4096 columns, the shrink runs as k_shrink_dl, and where that does not
 // apply (sources of 4 GB, several projections of one input, set_narrow) as k_shrink_oct or k_shrink_quad:
-// blocks of (eight tiles, `steps` steps of 64 columns), at most 512 of them (twice as many slices: 98 us against 77 for
-// 32768 x 4096 at rank 64, their sums are written and read; half as many: 81).  Wider sources stay with k_shrink_pair (24
-// adapters of rank 8 to 64, 32768 x 4096 -> 14336: the training step takes 1037 us, with the wide dy on k_shrink_oct 1054).
+// blocks of (eight tiles, `steps` steps of 64 columns), at most 512 of them.  The figures behind this plan are those of
+// k_shrink_oct and k_shrink_quad, for which it was made; k_shrink_dl takes it over and was not measured with another one.
+// Twice as many slices: 98 us against 77 for 32768 x 4096 at rank 64 (their sums are written and read), half as many: 81.
+// Wider sources stay with k_shrink_pair (24 adapters of rank 8 to 64, 32768 x 4096 -> 14336: the training step takes 1037
+// us, with the wide dy on k_shrink_oct 1054).
 constexpr int kSetBlocks = 512;
 // A CU holds one block of k_shrink_oct or two of k_shrink_quad (registers).  The eight waves read 256 contiguous bytes of a
 // row per step and are faster while every block has a CU of its own; past that they run in rounds.  Shrink with its slice

@@ -164,7 +164,7 @@ class AdapterGroups:
 
     def host_groups(self):
         """This object as the C++ nodes know it; ``None`` with master weights or adapters of a tensor subclass, which only the
-        Python nodes serve."""
+        Python nodes serve.  Laid out at an object's first call, so an object of few calls sees less of what those nodes save."""
         if self.master_a is not None:
             return None
         if self._host is None:
